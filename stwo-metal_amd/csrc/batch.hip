@@ -23,6 +23,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "fft_matrix.hpp"
 #include "field.hpp"
 #include "internal.hpp"
 
@@ -57,6 +58,10 @@ struct LevelLaunch {
   int kind;  // launch_fft_multi's (or launch_lde_multi's) schedule kind for every group of the launch
   size_t groups_off, fwd_off, wgs_off;  // offsets into the device buffer
   uint32_t n_groups, total_wgs, wg_log;
+  // matrix passes (groups_off: MxTop or MxLow descriptors): layers of a top
+  // pass with its directions, or the low pass (mx_layers = 0)
+  bool matrix = false, mx_inv = false, mx_fwd = false;
+  uint32_t mx_layers = 0;
 };
 
 // One tree's Merkle launches: its layer tables and shape.
@@ -189,7 +194,7 @@ int batch_create_trees(stwo_hip_ctx *ctx, const BatchTree *trees, size_t n_trees
   // 4 passes), plus the 256-byte alignment of two or three tables per launch
   // (2 directions x 4 levels x 2 workgroup sizes x at most 14 schedule kinds,
   // and the fused launches).
-  size_t desc_bytes = 2 * 4 * gt.size() * (sizeof(FftPass2) + 8) + 2 * 4 * 2 * 14 * 2 * 256 + 8192;
+  size_t desc_bytes = gt.size() * (sizeof(MxTop) + 2 * sizeof(MxLow)) + 8 * 256 + 2 * 4 * gt.size() * (sizeof(FftPass2) + 8) + 2 * 4 * 2 * 14 * 2 * 256 + 8192;
   int arc = device_alloc(ctx, tables_bytes + desc_bytes, &dmem, &from_job);
   if (arc) return arc;
   auto release = [&]() { device_free(dmem, from_job); };
@@ -199,6 +204,8 @@ int batch_create_trees(stwo_hip_ctx *ctx, const BatchTree *trees, size_t n_trees
   struct GroupPasses {
     std::vector<PassLaunch> inv, fwd;
     bool fused = false;
+    bool matrix = false;  // first and last passes on the matrix cores
+    MxPlan mx;
   };
   std::vector<GroupPasses> gp(gt.size());
   for (size_t gi = 0; gi < gt.size(); gi++) {
@@ -215,6 +222,32 @@ int batch_create_trees(stwo_hip_ctx *ctx, const BatchTree *trees, size_t n_trees
         release();
         return rc;
       }
+    }
+    GroupPasses &G = gp[gi];
+    const bool has_inv = t.stage != BATCH_RFFT, has_fwd = t.stage != BATCH_IFFT;
+    if ((!has_inv || mx_plan(ctx, tw, t.n, 0, true, t.count, t.aligned16, true, &G.mx)) &&
+        (!has_fwd || mx_plan(ctx, tw, t.n, t.b, false, t.count, t.aligned16, true, &G.mx))) {
+      G.matrix = true;
+      // what is left to the vector passes: the default plan's middle pass
+      const FftTune def;
+      for (int dir = 0; dir < 2; dir++) {
+        std::vector<PassLaunch> &v = dir ? G.fwd : G.inv;
+        if (v.empty()) continue;
+        if (!G.mx.mid) {
+          v.clear();
+          continue;
+        }
+        const FftCol *in_place = (const FftCol *)(dbase + (dir ? t.inplace_off : t.ifft_off));
+        int rc = make_group_passes(ctx, t.n, t.n + (dir ? t.b : 0), !dir, in_place, in_place, t.count,
+                                   dir ? tw_end : itw_end, true, v, &def);
+        if (!rc && v.size() != 3) rc = set_error(ctx, STWO_HIP_EINVAL, "internal: %zu passes of 2^%u", v.size(), t.n);
+        if (rc) {
+          release();
+          return rc;
+        }
+        v = {v[1]};
+      }
+      continue;
     }
     gp[gi].fused = t.stage == BATCH_LDE && lde_fusable(gp[gi].inv.back(), gp[gi].fwd.front(), t.b);
   }
@@ -252,8 +285,84 @@ int batch_create_trees(stwo_hip_ctx *ctx, const BatchTree *trees, size_t n_trees
     }
     return STWO_HIP_OK;
   };
+  // The matrix passes of every group that takes them.  The low pass is the
+  // first of the inverse levels and the last of the forward ones; the top pass
+  // runs after the inverse levels, fused with the forward one where the set
+  // has both.
+  auto add_mx_low = [&](bool inverse) -> int {
+    uint64_t units = 0, acc = 0;
+    auto takes = [&](size_t gi) { return gp[gi].matrix && gt[gi].stage != (inverse ? BATCH_RFFT : BATCH_IFFT); };
+    for (size_t gi = 0; gi < gt.size(); gi++)
+      if (takes(gi)) units += mx_low_units(gt[gi].count, gt[gi].n + (inverse ? 0 : gt[gi].b));
+    std::vector<MxLow> descs;
+    for (size_t gi = 0; gi < gt.size(); gi++) {
+      if (!takes(gi)) continue;
+      const GroupTabs &t = gt[gi];
+      const size_t tab = inverse ? t.ifft_off : gp[gi].mx.top_layers ? t.inplace_off : t.rfft_off;
+      uint32_t wgs = 0;
+      descs.push_back(mx_low(tw, (const FftCol *)(dbase + tab), t.count, t.n, t.n + (inverse ? 0 : t.b), inverse,
+                             gp[gi].mx, units, true, &wgs));
+      descs.back().wg_start = wgs;
+    }
+    if (descs.empty()) return STWO_HIP_OK;
+    // the longest workgroups start first
+    std::stable_sort(descs.begin(), descs.end(), [](const MxLow &a, const MxLow &c) { return a.iters > c.iters; });
+    for (MxLow &d : descs) {
+      const uint32_t wgs = d.wg_start;
+      d.wg_start = (uint32_t)acc;
+      acc += wgs;
+    }
+    if (acc >= (1ull << 31)) return set_error(ctx, STWO_HIP_EINVAL, "batch_create: grid too large");
+    LevelLaunch ll{};
+    ll.inverse = inverse;
+    ll.matrix = true;
+    ll.groups_off = st.put(descs.data(), descs.size() * sizeof(MxLow));
+    ll.n_groups = (uint32_t)descs.size();
+    ll.total_wgs = (uint32_t)acc;
+    levels.push_back(ll);
+    return STWO_HIP_OK;
+  };
+  auto add_mx_tops = [&](int stage) -> int {
+    for (uint32_t layers : {8u, 4u}) {
+      uint64_t units = 0, acc = 0;
+      auto takes = [&](size_t gi) {
+        return gp[gi].matrix && gt[gi].stage == stage && gp[gi].mx.top_layers == layers;
+      };
+      for (size_t gi = 0; gi < gt.size(); gi++)
+        if (takes(gi)) units += mx_top_units(gt[gi].count, gt[gi].n, gp[gi].mx);
+      std::vector<MxTop> descs;
+      for (size_t gi = 0; gi < gt.size(); gi++) {
+        if (!takes(gi)) continue;
+        const GroupTabs &t = gt[gi];
+        uint32_t wgs = 0;
+        descs.push_back(mx_top(tw, (const FftCol *)(dbase + t.ifft_off), (const FftCol *)(dbase + t.rfft_off), t.count,
+                               t.n, t.b, stage == BATCH_IFFT || !(flags & STWO_HIP_BATCH_DROP_COEFFS), gp[gi].mx, units,
+                               true, &wgs));
+        descs.back().wg_start = (uint32_t)acc;
+        acc += wgs;
+      }
+      if (descs.empty()) continue;
+      if (acc >= (1ull << 31)) return set_error(ctx, STWO_HIP_EINVAL, "batch_create: grid too large");
+      LevelLaunch ll{};
+      ll.matrix = true;
+      ll.mx_layers = layers;
+      ll.mx_inv = stage != BATCH_RFFT;
+      ll.mx_fwd = stage != BATCH_IFFT;
+      ll.groups_off = st.put(descs.data(), descs.size() * sizeof(MxTop));
+      ll.n_groups = (uint32_t)descs.size();
+      ll.total_wgs = (uint32_t)acc;
+      levels.push_back(ll);
+    }
+    return STWO_HIP_OK;
+  };
   for (int dir = 0; dir < 2; dir++) {
     const bool inverse = dir == 0;
+    int mrc = inverse ? add_mx_low(true) : add_mx_tops(BATCH_LDE);
+    if (!mrc && !inverse) mrc = add_mx_tops(BATCH_RFFT);
+    if (mrc) {
+      release();
+      return mrc;
+    }
     // (level, workgroup size) -> passes of every group (the fused ones aside)
     std::map<std::pair<uint32_t, uint32_t>, std::vector<PassLaunch>> by_level;
     for (const GroupPasses &g : gp) {
@@ -261,6 +370,7 @@ int batch_create_trees(stwo_hip_ctx *ctx, const BatchTree *trees, size_t n_trees
       const size_t k0 = (!inverse && g.fused) ? 1 : 0, k1 = passes.size() - ((inverse && g.fused) ? 1 : 0);
       for (size_t k = k0; k < k1; k++) {
         uint32_t level = inverse ? (uint32_t)k : (uint32_t)(passes.size() - 1 - k);
+        if (g.matrix) level = 1;  // the middle one of three
         by_level[{level, passes[k].wg_log}].push_back(passes[k]);
       }
     }
@@ -307,6 +417,11 @@ int batch_create_trees(stwo_hip_ctx *ctx, const BatchTree *trees, size_t n_trees
         return rc;
       }
     }
+    mrc = inverse ? add_mx_tops(BATCH_IFFT) : add_mx_low(false);
+    if (mrc) {
+      release();
+      return mrc;
+    }
   }
   if (st.host.size() > tables_bytes + desc_bytes) {
     release();
@@ -334,6 +449,15 @@ int batch_create_trees(stwo_hip_ctx *ctx, const BatchTree *trees, size_t n_trees
   const uint32_t keep_coeffs = (flags & STWO_HIP_BATCH_DROP_COEFFS) ? 0u : 1u;
   b->issue = [levels, tl, dbase, keep_coeffs](stwo_hip_ctx *c) -> int {
     for (const LevelLaunch &ll : levels) {
+      if (ll.matrix) {
+        int rc = ll.mx_layers
+                     ? launch_mx_top(c, nullptr, (const MxTop *)(dbase + ll.groups_off), ll.n_groups, ll.total_wgs,
+                                     ll.mx_layers, ll.mx_inv, ll.mx_fwd)
+                     : launch_mx_low(c, nullptr, (const MxLow *)(dbase + ll.groups_off), ll.n_groups, ll.total_wgs,
+                                     ll.inverse);
+        if (rc) return rc;
+        continue;
+      }
       int rc = ll.fused ? launch_lde_multi(c, (const FftPass2 *)(dbase + ll.groups_off),
                                            (const FftPass2 *)(dbase + ll.fwd_off),
                                            (const uint32_t *)(dbase + ll.wgs_off), ll.n_groups, ll.total_wgs,

@@ -22,6 +22,7 @@ struct stwo_hip_twiddles {
   uint32_t *d_itw;     // elementwise inverses
   uint32_t *d_tw2;     // both trees doubled (2 * t < 2^32), the radix-16 FFT's operands
   uint32_t *d_itw2;
+  uint32_t *d_mx = nullptr;  // matrix table of the matrix FFT passes (NULL below their sizes)
 };
 
 namespace stwo_hip {
@@ -33,7 +34,7 @@ struct FftTune {
   uint8_t t0 = 12;   // tile log of the contiguous low pass (10..13)
   uint8_t smax = 8;  // most layers per strided pass (5..8)
   uint8_t wg = 0;    // workgroup log: 0 = max(8, T - 4); 9 = 512 lanes for every tile size
-  uint8_t pad = 0;
+  uint8_t chosen = 0;  // set for the shape (by a caller or as the tuner's fastest): the vector plan is taken as given
 };
 inline uint64_t fft_tune_key(uint32_t n, uint32_t N, bool inverse) {
   return ((uint64_t)n << 16) | ((uint64_t)N << 1) | (inverse ? 1u : 0u);

@@ -30,6 +30,8 @@
 #include <vector>
 
 #include "common.hpp"
+#include "fft_dev.hpp"
+#include "fft_matrix.hpp"
 #include "field.hpp"
 #include "internal.hpp"
 
@@ -269,98 +271,6 @@ __global__ void __launch_bounds__(kBrThreads) bit_reverse_tiled_kernel(uint32_t 
 // consecutive words of tree level s per layer -- 15 words per lane per
 // stage, loaded once.  The circle layer (s = 0) reads 4 words (two (x, y)
 // pairs of line layer 0) for its 8 pairs.
-
-// `t2` is the twiddle doubled (the passes read the doubled trees).
-template <bool INV>
-__device__ __forceinline__ void bfly(uint32_t &a, uint32_t &b, uint32_t t2) {
-  if (INV) {
-    uint32_t s = m31_add(a, b);
-    b = m31_mul_dbl(m31_sub(a, b), t2);
-    a = s;
-  } else {
-    uint32_t tmp = m31_mul_dbl(b, t2);
-    b = m31_sub(a, tmp);
-    a = m31_add(a, tmp);
-  }
-}
-
-// Twiddles of one stage: for register bit r, 8 >> r consecutive words of
-// tree level s = sh + r starting at gb >> (s + 1); the circle layer (s = 0)
-// is expanded from two (x, y) pairs of line layer 0 into [y, -y, -x, x].
-struct StageTw {
-  uint32_t t0[8], t1[4], t2[2], t3[1];
-};
-
-// Word `byte_off / 4` of a table whose base is wave-uniform: the base stays
-// in SGPRs and the lane part is a 32-bit offset (global_load ... saddr).
-__device__ __forceinline__ uint32_t gld(const uint32_t *base, uint32_t byte_off) {
-  return *(gconst_u32 *)((gconst_u8 *)as_global(base) + byte_off);
-}
-__device__ __forceinline__ void gst(uint32_t *base, uint32_t byte_off, uint32_t v) {
-  *(g_u32 *)((g_u8 *)as_global(base) + byte_off) = v;
-}
-__device__ __forceinline__ u32x4 gld4(const uint32_t *base, uint32_t byte_off) {
-  return *(gconst_u4 *)((gconst_u8 *)as_global(base) + byte_off);
-}
-__device__ __forceinline__ void gst4(uint32_t *base, uint32_t byte_off, u32x4 v) {
-  *(g_u4 *)((g_u8 *)as_global(base) + byte_off) = v;
-}
-
-__device__ __forceinline__ void load_level(uint32_t *dst, int cnt, const uint32_t *tw_end, uint32_t N, uint32_t s,
-                                           uint32_t gb) {
-  const uint32_t hs = gb >> (s + 1);
-  if (s == 0) {
-    const uint32_t *l0 = tw_end - ((size_t)1 << (N - 1));
-    const uint32_t o = (hs >> 1) << 2;
-    uint32_t w4[4];
-#pragma unroll
-    for (int k = 0; k < 4; k++) w4[k] = gld(l0, o + 4 * k);
-#pragma unroll
-    for (int u = 0; u < 8; u++) {
-      uint32_t xx = w4[2 * (u >> 2)], yy = w4[2 * (u >> 2) + 1];
-      uint32_t v = (u & 2) ? xx : yy;
-      // doubled negation: 2 (P - v / 2) = 2P - v < 2^32 (for v = 0 it is 2P, still 0 mod P)
-      dst[u] = ((u & 3) == 1 || (u & 3) == 2) ? 2u * P - v : v;
-    }
-    return;
-  }
-  const uint32_t *lv = tw_end - ((size_t)1 << (N - s));
-  const uint32_t o = hs << 2;
-#pragma unroll
-  for (int u = 0; u < 8; u++)
-    if (u < cnt) dst[u] = gld(lv, o + 4 * u);
-}
-
-// Loads only the levels of the stage's active register bits [r_lo, r_hi).
-__device__ __forceinline__ void load_stage_twiddles(StageTw &t, const uint32_t *tw_end, uint32_t N, uint32_t sh,
-                                                    uint32_t gb, uint32_t r_lo, uint32_t r_hi) {
-  if (r_lo <= 0 && 0 < r_hi) load_level(t.t0, 8, tw_end, N, sh + 0, gb);
-  if (r_lo <= 1 && 1 < r_hi) load_level(t.t1, 4, tw_end, N, sh + 1, gb);
-  if (r_lo <= 2 && 2 < r_hi) load_level(t.t2, 2, tw_end, N, sh + 2, gb);
-  if (r_lo <= 3 && 3 < r_hi) load_level(t.t3, 1, tw_end, N, sh + 3, gb);
-}
-
-template <int R>
-__device__ __forceinline__ uint32_t stage_tw(const StageTw &t, int u) {
-  return R == 0 ? t.t0[u] : R == 1 ? t.t1[u] : R == 2 ? t.t2[u] : t.t3[u];
-}
-
-// Layers at register bits [RLO, RHI) of the group (forward: high to low).
-template <bool INV, int RLO, int RHI>
-__device__ __forceinline__ void stage_layers(uint32_t (&x)[16], const StageTw &t) {
-#pragma unroll
-  for (int rr = 0; rr < RHI - RLO; rr++) {
-    const int r = INV ? RLO + rr : RHI - 1 - rr;
-#pragma unroll
-    for (int j0 = 0; j0 < 16; j0++)
-      if (!((j0 >> r) & 1)) {
-        const int u = j0 >> (r + 1);
-        const uint32_t tw = r == 0 ? stage_tw<0>(t, u) : r == 1 ? stage_tw<1>(t, u) : r == 2 ? stage_tw<2>(t, u)
-                                                                                           : stage_tw<3>(t, u);
-        bfly<INV>(x[j0], x[j0 | (1 << r)], tw);
-      }
-  }
-}
 
 template <bool INV>
 __device__ __forceinline__ void stage_dispatch(uint32_t (&x)[16], const StageTw &t, uint32_t r_lo, uint32_t r_hi) {
@@ -1159,12 +1069,54 @@ int launch_fft_multi(stwo_hip_ctx *ctx, bool inverse, const FftPass2 *d_groups, 
 #undef STWO_MULTI
 }
 
+// The vector pass between the matrix passes of a column of more than 2^20
+// coefficients: the middle one of the default plan's three (top 8 layers,
+// n - 20, low 12).
+static int launch_mx_mid(stwo_hip_ctx *ctx, const FftCol *d_tab, uint32_t n_cols, uint32_t n, uint32_t N,
+                         const stwo_hip_twiddles *tw, bool inverse) {
+  const FftTune def;
+  std::vector<PassLaunch> ps;
+  int rc = make_group_passes(ctx, n, N, inverse, d_tab, d_tab, n_cols, (inverse ? tw->d_itw2 : tw->d_tw2) + tw->len,
+                             true, ps, &def);
+  if (rc) return rc;
+  STWO_HIP_CHECK_ARG(ctx, ps.size() == 3, "internal: %zu passes of 2^%u", ps.size(), n);
+  return launch_fft_pass(ctx, inverse, ps[1].p, ps[1].wgs, ps[1].wg_log);
+}
+
+// A group on the matrix passes.  d_tab: {in, out} of the first pass, d_inpl:
+// {out, out}.
+static int run_mx_group(stwo_hip_ctx *ctx, const FftCol *d_tab, const FftCol *d_inpl, uint32_t n_cols, uint32_t n,
+                        uint32_t N, const stwo_hip_twiddles *tw, bool inverse, const MxPlan &mx) {
+  uint32_t wl = 0, wt = 0;
+  const MxLow low = mx_low(tw, mx.top_layers && !inverse ? d_inpl : d_tab, n_cols, n, N, inverse, mx, mx_low_units(n_cols, N), false, &wl);
+  if (inverse) {
+    int rc = launch_mx_low(ctx, &low, nullptr, 0, wl, true);
+    if (rc || !mx.top_layers) return rc;
+    if (mx.mid && (rc = launch_mx_mid(ctx, d_tab, n_cols, n, N, tw, true))) return rc;
+    const MxTop top = mx_top(tw, d_tab, nullptr, n_cols, n, 0, true, mx, mx_top_units(n_cols, n, mx), false, &wt);
+    return launch_mx_top(ctx, &top, nullptr, 0, wt, mx.top_layers, true, false);
+  }
+  if (mx.top_layers) {
+    const MxTop top =
+        mx_top(tw, nullptr, d_tab, n_cols, n, N - n, false, mx, mx_top_units(n_cols, n, mx), false, &wt);
+    int rc = launch_mx_top(ctx, &top, nullptr, 0, wt, mx.top_layers, false, true);
+    if (rc) return rc;
+    if (mx.mid && (rc = launch_mx_mid(ctx, d_inpl, n_cols, n, N, tw, false))) return rc;
+  }
+  return launch_mx_low(ctx, &low, nullptr, 0, wl, false);
+}
+
 // Radix-16 path for N >= 4: one launch per pass over all columns of the group.
 static int run_fft_group2(stwo_hip_ctx *ctx, const std::vector<FftCol> &cols, void *dtab, void *dtab_out,
-                          uint32_t n, uint32_t N, const uint32_t *tw_end, bool inverse) {
+                          uint32_t n, uint32_t N, const stwo_hip_twiddles *tw, bool inverse) {
   bool aligned16 = true;
   for (const FftCol &c : cols)
     if ((((uintptr_t)c.in) | ((uintptr_t)c.out)) & 15) aligned16 = false;
+  const uint32_t *tw_end = (inverse ? tw->d_itw2 : tw->d_tw2) + tw->len;
+  MxPlan mx;
+  if (mx_plan(ctx, tw, n, N - n, inverse, cols.size(), aligned16, false, &mx))
+    return run_mx_group(ctx, (const FftCol *)dtab, (const FftCol *)dtab_out, (uint32_t)cols.size(), n, N, tw, inverse,
+                        mx);
   std::vector<PassLaunch> passes;
   int rc = make_group_passes(ctx, n, N, inverse, (const FftCol *)dtab, (const FftCol *)dtab_out,
                              (uint32_t)cols.size(), tw_end, aligned16, passes);
@@ -1196,6 +1148,25 @@ static int run_lde_group(stwo_hip_ctx *ctx, const std::vector<FftCol> &cols, con
     const size_t bytes[3] = {cols.size() * sizeof(FftCol), tf.size() * sizeof(FftCol), to.size() * sizeof(FftCol)};
     int rc = upload_tables(ctx, 3, srcs, bytes, d);
     if (rc) return rc;
+  }
+  MxPlan mx;
+  if (mx_plan(ctx, tw, n, 0, true, cols.size(), aligned16, false, &mx) &&
+      mx_plan(ctx, tw, n, b, false, cols.size(), aligned16, false, &mx)) {
+    const FftCol *ti = (const FftCol *)d[0], *tfw = (const FftCol *)d[1], *tio = (const FftCol *)d[2];
+    const uint32_t nc = (uint32_t)cols.size();
+    if (!mx.top_layers) {
+      int rc = run_mx_group(ctx, ti, ti, nc, n, n, tw, true, mx);
+      return rc ? rc : run_mx_group(ctx, tfw, tio, nc, n, N, tw, false, mx);
+    }
+    uint32_t w0 = 0, w1 = 0, w2 = 0;
+    const MxLow li = mx_low(tw, ti, nc, n, n, true, mx, mx_low_units(nc, n), false, &w0);
+    const MxLow lf = mx_low(tw, tio, nc, n, N, false, mx, mx_low_units(nc, N), false, &w2);
+    const MxTop top = mx_top(tw, ti, tfw, nc, n, b, store_coeffs, mx, mx_top_units(nc, n, mx), false, &w1);
+    int rc = launch_mx_low(ctx, &li, nullptr, 0, w0, true);
+    if (!rc && mx.mid) rc = launch_mx_mid(ctx, ti, nc, n, n, tw, true);
+    if (!rc) rc = launch_mx_top(ctx, &top, nullptr, 0, w1, mx.top_layers, true, true);
+    if (!rc && mx.mid) rc = launch_mx_mid(ctx, tio, nc, n, N, tw, false);
+    return rc ? rc : launch_mx_low(ctx, &lf, nullptr, 0, w2, false);
   }
   std::vector<PassLaunch> inv, fwd;
   int rc = make_group_passes(ctx, n, n, true, (const FftCol *)d[0], (const FftCol *)d[0], (uint32_t)cols.size(),
@@ -1268,7 +1239,7 @@ static int run_fft_group(stwo_hip_ctx *ctx, const std::vector<FftCol> &cols, uin
     return launch(ctx, "fft_small", fft_small_kernel, dim3((uint32_t)cols.size()), dim3(64), 0, a);
   }
   if (N >= 4)
-    return run_fft_group2(ctx, cols, dtab, dtab_out, n, N, (inverse ? tw->d_itw2 : tw->d_tw2) + tw->len, inverse);
+    return run_fft_group2(ctx, cols, dtab, dtab_out, n, N, tw, inverse);
   const uint32_t *tree = inverse ? tw->d_itw : tw->d_tw;
   const uint32_t *tw_end = tree + tw->len;
   uint32_t L = inverse ? N : n;
@@ -1481,7 +1452,8 @@ PlanKey plan_key(const std::vector<PassLaunch> &ps) {
   return k;
 }
 
-int time_passes(stwo_hip_ctx *ctx, bool inverse, const std::vector<PassLaunch> &ps, float *best_ms) {
+template <typename Fn>
+int time_launches(stwo_hip_ctx *ctx, Fn issue, float *best_ms) {
   hipEvent_t e0 = take_event(ctx), e1 = take_event(ctx);
   if (!e0 || !e1) return set_error(ctx, STWO_HIP_EDEVICE, "autotune: no events");
   int rc = STWO_HIP_OK;
@@ -1490,8 +1462,7 @@ int time_passes(stwo_hip_ctx *ctx, bool inverse, const std::vector<PassLaunch> &
   ctx->prof = false;
   for (int it = 0; it < 4 && rc == STWO_HIP_OK; it++) {
     if (hipEventRecord(e0, ctx->stream) != hipSuccess) rc = STWO_HIP_EDEVICE;
-    for (const PassLaunch &pl : ps)
-      if (rc == STWO_HIP_OK) rc = launch_fft_pass(ctx, inverse, pl.p, pl.wgs, pl.wg_log);
+    if (rc == STWO_HIP_OK) rc = issue();
     if (rc == STWO_HIP_OK && hipEventRecord(e1, ctx->stream) != hipSuccess) rc = STWO_HIP_EDEVICE;
     if (rc == STWO_HIP_OK && hipEventSynchronize(e1) != hipSuccess) rc = STWO_HIP_EDEVICE;
     float ms = 0;
@@ -1572,17 +1543,35 @@ int stwo_hip_fft_autotune(stwo_hip_ctx *ctx, const uint32_t *log_sizes, size_t n
           }
       float best = 1e30f, def_ms = 0;
       FftTune best_t = def;
+      // Without a choice the shape may take the matrix passes: then those are
+      // the default that a vector plan has to beat.
+      MxPlan mx;
+      ctx->fft_tune.erase(fft_tune_key(n, Nd, inverse));
+      const bool matrix = mx_plan(ctx, tw, n, Nd - n, inverse, c, true, false, &mx);
       for (auto &ck : cands) {
         rc = make_group_passes(ctx, n, Nd, inverse, first, inpl, (uint32_t)c, tw_end, true, ps, &ck.second);
         if (rc) return rc;
         float ms = 0;
-        rc = time_passes(ctx, inverse, ps, &ms);
+        rc = time_launches(
+            ctx,
+            [&]() {
+              int r = STWO_HIP_OK;
+              for (const PassLaunch &pl : ps)
+                if (!r) r = launch_fft_pass(ctx, inverse, pl.p, pl.wgs, pl.wg_log);
+              return r;
+            },
+            &ms);
         if (rc) return rc;
-        if (!(ck.first < def_key) && !(def_key < ck.first)) def_ms = ms;
+        if (!matrix && !(ck.first < def_key) && !(def_key < ck.first)) def_ms = ms;
         if (ms < best) {
           best = ms;
           best_t = ck.second;
         }
+      }
+      if (matrix) {
+        rc = time_launches(
+            ctx, [&]() { return run_mx_group(ctx, first, inpl, (uint32_t)c, n, Nd, tw, inverse, mx); }, &def_ms);
+        if (rc) return rc;
       }
       // Another plan must beat the default by kTuneMargin: timed alone a shape
       // gains a few percent from a run-time schedule, but inside a batched plan
@@ -1592,6 +1581,8 @@ int stwo_hip_fft_autotune(stwo_hip_ctx *ctx, const uint32_t *log_sizes, size_t n
       if (def_ms > 0 && best > def_ms * (1.0f - kTuneMargin)) {
         best = def_ms;
         best_t = def;
+      } else {
+        best_t.chosen = 1;
       }
       ctx->fft_tune[fft_tune_key(n, Nd, inverse)] = best_t;
       if (report && nr < max_report) {
@@ -1619,6 +1610,7 @@ int stwo_hip_fft_tune_set(stwo_hip_ctx *ctx, const uint32_t *entries, size_t n_e
     t.t0 = (uint8_t)e[3];
     t.smax = (uint8_t)e[4];
     t.wg = (uint8_t)e[5];
+    t.chosen = 1;
     ctx->fft_tune[fft_tune_key(e[0], e[1], e[2] != 0)] = t;
   }
   return STWO_HIP_OK;

@@ -13,6 +13,7 @@
 // index and sums the set bits' powers of the generator from a 31-entry
 // constant table.
 #include "common.hpp"
+#include "fft_matrix.hpp"
 #include "field.hpp"
 
 namespace stwo_hip {
@@ -84,8 +85,9 @@ int stwo_hip_twiddles_create(stwo_hip_ctx *ctx, stwo_hip_coset root, stwo_hip_tw
   tw->device = ctx->device;
   tw->root = {root.initial_index & IDX_MASK, root.log_size};
   tw->len = (size_t)1 << root.log_size;
-  // One allocation: tree | inverse tree | both doubled.
-  if (ctx_malloc(ctx, (void **)&tw->d_tw, tw->len * 16) != hipSuccess) {
+  // One allocation: tree | inverse tree | both doubled | matrix table.
+  const size_t mx_bytes = mx_table_bytes(root.log_size);
+  if (ctx_malloc(ctx, (void **)&tw->d_tw, tw->len * 16 + mx_bytes) != hipSuccess) {
     (void)hipGetLastError();  // clear the sticky error of the failed allocation
     delete tw;
     return set_error(ctx, STWO_HIP_ENOMEM, "twiddle tree of %zu entries: out of device memory", (size_t)1 << root.log_size);
@@ -95,6 +97,10 @@ int stwo_hip_twiddles_create(stwo_hip_ctx *ctx, stwo_hip_coset root, stwo_hip_tw
   tw->d_itw2 = tw->d_tw + 3 * tw->len;
   rc = launch(ctx, "twiddle_tree", twiddle_tree_kernel, dim3((uint32_t)((tw->len + 255) / 256)), dim3(256), 0,
               tw->d_tw, tw->d_itw, tw->d_tw2, tw->d_itw2, tw->root.initial_index, root.log_size);
+  if (rc == STWO_HIP_OK && mx_bytes) {
+    tw->d_mx = tw->d_tw + 4 * tw->len;
+    rc = mx_table_build(ctx, tw->d_tw + tw->len, tw->d_itw + tw->len, tw->d_mx);
+  }
   if (rc == STWO_HIP_OK && hipStreamSynchronize(ctx->stream) != hipSuccess)
     rc = set_error(ctx, STWO_HIP_EDEVICE, "twiddle tree build failed");
   if (rc) {
