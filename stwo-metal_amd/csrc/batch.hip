@@ -187,6 +187,10 @@ int batch_create_trees(stwo_hip_ctx *ctx, const BatchTree *trees, size_t n_trees
   }
   // Reserve the pass descriptor area after the tables: the descriptors hold
   // device addresses of the tables, known once the buffer exists.
+  // The plan's own counters: it may run on another context's stream than the
+  // one that made it.
+  const std::vector<uint32_t> zeros(tree_counters(all_max), 0);
+  const size_t counters_off = st.put(zeros.data(), zeros.size() * sizeof(uint32_t));
   size_t tables_bytes = (st.host.size() + 255) & ~(size_t)255;
   void *dmem = nullptr;
   bool from_job = false;
@@ -447,7 +451,8 @@ int batch_create_trees(stwo_hip_ctx *ctx, const BatchTree *trees, size_t n_trees
   b->d_mem = dmem;
   b->mem_from_job = from_job;
   const uint32_t keep_coeffs = (flags & STWO_HIP_BATCH_DROP_COEFFS) ? 0u : 1u;
-  b->issue = [levels, tl, dbase, keep_coeffs](stwo_hip_ctx *c) -> int {
+  b->issue = [levels, tl, dbase, keep_coeffs, counters_off](stwo_hip_ctx *c) -> int {
+    uint32_t *counters = (uint32_t *)(dbase + counters_off);
     for (const LevelLaunch &ll : levels) {
       if (ll.matrix) {
         int rc = ll.mx_layers
@@ -475,7 +480,7 @@ int batch_create_trees(stwo_hip_ctx *ctx, const BatchTree *trees, size_t n_trees
         int rc = launch_merkle_layer(c, nullptr, (const ColRef *)(dbase + t.off), t.count, max_log,
                                      layers + tree_layer_off(max_log), L.mode, true);
         if (rc) return rc;
-        rc = hash_node_layers(c, layers, max_log, 0, L.mode);
+        rc = hash_node_layers(c, layers, max_log, 0, L.mode, counters);
         if (rc) return rc;
         continue;
       }
@@ -493,7 +498,7 @@ int batch_create_trees(stwo_hip_ctx *ctx, const BatchTree *trees, size_t n_trees
           continue;
         }
         int next = ti < L.lt.size() ? (int)L.lt[ti].log_size : -1;
-        int rc = hash_node_layers(c, layers, (uint32_t)l + 1, (uint32_t)(next + 1), L.mode);
+        int rc = hash_node_layers(c, layers, (uint32_t)l + 1, (uint32_t)(next + 1), L.mode, counters);
         if (rc) return rc;
         l = next;
       }

@@ -90,6 +90,10 @@ struct stwo_hip_ctx {
   void *d_gather = nullptr;
   size_t gather_cap = 0;
 
+  // kTreeCounters zeros for the one-launch trees of this context's stream
+  // (every launch leaves them zero).
+  uint32_t *d_counters = nullptr;
+
   // Scratch device buffers kept across calls, keyed by purpose.
   std::map<std::string, std::pair<void *, size_t>> scratch;
   // Host copies of the tables upload_tables_cached last placed in its

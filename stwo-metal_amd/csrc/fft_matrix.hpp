@@ -9,7 +9,7 @@ namespace stwo_hip {
 
 constexpr uint32_t kMxMinLog = 12;     // smallest transform: one chunk of the low pass
 constexpr uint32_t kMxMaxLog = 24;     // largest: top 8 layers, at most 4 in between, low 12
-constexpr uint32_t kMxMaxBlowup = 4;   // blowups the matrix table covers
+constexpr uint32_t kMxMaxBlowup = 2;   // blowups the matrix table covers (0.7 MB; twice that a log further)
 
 // The top 4 or 8 layers of a group of columns of 2^n coefficients.  Inverse:
 // icols' in (evaluations) -> coefficients, stored to icols' out when `store`;

@@ -142,256 +142,347 @@ __global__ void alpha_pow2k_kernel(const uint32_t *in, uint32_t *out, uint32_t k
 // also copied to root_out.  The retry loop is bounded (each try fails with
 // probability about 2^-28); running out sets the error flag.
 // Run by the 4 lanes of one quad (lanes 0-3 of a wave, all active), each
-// compression shared by the quad (b2_compress_quad).
+// compression shared by the quad (b2_compress_quad).  In registers: m = the
+// digest (8 words) || the root; digest gets the new digest, the lane's word of
+// alpha is returned.
+__device__ __forceinline__ uint32_t channel_core(uint32_t m[16], uint32_t digest[8], uint32_t &n_draws, bool &ok) {
+  const b2_quad_iv iv = b2_quad_init();
+  uint32_t lo = iv.lo, hi = iv.hi;
+  b2_compress_quad(iv, lo, hi, m, b2_quad_d(iv, 64, true));
+  b2_quad_gather(lo, hi, digest);
+  const uint32_t d37 = b2_quad_d(iv, 37, true);
+  n_draws = 0;
+  ok = false;
+#pragma unroll 1
+  for (int tries = 0; tries < 64 && !ok; tries++) {
+#pragma unroll
+    for (int k = 0; k < 8; k++) m[k] = digest[k];
+    m[8] = n_draws;
+#pragma unroll
+    for (int k = 9; k < 16; k++) m[k] = 0;  // the 0x00 separator byte and zero padding
+    lo = iv.lo;
+    hi = iv.hi;
+    b2_compress_quad(iv, lo, hi, m, d37);
+    n_draws++;
+    const uint64_t bal = __ballot(lo < 2u * P && hi < 2u * P);
+    ok = ((bal >> (__lane_id() & ~3u)) & 0xF) == 0xF;
+  }
+  return b2_reduce_word(lo);
+}
 __device__ void channel_step(uint32_t *chan, const uint32_t *root, uint32_t *root_out, uint32_t *alpha_out) {
   const uint32_t j = __lane_id() & 3;
-  const uint32_t init_lo = b2_iv_lo(j), init_hi = b2_iv_hi(j);
-  uint32_t m[16];
+  uint32_t m[16], digest[8], n_draws;
+  bool ok;
   for (int k = 0; k < 8; k++) {
     m[k] = chan[k];
     m[8 + k] = root[k];
   }
   root_out[j] = root[j];
   root_out[4 + j] = root[4 + j];
-  uint32_t lo = init_lo, hi = init_hi;
-  b2_compress_quad(lo, hi, m, 64, true);
-  uint32_t digest[8];
-  b2_quad_gather(lo, hi, digest);
-  uint32_t n_draws = 0;
-  bool ok = false;
-  for (int tries = 0; tries < 64 && !ok; tries++) {
-    for (int k = 0; k < 8; k++) m[k] = digest[k];
-    m[8] = n_draws;
-    for (int k = 9; k < 16; k++) m[k] = 0;  // the 0x00 separator byte and zero padding
-    lo = init_lo;
-    hi = init_hi;
-    b2_compress_quad(lo, hi, m, 37, true);
-    n_draws++;
-    const uint64_t bal = __ballot(lo < 2u * P && hi < 2u * P);
-    ok = ((bal >> (__lane_id() & ~3u)) & 0xF) == 0xF;
-  }
+  const uint32_t al = channel_core(m, digest, n_draws, ok);
   chan[j] = digest[j];
   chan[4 + j] = digest[4 + j];
   if (j == 0) {
     chan[8] = n_draws;
     if (!ok) chan[9] = 1;
   }
-  alpha_out[j] = b2_reduce_word(lo);
+  alpha_out[j] = al;
 }
 
 // ---- the small layers in one launch ---------------------------------------
 //
-// Below kTailLog the per-layer work (a few thousand hashes) is far shorter
-// than the launches it takes (leaves, node layers, channel step, fold), so
-// one workgroup runs every remaining inner layer: lifted leaves of the 4
-// coordinate columns, the node layers, the channel step, then the line fold
-// into the next layer's evaluation, with a workgroup barrier between phases
-// (all of a workgroup's waves share one CU's L1, so its global writes are
-// visible to the workgroup after __syncthreads).  It writes the same trees,
-// roots, channel state and folded evaluations as the per-layer launches.
-constexpr uint32_t kTailLog = 10;
+// Below kTailLog a layer's work (a few hundred hashes) is far shorter than a
+// launch, so one workgroup runs every remaining inner layer: lifted leaves of
+// the 4 coordinate columns, the node layers, the channel step, then the line
+// fold into the next layer's evaluation.  The layer's values, its fold's
+// twiddles (loaded while the tree is hashed) and the channel stay in LDS from
+// phase to phase; the trees, roots, channel state and folded evaluations
+// written are the ones the per-layer launches write.  What bounds it is the
+// chain of compressions: lg + 3 a layer.  Layers of 2^9 and 2^10 cost one
+// workgroup as much as a launch over several costs (four compressions per
+// lane for the leaves of 2^10 alone).
+constexpr uint32_t kTailLog = 8;
 constexpr uint32_t kTailMax = 16;
-constexpr uint32_t kTailThreads = 1024;
 
 struct FriTailLayer {
-  const uint32_t *src[4];  // the layer's committed evaluation (log lg)
-  uint32_t *tree;          // its packed lifted tree
-  uint32_t *dst[4];        // the fold's output (log lg - step)
+  uint32_t *tree;    // the layer's packed lifted tree
+  uint32_t *dst[4];  // the fold's output (log lg - step)
   uint32_t lg, step, root_slot, pad;
 };
 struct FriTail {
+  const uint32_t *src[4];  // the first layer's evaluation
   FriTailLayer l[kTailMax];
   uint32_t n;
   const uint32_t *itw_end;
   uint32_t *chan, *roots, *alpha;
 };
 
-// Output i of the layer's fold (a run-time step of 1..4 at the call site).
+struct TailLds {
+  TreeLds t;
+  uint32_t v[4][1u << kTailLog], tw[1u << kTailLog], chan[8], alpha[4];
+};
+
+// Output i of STEP line folds of the layer in LDS (fold_line_at, from LDS).
 template <int STEP>
-__device__ __forceinline__ void tail_fold(const FriTailLayer &L, const uint32_t *itw_end, qm31 alpha, uint32_t i) {
-  Qm31ColsConst src;
+__device__ __forceinline__ qm31 tail_fold(const TailLds &S, uint32_t n, uint32_t i) {
+  constexpr int W = 1 << STEP;
+  qm31 a = qm31_make(S.alpha[0], S.alpha[1], S.alpha[2], S.alpha[3]), v[W];
 #pragma unroll
-  for (int k = 0; k < 4; k++) src.c[k] = L.src[k];
-  const qm31 r = fold_line_at<STEP>(src, itw_end, L.lg, alpha, i);
+  for (int j = 0; j < W; j++)
 #pragma unroll
-  for (int k = 0; k < 4; k++) L.dst[k][i] = r.v[k];
-}
-
-// Node levels top_log - 1 .. 0 of a packed tree, by one workgroup of
-// kTailThreads lanes: H(left || right), a quad per hash on levels of at most
-// kTailThreads / 4 hashes (their latency is the critical path), a lane per
-// hash above.  Every level is written to the tree and kept in LDS (lv[0] and
-// lv[1] in turn, at most kTailThreads digests each), and the next level reads
-// it from there: the global stores are never waited for.  Level top_log is
-// read from lv[0] when `in_lds` (written there by the caller), else from the
-// tree.  Starts with a barrier; returns the root (LDS, or the tree when
-// top_log = 0 and not in_lds) after a closing barrier.
-__device__ __forceinline__ const uint32_t *tree_levels_to_root(uint32_t *tree, uint32_t top_log,
-                                                               uint32_t (&lv)[2][kTailThreads * 8], bool in_lds) {
-  const uint32_t tid = threadIdx.x, q = tid >> 2, j = tid & 3;
-  uint32_t c = 0;  // lv[c] holds the level below the one being hashed
-  auto level = [&](const uint32_t *child, uint32_t l, uint32_t *keep) {
-    uint32_t *out = tree + tree_layer_off(l);
-    if ((1u << l) <= kTailThreads / 4) {
-      if (q < (1u << l)) {
-        uint32_t m[16];
+    for (int k = 0; k < 4; k++) v[j].v[k] = S.v[k][i * W + j];
 #pragma unroll
-        for (int k = 0; k < 16; k++) m[k] = child[16 * (size_t)q + k];
-        uint32_t lo = b2_iv_lo(j), hi = b2_iv_hi(j);
-        b2_compress_quad(lo, hi, m, 64, true);
-        out[8 * (size_t)q + j] = lo;
-        out[8 * (size_t)q + 4 + j] = hi;
-        keep[8 * q + j] = lo;
-        keep[8 * q + 4 + j] = hi;
+  for (int layer = 0; layer < STEP; layer++) {
+    const int half = W >> (layer + 1);
+    const uint32_t *lvl = S.tw + (n - (n >> layer));
+#pragma unroll
+    for (int j = 0; j < half; j++) {
+      const uint32_t xi = lvl[i * half + j];
+      qm31 f0, f1;
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        f0.v[k] = m31_add(v[2 * j].v[k], v[2 * j + 1].v[k]);
+        f1.v[k] = m31_mul(m31_sub(v[2 * j].v[k], v[2 * j + 1].v[k]), xi);
       }
-      return;
+      v[j] = qm31_add(f0, qm31_mul(a, f1));
     }
-    for (uint32_t i = tid; i < (1u << l); i += kTailThreads) {
-      uint32_t m[16];
-#pragma unroll
-      for (int k = 0; k < 16; k++) m[k] = child[16 * (size_t)i + k];
-      b2_state s;
-      b2_init(s);
-      b2_compress(s, m, 64, true);
-#pragma unroll
-      for (int k = 0; k < 8; k++) {
-        out[8 * (size_t)i + k] = s.h[k];
-        keep[8 * i + k] = s.h[k];
-      }
-    }
-  };
-  for (uint32_t l = top_log; l-- > 0;) {
-    __syncthreads();
-    if (!in_lds && l + 1 == top_log) {
-      level(tree + tree_layer_off(l + 1), l, lv[0]);
-      continue;  // the level is now in lv[0] = lv[c]
-    }
-    level(lv[c], l, lv[c ^ 1]);
-    c ^= 1;
+    if (layer + 1 < STEP) a = qm31_mul(a, a);
   }
-  __syncthreads();
-  return (top_log == 0 && !in_lds) ? tree : lv[c];
+  return v[0];
 }
 
-__global__ void __launch_bounds__(kTailThreads) fri_tail_kernel(FriTail t) {
-  __shared__ uint32_t lv[2][kTailThreads * 8];
-  const uint32_t tid = threadIdx.x;
+__global__ void __launch_bounds__(kTreeThreads) fri_tail_kernel(FriTail t) {
+  __shared__ __align__(16) TailLds S;
+  const uint32_t tid = threadIdx.x, q = tid >> 2, j = tid & 3;
+  uint32_t n = 1u << t.l[0].lg;
+  if (tid < n)
+#pragma unroll
+    for (int k = 0; k < 4; k++) S.v[k][tid] = t.src[k][tid];
+  if (tid < 8) S.chan[tid] = t.chan[tid];
+  uint32_t n_draws = 0;
+  bool ok = true;
+#pragma unroll 1
   for (uint32_t li = 0; li < t.n; li++) {
     const FriTailLayer &L = t.l[li];
+    n = 1u << L.lg;
+    __syncthreads();
+    // the fold's twiddles: levels lg, lg - 1, ... follow each other
+    const uint32_t n_out = n >> L.step;
+    uint32_t tw = 0;
+    if (tid < n - n_out) tw = t.itw_end[(ptrdiff_t)tid - (ptrdiff_t)n];
     // lifted leaves: H(le32 of the 4 coordinates), one 16-byte block
-    // Levels of at most kTailThreads / 4 hashes use a quad per hash (their
-    // latency is the layer's critical path), larger ones a lane per hash.
-    const uint32_t n = 1u << L.lg;
-    const uint32_t q = tid >> 2, j = tid & 3;
     uint32_t *leaves = L.tree + tree_layer_off(L.lg);
-    if (n <= kTailThreads / 4) {
-      if (q < n) {
-        uint32_t m[16];
+    uint32_t m[16];
 #pragma unroll
-        for (int k = 0; k < 4; k++) m[k] = L.src[k][q];
+    for (int k = 4; k < 16; k++) m[k] = 0;
+    if (n > 128) {
+      if (tid < n) {
 #pragma unroll
-        for (int k = 4; k < 16; k++) m[k] = 0;
-        uint32_t lo = b2_iv_lo(j), hi = b2_iv_hi(j);
-        b2_compress_quad(lo, hi, m, 16, true);
-        leaves[8 * (size_t)q + j] = lo;
-        leaves[8 * (size_t)q + 4 + j] = hi;
-        lv[0][8 * q + j] = lo;
-        lv[0][8 * q + 4 + j] = hi;
-      }
-    } else {
-      for (uint32_t i = tid; i < n; i += kTailThreads) {
-        uint32_t m[16];
-#pragma unroll
-        for (int k = 0; k < 4; k++) m[k] = L.src[k][i];
-#pragma unroll
-        for (int k = 4; k < 16; k++) m[k] = 0;
+        for (int k = 0; k < 4; k++) m[k] = S.v[k][tid];
         b2_state s;
         b2_init(s);
         b2_compress(s, m, 16, true);
+        store_hash(leaves + 8 * (size_t)tid, s, 0);
+        tree_keep(S.t, 0, tid, s);
+      }
+    } else {
+      for (uint32_t i = q; i < n; i += kTreeThreads / 4) {
 #pragma unroll
-        for (int k = 0; k < 8; k++) {
-          leaves[8 * (size_t)i + k] = s.h[k];
-          lv[0][8 * i + k] = s.h[k];
-        }
+        for (int k = 0; k < 4; k++) m[k] = S.v[k][i];
+        uint32_t lo = b2_iv_lo(j), hi = b2_iv_hi(j);
+        b2_compress_quad(lo, hi, m, 16, true);
+        as_global(leaves)[8 * i + j] = lo;
+        as_global(leaves)[8 * i + 4 + j] = hi;
+        tree_row(S.t, 0, i)[j] = lo;
+        tree_row(S.t, 0, i)[4 + j] = hi;
       }
     }
-    // node layers lg - 1 .. 0
-    const uint32_t *root = tree_levels_to_root(L.tree, L.lg, lv, true);
-    if (tid < 4) channel_step(t.chan, root, t.roots + 8 * L.root_slot, t.alpha);
+    S.tw[tid] = tw;
+    const uint32_t buf = tree_levels(S.t, 0, n, 0, L.lg, L.lg, L.tree, 0, false);
+    if (tid < 4) {
+      const uint32_t *root = tree_row(S.t, buf, 0);
+      uint32_t digest[8];
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        m[k] = S.chan[k];
+        m[8 + k] = root[k];
+      }
+      uint32_t *ro = t.roots + 8 * L.root_slot;
+      as_global(ro)[j] = root[j];
+      as_global(ro)[4 + j] = root[4 + j];
+      bool drawn;
+      S.alpha[j] = channel_core(m, digest, n_draws, drawn);
+      ok = ok && drawn;
+      if (j == 0)
+#pragma unroll
+        for (int k = 0; k < 8; k++) S.chan[k] = digest[k];
+    }
     __syncthreads();
-    const qm31 alpha = qm31_make(t.alpha[0], t.alpha[1], t.alpha[2], t.alpha[3]);
-    const uint32_t n_out = 1u << (L.lg - L.step);
-    for (uint32_t i = tid; i < n_out; i += kTailThreads) {
+    qm31 r;
+    if (tid < n_out) {
       switch (L.step) {
-        case 1: tail_fold<1>(L, t.itw_end, alpha, i); break;
-        case 2: tail_fold<2>(L, t.itw_end, alpha, i); break;
-        case 3: tail_fold<3>(L, t.itw_end, alpha, i); break;
-        default: tail_fold<4>(L, t.itw_end, alpha, i); break;
+        case 1: r = tail_fold<1>(S, n, tid); break;
+        case 2: r = tail_fold<2>(S, n, tid); break;
+        case 3: r = tail_fold<3>(S, n, tid); break;
+        default: r = tail_fold<4>(S, n, tid); break;
       }
     }
     __syncthreads();
+    if (tid < n_out)
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        as_global(L.dst[k])[tid] = r.v[k];
+        S.v[k][tid] = r.v[k];
+      }
+  }
+  if (tid < 8) t.chan[tid] = S.chan[tid];
+  if (tid < 4) t.alpha[tid] = S.alpha[tid];
+  if (tid == 0) {
+    t.chan[8] = n_draws;
+    if (!ok) t.chan[9] = 1;
   }
 }
 
-// ---- one FRI layer in two launches --------------------------------------
+// ---- one FRI layer in one launch ------------------------------------------
 //
-// Above kTailLog a layer is committed by fri_layer_kernel, which also runs
-// the fold that produces the layer (from the previous layer, with alpha from
-// the device channel), then hashes its lifted leaves and the first node
-// levels of every 256-leaf subtree; the remaining levels and the channel
-// step on the root run in fri_top_kernel (after merkle_nodes launches for
-// levels wider than 2^kTopLog).  The trees, roots, channel state and folded
-// evaluations written are the ones the separate fold, leaf, node and channel
-// launches write.
+// Above kTailLog a layer is committed by fri_layer_kernel: the fold that
+// produces it (from the previous layer, with alpha from the device channel),
+// its lifted leaves, the node levels (a subtree per workgroup, then the last
+// of each group of workgroups to finish, merkle_dev.hpp) and, in the workgroup
+// that hashes the root, the channel step.  The trees, roots, channel state and
+// folded evaluations written are the ones the separate fold, leaf, node and
+// channel launches write.
 constexpr int kFoldCircle = 5;    // fri_layer_kernel's FOLD for the circle fold
-constexpr uint32_t kTopLog = 10;  // fri_top_kernel starts at a level of at most 2^kTopLog nodes
 
-// FOLD = 0: the layer's values are src at i.  FOLD = 1..4: line folds of
-// that many steps from a layer of log lg + FOLD.  kFoldCircle: the circle
-// fold from log lg + 1.  A fold writes the layer to dst.  n_sub <= min(8, lg)
-// node levels follow the leaves in each workgroup.
+// The layer's value i: FOLD = 0, src at i; FOLD = 1..4, line folds of that many
+// steps from a layer of log lg + FOLD; kFoldCircle, the circle fold from log
+// lg + 1.  A fold writes the layer to dst.
 template <int FOLD>
-__global__ void __launch_bounds__(256) fri_layer_kernel(Qm31ColsConst src, Qm31Cols dst, const uint32_t *itw_end,
-                                                        const uint32_t *alpha_dev, uint32_t lg, uint32_t *tree,
-                                                        uint32_t n_sub) {
-  __shared__ uint32_t hs[256][9];
-  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-  if (i < (1u << lg)) {
+__device__ __forceinline__ qm31 fri_value(const Qm31ColsConst &src, const Qm31Cols &dst, const uint32_t *itw_end,
+                                          const qm31 &alpha, uint32_t lg, uint32_t i, bool store) {
+  if constexpr (FOLD == 0) {
+    return qm31_make(as_global(src.c[0])[i], as_global(src.c[1])[i], as_global(src.c[2])[i], as_global(src.c[3])[i]);
+  } else {
     qm31 v;
-    if constexpr (FOLD == 0) {
-      v = qm31_make(as_global(src.c[0])[i], as_global(src.c[1])[i], as_global(src.c[2])[i], as_global(src.c[3])[i]);
-    } else {
-      const qm31 alpha = load_qm31(alpha_dev);
-      if constexpr (FOLD == kFoldCircle)
-        v = fold_circle_at(src, itw_end, lg + 1, alpha, i);
-      else
-        v = fold_line_at<FOLD>(src, itw_end, lg + FOLD, alpha, i);
+    if constexpr (FOLD == kFoldCircle)
+      v = fold_circle_at(src, itw_end, lg + 1, alpha, i);
+    else
+      v = fold_line_at<FOLD>(src, itw_end, lg + FOLD, alpha, i);
+    if (store)
 #pragma unroll
       for (int k = 0; k < 4; k++) as_global(dst.c[k])[i] = v.v[k];
-    }
-    // lifted leaf: H(le32 of the 4 coordinates), one 16-byte block
-    uint32_t m[16];
+    return v;
+  }
+}
+
+// LEAVES per workgroup (tree_leaves_log): 64 with a quad per leaf, 256, 1,024.
+template <int FOLD, uint32_t LEAVES>
+__global__ void __launch_bounds__(kTreeThreads) fri_layer_kernel(Qm31ColsConst src, Qm31Cols dst,
+                                                                 const uint32_t *itw_end, uint32_t *alpha_dev,
+                                                                 uint32_t lg, uint32_t *tree, uint32_t *chan,
+                                                                 uint32_t *root_out, uint32_t *counters) {
+  __shared__ __align__(16) TreeLds S;
+  const uint32_t n = 1u << lg, first = blockIdx.x * LEAVES, tid = threadIdx.x;
+  const uint32_t q = tid >> 2, j = tid & 3;
+  uint32_t *leaves = tree + tree_layer_off(lg);
+  const qm31 alpha = FOLD ? load_qm31(alpha_dev) : qm31_make(0, 0, 0, 0);
+  // the channel, for the workgroup that hashes the root
+  uint32_t cm[16];
+  if (tid < 4)
+#pragma unroll
+    for (int k = 0; k < 8; k++) cm[k] = chan[k];
+  uint32_t top = lg, cnt = min(LEAVES, n), row0 = first;  // the level held in S
+  // lifted leaf: H(le32 of the 4 coordinates), one 16-byte block
+  uint32_t m[16];
+#pragma unroll
+  for (int k = 4; k < 16; k++) m[k] = 0;
+  auto leaf = [&](uint32_t i) {
+    const qm31 v = fri_value<FOLD>(src, dst, itw_end, alpha, lg, i, true);
 #pragma unroll
     for (int k = 0; k < 4; k++) m[k] = v.v[k];
-#pragma unroll
-    for (int k = 4; k < 16; k++) m[k] = 0;
     b2_state s;
     b2_init(s);
     b2_compress(s, m, 16, true);
-    store_hash(tree + tree_layer_off(lg) + 8 * (size_t)i, s, 0);
+    store_hash(leaves + 8 * (size_t)i, s, 0);
+    return s;
+  };
+  auto node = [&](const b2_state &a, const b2_state &b, uint32_t l, size_t i) {
+    uint32_t w[16];
 #pragma unroll
-    for (int k = 0; k < 8; k++) hs[threadIdx.x][k] = s.h[k];
+    for (int k = 0; k < 8; k++) {
+      w[k] = a.h[k];
+      w[8 + k] = b.h[k];
+    }
+    b2_state s;
+    b2_init(s);
+    b2_compress(s, w, 64, true);
+    store_hash(tree + tree_layer_off(l) + 8 * i, s, 0);
+    return s;
+  };
+  if constexpr (LEAVES == 64) {
+    const uint32_t i = first + q;
+    if (i < n) {  // the quad's lanes fold alike, the first stores
+      const qm31 v = fri_value<FOLD>(src, dst, itw_end, alpha, lg, i, j == 0);
+#pragma unroll
+      for (int k = 0; k < 4; k++) m[k] = v.v[k];
+      uint32_t lo = b2_iv_lo(j), hi = b2_iv_hi(j);
+      b2_compress_quad(lo, hi, m, 16, true);
+      as_global(leaves + 8 * (size_t)i)[j] = lo;
+      as_global(leaves + 8 * (size_t)i)[4 + j] = hi;
+      tree_row(S, 0, q)[j] = lo;
+      tree_row(S, 0, q)[4 + j] = hi;
+    }
+  } else if constexpr (LEAVES == 256) {
+    const uint32_t i = first + tid;
+    if (i < n) tree_keep(S, 0, tid, leaf(i));
+  } else {
+    // four leaves per lane and, from registers, the two levels above them
+    const uint32_t i = first + 4 * tid;
+    b2_state keep;
+#pragma unroll 1
+    for (uint32_t p = 0; p < 2; p++) {
+      const b2_state a = leaf(i + 2 * p), b = leaf(i + 2 * p + 1);
+      const b2_state c = node(a, b, lg - 1, i / 2 + p);
+      if (p == 0)
+        keep = c;
+      else
+        tree_keep(S, 0, tid, node(keep, c, lg - 2, i / 4));
+    }
+    top -= 2;
+    cnt >>= 2;
+    row0 >>= 2;
   }
-  subtree_levels(hs, tree, lg, n_sub, 0);
+  const uint32_t lv = 31 - __clz(cnt), l = top - lv;
+  uint32_t buf = tree_levels(S, 0, cnt, row0, top, lv, tree, 0, l > 0);
+  const int done = tree_finish(S, buf, blockIdx.x, l, 0, tree, 0, counters);
+  if (done < 0 || tid >= 4) return;
+  const uint32_t *root = tree_row(S, (uint32_t)done, 0);
+  uint32_t digest[8], n_draws;
+  bool ok;
+#pragma unroll
+  for (int k = 0; k < 8; k++) cm[8 + k] = root[k];
+  root_out[j] = root[j];
+  root_out[4 + j] = root[4 + j];
+  const uint32_t al = channel_core(cm, digest, n_draws, ok);
+  alpha_dev[j] = al;
+  if (j == 0) {
+#pragma unroll
+    for (int k = 0; k < 8; k++) chan[k] = digest[k];
+    chan[8] = n_draws;
+    if (!ok) chan[9] = 1;
+  }
 }
 
-// Levels top_log - 1 .. 0 (level top_log - 1 of at most 2^kTopLog nodes),
-// then the channel step on the root.
-__global__ void __launch_bounds__(kTailThreads) fri_top_kernel(uint32_t *tree, uint32_t top_log, uint32_t *chan,
-                                                               uint32_t *root_out, uint32_t *alpha_out) {
-  __shared__ uint32_t lv[2][kTailThreads * 8];
-  const uint32_t *root = tree_levels_to_root(tree, top_log, lv, false);
-  if (threadIdx.x < 4) channel_step(chan, root, root_out, alpha_out);
+template <int FOLD>
+static int launch_fri_layer(stwo_hip_ctx *ctx, const Qm31ColsConst &src, const Qm31Cols &dst, const uint32_t *itw_end,
+                            uint32_t *alpha, uint32_t lg, uint32_t *tree, uint32_t *chan, uint32_t *root_out) {
+  const uint32_t per = tree_leaves_log(lg);
+  const dim3 grid(1u << (lg > per ? lg - per : 0)), block(kTreeThreads);
+  return launch(ctx, "fri_layer",
+                per == 6   ? fri_layer_kernel<FOLD, 64>
+                : per == 8 ? fri_layer_kernel<FOLD, 256>
+                           : fri_layer_kernel<FOLD, 1024>,
+                grid, block, 0, src, dst, itw_end, alpha, lg, tree, chan, root_out, ctx->d_counters);
 }
 
 // chan = [digest, n_draws, 0] (the device channel's starting state).
@@ -763,7 +854,7 @@ static int fri_commit_impl(stwo_hip_ctx *ctx, uint8_t channel_digest[32], uint32
   if (keep && keep->layers.size() != sched.size())
     return set_error(ctx, STWO_HIP_EINVAL, "internal: FRI prover storage does not match the schedule");
   // The layer loop runs on the stream without host round trips: after each
-  // layer's Merkle commit, the kernel that hashes its root (fri_top_kernel,
+  // layer's Merkle commit, the kernel that hashes its root (fri_layer_kernel
   // or the tail) mixes the root into the device copy of the channel and
   // draws the next alpha, which the folds read from device memory.  The host reads the roots, the channel
   // and the last layer once, at the end.
@@ -842,27 +933,17 @@ static int fri_commit_impl(stwo_hip_ctx *ctx, uint8_t channel_digest[32], uint32
       if (r) return r;
       for (int k = 0; k < 4; k++) src.c[k] = cols[k];
     }
-    const uint32_t n_sub = std::min<uint32_t>(8, lg);
-    const dim3 grid((uint32_t)(((1ull << lg) + 255) / 256)), block(256);
     const uint32_t *itw_end = tw->d_itw + tw->len;
+    uint32_t *root_out = d_roots + 8 * nr;
     int r;
     switch (fold) {
-      case 0: r = launch(ctx, "fri_layer", fri_layer_kernel<0>, grid, block, 0, src, dst, itw_end, (const uint32_t *)d_alpha, lg, tree, n_sub); break;
-      case 1: r = launch(ctx, "fri_layer", fri_layer_kernel<1>, grid, block, 0, src, dst, itw_end, (const uint32_t *)d_alpha, lg, tree, n_sub); break;
-      case 2: r = launch(ctx, "fri_layer", fri_layer_kernel<2>, grid, block, 0, src, dst, itw_end, (const uint32_t *)d_alpha, lg, tree, n_sub); break;
-      case 3: r = launch(ctx, "fri_layer", fri_layer_kernel<3>, grid, block, 0, src, dst, itw_end, (const uint32_t *)d_alpha, lg, tree, n_sub); break;
-      case 4: r = launch(ctx, "fri_layer", fri_layer_kernel<4>, grid, block, 0, src, dst, itw_end, (const uint32_t *)d_alpha, lg, tree, n_sub); break;
-      default: r = launch(ctx, "fri_layer", fri_layer_kernel<kFoldCircle>, grid, block, 0, src, dst, itw_end, (const uint32_t *)d_alpha, lg, tree, n_sub); break;
+      case 0: r = launch_fri_layer<0>(ctx, src, dst, itw_end, d_alpha, lg, tree, d_chan, root_out); break;
+      case 1: r = launch_fri_layer<1>(ctx, src, dst, itw_end, d_alpha, lg, tree, d_chan, root_out); break;
+      case 2: r = launch_fri_layer<2>(ctx, src, dst, itw_end, d_alpha, lg, tree, d_chan, root_out); break;
+      case 3: r = launch_fri_layer<3>(ctx, src, dst, itw_end, d_alpha, lg, tree, d_chan, root_out); break;
+      case 4: r = launch_fri_layer<4>(ctx, src, dst, itw_end, d_alpha, lg, tree, d_chan, root_out); break;
+      default: r = launch_fri_layer<kFoldCircle>(ctx, src, dst, itw_end, d_alpha, lg, tree, d_chan, root_out); break;
     }
-    if (r) return r;
-    uint32_t top = lg - n_sub;
-    if (top > kTopLog + 1) {
-      r = hash_node_layers(ctx, tree, top, kTopLog + 1, STWO_HIP_HASH_BLAKE2S);
-      if (r) return r;
-      top = kTopLog + 1;
-    }
-    r = launch(ctx, "fri_top", fri_top_kernel, dim3(1), dim3(kTailThreads), 0, tree, top, d_chan, d_roots + 8 * nr,
-               d_alpha);
     if (r) return r;
     nr++;
     return STWO_HIP_OK;
@@ -903,6 +984,7 @@ static int fri_commit_impl(stwo_hip_ctx *ctx, uint8_t channel_digest[32], uint32
         t.chan = d_chan;
         t.roots = d_roots;
         t.alpha = d_alpha;
+        for (int k = 0; k < 4; k++) t.src[k] = cur[k];
         for (;;) {
           last = !(lg > last_log + cfg.line_fold_step);
           step = last ? lg - last_log : cfg.line_fold_step;
@@ -911,7 +993,6 @@ static int fri_commit_impl(stwo_hip_ctx *ctx, uint8_t channel_digest[32], uint32
           FriTailLayer &L = t.l[t.n++];
           L.tree = keep ? keep->layers[nr].tree : scratch_tree;
           for (int k = 0; k < 4; k++) {
-            L.src[k] = cur[k];
             if (keep) keep->layers[nr].cols[k] = cur[k];
             L.dst[k] = layer_buf(n_folds, lg - step, k);
             cur[k] = L.dst[k];
@@ -924,7 +1005,7 @@ static int fri_commit_impl(stwo_hip_ctx *ctx, uint8_t channel_digest[32], uint32
           lg -= step;
           if (last) break;
         }
-        rc = launch(ctx, "fri_tail", fri_tail_kernel, dim3(1), dim3(kTailThreads), 0, t);
+        rc = launch(ctx, "fri_tail", fri_tail_kernel, dim3(1), dim3(kTreeThreads), 0, t);
         if (rc) return rc;
         break;
       }

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "common.hpp"
@@ -267,7 +268,16 @@ struct ColRef {
 int launch_merkle_layer(stwo_hip_ctx *ctx, const uint32_t *prev, const ColRef *d_cols, uint32_t n_cols,
                         uint32_t log_size, uint32_t *out, int mode, bool lifted);
 // Node layers [stop_log, top_log) of a packed tree whose layer top_log is filled.
-int hash_node_layers(stwo_hip_ctx *ctx, uint32_t *layers, uint32_t top_log, uint32_t stop_log, int mode);
+int hash_node_layers(stwo_hip_ctx *ctx, uint32_t *layers, uint32_t top_log, uint32_t stop_log, int mode,
+                     uint32_t *counters);
+// Counters of the one-launch trees: a word per group of workgroups that hand
+// their digests on, stage by stage; 2^12 + 2^5 + 1 for 2^30 leaves, and at most
+// 2^(lg / 2) for 2^lg (a tree's stages take equal shares of the levels above the
+// first 2^6, 2^8 or 2^10 digests).
+constexpr uint32_t kTreeCounters = 1u << 13;
+inline uint32_t tree_counters(uint32_t lg) { return std::min(kTreeCounters, 1u << ((lg + 1) / 2)); }
+// log2 of the first digests a workgroup of a one-launch tree of 2^lg takes.
+inline uint32_t tree_leaves_log(uint32_t lg) { return lg <= 14 ? 6 : lg < 18 ? 8 : 10; }
 
 __host__ __device__ inline size_t tree_layer_off(uint32_t l) { return (((size_t)1 << l) - 1) * 8; }
 

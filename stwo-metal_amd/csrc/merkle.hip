@@ -14,10 +14,10 @@
 // wave.  Column pointers come from a per-call device table (uniform across
 // the wave -> scalar loads).
 //
-// Node layers without injected columns run in `merkle_nodes_kernel`, which
-// hashes up to 8 consecutive layers per launch: each 256-lane workgroup
-// hashes 256 nodes, keeps the digests in LDS and halves the active lanes per
-// layer, writing every layer to global memory.
+// A run of node layers without injected columns, to the next injected layer or
+// the root, is one launch of `merkle_nodes_kernel`: each workgroup hashes a
+// subtree through LDS, writing every layer to global memory, and the last of
+// each group of workgroups to finish hashes on (merkle_dev.hpp).
 #include <algorithm>
 #include <vector>
 
@@ -40,6 +40,33 @@ __device__ __forceinline__ void load_block64(uint32_t m[16], const uint32_t *src
     m[4 * k + 2] = v.z;
     m[4 * k + 3] = v.w;
   }
+}
+
+__device__ __forceinline__ b2_state hash_block(const uint32_t m[16], uint32_t m31) {
+  b2_state s;
+  b2_init(s);
+  b2_compress(s, m, 64, true);
+  if (m31)
+#pragma unroll
+    for (int k = 0; k < 8; k++) s.h[k] = b2_reduce_word(s.h[k]);
+  return s;
+}
+// Node i: H(prev[2i] || prev[2i+1]), stored to out.
+__device__ __forceinline__ b2_state hash_node(const uint32_t *prev, uint32_t i, uint32_t *out, uint32_t m31) {
+  uint32_t m[16];
+  load_block64(m, prev + 16 * (size_t)i);
+  const b2_state s = hash_block(m, m31);
+  store_hash(out + 8 * (size_t)i, s, 0);
+  return s;
+}
+__device__ __forceinline__ b2_state hash_pair(const b2_state &a, const b2_state &b, uint32_t m31) {
+  uint32_t m[16];
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    m[k] = a.h[k];
+    m[8 + k] = b.h[k];
+  }
+  return hash_block(m, m31);
 }
 
 // Word idx of a column.  Layers are at most 2^30 rows, so the byte offset
@@ -231,28 +258,63 @@ __global__ void __launch_bounds__(256) merkle_layer_quad_lds_kernel(const uint32
   o[4 + j] = hi;
 }
 
-// Hashes `n_layers` (<= 8) consecutive node layers below `prev` (of log size
-// out_log + 1).  Layer k (k = 0 first) has log size out_log - k and is
-// written at out_base + offset(out_log - k) in the packed layout.
-__global__ void __launch_bounds__(256) merkle_nodes_kernel(const uint32_t *prev, uint32_t *packed, uint32_t out_log,
-                                                           uint32_t n_layers, uint32_t m31) {
-  __shared__ uint32_t hs[256][9];
-  const uint32_t n = 1u << out_log;
-  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-  uint32_t m[16];
-  b2_state s;
-  if (i < n) {
-    load_block64(m, prev + 16 * (size_t)i);
-    b2_init(s);
-    b2_compress(s, m, 64, true);
-    if (m31)
-#pragma unroll
-      for (int k = 0; k < 8; k++) s.h[k] = b2_reduce_word(s.h[k]);
-    store_hash(packed + (((size_t)1 << out_log) - 1) * 8 + 8 * (size_t)i, s, 0);
-#pragma unroll
-    for (int k = 0; k < 8; k++) hs[threadIdx.x][k] = s.h[k];
+// Node layers out_log .. stop_log below `prev` (of log size out_log + 1), each
+// written at its place in the packed layout.  A workgroup takes NODES nodes of
+// layer out_log: 1,024 (four per lane, with the two levels above them from
+// registers) where there are enough of them, which leaves little of a subtree to
+// its narrow levels; 64 (a quad each) in small trees, where latency counts; 256
+// between.
+template <uint32_t NODES>
+__global__ void __launch_bounds__(kTreeThreads) merkle_nodes_kernel(const uint32_t *prev, uint32_t *packed,
+                                                                    uint32_t out_log, uint32_t stop_log, uint32_t m31,
+                                                                    uint32_t *counters) {
+  __shared__ __align__(16) TreeLds S;
+  const uint32_t n = 1u << out_log, first = blockIdx.x * NODES, tid = threadIdx.x;
+  uint32_t *out = packed + tree_layer_off(out_log);
+  uint32_t lg = out_log, cnt = min(NODES, n), row0 = first;  // the level held in S
+  if constexpr (NODES == 64) {
+    const uint32_t q = tid >> 2, j = tid & 3, i = first + q;
+    if (i < n) {
+      uint32_t m[16];
+      load_block64(m, prev + 16 * (size_t)i);
+      uint32_t lo = b2_iv_lo(j), hi = b2_iv_hi(j);
+      b2_compress_quad(lo, hi, m, 64, true);
+      if (m31) {
+        lo = b2_reduce_word(lo);
+        hi = b2_reduce_word(hi);
+      }
+      as_global(out + 8 * (size_t)i)[j] = lo;
+      as_global(out + 8 * (size_t)i)[4 + j] = hi;
+      tree_row(S, 0, q)[j] = lo;
+      tree_row(S, 0, q)[4 + j] = hi;
+    }
+  } else if constexpr (NODES == 256) {
+    const uint32_t i = first + tid;
+    if (i < n) tree_keep(S, 0, tid, hash_node(prev, i, out, m31));
+  } else {
+    // four nodes per lane and, from registers, the two levels above them
+    const uint32_t i = first + 4 * tid;
+    b2_state keep;
+#pragma unroll 1
+    for (uint32_t p = 0; p < 2; p++) {
+      const b2_state a = hash_node(prev, i + 2 * p, out, m31), b = hash_node(prev, i + 2 * p + 1, out, m31);
+      const b2_state c = hash_pair(a, b, m31);
+      store_hash(packed + tree_layer_off(out_log - 1) + 8 * (size_t)(i / 2 + p), c, 0);
+      if (p == 0) {
+        keep = c;
+      } else {
+        const b2_state t = hash_pair(keep, c, m31);
+        store_hash(packed + tree_layer_off(out_log - 2) + 8 * (size_t)(i / 4), t, 0);
+        tree_keep(S, 0, tid, t);
+      }
+    }
+    lg -= 2;
+    cnt >>= 2;
+    row0 >>= 2;
   }
-  subtree_levels(hs, packed, out_log, n_layers - 1, m31);
+  const uint32_t lv = min(31 - __clz(cnt), lg - stop_log), l = lg - lv;
+  const uint32_t buf = tree_levels(S, 0, cnt, row0, lg, lv, packed, m31, l > stop_log);
+  tree_finish(S, buf, blockIdx.x, l, stop_log, packed, m31, counters);
 }
 
 static inline size_t layer_off(uint32_t l) { return tree_layer_off(l); }
@@ -289,26 +351,23 @@ static int launch_layer(stwo_hip_ctx *ctx, const uint32_t *prev, const std::vect
   return launch_merkle_layer(ctx, prev, (const ColRef *)dtab, (uint32_t)cols.size(), log_size, out, mode, lifted);
 }
 
-// Hashes node layers top_log-1 .. stop_log of a packed tree whose layer top_log is filled.
-int hash_node_layers(stwo_hip_ctx *ctx, uint32_t *layers, uint32_t top_log, uint32_t stop_log, int mode) {
-  // layers [stop_log, top_log) are produced, from top_log - 1 down.
+// Hashes node layers top_log-1 .. stop_log of a packed tree whose layer top_log
+// is filled.  counters: kTreeCounters zeros, left zero, used by no launch that
+// may overlap this one.
+int hash_node_layers(stwo_hip_ctx *ctx, uint32_t *layers, uint32_t top_log, uint32_t stop_log, int mode,
+                     uint32_t *counters) {
   STWO_HIP_CHECK_ARG(ctx, mode == STWO_HIP_HASH_BLAKE2S || mode == STWO_HIP_HASH_BLAKE2S_M31,
                      "merkle: unknown hash mode %d", mode);
-  uint32_t l = top_log;
-  while (l > stop_log) {
-    uint32_t out_log = l - 1;
-    uint32_t n_layers = std::min<uint32_t>(8, out_log - stop_log + 1);
-    // within one workgroup of 256 outputs we can go down at most 8 layers
-    uint32_t n_out = 1u << out_log;
-    uint32_t blocks = (n_out + 255) / 256;
-    if (n_out < 256) n_layers = std::min<uint32_t>(n_layers, out_log + 1);
-    int rc = launch(ctx, "merkle_nodes", merkle_nodes_kernel, dim3(blocks), dim3(256), 0,
-                    (const uint32_t *)(layers + layer_off(l)), layers, out_log, n_layers,
-                    (uint32_t)(mode == STWO_HIP_HASH_BLAKE2S_M31));
-    if (rc) return rc;
-    l = out_log + 1 - n_layers;
-  }
-  return STWO_HIP_OK;
+  if (top_log <= stop_log) return STWO_HIP_OK;
+  const uint32_t out_log = top_log - 1;
+  // (four nodes per lane take the two levels above along)
+  const uint32_t per = std::min<uint32_t>(tree_leaves_log(out_log), out_log >= stop_log + 2 ? 10 : 8);
+  const dim3 grid(1u << (out_log > per ? out_log - per : 0)), block(kTreeThreads);
+  const uint32_t *prev = layers + layer_off(top_log);
+  const uint32_t m31 = (uint32_t)(mode == STWO_HIP_HASH_BLAKE2S_M31);
+  return launch(ctx, "merkle_nodes",
+                per == 6 ? merkle_nodes_kernel<64> : per == 8 ? merkle_nodes_kernel<256> : merkle_nodes_kernel<1024>,
+                grid, block, 0, prev, layers, out_log, stop_log, m31, counters);
 }
 
 }  // namespace stwo_hip
@@ -353,7 +412,7 @@ int stwo_hip_merkle_commit(stwo_hip_ctx *ctx, const uint32_t *const *cols, const
       for (size_t c = 0; c < n_cols; c++)
         if ((int)log_sizes[c] < l) next = std::max(next, (int)log_sizes[c]);
       uint32_t stop = (uint32_t)(next + 1);
-      int rc = hash_node_layers(ctx, layers, (uint32_t)l + 1, stop, hash_mode);
+      int rc = hash_node_layers(ctx, layers, (uint32_t)l + 1, stop, hash_mode, ctx->d_counters);
       if (rc) return rc;
       l = (int)stop - 1;
       continue;
@@ -399,7 +458,7 @@ int stwo_hip_merkle_lifted_commit(stwo_hip_ctx *ctx, const uint32_t *const *cols
   int rc = stwo_hip_merkle_lifted_build_leaves(ctx, cols, log_sizes, n_cols, lifting_log_size,
                                                layers + layer_off(lifting_log_size), hash_mode);
   if (rc) return rc;
-  return hash_node_layers(ctx, layers, lifting_log_size, 0, hash_mode);
+  return hash_node_layers(ctx, layers, lifting_log_size, 0, hash_mode, ctx->d_counters);
 }
 
 }  // extern "C"

@@ -9,6 +9,7 @@
 #include <algorithm>
 
 #include "common.hpp"
+#include "internal.hpp"
 #include "field.hpp"
 
 namespace stwo_hip {
@@ -67,7 +68,9 @@ static const int kEventPoolInit = 16;
 
 static int arena_init(stwo_hip_ctx *ctx) {
   STWO_HIP_TRY(ctx, hipHostMalloc((void **)&ctx->h_arena, kArenaBytes, hipHostMallocDefault));
-  STWO_HIP_TRY(ctx, hipMalloc((void **)&ctx->d_arena, kArenaBytes));
+  STWO_HIP_TRY(ctx, hipMalloc((void **)&ctx->d_arena, kArenaBytes + kTreeCounters * 4));
+  ctx->d_counters = (uint32_t *)(ctx->d_arena + kArenaBytes);
+  STWO_HIP_TRY(ctx, hipMemsetAsync(ctx->d_counters, 0, kTreeCounters * 4, ctx->stream));
   ctx->arena_cap = kArenaBytes;
   ctx->arena_head = 0;
   STWO_HIP_TRY(ctx, hipHostMalloc((void **)&ctx->h_stage, kStageBytes, hipHostMallocDefault));
