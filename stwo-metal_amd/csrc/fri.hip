@@ -189,32 +189,73 @@ __device__ void channel_step(uint32_t *chan, const uint32_t *root, uint32_t *roo
   alpha_out[j] = al;
 }
 
+// The device words of one FRI commit: the channel (digest, n_draws, error flag),
+// the alpha drawn last, a slot for its powers, the root mixed before the first
+// layer (commits of a group), the roots, then flags, the grind's
+// best nonce (8-byte aligned) and prefix, and the last layer: its coefficients
+// when the end runs on the device, its evaluation otherwise.
+constexpr uint32_t kMaxRoots = 32;  // one per layer, at most log_size <= 28
+constexpr uint32_t kDevLastMax = 6;  // largest log of a last layer held here
+constexpr uint32_t kAlphaOff = 10, kAlphaTmpOff = 14, kMixedOff = 18, kRootsOff = 32, kFlagsOff = kRootsOff + 8 * kMaxRoots,
+                   kBestOff = kFlagsOff + 2, kPrefixOff = kBestOff + 2, kPolyOff = kPrefixOff + 8,
+                   kFriStateWords = kPolyOff + (4u << kDevLastMax);
+static_assert(kBestOff % 2 == 0, "best nonce alignment");
+
+// FRI commits that run side by side (fri_commit_jobs): blockIdx.y.
+constexpr uint32_t kFriJobs = 16;
+
+constexpr int kFoldCircle = 5;  // FOLD for the circle fold
+
+// A layer's value i: FOLD = 0, src at i; FOLD = 1..4, line folds of that many
+// steps from a layer of log lg + FOLD; kFoldCircle, the circle fold from log
+// lg + 1.  A fold writes the layer to dst (coordinates 2^lg words apart).
+template <int FOLD>
+__device__ __forceinline__ qm31 fri_value(const Qm31ColsConst &src, uint32_t *dst, const uint32_t *itw_end,
+                                          const qm31 &alpha, uint32_t lg, uint32_t i, bool store) {
+  if constexpr (FOLD == 0) {
+    return qm31_make(as_global(src.c[0])[i], as_global(src.c[1])[i], as_global(src.c[2])[i], as_global(src.c[3])[i]);
+  } else {
+    qm31 v;
+    if constexpr (FOLD == kFoldCircle)
+      v = fold_circle_at(src, itw_end, lg + 1, alpha, i);
+    else
+      v = fold_line_at<FOLD>(src, itw_end, lg + FOLD, alpha, i);
+    if (store)
+#pragma unroll
+      for (int k = 0; k < 4; k++) as_global(dst + ((size_t)k << lg))[i] = v.v[k];
+    return v;
+  }
+}
+
 // ---- the small layers in one launch ---------------------------------------
 //
 // Below kTailLog a layer's work (a few hundred hashes) is far shorter than a
-// launch, so one workgroup runs every remaining inner layer: lifted leaves of
-// the 4 coordinate columns, the node layers, the channel step, then the line
+// launch, so one workgroup runs every remaining inner layer: the fold that
+// produces the first of them, then per layer the lifted leaves of
+// the 4 coordinate columns, the node layers, the channel step and the line
 // fold into the next layer's evaluation.  The layer's values, its fold's
 // twiddles (loaded while the tree is hashed) and the channel stay in LDS from
 // phase to phase; the trees, roots, channel state and folded evaluations
 // written are the ones the per-layer launches write.  What bounds it is the
 // chain of compressions: lg + 3 a layer.  Layers of 2^9 and 2^10 cost one
 // workgroup as much as a launch over several costs (four compressions per
-// lane for the leaves of 2^10 alone).
+// lane for the leaves of 2^10 alone).  The commits of a group take a workgroup
+// each.
 constexpr uint32_t kTailLog = 8;
 constexpr uint32_t kTailMax = 16;
 
 struct FriTailLayer {
-  uint32_t *tree;    // the layer's packed lifted tree
-  uint32_t *dst[4];  // the fold's output (log lg - step)
-  uint32_t lg, step, root_slot, pad;
+  uint32_t *tree;  // the layer's packed lifted tree
+  uint32_t *dst;   // the fold's output (log lg - step, coordinates that far apart)
+  uint32_t lg, step;
 };
 struct FriTail {
-  const uint32_t *src[4];  // the first layer's evaluation
+  Qm31ColsConst src;  // what `fold` folds into the first layer's evaluation first (fold = 0: that evaluation)
+  uint32_t *first;
   FriTailLayer l[kTailMax];
-  uint32_t n;
+  uint32_t n, fold, root;  // root: the first layer's slot
   const uint32_t *itw_end;
-  uint32_t *chan, *roots, *alpha;
+  uint32_t *state;
 };
 
 struct TailLds {
@@ -251,14 +292,27 @@ __device__ __forceinline__ qm31 tail_fold(const TailLds &S, uint32_t n, uint32_t
   return v[0];
 }
 
-__global__ void __launch_bounds__(kTreeThreads) fri_tail_kernel(FriTail t) {
+__device__ __forceinline__ void fri_tail(const FriTail &t) {
   __shared__ __align__(16) TailLds S;
   const uint32_t tid = threadIdx.x, q = tid >> 2, j = tid & 3;
+  uint32_t *chan = t.state, *alpha = t.state + kAlphaOff;
   uint32_t n = 1u << t.l[0].lg;
-  if (tid < n)
+  if (tid < n) {
+    const uint32_t lg = t.l[0].lg;
+    qm31 v, a = qm31_make(0, 0, 0, 0);
+    if (t.fold) a = load_qm31(alpha);
+    switch (t.fold) {
+      case 0: v = fri_value<0>(t.src, t.first, t.itw_end, a, lg, tid, false); break;
+      case 1: v = fri_value<1>(t.src, t.first, t.itw_end, a, lg, tid, true); break;
+      case 2: v = fri_value<2>(t.src, t.first, t.itw_end, a, lg, tid, true); break;
+      case 3: v = fri_value<3>(t.src, t.first, t.itw_end, a, lg, tid, true); break;
+      case 4: v = fri_value<4>(t.src, t.first, t.itw_end, a, lg, tid, true); break;
+      default: v = fri_value<kFoldCircle>(t.src, t.first, t.itw_end, a, lg, tid, true); break;
+    }
 #pragma unroll
-    for (int k = 0; k < 4; k++) S.v[k][tid] = t.src[k][tid];
-  if (tid < 8) S.chan[tid] = t.chan[tid];
+    for (int k = 0; k < 4; k++) S.v[k][tid] = v.v[k];
+  }
+  if (tid < 8) S.chan[tid] = chan[tid];
   uint32_t n_draws = 0;
   bool ok = true;
 #pragma unroll 1
@@ -307,7 +361,7 @@ __global__ void __launch_bounds__(kTreeThreads) fri_tail_kernel(FriTail t) {
         m[k] = S.chan[k];
         m[8 + k] = root[k];
       }
-      uint32_t *ro = t.roots + 8 * L.root_slot;
+      uint32_t *ro = t.state + kRootsOff + 8 * (t.root + li);
       as_global(ro)[j] = root[j];
       as_global(ro)[4 + j] = root[4 + j];
       bool drawn;
@@ -331,17 +385,19 @@ __global__ void __launch_bounds__(kTreeThreads) fri_tail_kernel(FriTail t) {
     if (tid < n_out)
 #pragma unroll
       for (int k = 0; k < 4; k++) {
-        as_global(L.dst[k])[tid] = r.v[k];
+        as_global(L.dst + ((size_t)k << (L.lg - L.step)))[tid] = r.v[k];
         S.v[k][tid] = r.v[k];
       }
   }
-  if (tid < 8) t.chan[tid] = S.chan[tid];
-  if (tid < 4) t.alpha[tid] = S.alpha[tid];
+  if (tid < 8) chan[tid] = S.chan[tid];
+  if (tid < 4) alpha[tid] = S.alpha[tid];
   if (tid == 0) {
-    t.chan[8] = n_draws;
-    if (!ok) t.chan[9] = 1;
+    chan[8] = n_draws;
+    if (!ok) chan[9] = 1;
   }
 }
+__global__ void __launch_bounds__(kTreeThreads) fri_tail_kernel(FriTail t) { fri_tail(t); }
+__global__ void __launch_bounds__(kTreeThreads) fri_tails_kernel(const FriTail *t) { fri_tail(t[blockIdx.x]); }
 
 // ---- one FRI layer in one launch ------------------------------------------
 //
@@ -352,36 +408,25 @@ __global__ void __launch_bounds__(kTreeThreads) fri_tail_kernel(FriTail t) {
 // that hashes the root, the channel step.  The trees, roots, channel state and
 // folded evaluations written are the ones the separate fold, leaf, node and
 // channel launches write.
-constexpr int kFoldCircle = 5;    // fri_layer_kernel's FOLD for the circle fold
-
-// The layer's value i: FOLD = 0, src at i; FOLD = 1..4, line folds of that many
-// steps from a layer of log lg + FOLD; kFoldCircle, the circle fold from log
-// lg + 1.  A fold writes the layer to dst.
-template <int FOLD>
-__device__ __forceinline__ qm31 fri_value(const Qm31ColsConst &src, const Qm31Cols &dst, const uint32_t *itw_end,
-                                          const qm31 &alpha, uint32_t lg, uint32_t i, bool store) {
-  if constexpr (FOLD == 0) {
-    return qm31_make(as_global(src.c[0])[i], as_global(src.c[1])[i], as_global(src.c[2])[i], as_global(src.c[3])[i]);
-  } else {
-    qm31 v;
-    if constexpr (FOLD == kFoldCircle)
-      v = fold_circle_at(src, itw_end, lg + 1, alpha, i);
-    else
-      v = fold_line_at<FOLD>(src, itw_end, lg + FOLD, alpha, i);
-    if (store)
-#pragma unroll
-      for (int k = 0; k < 4; k++) as_global(dst.c[k])[i] = v.v[k];
-    return v;
-  }
-}
+struct FriLayerJob {
+  const uint32_t *src[4];
+  uint32_t *dst;  // a fold's output, coordinates 2^lg words apart
+  uint32_t *tree, *state, *counters;
+  uint32_t root;  // the layer's slot
+};
+struct FriLayerJobs {
+  FriLayerJob j[kFriJobs];
+};
 
 // LEAVES per workgroup (tree_leaves_log): 64 with a quad per leaf, 256, 1,024.
 template <int FOLD, uint32_t LEAVES>
-__global__ void __launch_bounds__(kTreeThreads) fri_layer_kernel(Qm31ColsConst src, Qm31Cols dst,
-                                                                 const uint32_t *itw_end, uint32_t *alpha_dev,
-                                                                 uint32_t lg, uint32_t *tree, uint32_t *chan,
-                                                                 uint32_t *root_out, uint32_t *counters) {
+__global__ void __launch_bounds__(kTreeThreads) fri_layer_kernel(FriLayerJobs jobs, const uint32_t *itw_end,
+                                                                 uint32_t lg) {
   __shared__ __align__(16) TreeLds S;
+  const FriLayerJob &J = jobs.j[blockIdx.y];
+  const Qm31ColsConst src = {{J.src[0], J.src[1], J.src[2], J.src[3]}};
+  uint32_t *dst = J.dst, *tree = J.tree, *counters = J.counters;
+  uint32_t *chan = J.state, *alpha_dev = J.state + kAlphaOff, *root_out = J.state + kRootsOff + 8 * J.root;
   const uint32_t n = 1u << lg, first = blockIdx.x * LEAVES, tid = threadIdx.x;
   const uint32_t q = tid >> 2, j = tid & 3;
   uint32_t *leaves = tree + tree_layer_off(lg);
@@ -474,15 +519,15 @@ __global__ void __launch_bounds__(kTreeThreads) fri_layer_kernel(Qm31ColsConst s
 }
 
 template <int FOLD>
-static int launch_fri_layer(stwo_hip_ctx *ctx, const Qm31ColsConst &src, const Qm31Cols &dst, const uint32_t *itw_end,
-                            uint32_t *alpha, uint32_t lg, uint32_t *tree, uint32_t *chan, uint32_t *root_out) {
+static int launch_fri_layer(stwo_hip_ctx *ctx, const FriLayerJobs &jobs, uint32_t n_jobs, const uint32_t *itw_end,
+                            uint32_t lg) {
   const uint32_t per = tree_leaves_log(lg);
-  const dim3 grid(1u << (lg > per ? lg - per : 0)), block(kTreeThreads);
+  const dim3 grid(1u << (lg > per ? lg - per : 0), n_jobs), block(kTreeThreads);
   return launch(ctx, "fri_layer",
                 per == 6   ? fri_layer_kernel<FOLD, 64>
                 : per == 8 ? fri_layer_kernel<FOLD, 256>
                            : fri_layer_kernel<FOLD, 1024>,
-                grid, block, 0, src, dst, itw_end, alpha, lg, tree, chan, root_out, ctx->d_counters);
+                grid, block, 0, jobs, itw_end, lg);
 }
 
 // chan = [digest, n_draws, 0] (the device channel's starting state).
@@ -491,6 +536,36 @@ struct ChanInit {
 };
 __global__ void chan_init_kernel(ChanInit init, uint32_t *chan) {
   if (threadIdx.x < 10) chan[threadIdx.x] = init.w[threadIdx.x];
+}
+
+// The starting states of a group of commits (blockIdx.x): a fresh channel that
+// has mixed the root at the head of `tree`, kept in the state (the commit's own
+// layers overwrite that tree), and the counters cleared.
+struct ChanInits {
+  struct {
+    uint32_t *state;
+    const uint32_t *tree;
+    uint32_t *counters, n_counters;
+  } c[kFriJobs];
+};
+__global__ void __launch_bounds__(64) chan_inits_kernel(ChanInits init) {
+  const auto &c = init.c[blockIdx.x];
+  const uint32_t tid = threadIdx.x;
+  for (uint32_t k = tid; k < c.n_counters; k += 64) c.counters[k] = 0;
+  if (tid >= 4) return;
+  const b2_quad_iv iv = b2_quad_init();
+  uint32_t m[16], lo = iv.lo, hi = iv.hi;
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    m[k] = 0;
+    m[8 + k] = c.tree[k];
+  }
+  c.state[kMixedOff + tid] = c.tree[tid];
+  c.state[kMixedOff + 4 + tid] = c.tree[4 + tid];
+  b2_compress_quad(iv, lo, hi, m, b2_quad_d(iv, 64, true));
+  c.state[tid] = lo;
+  c.state[4 + tid] = hi;
+  if (tid < 2) c.state[8 + tid] = 0;
 }
 
 // One Fiat-Shamir step of the prove on the device: chan (optionally first
@@ -565,7 +640,6 @@ int prove_channel_step(stwo_hip_ctx *ctx, uint32_t *chan, const uint8_t *init_di
 // The natural-order butterfly i of a line domain of log m uses the inverse x
 // of point i, held at itw_end - 2^m + bitrev_{m-1}(i) (the tree keeps each
 // doubling's x's of the first half in bit-reversed order).
-constexpr uint32_t kDevLastMax = 6;
 struct LastLayerArgs {
   const uint32_t *src[4];
   const uint32_t *itw_end;
@@ -830,10 +904,6 @@ static int check_fri_args(stwo_hip_ctx *ctx, const stwo_hip_fri_config &cfg, uin
   return check_line_domain(ctx, dom, tw);
 }
 
-// FriProver::commit.  With `keep`, every committed layer's tree and every
-// folded evaluation stays in `keep->mem` (laid out by the caller from
-// fri_schedule); without, one scratch tree and two scratch layer buffers
-// are reused.
 // grind: NULL, or (prove) the end of the commit and the proof of work's first
 // search range run on the device when the last layer allows
 // (fri_last_layer_kernel): grind->found then says whether that range held
@@ -843,205 +913,260 @@ struct FriGrind {
   bool found;
   uint64_t nonce;
 };
+// A commit on its way through the layers (FriProver::commit).  With `keep`,
+// every committed layer's tree and every folded evaluation stays in
+// `keep->mem` (laid out by the caller from fri_schedule); without, one scratch
+// tree and two layer buffers are reused, and a last layer of at most
+// 2^kDevLastMax values lies in the state, for one download of both.
+struct FriChain {
+  stwo_hip_fri_config cfg;
+  uint32_t log_size;
+  const uint32_t *column[4];
+  uint32_t *tree, *lay[2], *state, *counters;
+  stwo_hip_fri_prover *keep;
+
+  // The layer to commit next (done: the last layer, not committed): its log,
+  // its evaluation (from cur on, coordinates 2^lg words apart; the first
+  // layer's is `column`) and the fold that writes it from src, if not launched
+  // yet: the circle fold or `pending` line folds.
+  uint32_t lg, last_log, nr, n_folds, line_init, pending;
+  bool first, circle, done;
+  uint32_t *cur;
+  const uint32_t *src[4];
+
+  void start() {
+    last_log = cfg.log_last_layer_degree_bound + cfg.log_blowup_factor;
+    lg = log_size;
+    nr = n_folds = line_init = pending = 0;
+    first = true;
+    circle = done = false;
+    cur = nullptr;
+    for (int k = 0; k < 4; k++) src[k] = column[k];
+  }
+  bool last_in_state() const { return !keep && last_log <= kDevLastMax; }
+  uint32_t *layer_tree() const { return keep ? keep->layers[nr].tree : tree; }
+  // The layer at lg is committed: on to the next (fri.rs:188-262).
+  void next() {
+    const uint32_t step = first ? 1 : std::min(cfg.line_fold_step, lg - last_log);
+    for (int k = 0; k < 4; k++) {
+      src[k] = first ? column[k] : cur + ((size_t)k << lg);
+      if (keep) keep->layers[nr].cols[k] = src[k];
+    }
+    lg -= step;
+    line_init = first ? half_odds_initial(lg) : (uint32_t)(((uint64_t)line_init << step) & IDX_MASK);
+    circle = first;
+    pending = step;
+    first = false;
+    done = lg == last_log;
+    cur = keep                      ? keep->evals[n_folds]
+          : done && last_in_state() ? state + kPolyOff
+                                    : lay[n_folds & 1];
+    n_folds++;
+    nr++;
+  }
+  // The remaining layers are the tail's.
+  bool in_tail() const { return !first && lg <= kTailLog && cfg.line_fold_step <= 4; }
+};
+
+// Launches the pending fold on its own (a line fold of more than 4 steps, or
+// the fold into the last layer when no tail runs).
+static int fri_flush(stwo_hip_ctx *ctx, FriChain &c, const stwo_hip_twiddles *tw) {
+  if (!c.pending) return STWO_HIP_OK;
+  const qm31 unused = qm31_make(0, 0, 0, 0);
+  uint32_t *dst[4];
+  for (int k = 0; k < 4; k++) dst[k] = c.cur + ((size_t)k << c.lg);
+  const uint32_t src_log = c.lg + c.pending, step = c.pending;
+  uint32_t *alpha = c.state + kAlphaOff;
+  int rc = c.circle ? fold_circle(ctx, dst, c.src, src_log, unused, tw, false, alpha)
+                    : fold_line_steps(ctx, c.src, src_log, unused, step, tw, dst, alpha, c.state + kAlphaTmpOff);
+  c.pending = 0;
+  for (int k = 0; k < 4; k++) c.src[k] = dst[k];
+  return rc;
+}
+
+// Runs the chains (each with its channel in its state) up to their last layers:
+// on the stream, without host round trips.  After each
+// layer's Merkle commit, the kernel that hashes its root (fri_layer_kernel
+// or the tail) mixes the root into the device copy of the channel and
+// draws the next alpha, which the folds read from device memory.
+//
+// A chain is a row of dependent launches that leave the device nearly idle, so
+// chains that stand at the same layer size share theirs (the larger ones begin
+// alone): 12 commits of 2^14 to 2^19 one after another took 2.6 ms of
+// device time, side by side they take 0.5 ms.
+static int fri_run(stwo_hip_ctx *ctx, FriChain *const *chains, size_t n, const stwo_hip_twiddles *tw) {
+  const uint32_t *itw_end = tw->d_itw + tw->len;
+  int rc;
+  for (;;) {
+    FriChain *lead = nullptr;
+    for (size_t i = 0; i < n; i++) {
+      FriChain *c = chains[i];
+      if (!c->done && !c->in_tail() && (!lead || c->lg > lead->lg)) lead = c;
+    }
+    if (!lead) break;
+    auto kind = [](const FriChain &c) { return c.circle && c.pending ? kFoldCircle : (int)c.pending; };
+    if (lead->pending > 4) {
+      rc = fri_flush(ctx, *lead, tw);
+      if (rc) return rc;
+    }
+    const int fold = kind(*lead);
+    const uint32_t lg = lead->lg;
+    FriLayerJobs jobs{};
+    uint32_t nj = 0;
+    for (size_t i = 0; i < n && nj < kFriJobs; i++) {
+      FriChain &c = *chains[i];
+      if (c.done || c.in_tail() || c.lg != lg || kind(c) != fold) continue;
+      if (c.nr >= kMaxRoots || (c.keep && c.nr >= c.keep->layers.size()))
+        return set_error(ctx, STWO_HIP_EINVAL, "internal: FRI layer overflow");
+      FriLayerJob &j = jobs.j[nj++];
+      for (int k = 0; k < 4; k++) j.src[k] = c.src[k];
+      j.dst = c.cur;
+      j.tree = c.layer_tree();
+      j.state = c.state;
+      j.counters = c.counters;
+      j.root = c.nr;
+      c.next();
+    }
+    switch (fold) {
+      case 0: rc = launch_fri_layer<0>(ctx, jobs, nj, itw_end, lg); break;
+      case 1: rc = launch_fri_layer<1>(ctx, jobs, nj, itw_end, lg); break;
+      case 2: rc = launch_fri_layer<2>(ctx, jobs, nj, itw_end, lg); break;
+      case 3: rc = launch_fri_layer<3>(ctx, jobs, nj, itw_end, lg); break;
+      case 4: rc = launch_fri_layer<4>(ctx, jobs, nj, itw_end, lg); break;
+      default: rc = launch_fri_layer<kFoldCircle>(ctx, jobs, nj, itw_end, lg); break;
+    }
+    if (rc) return rc;
+  }
+  // Every remaining inner layer of a chain (at most kTailLog of them) in one workgroup.
+  std::vector<FriTail> tails;
+  for (size_t i = 0; i < n; i++) {
+    FriChain &c = *chains[i];
+    if (c.done) {
+      rc = fri_flush(ctx, c, tw);
+      if (rc) return rc;
+      continue;
+    }
+    tails.emplace_back();
+    FriTail &t = tails.back();
+    memset(&t, 0, sizeof(t));
+    for (int k = 0; k < 4; k++) t.src.c[k] = c.src[k];
+    t.first = c.cur;
+    t.fold = c.circle ? kFoldCircle : c.pending;
+    t.root = c.nr;
+    t.itw_end = itw_end;
+    t.state = c.state;
+    while (!c.done) {
+      if (t.n >= kTailMax || c.nr >= kMaxRoots || (c.keep && c.nr >= c.keep->layers.size()))
+        return set_error(ctx, STWO_HIP_EINVAL, "internal: FRI tail overflow");
+      FriTailLayer &L = t.l[t.n++];
+      L.lg = c.lg;
+      L.tree = c.layer_tree();
+      c.next();
+      L.step = c.pending;
+      L.dst = c.cur;
+    }
+    c.pending = 0;
+  }
+  if (tails.empty()) return STWO_HIP_OK;
+  if (tails.size() == 1)
+    return launch(ctx, "fri_tail", fri_tail_kernel, dim3(1), dim3(kTreeThreads), 0, tails[0]);
+  void *d_tails = nullptr;
+  rc = upload_table(ctx, tails.data(), tails.size() * sizeof(FriTail), &d_tails);
+  if (rc) return rc;
+  return launch(ctx, "fri_tail", fri_tails_kernel, dim3((uint32_t)tails.size()), dim3(kTreeThreads), 0,
+                (const FriTail *)d_tails);
+}
+
+// The end of a commit on the host, from the downloaded state and the last
+// layer's evaluation (4 coordinates of 2^lg words): fri.rs:274-291.
+static int fri_finish(stwo_hip_ctx *ctx, const FriChain &c, const uint32_t *st, const uint32_t *h,
+                      uint8_t channel_digest[32], uint32_t *channel_n_draws, uint32_t *roots, uint32_t *n_roots,
+                      uint32_t *last_layer_poly) {
+  if (st[9]) return set_error(ctx, STWO_HIP_EDEVICE, "fri_commit: channel draw did not terminate");
+  memcpy(roots, st + kRootsOff, 32 * c.nr);
+  HostChannel ch;
+  memcpy(ch.digest, st, 32);
+  ch.n_draws = st[8];
+  const size_t n = (size_t)1 << c.lg;
+  std::vector<qm31> vals(n);
+  for (size_t i = 0; i < n; i++) vals[i] = qm31_make(h[i], h[n + i], h[2 * n + i], h[3 * n + i]);
+  host_line_interpolate(vals, c.line_init, c.lg);
+  // into_ordered_coefficients: bit reverse (line.rs:157-160)
+  for (size_t i = 0; i < n; i++) {
+    size_t j = bitrev32((uint32_t)i, c.lg);
+    if (j > i) std::swap(vals[i], vals[j]);
+  }
+  size_t bound = (size_t)1 << c.cfg.log_last_layer_degree_bound;
+  for (size_t i = bound; i < n; i++)
+    for (int k = 0; k < 4; k++)
+      if (vals[i].v[k]) return set_error(ctx, STWO_HIP_EDEGREE, "invalid degree");
+  // from_ordered_coefficients bit-reverses the kept coefficients (line.rs:167-170)
+  for (size_t i = 0; i < bound; i++) {
+    size_t j = bitrev32((uint32_t)i, c.cfg.log_last_layer_degree_bound);
+    for (int k = 0; k < 4; k++) last_layer_poly[4 * j + k] = vals[i].v[k];
+  }
+  ch.mix_felts(last_layer_poly, bound);
+  memcpy(channel_digest, ch.digest, 32);
+  *channel_n_draws = ch.n_draws;
+  *n_roots = c.nr;
+  return STWO_HIP_OK;
+}
+
 static int fri_commit_impl(stwo_hip_ctx *ctx, uint8_t channel_digest[32], uint32_t *channel_n_draws,
                            const stwo_hip_fri_config &cfg, const uint32_t *const column[4], uint32_t log_size,
                            const stwo_hip_twiddles *tw, uint32_t *roots, uint32_t *n_roots, uint32_t *last_layer_poly,
                            stwo_hip_fri_prover *keep, FriGrind *grind = nullptr) {
   int rc = check_fri_args(ctx, cfg, log_size, tw);
   if (rc) return rc;
-  const uint32_t last_log = cfg.log_last_layer_degree_bound + cfg.log_blowup_factor;
-  const std::vector<FriLayerShape> sched = fri_schedule(cfg, log_size);
-  if (keep && keep->layers.size() != sched.size())
+  if (keep && keep->layers.size() != fri_schedule(cfg, log_size).size())
     return set_error(ctx, STWO_HIP_EINVAL, "internal: FRI prover storage does not match the schedule");
-  // The layer loop runs on the stream without host round trips: after each
-  // layer's Merkle commit, the kernel that hashes its root (fri_layer_kernel
-  // or the tail) mixes the root into the device copy of the channel and
-  // draws the next alpha, which the folds read from device memory.  The host reads the roots, the channel
-  // and the last layer once, at the end.
-  constexpr uint32_t kMaxRoots = 32;
-  // chan[0..10) | alpha[10..14) | alpha_tmp[14..18) | pad | roots[32 ..)
-  constexpr uint32_t kRootsOff = 32;
-  // One root per layer and at most log_size layers (log_size <= 28).
-  static_assert(kMaxRoots >= 28, "root slots");
-  void *tree_p = nullptr, *lay_a = nullptr, *lay_b = nullptr, *state_p = nullptr;
+  FriChain c{};
+  c.cfg = cfg;
+  c.log_size = log_size;
+  c.keep = keep;
+  c.counters = ctx->d_counters;
+  for (int k = 0; k < 4; k++) c.column[k] = column[k];
+  void *p = nullptr;
   if (!keep) {
-    rc = get_scratch(ctx, "fri_tree", layer_off(log_size + 1) * 4, &tree_p);
+    rc = get_scratch(ctx, "fri_tree", layer_off(log_size + 1) * 4, &p);
     if (rc) return rc;
-    rc = get_scratch(ctx, "fri_layer_a", ((size_t)4 << (log_size - 1)) * 4, &lay_a);
-    if (rc) return rc;
-    rc = get_scratch(ctx, "fri_layer_b", ((size_t)4 << (log_size - 1)) * 4, &lay_b);
-    if (rc) return rc;
+    c.tree = (uint32_t *)p;
+    for (int k = 0; k < 2; k++) {
+      rc = get_scratch(ctx, k ? "fri_layer_b" : "fri_layer_a", ((size_t)4 << (log_size - 1)) * 4, &p);
+      if (rc) return rc;
+      c.lay[k] = (uint32_t *)p;
+    }
   }
-  // then flags[kFlagsOff], the grind's best nonce (8-byte aligned), the
-  // grind prefix and the last layer's coefficients (device end only)
-  constexpr uint32_t kFlagsOff = kRootsOff + 8 * kMaxRoots, kBestOff = kFlagsOff + 2, kPrefixOff = kBestOff + 2,
-                     kPolyOff = kPrefixOff + 8;
-  static_assert(kBestOff % 2 == 0, "best nonce alignment");
-  rc = get_scratch(ctx, "fri_state", (kPolyOff + (4u << kDevLastMax)) * 4, &state_p);
+  rc = get_scratch(ctx, "fri_state", kFriStateWords * 4, &p);
   if (rc) return rc;
-  uint32_t *scratch_tree = (uint32_t *)tree_p;
-  uint32_t *state = (uint32_t *)state_p;
-  uint32_t *d_chan = state, *d_alpha = state + 10, *d_alpha_tmp = state + 14, *d_roots = state + kRootsOff;
+  uint32_t *state = c.state = (uint32_t *)p;
   {
     // set by a launch, in stream order: no synchronization
     ChanInit init{};
     memcpy(init.w, channel_digest, 32);
     init.w[8] = *channel_n_draws;
     init.w[9] = 0;
-    rc = launch(ctx, "fri_chan_init", chan_init_kernel, dim3(1), dim3(64), 0, init, d_chan);
+    rc = launch(ctx, "fri_chan_init", chan_init_kernel, dim3(1), dim3(64), 0, init, state);
     if (rc) return rc;
   }
-  uint32_t nr = 0;
-
-  // A fold not launched yet: the circle fold after the first layer or a line
-  // fold of `step` steps.  The next layer's commit runs it in its own launch
-  // (fri_layer_kernel) when the step is at most 4; otherwise, and before the
-  // tail or the end, it runs on its own.
-  struct PendingFold {
-    bool on, circle;
-    uint32_t step, src_log;
-    const uint32_t *src[4];
-    uint32_t *dst[4];
-  } pend{};
-  const qm31 unused = qm31_make(0, 0, 0, 0);
-  auto flush = [&]() -> int {
-    if (!pend.on) return STWO_HIP_OK;
-    pend.on = false;
-    if (pend.circle) return fold_circle(ctx, pend.dst, pend.src, pend.src_log, unused, tw, false, d_alpha);
-    return fold_line_steps(ctx, pend.src, pend.src_log, unused, pend.step, tw, pend.dst, d_alpha, d_alpha_tmp);
-  };
-
-  // Commits the layer `cols` of log lg (running the pending fold that writes
-  // it, if it fuses), then mixes its root into the channel and draws alpha.
-  auto commit_layer = [&](const uint32_t *const cols[4], uint32_t lg) -> int {
-    if (keep && nr >= keep->layers.size()) return set_error(ctx, STWO_HIP_EINVAL, "internal: FRI layer overflow");
-    uint32_t *tree = keep ? keep->layers[nr].tree : scratch_tree;
-    if (keep)
-      for (int k = 0; k < 4; k++) keep->layers[nr].cols[k] = cols[k];
-    Qm31ColsConst src;
-    Qm31Cols dst{};
-    int fold = 0;
-    if (pend.on && (pend.circle || pend.step <= 4)) {
-      fold = pend.circle ? kFoldCircle : (int)pend.step;
-      for (int k = 0; k < 4; k++) {
-        src.c[k] = pend.src[k];
-        dst.c[k] = pend.dst[k];
-      }
-      pend.on = false;
-    } else {
-      int r = flush();
-      if (r) return r;
-      for (int k = 0; k < 4; k++) src.c[k] = cols[k];
-    }
-    const uint32_t *itw_end = tw->d_itw + tw->len;
-    uint32_t *root_out = d_roots + 8 * nr;
-    int r;
-    switch (fold) {
-      case 0: r = launch_fri_layer<0>(ctx, src, dst, itw_end, d_alpha, lg, tree, d_chan, root_out); break;
-      case 1: r = launch_fri_layer<1>(ctx, src, dst, itw_end, d_alpha, lg, tree, d_chan, root_out); break;
-      case 2: r = launch_fri_layer<2>(ctx, src, dst, itw_end, d_alpha, lg, tree, d_chan, root_out); break;
-      case 3: r = launch_fri_layer<3>(ctx, src, dst, itw_end, d_alpha, lg, tree, d_chan, root_out); break;
-      case 4: r = launch_fri_layer<4>(ctx, src, dst, itw_end, d_alpha, lg, tree, d_chan, root_out); break;
-      default: r = launch_fri_layer<kFoldCircle>(ctx, src, dst, itw_end, d_alpha, lg, tree, d_chan, root_out); break;
-    }
-    if (r) return r;
-    nr++;
-    return STWO_HIP_OK;
-  };
-
-  // First layer (fri.rs:176-183, 360-369).
-  rc = commit_layer(column, log_size);
+  c.start();
+  FriChain *chain = &c;
+  rc = fri_run(ctx, &chain, 1, tw);
   if (rc) return rc;
-  // Inner layers (fri.rs:188-262).
-  uint32_t lg = log_size - 1;
-  uint32_t line_init = half_odds_initial(lg);
-  uint32_t *bufs[2] = {(uint32_t *)lay_a, (uint32_t *)lay_b};
-  uint32_t *cur[4];
-  // Evaluation buffer of the layer of log `l` that fold number `f` writes.
-  auto layer_buf = [&](int f, uint32_t l, int k) -> uint32_t * {
-    return keep ? keep->evals[f] + ((size_t)k << l) : bufs[f & 1] + ((size_t)k << l);
-  };
-  for (int k = 0; k < 4; k++) cur[k] = layer_buf(0, lg, k);
-  int n_folds = 1;
-  pend.on = true;
-  pend.circle = true;
-  pend.step = 1;
-  pend.src_log = log_size;
-  for (int k = 0; k < 4; k++) {
-    pend.src[k] = column[k];
-    pend.dst[k] = cur[k];
-  }
-  if (lg != last_log) {
-    for (;;) {
-      bool last = !(lg > last_log + cfg.line_fold_step);
-      uint32_t step = last ? lg - last_log : cfg.line_fold_step;
-      if (lg <= kTailLog && cfg.line_fold_step <= 4) {
-        rc = flush();
-        if (rc) return rc;
-        // Every remaining inner layer (at most kTailLog of them) in one launch.
-        FriTail t{};
-        t.itw_end = tw->d_itw + tw->len;
-        t.chan = d_chan;
-        t.roots = d_roots;
-        t.alpha = d_alpha;
-        for (int k = 0; k < 4; k++) t.src[k] = cur[k];
-        for (;;) {
-          last = !(lg > last_log + cfg.line_fold_step);
-          step = last ? lg - last_log : cfg.line_fold_step;
-          if (t.n >= kTailMax || (keep && nr >= keep->layers.size()))
-            return set_error(ctx, STWO_HIP_EINVAL, "internal: FRI tail overflow");
-          FriTailLayer &L = t.l[t.n++];
-          L.tree = keep ? keep->layers[nr].tree : scratch_tree;
-          for (int k = 0; k < 4; k++) {
-            if (keep) keep->layers[nr].cols[k] = cur[k];
-            L.dst[k] = layer_buf(n_folds, lg - step, k);
-            cur[k] = L.dst[k];
-          }
-          L.lg = lg;
-          L.step = step;
-          L.root_slot = nr++;
-          n_folds++;
-          line_init = (uint32_t)(((uint64_t)line_init << step) & IDX_MASK);
-          lg -= step;
-          if (last) break;
-        }
-        rc = launch(ctx, "fri_tail", fri_tail_kernel, dim3(1), dim3(kTreeThreads), 0, t);
-        if (rc) return rc;
-        break;
-      }
-      rc = commit_layer(cur, lg);
-      if (rc) return rc;
-      pend.on = true;
-      pend.circle = false;
-      pend.step = step;
-      pend.src_log = lg;
-      for (int k = 0; k < 4; k++) {
-        pend.src[k] = cur[k];
-        pend.dst[k] = layer_buf(n_folds, lg - step, k);
-        cur[k] = pend.dst[k];
-      }
-      n_folds++;
-      line_init = (uint32_t)(((uint64_t)line_init << step) & IDX_MASK);
-      lg -= step;
-      if (last) break;
-    }
-  }
-  // The fold into the last layer when no tail ran (or the circle fold alone).
-  rc = flush();
-  if (rc) return rc;
+  const uint32_t nr = c.nr, lg = c.lg;
   if (grind) grind->found = false;
   if (grind && lg <= kDevLastMax && grind->pow_bits + 6 < 20) {
     // The last layer, the channel mix and the grind's first range on the
     // device, then one synchronization.
     const uint32_t bound_log = cfg.log_last_layer_degree_bound;
     LastLayerArgs la{};
-    for (int k = 0; k < 4; k++) la.src[k] = cur[k];
+    for (int k = 0; k < 4; k++) la.src[k] = c.cur + ((size_t)k << lg);
     la.itw_end = tw->d_itw + tw->len;
     la.lg = lg;
     la.bound_log = bound_log;
     la.pow_bits = grind->pow_bits;
     la.n_inv = m31_inv((uint32_t)(((uint64_t)1 << lg) % P));
-    la.chan = d_chan;
+    la.chan = state;
     la.poly = state + kPolyOff;
     la.prefixed = state + kPrefixOff;
     la.flags = state + kFlagsOff;
@@ -1058,7 +1183,6 @@ static int fri_commit_impl(stwo_hip_ctx *ctx, uint8_t channel_digest[32], uint32
       if (rc) return rc;
     }
     if (st[9]) return set_error(ctx, STWO_HIP_EDEVICE, "fri_commit: channel draw did not terminate");
-    if (nr != sched.size()) return set_error(ctx, STWO_HIP_EDEVICE, "internal: FRI schedule mismatch");
     if (st[kFlagsOff]) return set_error(ctx, STWO_HIP_EDEGREE, "invalid degree");
     memcpy(roots, st.data() + kRootsOff, 32 * nr);
     if (keep)
@@ -1076,57 +1200,90 @@ static int fri_commit_impl(stwo_hip_ctx *ctx, uint8_t channel_digest[32], uint32
     if (keep) {
       keep->last_layer_poly.assign(last_layer_poly, last_layer_poly + 4 * bound);
       keep->last_log = lg;
-      for (int k = 0; k < 4; k++) keep->last_layer_eval[k] = cur[k];
+      for (int k = 0; k < 4; k++) keep->last_layer_eval[k] = c.cur + ((size_t)k << lg);
     }
     return STWO_HIP_OK;
   }
   // One synchronization for the channel state, the roots and the last layer.
-  std::vector<uint32_t> st(kRootsOff + 8 * nr);
-  size_t n = (size_t)1 << lg;
-  std::vector<uint32_t> h(4 * n);
+  std::vector<uint32_t> st(kPolyOff + ((size_t)4 << lg));
   {
-    const DownloadReq reqs[5] = {{st.data(), state, st.size()},
-                                 {h.data(), cur[0], n},
-                                 {h.data() + n, cur[1], n},
-                                 {h.data() + 2 * n, cur[2], n},
-                                 {h.data() + 3 * n, cur[3], n}};
-    rc = download_many(ctx, reqs, 5);
+    const bool one = c.last_in_state();
+    const DownloadReq reqs[2] = {{st.data(), state, one ? st.size() : kRootsOff + 8 * nr},
+                                 {st.data() + kPolyOff, c.cur, (size_t)4 << lg}};
+    rc = download_many(ctx, reqs, one ? 1 : 2);
     if (rc) return rc;
   }
-  if (st[9]) return set_error(ctx, STWO_HIP_EDEVICE, "fri_commit: channel draw did not terminate");
-  if (nr != sched.size()) return set_error(ctx, STWO_HIP_EDEVICE, "internal: FRI schedule mismatch");
-  memcpy(roots, st.data() + kRootsOff, 32 * nr);
-  if (keep)
-    for (uint32_t k = 0; k < nr; k++) memcpy(keep->layers[k].root, roots + 8 * k, 32);
-  HostChannel ch;
-  memcpy(ch.digest, st.data(), 32);
-  ch.n_draws = st[8];
-  // Last layer (fri.rs:274-291).
-  std::vector<qm31> vals(n);
-  for (size_t i = 0; i < n; i++) vals[i] = qm31_make(h[i], h[n + i], h[2 * n + i], h[3 * n + i]);
-  host_line_interpolate(vals, line_init, lg);
-  // into_ordered_coefficients: bit reverse (line.rs:157-160)
-  for (size_t i = 0; i < n; i++) {
-    size_t j = bitrev32((uint32_t)i, lg);
-    if (j > i) std::swap(vals[i], vals[j]);
-  }
-  size_t bound = (size_t)1 << cfg.log_last_layer_degree_bound;
-  for (size_t i = bound; i < n; i++)
-    for (int k = 0; k < 4; k++)
-      if (vals[i].v[k]) return set_error(ctx, STWO_HIP_EDEGREE, "invalid degree");
-  // from_ordered_coefficients bit-reverses the kept coefficients (line.rs:167-170)
-  for (size_t i = 0; i < bound; i++) {
-    size_t j = bitrev32((uint32_t)i, cfg.log_last_layer_degree_bound);
-    for (int k = 0; k < 4; k++) last_layer_poly[4 * j + k] = vals[i].v[k];
-  }
-  ch.mix_felts(last_layer_poly, bound);
-  memcpy(channel_digest, ch.digest, 32);
-  *channel_n_draws = ch.n_draws;
-  *n_roots = nr;
+  rc = fri_finish(ctx, c, st.data(), st.data() + kPolyOff, channel_digest, channel_n_draws, roots, n_roots,
+                  last_layer_poly);
+  if (rc) return rc;
   if (keep) {
-    keep->last_layer_poly.assign(last_layer_poly, last_layer_poly + 4 * bound);
+    for (uint32_t k = 0; k < nr; k++) memcpy(keep->layers[k].root, roots + 8 * k, 32);
+    keep->last_layer_poly.assign(last_layer_poly, last_layer_poly + ((size_t)4 << cfg.log_last_layer_degree_bound));
     keep->last_log = lg;
-    for (int k = 0; k < 4; k++) keep->last_layer_eval[k] = cur[k];
+    for (int k = 0; k < 4; k++) keep->last_layer_eval[k] = c.cur + ((size_t)k << lg);
+  }
+  return STWO_HIP_OK;
+}
+
+size_t fri_job_words(uint32_t log_size) { return kFriStateWords + tree_counters(log_size); }
+
+int fri_commit_jobs(stwo_hip_ctx *ctx, FriJob *jobs, size_t n, const stwo_hip_twiddles *tw, uint32_t *mem) {
+  int rc;
+  std::vector<FriChain> chains(n);
+  std::vector<FriChain *> order(n);
+  // the states, then every job's counters
+  uint32_t *counters = mem + n * kFriStateWords;
+  ChanInits init{};
+  uint32_t ni = 0;
+  auto send = [&]() {
+    const int r = launch(ctx, "fri_chan_init", chan_inits_kernel, dim3(ni), dim3(64), 0, init);
+    ni = 0;
+    return r;
+  };
+  for (size_t i = 0; i < n; i++) {
+    FriJob &j = jobs[i];
+    rc = check_fri_args(ctx, j.cfg, j.log_size, tw);
+    if (rc) return rc;
+    FriChain &c = chains[i];
+    c = FriChain{};
+    c.cfg = j.cfg;
+    c.log_size = j.log_size;
+    for (int k = 0; k < 4; k++) c.column[k] = j.column[k];
+    c.tree = j.tree;
+    c.lay[0] = j.layers;
+    c.lay[1] = j.layers + ((size_t)4 << (j.log_size - 1));
+    c.state = mem + i * kFriStateWords;
+    c.counters = counters;
+    init.c[ni++] = {c.state, j.tree, counters, tree_counters(j.log_size)};
+    counters += tree_counters(j.log_size);
+    c.start();
+    order[i] = &c;
+    if (ni == kFriJobs || i + 1 == n) {
+      rc = send();
+      if (rc) return rc;
+    }
+  }
+  rc = fri_run(ctx, order.data(), n, tw);
+  if (rc) return rc;
+  // One download of the states, with the last layers of the usual sizes in them.
+  std::vector<uint32_t> st(n * kFriStateWords);
+  std::vector<std::vector<uint32_t>> big(n);
+  std::vector<DownloadReq> reqs = {{st.data(), mem, st.size()}};
+  for (size_t i = 0; i < n; i++) {
+    const FriChain &c = chains[i];
+    if (c.last_in_state()) continue;
+    big[i].resize((size_t)4 << c.lg);
+    reqs.push_back({big[i].data(), c.cur, big[i].size()});
+  }
+  rc = download_many(ctx, reqs.data(), reqs.size());
+  if (rc) return rc;
+  for (size_t i = 0; i < n; i++) {
+    const uint32_t *s = st.data() + i * kFriStateWords;
+    memcpy(jobs[i].mixed_root, s + kMixedOff, 32);
+    uint32_t n_draws = 0;
+    rc = fri_finish(ctx, chains[i], s, big[i].empty() ? s + kPolyOff : big[i].data(), jobs[i].digest, &n_draws,
+                    jobs[i].roots, &jobs[i].n_roots, jobs[i].last_layer_poly);
+    if (rc) return rc;
   }
   return STWO_HIP_OK;
 }

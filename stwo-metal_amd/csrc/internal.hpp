@@ -218,6 +218,24 @@ struct stwo_hip_fri_prover {
 
 namespace stwo_hip {
 
+// FriProver::commit of several evaluations side by side, each on a fresh channel
+// that first mixes the root at the head of `tree`: the server's commit jobs.
+// tree: then the scratch of the layers' trees (2^(log_size + 1) - 1 hashes);
+// layers: the folded evaluations (3 << log_size words).
+struct FriJob {
+  stwo_hip_fri_config cfg;
+  uint32_t log_size;
+  const uint32_t *column[4];
+  uint32_t *tree, *layers;
+  // results
+  uint32_t mixed_root[8];
+  uint8_t digest[32];
+  uint32_t *roots, n_roots, *last_layer_poly;
+};
+// mem: the jobs' fri_job_words each.
+size_t fri_job_words(uint32_t log_size);
+int fri_commit_jobs(stwo_hip_ctx *ctx, FriJob *jobs, size_t n, const stwo_hip_twiddles *tw, uint32_t *mem);
+
 // stwo_hip_fri_prover_commit whose memory is the context's scratch buffer
 // `scratch_key` (kept by the context, reused by the next call with the same
 // key) when scratch_key is not NULL.  One such prover per key at a time.

@@ -16,10 +16,10 @@
 // memory; ONE batched plan interpolates, evaluates and commits every job's
 // columns -- columns of equal size and blowup from all jobs share each FFT
 // pass launch -- into one lifted Blake2s tree per job (the PCS form,
-// CommitmentTreeProver::new, STWO/prover/pcs/mod.rs:766-803); then per job
-// the trace root is mixed into a fresh Blake2s channel and FRI commits the
+// CommitmentTreeProver::new, STWO/prover/pcs/mod.rs:766-803); then each job's
+// trace root is mixed into a fresh Blake2s channel and FRI commits the
 // QM31 column formed by its first four evaluations (FriProver::commit,
-// STWO/prover/fri.rs:133-291).  A prove group runs stwo_hip_wide_fib_prove.
+// STWO/prover/fri.rs:133-291), the jobs' layers of equal size sharing a launch.  A prove group runs stwo_hip_wide_fib_prove.
 // While a group runs, every device buffer the library takes for itself
 // (plan tables, FRI trees, prove buffers) is carved from the group's block
 // (job_mem_begin).  Results depend only on the job: each has its own
@@ -115,21 +115,21 @@ struct Group {
 inline size_t words_tree(uint32_t max_log) { return (((size_t)2 << max_log) - 1) * 8; }
 inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// A commit job's own data: columns, evaluations, tree.
+// A commit job's own data: columns, evaluations, tree and FRI state.  Once the
+// evaluations are committed the rest is the FRI commit's: its folded evaluations
+// lie over the columns (3 << L words), its trees over the trace's.
+size_t commit_cols_bytes(const stwo_hip_job_desc &d) {
+  const uint32_t L = d.log_size + d.log_blowup;
+  return align256(std::max((size_t)d.n_cols << d.log_size, (size_t)3 << L) * 4);
+}
 size_t commit_data_bytes(const stwo_hip_job_desc &d) {
   const uint32_t L = d.log_size + d.log_blowup;
-  return align256(((size_t)d.n_cols << d.log_size) * 4) + align256(((size_t)d.n_cols << L) * 4) +
-         align256(words_tree(L) * 4);
-}
-// FriProver::commit's scratch for a first layer of 2^L (fri_commit_impl:
-// tree, two layer buffers, channel state).
-size_t fri_scratch_bytes(uint32_t L) {
-  return align256(words_tree(L) * 4) + 2 * align256(((size_t)4 << (L - 1)) * 4) + align256((32 + 8 * 32) * 4);
+  return commit_cols_bytes(d) + align256(((size_t)d.n_cols << L) * 4) + align256(words_tree(L) * 4) +
+         fri_job_words(L) * 4;
 }
 // Device bytes of a group: every commit job's data, the batched plan's
-// tables (column tables and pass descriptors), the largest FRI scratch (the
-// FRI commits run largest first, so later ones reuse it); a prove job's
-// buffers and its seeded inputs.
+// tables (column tables and pass descriptors); a prove job's buffers and its
+// seeded inputs.
 size_t group_bytes(const std::vector<const stwo_hip_job_desc *> &g) {
   if (g.size() == 1 && g[0]->kind == STWO_HIP_JOB_PROVE) {
     const stwo_hip_job_desc &d = *g[0];
@@ -137,14 +137,11 @@ size_t group_bytes(const std::vector<const stwo_hip_job_desc *> &g) {
            ((size_t)1 << 20);
   }
   size_t b = 0, cols = 0;
-  uint32_t max_L = 0;
   for (const stwo_hip_job_desc *d : g) {
     b += commit_data_bytes(*d);
     cols += d->n_cols;
-    max_L = std::max(max_L, d->log_size + d->log_blowup);
   }
-  b += (size_t)256 * 1024 + 128 * cols;  // plan tables and descriptors
-  b += fri_scratch_bytes(max_L) + (size_t)64 * 1024;
+  b += (size_t)320 * 1024 + 128 * cols;  // plan tables and descriptors
   return align256(b);
 }
 
@@ -203,88 +200,156 @@ int check_job(const stwo_hip_server *s, const stwo_hip_job_desc &d) {
   return STWO_HIP_OK;
 }
 
+// The callers' device columns of a group into its memory, one launch: a copy
+// call per column costs the stream 1.9 us, 1.2 of 5.2 ms for 624 columns of 2^12
+// to 2^17; this moves them in 13 us (bound by memory).  16 bytes a lane where
+// the column is aligned to that.
+struct ColCopy {
+  const uint32_t *src;
+  uint32_t *dst;
+  size_t words;  // 2^log >= 16
+};
+constexpr uint32_t kCopyWords = 8192;  // per workgroup
+__global__ void __launch_bounds__(256) copy_columns_kernel(const ColCopy *cols) {
+  const ColCopy c = cols[blockIdx.y];
+  const size_t first = (size_t)blockIdx.x * kCopyWords;
+  if (first >= c.words) return;
+  const size_t end = c.words - first < kCopyWords ? c.words : first + kCopyWords;
+  if (((uintptr_t)c.src & 15) == 0) {
+    for (size_t i = first + 4 * threadIdx.x; i < end; i += 4 * 256)
+      *reinterpret_cast<uint4 *>(c.dst + i) = *reinterpret_cast<const uint4 *>(c.src + i);
+  } else {
+    for (size_t i = first + threadIdx.x; i < end; i += 256) c.dst[i] = c.src[i];
+  }
+}
+
+// Whether a kernel of this device may read [p, p + bytes): whole words of one
+// allocation on it.  Neighbouring columns mostly share theirs, so the last
+// allocation found is tried first.
+struct DeviceRange {
+  uintptr_t base = 0, end = 0;
+  bool readable(int device, const void *p, size_t bytes) {
+    const uintptr_t b = (uintptr_t)p;
+    if (b & 3) return false;
+    if (b >= base && b < end) return bytes <= end - b;
+    hipDeviceptr_t at = nullptr;
+    size_t size = 0;
+    hipPointerAttribute_t attr;
+    if (hipMemGetAddressRange(&at, &size, (hipDeviceptr_t)p) != hipSuccess ||
+        hipPointerGetAttributes(&attr, p) != hipSuccess || attr.type != hipMemoryTypeDevice ||
+        attr.device != device) {
+      (void)hipGetLastError();
+      return false;
+    }
+    base = (uintptr_t)at;
+    end = base + size;
+    return b >= base && b < end && bytes <= end - b;
+  }
+};
+
 // Columns of a job into `dst` (n_cols x 2^log_size): the caller's device
-// columns, its host data, or the seed.
-int load_columns(stwo_hip_ctx *ctx, const stwo_hip_job_desc &d, uint32_t n_cols, uint32_t *dst) {
+// columns (by `copies` where a kernel may read them), its host data, or the seed.
+int load_columns(stwo_hip_ctx *ctx, const stwo_hip_job_desc &d, uint32_t n_cols, uint32_t *dst, DeviceRange &range,
+                 std::vector<ColCopy> &copies) {
   const size_t n = (size_t)1 << d.log_size;
+  if (!d.cols && d.host) {
+    STWO_HIP_TRY(ctx, hipMemcpyAsync(dst, d.host, n_cols * n * 4, hipMemcpyHostToDevice, ctx->stream));
+    return STWO_HIP_OK;
+  }
   for (uint32_t c = 0; c < n_cols; c++) {
     uint32_t *col = dst + c * n;
-    if (d.cols) {
-      STWO_HIP_CHECK_ARG(ctx, d.cols[c], "job column %u is NULL", c);
-      STWO_HIP_TRY(ctx, hipMemcpyAsync(col, d.cols[c], n * 4, hipMemcpyDeviceToDevice, ctx->stream));
-    } else if (d.host) {
-      STWO_HIP_TRY(ctx, hipMemcpyAsync(col, d.host + c * n, n * 4, hipMemcpyHostToDevice, ctx->stream));
-    } else {
+    if (!d.cols) {
       int rc = stwo_hip_fill_random(ctx, col, n, d.seed, c);
       if (rc) return rc;
+      continue;
     }
+    STWO_HIP_CHECK_ARG(ctx, d.cols[c], "job column %u is NULL", c);
+    if (range.readable(ctx->device, d.cols[c], n * 4))
+      copies.push_back({d.cols[c], col, n});
+    else
+      STWO_HIP_TRY(ctx, hipMemcpyAsync(col, d.cols[c], n * 4, hipMemcpyDeviceToDevice, ctx->stream));
+  }
+  return STWO_HIP_OK;
+}
+
+int copy_columns(stwo_hip_ctx *ctx, const std::vector<ColCopy> &copies) {
+  constexpr size_t kMaxRows = 4096;  // columns per launch: a table within the upload ring
+  for (size_t at = 0; at < copies.size(); at += kMaxRows) {
+    const size_t rows = std::min(kMaxRows, copies.size() - at);
+    size_t words = 0;
+    for (size_t k = 0; k < rows; k++) words = std::max(words, copies[at + k].words);
+    void *table = nullptr;
+    int rc = upload_table(ctx, copies.data() + at, rows * sizeof(ColCopy), &table);
+    if (rc) return rc;
+    rc = launch(ctx, "copy_columns", copy_columns_kernel,
+                dim3((uint32_t)((words + kCopyWords - 1) / kCopyWords), (uint32_t)rows), dim3(256), 0,
+                (const ColCopy *)table);
+    if (rc) return rc;
   }
   return STWO_HIP_OK;
 }
 
 int run_commit_group(stwo_hip_server *s, stwo_hip_ctx *ctx, Group &g) {
   uint8_t *p = g.mem;
-  std::vector<std::vector<uint32_t *>> cols(g.jobs.size()), outs(g.jobs.size());
-  std::vector<std::vector<uint32_t>> logs(g.jobs.size());
-  std::vector<uint32_t *> trees(g.jobs.size());
-  std::vector<BatchTree> sets(g.jobs.size());
-  for (size_t k = 0; k < g.jobs.size(); k++) {
+  const size_t n_jobs = g.jobs.size();
+  std::vector<std::vector<uint32_t *>> cols(n_jobs), outs(n_jobs);
+  std::vector<std::vector<uint32_t>> logs(n_jobs);
+  std::vector<BatchTree> sets(n_jobs);
+  std::vector<FriJob> fri(n_jobs);
+  std::vector<ColCopy> copies;
+  DeviceRange range;
+  for (size_t k = 0; k < n_jobs; k++) {
     const stwo_hip_job_desc &d = g.jobs[k]->desc;
     const uint32_t n = d.log_size, L = n + d.log_blowup;
     uint32_t *in = (uint32_t *)p;
-    p += align256(((size_t)d.n_cols << n) * 4);
+    p += commit_cols_bytes(d);
     uint32_t *out = (uint32_t *)p;
     p += align256(((size_t)d.n_cols << L) * 4);
-    trees[k] = (uint32_t *)p;
+    uint32_t *tree = (uint32_t *)p;
     p += align256(words_tree(L) * 4);
-    int rc = load_columns(ctx, d, d.n_cols, in);
+    int rc = load_columns(ctx, d, d.n_cols, in, range, copies);
     if (rc) return rc;
     for (uint32_t c = 0; c < d.n_cols; c++) {
       cols[k].push_back(in + ((size_t)c << n));
       outs[k].push_back(out + ((size_t)c << L));
     }
     logs[k].assign(d.n_cols, n);
-    sets[k] = {cols[k].data(), logs[k].data(), d.n_cols, d.log_blowup, outs[k].data(), trees[k],
+    sets[k] = {cols[k].data(), logs[k].data(), d.n_cols, d.log_blowup, outs[k].data(), tree,
                STWO_HIP_TREE_LIFTED, STWO_HIP_HASH_BLAKE2S};
+    FriJob &f = fri[k];
+    f.cfg = d.fri;
+    f.log_size = L;
+    for (int j = 0; j < 4; j++) f.column[j] = outs[k][j];
+    f.tree = tree;
+    f.layers = in;
+    f.roots = g.jobs[k]->res.fri_roots;
+    f.n_roots = 0;
+    f.last_layer_poly = g.jobs[k]->res.last_layer_poly;
   }
+  uint32_t *fri_mem = (uint32_t *)p;
+  for (const FriJob &f : fri) p += fri_job_words(f.log_size) * 4;
+  p = g.mem + align256(p - g.mem);
   job_mem_begin(ctx, p, g.mem + g.bytes - p);
+  int rc = copy_columns(ctx, copies);
   stwo_hip_batch *plan = nullptr;
-  int rc = batch_create_trees(ctx, sets.data(), sets.size(), s->tw, STWO_HIP_BATCH_DROP_COEFFS, &plan);
+  if (rc == STWO_HIP_OK)
+    rc = batch_create_trees(ctx, sets.data(), sets.size(), s->tw, STWO_HIP_BATCH_DROP_COEFFS, &plan);
   if (rc == STWO_HIP_OK) rc = stwo_hip_batch_run(ctx, plan);
-  if (rc == STWO_HIP_OK) {
-    std::vector<DownloadReq> reqs;
-    for (size_t k = 0; k < g.jobs.size(); k++) reqs.push_back({g.jobs[k]->res.trace_root, trees[k], 8});
-    rc = download_many(ctx, reqs.data(), reqs.size());
-  }
+  // FRI of every job side by side, on channels that mix the trace roots (evals
+  // 0..3 as QM31 coordinates)
+  if (rc == STWO_HIP_OK) rc = fri_commit_jobs(ctx, fri.data(), n_jobs, s->tw, fri_mem);
   if (plan) stwo_hip_batch_destroy(ctx, plan);
-  // FRI per job, largest first (the FRI scratch carved for the first serves the others)
-  std::vector<size_t> order(g.jobs.size());
-  for (size_t k = 0; k < order.size(); k++) order[k] = k;
-  std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) {
-    return g.jobs[a]->desc.log_size + g.jobs[a]->desc.log_blowup > g.jobs[b]->desc.log_size + g.jobs[b]->desc.log_blowup;
-  });
-  for (size_t k : order) {
-    if (rc) break;
-    Job &j = *g.jobs[k];
-    const stwo_hip_job_desc &d = j.desc;
-    const uint32_t L = d.log_size + d.log_blowup;
-    // Channel: mix the trace root, then FRI on (evals 0..3) as QM31 coordinates.
-    b2_host h;
-    uint8_t zero[32] = {0};
-    h.update(zero, 32);
-    h.update(j.res.trace_root, 32);
-    uint8_t digest[32];
-    h.finalize(digest);
-    uint32_t n_draws = 0;
-    const uint32_t *coords[4] = {outs[k][0], outs[k][1], outs[k][2], outs[k][3]};
-    uint32_t n_roots = 0;
-    rc = stwo_hip_fri_commit(ctx, digest, &n_draws, d.fri, coords, L, s->tw, j.res.fri_roots, &n_roots,
-                             j.res.last_layer_poly);
-    if (rc) break;
-    j.res.n_fri_roots = n_roots;
-    memcpy(j.res.final_digest, digest, 32);
+  if (rc == STWO_HIP_OK) {
+    for (size_t k = 0; k < n_jobs; k++) {
+      stwo_hip_job_result &res = g.jobs[k]->res;
+      memcpy(res.trace_root, fri[k].mixed_root, 32);
+      res.n_fri_roots = fri[k].n_roots;
+      memcpy(res.final_digest, fri[k].digest, 32);
+    }
   }
-  if (rc == STWO_HIP_OK) rc = stwo_hip_sync(ctx);
+  // also after a failure: the group's memory goes to another slot
+  const int src = stwo_hip_sync(ctx);
+  if (rc == STWO_HIP_OK) rc = src;
   job_mem_end(ctx);
   return rc;
 }
@@ -301,7 +366,9 @@ int run_prove_group(stwo_hip_server *s, stwo_hip_ctx *ctx, Group &g) {
     b = d.cols[1];
   } else {
     uint32_t *ab = (uint32_t *)p;
-    rc = load_columns(ctx, d, 2, ab);
+    DeviceRange range;
+    std::vector<ColCopy> none;  // no device columns on this path
+    rc = load_columns(ctx, d, 2, ab, range, none);
     a = ab;
     b = ab + n;
   }
