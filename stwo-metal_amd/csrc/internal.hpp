@@ -282,12 +282,33 @@ struct ColRef {
   uint32_t pad;
 };
 
-// One Merkle layer over a device table of columns (mixed layer or lifted leaves).
-int launch_merkle_layer(stwo_hip_ctx *ctx, const uint32_t *prev, const ColRef *d_cols, uint32_t n_cols,
-                        uint32_t log_size, uint32_t *out, int mode, bool lifted);
-// Node layers [stop_log, top_log) of a packed tree whose layer top_log is filled.
-int hash_node_layers(stwo_hip_ctx *ctx, uint32_t *layers, uint32_t top_log, uint32_t stop_log, int mode,
-                     uint32_t *counters);
+// A tree's launches: a layer with columns, or a run of node layers.
+struct MerkleLayer {
+  const uint32_t *prev;  // layer log_size + 1, or NULL
+  const ColRef *cols;
+  uint32_t *out;
+  uint32_t n_cols, log_size, m31, lifted;
+  uint32_t wg_start;  // first workgroup, in a launch of several
+};
+struct MerkleNodes {
+  uint32_t *packed, *counters;
+  uint32_t out_log, stop_log, m31, wg_start;
+};
+enum : uint32_t {
+  kMerkleLayer, kMerkleAhead, kMerkleQuad, kMerkleQuadLds, kMerkleNodes64, kMerkleNodes256, kMerkleNodes1024
+};
+struct MerkleStep {
+  uint32_t kind, wgs;  // steps of one kind, of different trees, may share a launch
+  MerkleLayer layer;   // kinds below kMerkleNodes64
+  MerkleNodes nodes;
+};
+MerkleStep merkle_layer_step(const uint32_t *prev, const ColRef *d_cols, uint32_t n_cols, uint32_t log_size,
+                             uint32_t *out, int mode, bool lifted);
+MerkleStep merkle_nodes_step(uint32_t *layers, uint32_t top_log, uint32_t stop_log, int mode, uint32_t *counters);
+int launch_merkle(stwo_hip_ctx *ctx, const MerkleStep &s);
+// n steps of one kind from a table of MerkleLayer or MerkleNodes.
+int launch_merkle_multi(stwo_hip_ctx *ctx, uint32_t kind, bool lifted, const void *d_steps, uint32_t n, uint32_t wgs);
+
 // Counters of the one-launch trees: a word per group of workgroups that hand
 // their digests on, stage by stage; 2^12 + 2^5 + 1 for 2^30 leaves, and at most
 // 2^(lg / 2) for 2^lg (a tree's stages take equal shares of the levels above the

@@ -84,11 +84,11 @@ __device__ __forceinline__ uint32_t ld_col_word(const uint32_t *col, uint32_t id
 // large layers the other waves hide the latency and the extra registers and
 // copies cost more than they save.
 template <bool AHEAD>
-__global__ void __launch_bounds__(256) merkle_layer_kernel(const uint32_t *prev, const ColRef *cols, uint32_t n_cols,
-                                                           uint32_t log_size, uint32_t *out, uint32_t m31,
-                                                           uint32_t lifted) {
-  const uint32_t n = 1u << log_size;
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void merkle_layer(const MerkleLayer &L, uint32_t wg) {
+  const uint32_t *prev = L.prev;
+  const ColRef *cols = L.cols;
+  const uint32_t n_cols = L.n_cols, lifted = L.lifted, n = 1u << L.log_size;
+  const uint32_t i = wg * 256 + threadIdx.x;
   if (i >= n) return;
   // The words of columns c0 .. c0 + 15 at this row (zeros past n_cols).
   auto load_cols = [&](uint32_t c0, uint32_t (&dst)[16]) {
@@ -130,7 +130,7 @@ __global__ void __launch_bounds__(256) merkle_layer_kernel(const uint32_t *prev,
     t += 4 * cnt;
     b2_compress(s, m, t, c0 + 16 >= n_cols);
   }
-  store_hash(out + 8 * (size_t)i, s, m31);
+  store_hash(L.out + 8 * (size_t)i, s, L.m31);
 }
 
 // Layers of few nodes, where a node's chain of blocks is the launch's
@@ -138,11 +138,11 @@ __global__ void __launch_bounds__(256) merkle_layer_kernel(const uint32_t *prev,
 // instructions per lane instead of 960 on one lane), each block's column
 // words loaded one compression ahead.  Same inputs and outputs as
 // merkle_layer_kernel; the grid has 4 lanes per node.
-__global__ void __launch_bounds__(256) merkle_layer_quad_kernel(const uint32_t *prev, const ColRef *cols,
-                                                                uint32_t n_cols, uint32_t log_size, uint32_t *out,
-                                                                uint32_t m31, uint32_t lifted) {
-  const uint32_t n = 1u << log_size;
-  const uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) >> 2, j = threadIdx.x & 3;
+__device__ __forceinline__ void merkle_layer_quad(const MerkleLayer &L, uint32_t wg) {
+  const uint32_t *prev = L.prev;
+  const ColRef *cols = L.cols;
+  const uint32_t n_cols = L.n_cols, lifted = L.lifted, m31 = L.m31, n = 1u << L.log_size;
+  const uint32_t i = (wg * 256 + threadIdx.x) >> 2, j = threadIdx.x & 3;
   if (i >= n) return;  // a quad's four lanes share i and leave together
   auto load_cols = [&](uint32_t c0, uint32_t (&dst)[16]) {
     const uint32_t cnt = min(16u, n_cols - c0);
@@ -182,7 +182,7 @@ __global__ void __launch_bounds__(256) merkle_layer_quad_kernel(const uint32_t *
     lo = b2_reduce_word(lo);
     hi = b2_reduce_word(hi);
   }
-  g_u32 *o = as_global(out + 8 * (size_t)i);
+  g_u32 *o = as_global(L.out + 8 * (size_t)i);
   o[j] = lo;
   o[4 + j] = hi;
 }
@@ -197,14 +197,14 @@ __global__ void __launch_bounds__(256) merkle_layer_quad_kernel(const uint32_t *
 // round trips and its blocks then read their words from LDS.  Same inputs
 // and outputs as merkle_layer_kernel (mixed layers only, not lifted).
 constexpr uint32_t MQ_CHUNK = 240;  // 15 blocks; 61,440 B of words + 1,920 B of pointers
-__global__ void __launch_bounds__(256) merkle_layer_quad_lds_kernel(const uint32_t *prev, const ColRef *cols,
-                                                                    uint32_t n_cols, uint32_t log_size,
-                                                                    uint32_t *out, uint32_t m31) {
+__device__ __forceinline__ void merkle_layer_quad_lds(const MerkleLayer &L, uint32_t wg) {
   __shared__ const uint32_t *ptrs[MQ_CHUNK];
   __shared__ uint32_t tile[MQ_CHUNK * 64];
-  const uint32_t n = 1u << log_size;
+  const uint32_t *prev = L.prev;
+  const ColRef *cols = L.cols;
+  const uint32_t n_cols = L.n_cols, m31 = L.m31, n = 1u << L.log_size;
   const uint32_t tid = threadIdx.x, node = tid >> 2, j = tid & 3;
-  const uint32_t i0 = blockIdx.x * 64, i = i0 + node;
+  const uint32_t i0 = wg * 64, i = i0 + node;
   const bool active = i < n;  // every lane stays for the barriers
   uint32_t lo = b2_iv_lo(j), hi = b2_iv_hi(j);
   uint32_t m[16];
@@ -253,7 +253,7 @@ __global__ void __launch_bounds__(256) merkle_layer_quad_lds_kernel(const uint32
     lo = b2_reduce_word(lo);
     hi = b2_reduce_word(hi);
   }
-  g_u32 *o = as_global(out + 8 * (size_t)i);
+  g_u32 *o = as_global(L.out + 8 * (size_t)i);
   o[j] = lo;
   o[4 + j] = hi;
 }
@@ -265,11 +265,12 @@ __global__ void __launch_bounds__(256) merkle_layer_quad_lds_kernel(const uint32
 // its narrow levels; 64 (a quad each) in small trees, where latency counts; 256
 // between.
 template <uint32_t NODES>
-__global__ void __launch_bounds__(kTreeThreads) merkle_nodes_kernel(const uint32_t *prev, uint32_t *packed,
-                                                                    uint32_t out_log, uint32_t stop_log, uint32_t m31,
-                                                                    uint32_t *counters) {
+__device__ __forceinline__ void merkle_nodes(const MerkleNodes &L, uint32_t wg) {
   __shared__ __align__(16) TreeLds S;
-  const uint32_t n = 1u << out_log, first = blockIdx.x * NODES, tid = threadIdx.x;
+  uint32_t *packed = L.packed;
+  const uint32_t out_log = L.out_log, stop_log = L.stop_log, m31 = L.m31;
+  const uint32_t *prev = packed + tree_layer_off(out_log + 1);
+  const uint32_t n = 1u << out_log, first = wg * NODES, tid = threadIdx.x;
   uint32_t *out = packed + tree_layer_off(out_log);
   uint32_t lg = out_log, cnt = min(NODES, n), row0 = first;  // the level held in S
   if constexpr (NODES == 64) {
@@ -314,60 +315,141 @@ __global__ void __launch_bounds__(kTreeThreads) merkle_nodes_kernel(const uint32
   }
   const uint32_t lv = min(31 - __clz(cnt), lg - stop_log), l = lg - lv;
   const uint32_t buf = tree_levels(S, 0, cnt, row0, lg, lv, packed, m31, l > stop_log);
-  tree_finish(S, buf, blockIdx.x, l, stop_log, packed, m31, counters);
+  tree_finish(S, buf, wg, l, stop_log, packed, m31, L.counters);
+}
+
+// The launches: one layer or run of node layers by value, or several from a
+// table, each owning the workgroups from its wg_start on (0, then increasing).
+template <typename T>
+__device__ __forceinline__ const T &step_of(const T *t, uint32_t n) {
+  uint32_t g = 0, hi = n;
+  while (hi - g > 1) {
+    const uint32_t mid = (g + hi) / 2;
+    if (t[mid].wg_start <= blockIdx.x) g = mid; else hi = mid;
+  }
+  return t[g];
+}
+template <bool AHEAD>
+__global__ void __launch_bounds__(256) merkle_layer_kernel(MerkleLayer L) {
+  merkle_layer<AHEAD>(L, blockIdx.x);
+}
+template <bool AHEAD>
+__global__ void __launch_bounds__(256) merkle_layer_multi_kernel(const MerkleLayer *t, uint32_t n) {
+  const MerkleLayer L = step_of(t, n);
+  merkle_layer<AHEAD>(L, blockIdx.x - L.wg_start);
+}
+__global__ void __launch_bounds__(256) merkle_layer_quad_kernel(MerkleLayer L) { merkle_layer_quad(L, blockIdx.x); }
+__global__ void __launch_bounds__(256) merkle_layer_quad_multi_kernel(const MerkleLayer *t, uint32_t n) {
+  const MerkleLayer L = step_of(t, n);
+  merkle_layer_quad(L, blockIdx.x - L.wg_start);
+}
+__global__ void __launch_bounds__(256) merkle_layer_quad_lds_kernel(MerkleLayer L) {
+  merkle_layer_quad_lds(L, blockIdx.x);
+}
+__global__ void __launch_bounds__(256) merkle_layer_quad_lds_multi_kernel(const MerkleLayer *t, uint32_t n) {
+  const MerkleLayer L = step_of(t, n);
+  merkle_layer_quad_lds(L, blockIdx.x - L.wg_start);
+}
+template <uint32_t NODES>
+__global__ void __launch_bounds__(kTreeThreads) merkle_nodes_kernel(MerkleNodes L) {
+  merkle_nodes<NODES>(L, blockIdx.x);
+}
+template <uint32_t NODES>
+__global__ void __launch_bounds__(kTreeThreads) merkle_nodes_multi_kernel(const MerkleNodes *t, uint32_t n) {
+  const MerkleNodes L = step_of(t, n);
+  merkle_nodes<NODES>(L, blockIdx.x - L.wg_start);
 }
 
 static inline size_t layer_off(uint32_t l) { return tree_layer_off(l); }
 
-int launch_merkle_layer(stwo_hip_ctx *ctx, const uint32_t *prev, const ColRef *d_cols, uint32_t n_cols,
-                        uint32_t log_size, uint32_t *out, int mode, bool lifted) {
+// Up to 2^14 nodes with more than one block per node, the layer is
+// latency-bound even at four lanes per node: a quad per node (mixed layers
+// with the columns staged through LDS, lifted ones loading a block ahead).  Below 2^16
+// nodes, a lane per node with the loads one block ahead.
+MerkleStep merkle_layer_step(const uint32_t *prev, const ColRef *d_cols, uint32_t n_cols, uint32_t log_size,
+                             uint32_t *out, int mode, bool lifted) {
+  MerkleStep s{};
+  s.layer = {prev, d_cols, out, n_cols, log_size, (uint32_t)(mode == STWO_HIP_HASH_BLAKE2S_M31), (uint32_t)lifted, 0};
+  const uint32_t n = 1u << log_size;
+  const bool quad = log_size <= 14 && n_cols > 16;
+  s.kind = quad                             ? (lifted ? kMerkleQuad : kMerkleQuadLds)
+           : log_size < 16 && n_cols > 16 ? kMerkleAhead
+                                            : kMerkleLayer;
+  s.wgs = quad ? (n + 63) / 64 : (n + 255) / 256;
+  return s;
+}
+
+// Node layers top_log-1 .. stop_log (< top_log) of a packed tree whose layer
+// top_log is filled.  counters: tree_counters(top_log) zeros, left zero, used by
+// no launch that may overlap this one.
+MerkleStep merkle_nodes_step(uint32_t *layers, uint32_t top_log, uint32_t stop_log, int mode, uint32_t *counters) {
+  MerkleStep s{};
+  const uint32_t out_log = top_log - 1;
+  // (four nodes per lane take the two levels above along)
+  const uint32_t per = std::min<uint32_t>(tree_leaves_log(out_log), out_log >= stop_log + 2 ? 10 : 8);
+  s.nodes = {layers, counters, out_log, stop_log, (uint32_t)(mode == STWO_HIP_HASH_BLAKE2S_M31), 0};
+  s.kind = per == 6 ? kMerkleNodes64 : per == 8 ? kMerkleNodes256 : kMerkleNodes1024;
+  s.wgs = 1u << (out_log > per ? out_log - per : 0);
+  return s;
+}
+
+static const char *step_name(uint32_t kind, bool lifted) {
+  return kind >= kMerkleNodes64 ? "merkle_nodes" : lifted ? "merkle_lifted_leaves" : "merkle_commit_on_layer";
+}
+
+int launch_merkle(stwo_hip_ctx *ctx, const MerkleStep &s) {
+  const char *name = step_name(s.kind, s.layer.lifted);
+  const dim3 grid(s.wgs), block(256);
+  switch (s.kind) {
+    case kMerkleLayer: return launch(ctx, name, merkle_layer_kernel<false>, grid, block, 0, s.layer);
+    case kMerkleAhead: return launch(ctx, name, merkle_layer_kernel<true>, grid, block, 0, s.layer);
+    case kMerkleQuad: return launch(ctx, name, merkle_layer_quad_kernel, grid, block, 0, s.layer);
+    case kMerkleQuadLds: return launch(ctx, name, merkle_layer_quad_lds_kernel, grid, block, 0, s.layer);
+    case kMerkleNodes64: return launch(ctx, name, merkle_nodes_kernel<64>, grid, block, 0, s.nodes);
+    case kMerkleNodes256: return launch(ctx, name, merkle_nodes_kernel<256>, grid, block, 0, s.nodes);
+    default: return launch(ctx, name, merkle_nodes_kernel<1024>, grid, block, 0, s.nodes);
+  }
+}
+
+int launch_merkle_multi(stwo_hip_ctx *ctx, uint32_t kind, bool lifted, const void *d_steps, uint32_t n, uint32_t wgs) {
+  const char *name = step_name(kind, lifted);
+  const dim3 grid(wgs), block(256);
+  const MerkleLayer *l = (const MerkleLayer *)d_steps;
+  const MerkleNodes *t = (const MerkleNodes *)d_steps;
+  switch (kind) {
+    case kMerkleLayer: return launch(ctx, name, merkle_layer_multi_kernel<false>, grid, block, 0, l, n);
+    case kMerkleAhead: return launch(ctx, name, merkle_layer_multi_kernel<true>, grid, block, 0, l, n);
+    case kMerkleQuad: return launch(ctx, name, merkle_layer_quad_multi_kernel, grid, block, 0, l, n);
+    case kMerkleQuadLds: return launch(ctx, name, merkle_layer_quad_lds_multi_kernel, grid, block, 0, l, n);
+    case kMerkleNodes64: return launch(ctx, name, merkle_nodes_multi_kernel<64>, grid, block, 0, t, n);
+    case kMerkleNodes256: return launch(ctx, name, merkle_nodes_multi_kernel<256>, grid, block, 0, t, n);
+    default: return launch(ctx, name, merkle_nodes_multi_kernel<1024>, grid, block, 0, t, n);
+  }
+}
+
+static int check_mode(stwo_hip_ctx *ctx, int mode) {
   STWO_HIP_CHECK_ARG(ctx, mode == STWO_HIP_HASH_BLAKE2S || mode == STWO_HIP_HASH_BLAKE2S_M31,
                      "merkle: unknown hash mode %d", mode);
-  uint32_t n = 1u << log_size;
-  const char *name = lifted ? "merkle_lifted_leaves" : "merkle_commit_on_layer";
-  const uint32_t m31 = (uint32_t)(mode == STWO_HIP_HASH_BLAKE2S_M31);
-  // Up to 2^14 nodes with more than one block per node, the layer is
-  // latency-bound even at four lanes per node: a quad per node (mixed layers
-  // with the columns staged through LDS, lifted ones loading a block ahead).  Below 2^16
-  // nodes, a lane per node with the loads one block ahead.
-  if (log_size <= 14 && n_cols > 16 && !lifted)
-    return launch(ctx, name, merkle_layer_quad_lds_kernel, dim3((n + 63) / 64), dim3(256), 0, prev, d_cols, n_cols,
-                  log_size, out, m31);
-  if (log_size <= 14 && n_cols > 16)
-    return launch(ctx, name, merkle_layer_quad_kernel, dim3((4 * n + 255) / 256), dim3(256), 0, prev, d_cols, n_cols,
-                  log_size, out, m31, (uint32_t)lifted);
-  const bool ahead = log_size < 16 && n_cols > 16;
-  return launch(ctx, name, ahead ? merkle_layer_kernel<true> : merkle_layer_kernel<false>, dim3((n + 255) / 256),
-                dim3(256), 0, prev, d_cols, n_cols, log_size, out, m31, (uint32_t)lifted);
+  return STWO_HIP_OK;
 }
 
 static int launch_layer(stwo_hip_ctx *ctx, const uint32_t *prev, const std::vector<ColRef> &cols, uint32_t log_size,
                         uint32_t *out, int mode, bool lifted) {
+  int rc = check_mode(ctx, mode);
+  if (rc) return rc;
   void *dtab = nullptr;
   if (!cols.empty()) {
-    int rc = upload_table(ctx, cols.data(), cols.size() * sizeof(ColRef), &dtab);
+    rc = upload_table(ctx, cols.data(), cols.size() * sizeof(ColRef), &dtab);
     if (rc) return rc;
   }
-  return launch_merkle_layer(ctx, prev, (const ColRef *)dtab, (uint32_t)cols.size(), log_size, out, mode, lifted);
+  return launch_merkle(
+      ctx, merkle_layer_step(prev, (const ColRef *)dtab, (uint32_t)cols.size(), log_size, out, mode, lifted));
 }
 
-// Hashes node layers top_log-1 .. stop_log of a packed tree whose layer top_log
-// is filled.  counters: kTreeCounters zeros, left zero, used by no launch that
-// may overlap this one.
-int hash_node_layers(stwo_hip_ctx *ctx, uint32_t *layers, uint32_t top_log, uint32_t stop_log, int mode,
-                     uint32_t *counters) {
-  STWO_HIP_CHECK_ARG(ctx, mode == STWO_HIP_HASH_BLAKE2S || mode == STWO_HIP_HASH_BLAKE2S_M31,
-                     "merkle: unknown hash mode %d", mode);
-  if (top_log <= stop_log) return STWO_HIP_OK;
-  const uint32_t out_log = top_log - 1;
-  // (four nodes per lane take the two levels above along)
-  const uint32_t per = std::min<uint32_t>(tree_leaves_log(out_log), out_log >= stop_log + 2 ? 10 : 8);
-  const dim3 grid(1u << (out_log > per ? out_log - per : 0)), block(kTreeThreads);
-  const uint32_t *prev = layers + layer_off(top_log);
-  const uint32_t m31 = (uint32_t)(mode == STWO_HIP_HASH_BLAKE2S_M31);
-  return launch(ctx, "merkle_nodes",
-                per == 6 ? merkle_nodes_kernel<64> : per == 8 ? merkle_nodes_kernel<256> : merkle_nodes_kernel<1024>,
-                grid, block, 0, prev, layers, out_log, stop_log, m31, counters);
+static int hash_node_layers(stwo_hip_ctx *ctx, uint32_t *layers, uint32_t top_log, uint32_t stop_log, int mode) {
+  int rc = check_mode(ctx, mode);
+  if (rc || top_log <= stop_log) return rc;
+  return launch_merkle(ctx, merkle_nodes_step(layers, top_log, stop_log, mode, ctx->d_counters));
 }
 
 }  // namespace stwo_hip
@@ -412,7 +494,7 @@ int stwo_hip_merkle_commit(stwo_hip_ctx *ctx, const uint32_t *const *cols, const
       for (size_t c = 0; c < n_cols; c++)
         if ((int)log_sizes[c] < l) next = std::max(next, (int)log_sizes[c]);
       uint32_t stop = (uint32_t)(next + 1);
-      int rc = hash_node_layers(ctx, layers, (uint32_t)l + 1, stop, hash_mode, ctx->d_counters);
+      int rc = hash_node_layers(ctx, layers, (uint32_t)l + 1, stop, hash_mode);
       if (rc) return rc;
       l = (int)stop - 1;
       continue;
@@ -458,7 +540,7 @@ int stwo_hip_merkle_lifted_commit(stwo_hip_ctx *ctx, const uint32_t *const *cols
   int rc = stwo_hip_merkle_lifted_build_leaves(ctx, cols, log_sizes, n_cols, lifting_log_size,
                                                layers + layer_off(lifting_log_size), hash_mode);
   if (rc) return rc;
-  return hash_node_layers(ctx, layers, lifting_log_size, 0, hash_mode, ctx->d_counters);
+  return hash_node_layers(ctx, layers, lifting_log_size, 0, hash_mode);
 }
 
 }  // extern "C"

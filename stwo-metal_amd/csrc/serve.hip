@@ -115,7 +115,8 @@ struct Group {
 inline size_t words_tree(uint32_t max_log) { return (((size_t)2 << max_log) - 1) * 8; }
 inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// A commit job's own data: columns, evaluations, tree and FRI state.  Once the
+// A commit job's own data: columns, evaluations, tree, FRI state and its tree's
+// part of the plan's tables.  Once the
 // evaluations are committed the rest is the FRI commit's: its folded evaluations
 // lie over the columns (3 << L words), its trees over the trace's.
 size_t commit_cols_bytes(const stwo_hip_job_desc &d) {
@@ -125,7 +126,7 @@ size_t commit_cols_bytes(const stwo_hip_job_desc &d) {
 size_t commit_data_bytes(const stwo_hip_job_desc &d) {
   const uint32_t L = d.log_size + d.log_blowup;
   return commit_cols_bytes(d) + align256(((size_t)d.n_cols << L) * 4) + align256(words_tree(L) * 4) +
-         fri_job_words(L) * 4;
+         fri_job_words(L) * 4 + align256(tree_counters(L) * 4) + 1024;
 }
 // Device bytes of a group: every commit job's data, the batched plan's
 // tables (column tables and pass descriptors); a prove job's buffers and its
