@@ -84,6 +84,305 @@ struct TreeWave {
   uint32_t n, wgs;
 };
 
+// One group of same-size columns: its tables' places in the staging.
+struct GroupTabs {
+  uint32_t n, b;
+  int stage;
+  size_t ifft_off, rfft_off, inplace_off;
+  uint32_t count;
+  bool aligned16;  // every column pointer of the group is 16-byte aligned
+};
+
+// A group of columns {in, out} (in place but for the evaluations).
+GroupTabs put_group(Staging &st, uint32_t n, uint32_t b, int stage, const std::vector<FftCol> &cols) {
+  std::vector<FftCol> a, c;
+  GroupTabs t{};
+  t.n = n;
+  t.b = b;
+  t.stage = stage;
+  t.count = (uint32_t)cols.size();
+  t.aligned16 = true;
+  for (const FftCol &f : cols) {
+    if (stage != BATCH_RFFT) a.push_back({f.in, (uint32_t *)f.in});
+    c.push_back({f.out, f.out});
+    if ((((uintptr_t)f.in) | ((uintptr_t)f.out)) & 15) t.aligned16 = false;
+  }
+  if (stage != BATCH_RFFT) t.ifft_off = st.put(a.data(), a.size() * sizeof(FftCol));
+  if (stage != BATCH_IFFT) {
+    t.rfft_off = st.put(cols.data(), cols.size() * sizeof(FftCol));
+    t.inplace_off = st.put(c.data(), c.size() * sizeof(FftCol));
+  } else {
+    t.rfft_off = t.inplace_off = t.ifft_off;
+  }
+  return t;
+}
+
+// Upper bound on the descriptors that build_levels adds: one per group and pass
+// (2 directions, at most 4 passes), plus the 256-byte alignment of two or three
+// tables per launch (2 directions x 4 levels x 2 workgroup sizes x at most 14
+// schedule kinds, and the fused launches).
+size_t levels_bound(size_t n_groups) {
+  return n_groups * (sizeof(MxTop) + 2 * sizeof(MxLow)) + 8 * 256 + 2 * 4 * n_groups * (sizeof(FftPass2) + 8) +
+         2 * 4 * 2 * 14 * 2 * 256 + 8192;
+}
+
+// Two workgroups of the vector passes a CU, half of what it holds (16 KB
+// of LDS and 256 lanes each).
+constexpr uint64_t kShareWgs = 512;
+
+// The launches of the groups' transforms, over their tables and the descriptors
+// put after them, all at dbase once uploaded.  drop: the fused passes need not
+// store the coefficients.  matrix: groups that can take the matrix passes do.
+int build_levels(stwo_hip_ctx *ctx, const stwo_hip_twiddles *tw, const std::vector<GroupTabs> &gt, uint8_t *dbase,
+                 bool store_coeffs, bool matrix, Staging &st, std::vector<LevelLaunch> &levels) {
+  // The radix-16 passes take the doubled trees.
+  const uint32_t *itw_end = tw->d_itw2 + tw->len, *tw_end = tw->d_tw2 + tw->len;
+  // Both transforms' passes of every group; where the IFFT's last pass and
+  // the RFFT's first pass tile alike they become one fused pass.
+  struct GroupPasses {
+    std::vector<PassLaunch> inv, fwd;
+    bool fused = false;
+    bool matrix = false;  // first and last passes on the matrix cores
+    MxPlan mx;
+  };
+  std::vector<GroupPasses> gp(gt.size());
+  for (size_t gi = 0; gi < gt.size(); gi++) {
+    const GroupTabs &t = gt[gi];
+    for (int dir = 0; dir < 2; dir++) {
+      const bool inverse = dir == 0;
+      if ((inverse && t.stage == BATCH_RFFT) || (!inverse && t.stage == BATCH_IFFT)) continue;
+      const uint32_t n = t.n, N = t.n + (inverse ? 0 : t.b);
+      const FftCol *first = (const FftCol *)(dbase + (inverse ? t.ifft_off : t.rfft_off));
+      const FftCol *inpl = (const FftCol *)(dbase + t.inplace_off);
+      int rc = make_group_passes(ctx, inverse ? N : n, N, inverse, first, inpl, t.count, inverse ? itw_end : tw_end,
+                                 t.aligned16, inverse ? gp[gi].inv : gp[gi].fwd);
+      if (rc) return rc;
+    }
+    GroupPasses &G = gp[gi];
+    const bool has_inv = t.stage != BATCH_RFFT, has_fwd = t.stage != BATCH_IFFT;
+    if (matrix &&
+        (!has_inv || mx_plan(ctx, tw, t.n, 0, true, t.count, t.aligned16, true, &G.mx)) &&
+        (!has_fwd || mx_plan(ctx, tw, t.n, t.b, false, t.count, t.aligned16, true, &G.mx))) {
+      G.matrix = true;
+      // what is left to the vector passes: the default plan's middle pass
+      const FftTune def;
+      for (int dir = 0; dir < 2; dir++) {
+        std::vector<PassLaunch> &v = dir ? G.fwd : G.inv;
+        if (v.empty()) continue;
+        if (!G.mx.mid) {
+          v.clear();
+          continue;
+        }
+        const FftCol *in_place = (const FftCol *)(dbase + (dir ? t.inplace_off : t.ifft_off));
+        int rc = make_group_passes(ctx, t.n, t.n + (dir ? t.b : 0), !dir, in_place, in_place, t.count,
+                                   dir ? tw_end : itw_end, true, v, &def);
+        if (!rc && v.size() != 3) rc = set_error(ctx, STWO_HIP_EINVAL, "internal: %zu passes of 2^%u", v.size(), t.n);
+        if (rc) return rc;
+        v = {v[1]};
+      }
+      continue;
+    }
+    gp[gi].fused = t.stage == BATCH_LDE && lde_fusable(gp[gi].inv.back(), gp[gi].fwd.front(), t.b);
+  }
+  auto add_level = [&](bool inverse, uint32_t wg_log, std::vector<PassLaunch> &v) -> int {
+    // Groups whose pass matches a compile-time schedule get a launch per
+    // schedule with that schedule's kernel; the rest share one.  Schedules that
+    // together do not fill the device once (kShareWgs) share the run-time
+    // schedule's launch instead: a launch costs more than the schedule gains
+    // there (six schedules of 512 workgroups in all: 27 us in six launches, 12 us in
+    // one).
+    std::map<uint32_t, uint64_t> kinds;  // schedule -> workgroups
+    for (auto &pl : v) kinds[pl.p.fixed] += pl.wgs;
+    std::vector<std::pair<uint64_t, uint32_t>> by_wgs;
+    for (auto &k : kinds) by_wgs.push_back({k.second, k.first});
+    std::sort(by_wgs.begin(), by_wgs.end());
+    uint64_t small = 0;
+    std::vector<std::vector<uint32_t>> launches(1);
+    for (auto &k : by_wgs)
+      if ((small += k.first) <= kShareWgs)
+        launches[0].push_back(k.second);
+      else
+        launches.push_back({k.second});
+    for (const std::vector<uint32_t> &kds : launches) {
+      const uint32_t kd = kds.size() == 1 ? kds[0] : 0;
+      std::vector<FftPass2> descs;
+      std::vector<uint32_t> starts;
+      uint64_t acc = 0;
+      bool uniform = true;
+      for (auto &pl : v) {
+        if (std::find(kds.begin(), kds.end(), pl.p.fixed) == kds.end()) continue;
+        descs.push_back(pl.p);
+        starts.push_back((uint32_t)acc);
+        acc += pl.wgs;
+        if (pl.p.T < 10) uniform = false;
+      }
+      if (descs.empty()) continue;
+      if (acc >= (1ull << 31)) return set_error(ctx, STWO_HIP_EINVAL, "FFT groups too large for one launch");
+      LevelLaunch ll{};
+      ll.inverse = inverse;
+      ll.fused = false;
+      ll.kind = kd != 0 ? (int)kd : (uniform ? -1 : 0);
+      ll.groups_off = st.put(descs.data(), descs.size() * sizeof(FftPass2));
+      ll.wgs_off = st.put(starts.data(), starts.size() * sizeof(uint32_t));
+      ll.n_groups = (uint32_t)descs.size();
+      ll.total_wgs = (uint32_t)acc;
+      ll.wg_log = wg_log;
+      levels.push_back(ll);
+    }
+    return STWO_HIP_OK;
+  };
+  // The matrix passes of every group that takes them.  The low pass is the
+  // first of the inverse levels and the last of the forward ones; the top pass
+  // runs after the inverse levels, fused with the forward one where the set
+  // has both.
+  auto add_mx_low = [&](bool inverse) -> int {
+    uint64_t units = 0, acc = 0;
+    auto takes = [&](size_t gi) { return gp[gi].matrix && gt[gi].stage != (inverse ? BATCH_RFFT : BATCH_IFFT); };
+    for (size_t gi = 0; gi < gt.size(); gi++)
+      if (takes(gi)) units += mx_low_units(gt[gi].count, gt[gi].n + (inverse ? 0 : gt[gi].b));
+    std::vector<MxLow> descs;
+    for (size_t gi = 0; gi < gt.size(); gi++) {
+      if (!takes(gi)) continue;
+      const GroupTabs &t = gt[gi];
+      const size_t tab = inverse ? t.ifft_off : gp[gi].mx.top_layers ? t.inplace_off : t.rfft_off;
+      uint32_t wgs = 0;
+      descs.push_back(mx_low(tw, (const FftCol *)(dbase + tab), t.count, t.n, t.n + (inverse ? 0 : t.b), inverse,
+                             gp[gi].mx, units, true, &wgs));
+      descs.back().wg_start = wgs;
+    }
+    if (descs.empty()) return STWO_HIP_OK;
+    // the longest workgroups start first
+    std::stable_sort(descs.begin(), descs.end(), [](const MxLow &a, const MxLow &c) { return a.iters > c.iters; });
+    for (MxLow &d : descs) {
+      const uint32_t wgs = d.wg_start;
+      d.wg_start = (uint32_t)acc;
+      acc += wgs;
+    }
+    if (acc >= (1ull << 31)) return set_error(ctx, STWO_HIP_EINVAL, "FFT groups too large for one launch");
+    LevelLaunch ll{};
+    ll.inverse = inverse;
+    ll.matrix = true;
+    ll.groups_off = st.put(descs.data(), descs.size() * sizeof(MxLow));
+    ll.n_groups = (uint32_t)descs.size();
+    ll.total_wgs = (uint32_t)acc;
+    levels.push_back(ll);
+    return STWO_HIP_OK;
+  };
+  auto add_mx_tops = [&](int stage) -> int {
+    for (uint32_t layers : {8u, 4u}) {
+      uint64_t units = 0, acc = 0;
+      auto takes = [&](size_t gi) {
+        return gp[gi].matrix && gt[gi].stage == stage && gp[gi].mx.top_layers == layers;
+      };
+      for (size_t gi = 0; gi < gt.size(); gi++)
+        if (takes(gi)) units += mx_top_units(gt[gi].count, gt[gi].n, gp[gi].mx);
+      std::vector<MxTop> descs;
+      for (size_t gi = 0; gi < gt.size(); gi++) {
+        if (!takes(gi)) continue;
+        const GroupTabs &t = gt[gi];
+        uint32_t wgs = 0;
+        descs.push_back(mx_top(tw, (const FftCol *)(dbase + t.ifft_off), (const FftCol *)(dbase + t.rfft_off), t.count,
+                               t.n, t.b, stage == BATCH_IFFT || store_coeffs, gp[gi].mx, units,
+                               true, &wgs));
+        descs.back().wg_start = (uint32_t)acc;
+        acc += wgs;
+      }
+      if (descs.empty()) continue;
+      if (acc >= (1ull << 31)) return set_error(ctx, STWO_HIP_EINVAL, "FFT groups too large for one launch");
+      LevelLaunch ll{};
+      ll.matrix = true;
+      ll.mx_layers = layers;
+      ll.mx_inv = stage != BATCH_RFFT;
+      ll.mx_fwd = stage != BATCH_IFFT;
+      ll.groups_off = st.put(descs.data(), descs.size() * sizeof(MxTop));
+      ll.n_groups = (uint32_t)descs.size();
+      ll.total_wgs = (uint32_t)acc;
+      levels.push_back(ll);
+    }
+    return STWO_HIP_OK;
+  };
+  for (int dir = 0; dir < 2; dir++) {
+    const bool inverse = dir == 0;
+    int mrc = inverse ? add_mx_low(true) : add_mx_tops(BATCH_LDE);
+    if (!mrc && !inverse) mrc = add_mx_tops(BATCH_RFFT);
+    if (mrc) return mrc;
+    // (level, workgroup size) -> passes of every group (the fused ones aside)
+    std::map<std::pair<uint32_t, uint32_t>, std::vector<PassLaunch>> by_level;
+    for (const GroupPasses &g : gp) {
+      const std::vector<PassLaunch> &passes = inverse ? g.inv : g.fwd;
+      const size_t k0 = (!inverse && g.fused) ? 1 : 0, k1 = passes.size() - ((inverse && g.fused) ? 1 : 0);
+      for (size_t k = k0; k < k1; k++) {
+        uint32_t level = inverse ? (uint32_t)k : (uint32_t)(passes.size() - 1 - k);
+        if (g.matrix) level = 1;  // the middle one of three
+        by_level[{level, passes[k].wg_log}].push_back(passes[k]);
+      }
+    }
+    if (!inverse) {
+      // the fused passes run after every IFFT level and before every RFFT one
+      std::map<std::pair<uint32_t, int>, std::vector<size_t>> fused;  // (wg_log, kind) -> groups
+      for (size_t gi = 0; gi < gp.size(); gi++)
+        if (gp[gi].fused)
+          fused[{gp[gi].inv.back().wg_log, lde_kind(gp[gi].inv.back(), gp[gi].fwd.front())}].push_back(gi);
+      for (auto &kv : fused) {
+        std::vector<FftPass2> pis, pfs;
+        std::vector<uint32_t> starts;
+        uint64_t acc = 0;
+        for (size_t gi : kv.second) {
+          pis.push_back(gp[gi].inv.back().p);
+          pfs.push_back(gp[gi].fwd.front().p);
+          starts.push_back((uint32_t)acc);
+          acc += gp[gi].inv.back().wgs;
+        }
+        if (acc >= (1ull << 31)) return set_error(ctx, STWO_HIP_EINVAL, "FFT groups too large for one launch");
+        LevelLaunch ll{};
+        ll.inverse = false;
+        ll.fused = true;
+        ll.kind = kv.first.second;
+        ll.groups_off = st.put(pis.data(), pis.size() * sizeof(FftPass2));
+        ll.fwd_off = st.put(pfs.data(), pfs.size() * sizeof(FftPass2));
+        ll.wgs_off = st.put(starts.data(), starts.size() * sizeof(uint32_t));
+        ll.n_groups = (uint32_t)pis.size();
+        ll.total_wgs = (uint32_t)acc;
+        ll.wg_log = kv.first.first;
+        levels.push_back(ll);
+      }
+    }
+    std::vector<std::pair<uint32_t, uint32_t>> order;
+    for (auto &kv : by_level) order.push_back(kv.first);
+    if (!inverse) std::reverse(order.begin(), order.end());  // forward: highest level first
+    for (const auto &key : order) {
+      int rc = add_level(inverse, key.second, by_level[key]);
+      if (rc) return rc;
+    }
+    mrc = inverse ? add_mx_tops(BATCH_IFFT) : add_mx_low(false);
+    if (mrc) return mrc;
+  }
+  return STWO_HIP_OK;
+}
+
+int issue_levels(stwo_hip_ctx *c, const std::vector<LevelLaunch> &levels, uint8_t *dbase, uint32_t keep_coeffs) {
+  for (const LevelLaunch &ll : levels) {
+    if (ll.matrix) {
+      int rc = ll.mx_layers
+                   ? launch_mx_top(c, nullptr, (const MxTop *)(dbase + ll.groups_off), ll.n_groups, ll.total_wgs,
+                                   ll.mx_layers, ll.mx_inv, ll.mx_fwd)
+                   : launch_mx_low(c, nullptr, (const MxLow *)(dbase + ll.groups_off), ll.n_groups, ll.total_wgs,
+                                   ll.inverse);
+      if (rc) return rc;
+      continue;
+    }
+    int rc = ll.fused ? launch_lde_multi(c, (const FftPass2 *)(dbase + ll.groups_off),
+                                         (const FftPass2 *)(dbase + ll.fwd_off),
+                                         (const uint32_t *)(dbase + ll.wgs_off), ll.n_groups, ll.total_wgs,
+                                         ll.wg_log, ll.kind, keep_coeffs)
+                      : launch_fft_multi(c, ll.inverse, (const FftPass2 *)(dbase + ll.groups_off),
+                                         (const uint32_t *)(dbase + ll.wgs_off), ll.n_groups, ll.total_wgs,
+                                         ll.wg_log, ll.kind);
+    if (rc) return rc;
+  }
+  return STWO_HIP_OK;
+}
+
 }  // namespace
 
 int batch_create_trees(stwo_hip_ctx *ctx, const BatchTree *trees, size_t n_trees, const stwo_hip_twiddles *tw,
@@ -120,8 +419,6 @@ int batch_create_trees(stwo_hip_ctx *ctx, const BatchTree *trees, size_t n_trees
   uint32_t rl = tw->root.log_size;
   STWO_HIP_CHECK_ARG(ctx, all_max - 1 <= rl && tw->root.initial_index == half_odds_initial(rl),
                      "batch_create: twiddle root must be half_odds(r) with r >= %u", all_max - 1);
-  // The radix-16 passes take the doubled trees.
-  const uint32_t *itw_end = tw->d_itw2 + tw->len, *tw_end = tw->d_tw2 + tw->len;
 
   // Groups by (log size, blowup, stage) over every set, largest first (their
   // workgroups start first): columns of different sets share launches.
@@ -133,34 +430,15 @@ int batch_create_trees(stwo_hip_ctx *ctx, const BatchTree *trees, size_t n_trees
           .push_back({t, i});
 
   Staging st;
-  struct GroupTabs {
-    uint32_t n, b;
-    int stage;
-    size_t ifft_off, rfft_off, inplace_off;
-    uint32_t count;
-    bool aligned16;  // every column pointer of the group is 16-byte aligned
-  };
   std::vector<GroupTabs> gt;
   for (auto &g : groups) {
-    std::vector<FftCol> a, bb, c;
-    GroupTabs t;
-    t.aligned16 = true;
-    t.stage = std::get<2>(g.first);
+    const int stage = std::get<2>(g.first);
+    std::vector<FftCol> cols;
     for (auto &ti : g.second) {
       uint32_t *col = trees[ti.first].cols[ti.second];
-      uint32_t *o = t.stage == BATCH_IFFT ? col : trees[ti.first].outs[ti.second];
-      a.push_back({col, col});
-      bb.push_back({col, o});
-      c.push_back({o, o});
-      if ((((uintptr_t)col) | ((uintptr_t)o)) & 15) t.aligned16 = false;
+      cols.push_back({col, stage == BATCH_IFFT ? col : trees[ti.first].outs[ti.second]});
     }
-    t.n = std::get<0>(g.first);
-    t.b = std::get<1>(g.first);
-    t.count = (uint32_t)g.second.size();
-    t.ifft_off = st.put(a.data(), a.size() * sizeof(FftCol));
-    t.rfft_off = st.put(bb.data(), bb.size() * sizeof(FftCol));
-    t.inplace_off = st.put(c.data(), c.size() * sizeof(FftCol));
-    gt.push_back(t);
+    gt.push_back(put_group(st, std::get<0>(g.first), std::get<1>(g.first), stage, cols));
   }
   // Merkle column tables, per set.
   std::vector<TreeLaunches> tl;
@@ -208,244 +486,21 @@ int batch_create_trees(stwo_hip_ctx *ctx, const BatchTree *trees, size_t n_trees
   size_t tree_steps_bound = 0;
   if (tl.size() > 1)
     for (const TreeLaunches &L : tl) tree_steps_bound += 2 * L.lt.size() * (sizeof(MerkleLayer) + 256);
-  // Upper bound on descriptors: one per group and pass (2 directions, at most
-  // 4 passes), plus the 256-byte alignment of two or three tables per launch
-  // (2 directions x 4 levels x 2 workgroup sizes x at most 14 schedule kinds,
-  // and the fused launches).
-  size_t desc_bytes = gt.size() * (sizeof(MxTop) + 2 * sizeof(MxLow)) + 8 * 256 + 2 * 4 * gt.size() * (sizeof(FftPass2) + 8) + 2 * 4 * 2 * 14 * 2 * 256 + 8192 +
-                      tree_steps_bound;
+  const size_t desc_bytes = levels_bound(gt.size()) + tree_steps_bound;
   int arc = device_alloc(ctx, tables_bytes + desc_bytes, &dmem, &from_job);
   if (arc) return arc;
   auto release = [&]() { device_free(dmem, from_job); };
   uint8_t *dbase = (uint8_t *)dmem;
-  // Both transforms' passes of every group; where the IFFT's last pass and
-  // the RFFT's first pass tile alike they become one fused pass.
-  struct GroupPasses {
-    std::vector<PassLaunch> inv, fwd;
-    bool fused = false;
-    bool matrix = false;  // first and last passes on the matrix cores
-    MxPlan mx;
-  };
-  std::vector<GroupPasses> gp(gt.size());
-  for (size_t gi = 0; gi < gt.size(); gi++) {
-    const GroupTabs &t = gt[gi];
-    for (int dir = 0; dir < 2; dir++) {
-      const bool inverse = dir == 0;
-      if ((inverse && t.stage == BATCH_RFFT) || (!inverse && t.stage == BATCH_IFFT)) continue;
-      const uint32_t n = t.n, N = t.n + (inverse ? 0 : t.b);
-      const FftCol *first = (const FftCol *)(dbase + (inverse ? t.ifft_off : t.rfft_off));
-      const FftCol *inpl = (const FftCol *)(dbase + t.inplace_off);
-      int rc = make_group_passes(ctx, inverse ? N : n, N, inverse, first, inpl, t.count, inverse ? itw_end : tw_end,
-                                 t.aligned16, inverse ? gp[gi].inv : gp[gi].fwd);
-      if (rc) {
-        release();
-        return rc;
-      }
-    }
-    GroupPasses &G = gp[gi];
-    const bool has_inv = t.stage != BATCH_RFFT, has_fwd = t.stage != BATCH_IFFT;
-    if ((!has_inv || mx_plan(ctx, tw, t.n, 0, true, t.count, t.aligned16, true, &G.mx)) &&
-        (!has_fwd || mx_plan(ctx, tw, t.n, t.b, false, t.count, t.aligned16, true, &G.mx))) {
-      G.matrix = true;
-      // what is left to the vector passes: the default plan's middle pass
-      const FftTune def;
-      for (int dir = 0; dir < 2; dir++) {
-        std::vector<PassLaunch> &v = dir ? G.fwd : G.inv;
-        if (v.empty()) continue;
-        if (!G.mx.mid) {
-          v.clear();
-          continue;
-        }
-        const FftCol *in_place = (const FftCol *)(dbase + (dir ? t.inplace_off : t.ifft_off));
-        int rc = make_group_passes(ctx, t.n, t.n + (dir ? t.b : 0), !dir, in_place, in_place, t.count,
-                                   dir ? tw_end : itw_end, true, v, &def);
-        if (!rc && v.size() != 3) rc = set_error(ctx, STWO_HIP_EINVAL, "internal: %zu passes of 2^%u", v.size(), t.n);
-        if (rc) {
-          release();
-          return rc;
-        }
-        v = {v[1]};
-      }
-      continue;
-    }
-    gp[gi].fused = t.stage == BATCH_LDE && lde_fusable(gp[gi].inv.back(), gp[gi].fwd.front(), t.b);
-  }
   std::vector<LevelLaunch> levels;
-  auto add_level = [&](bool inverse, uint32_t wg_log, std::vector<PassLaunch> &v) -> int {
-    // Groups whose pass matches a compile-time schedule get a launch per
-    // schedule with that schedule's kernel; the rest share one.
-    std::vector<uint32_t> kinds;
-    for (auto &pl : v)
-      if (std::find(kinds.begin(), kinds.end(), pl.p.fixed) == kinds.end()) kinds.push_back(pl.p.fixed);
-    for (uint32_t kd : kinds) {
-      std::vector<FftPass2> descs;
-      std::vector<uint32_t> starts;
-      uint64_t acc = 0;
-      bool uniform = true;
-      for (auto &pl : v) {
-        if (pl.p.fixed != kd) continue;
-        descs.push_back(pl.p);
-        starts.push_back((uint32_t)acc);
-        acc += pl.wgs;
-        if (pl.p.T < 10) uniform = false;
-      }
-      if (descs.empty()) continue;
-      if (acc >= (1ull << 31)) return set_error(ctx, STWO_HIP_EINVAL, "batch_create: grid too large");
-      LevelLaunch ll{};
-      ll.inverse = inverse;
-      ll.fused = false;
-      ll.kind = kd != 0 ? (int)kd : (uniform ? -1 : 0);
-      ll.groups_off = st.put(descs.data(), descs.size() * sizeof(FftPass2));
-      ll.wgs_off = st.put(starts.data(), starts.size() * sizeof(uint32_t));
-      ll.n_groups = (uint32_t)descs.size();
-      ll.total_wgs = (uint32_t)acc;
-      ll.wg_log = wg_log;
-      levels.push_back(ll);
-    }
-    return STWO_HIP_OK;
-  };
-  // The matrix passes of every group that takes them.  The low pass is the
-  // first of the inverse levels and the last of the forward ones; the top pass
-  // runs after the inverse levels, fused with the forward one where the set
-  // has both.
-  auto add_mx_low = [&](bool inverse) -> int {
-    uint64_t units = 0, acc = 0;
-    auto takes = [&](size_t gi) { return gp[gi].matrix && gt[gi].stage != (inverse ? BATCH_RFFT : BATCH_IFFT); };
-    for (size_t gi = 0; gi < gt.size(); gi++)
-      if (takes(gi)) units += mx_low_units(gt[gi].count, gt[gi].n + (inverse ? 0 : gt[gi].b));
-    std::vector<MxLow> descs;
-    for (size_t gi = 0; gi < gt.size(); gi++) {
-      if (!takes(gi)) continue;
-      const GroupTabs &t = gt[gi];
-      const size_t tab = inverse ? t.ifft_off : gp[gi].mx.top_layers ? t.inplace_off : t.rfft_off;
-      uint32_t wgs = 0;
-      descs.push_back(mx_low(tw, (const FftCol *)(dbase + tab), t.count, t.n, t.n + (inverse ? 0 : t.b), inverse,
-                             gp[gi].mx, units, true, &wgs));
-      descs.back().wg_start = wgs;
-    }
-    if (descs.empty()) return STWO_HIP_OK;
-    // the longest workgroups start first
-    std::stable_sort(descs.begin(), descs.end(), [](const MxLow &a, const MxLow &c) { return a.iters > c.iters; });
-    for (MxLow &d : descs) {
-      const uint32_t wgs = d.wg_start;
-      d.wg_start = (uint32_t)acc;
-      acc += wgs;
-    }
-    if (acc >= (1ull << 31)) return set_error(ctx, STWO_HIP_EINVAL, "batch_create: grid too large");
-    LevelLaunch ll{};
-    ll.inverse = inverse;
-    ll.matrix = true;
-    ll.groups_off = st.put(descs.data(), descs.size() * sizeof(MxLow));
-    ll.n_groups = (uint32_t)descs.size();
-    ll.total_wgs = (uint32_t)acc;
-    levels.push_back(ll);
-    return STWO_HIP_OK;
-  };
-  auto add_mx_tops = [&](int stage) -> int {
-    for (uint32_t layers : {8u, 4u}) {
-      uint64_t units = 0, acc = 0;
-      auto takes = [&](size_t gi) {
-        return gp[gi].matrix && gt[gi].stage == stage && gp[gi].mx.top_layers == layers;
-      };
-      for (size_t gi = 0; gi < gt.size(); gi++)
-        if (takes(gi)) units += mx_top_units(gt[gi].count, gt[gi].n, gp[gi].mx);
-      std::vector<MxTop> descs;
-      for (size_t gi = 0; gi < gt.size(); gi++) {
-        if (!takes(gi)) continue;
-        const GroupTabs &t = gt[gi];
-        uint32_t wgs = 0;
-        descs.push_back(mx_top(tw, (const FftCol *)(dbase + t.ifft_off), (const FftCol *)(dbase + t.rfft_off), t.count,
-                               t.n, t.b, stage == BATCH_IFFT || !(flags & STWO_HIP_BATCH_DROP_COEFFS), gp[gi].mx, units,
-                               true, &wgs));
-        descs.back().wg_start = (uint32_t)acc;
-        acc += wgs;
-      }
-      if (descs.empty()) continue;
-      if (acc >= (1ull << 31)) return set_error(ctx, STWO_HIP_EINVAL, "batch_create: grid too large");
-      LevelLaunch ll{};
-      ll.matrix = true;
-      ll.mx_layers = layers;
-      ll.mx_inv = stage != BATCH_RFFT;
-      ll.mx_fwd = stage != BATCH_IFFT;
-      ll.groups_off = st.put(descs.data(), descs.size() * sizeof(MxTop));
-      ll.n_groups = (uint32_t)descs.size();
-      ll.total_wgs = (uint32_t)acc;
-      levels.push_back(ll);
-    }
-    return STWO_HIP_OK;
-  };
-  for (int dir = 0; dir < 2; dir++) {
-    const bool inverse = dir == 0;
-    int mrc = inverse ? add_mx_low(true) : add_mx_tops(BATCH_LDE);
-    if (!mrc && !inverse) mrc = add_mx_tops(BATCH_RFFT);
-    if (mrc) {
-      release();
-      return mrc;
-    }
-    // (level, workgroup size) -> passes of every group (the fused ones aside)
-    std::map<std::pair<uint32_t, uint32_t>, std::vector<PassLaunch>> by_level;
-    for (const GroupPasses &g : gp) {
-      const std::vector<PassLaunch> &passes = inverse ? g.inv : g.fwd;
-      const size_t k0 = (!inverse && g.fused) ? 1 : 0, k1 = passes.size() - ((inverse && g.fused) ? 1 : 0);
-      for (size_t k = k0; k < k1; k++) {
-        uint32_t level = inverse ? (uint32_t)k : (uint32_t)(passes.size() - 1 - k);
-        if (g.matrix) level = 1;  // the middle one of three
-        by_level[{level, passes[k].wg_log}].push_back(passes[k]);
-      }
-    }
-    if (!inverse) {
-      // the fused passes run after every IFFT level and before every RFFT one
-      std::map<std::pair<uint32_t, int>, std::vector<size_t>> fused;  // (wg_log, kind) -> groups
-      for (size_t gi = 0; gi < gp.size(); gi++)
-        if (gp[gi].fused)
-          fused[{gp[gi].inv.back().wg_log, lde_kind(gp[gi].inv.back(), gp[gi].fwd.front())}].push_back(gi);
-      for (auto &kv : fused) {
-        std::vector<FftPass2> pis, pfs;
-        std::vector<uint32_t> starts;
-        uint64_t acc = 0;
-        for (size_t gi : kv.second) {
-          pis.push_back(gp[gi].inv.back().p);
-          pfs.push_back(gp[gi].fwd.front().p);
-          starts.push_back((uint32_t)acc);
-          acc += gp[gi].inv.back().wgs;
-        }
-        if (acc >= (1ull << 31)) {
-          release();
-          return set_error(ctx, STWO_HIP_EINVAL, "batch_create: grid too large");
-        }
-        LevelLaunch ll{};
-        ll.inverse = false;
-        ll.fused = true;
-        ll.kind = kv.first.second;
-        ll.groups_off = st.put(pis.data(), pis.size() * sizeof(FftPass2));
-        ll.fwd_off = st.put(pfs.data(), pfs.size() * sizeof(FftPass2));
-        ll.wgs_off = st.put(starts.data(), starts.size() * sizeof(uint32_t));
-        ll.n_groups = (uint32_t)pis.size();
-        ll.total_wgs = (uint32_t)acc;
-        ll.wg_log = kv.first.first;
-        levels.push_back(ll);
-      }
-    }
-    std::vector<std::pair<uint32_t, uint32_t>> order;
-    for (auto &kv : by_level) order.push_back(kv.first);
-    if (!inverse) std::reverse(order.begin(), order.end());  // forward: highest level first
-    for (const auto &key : order) {
-      int rc = add_level(inverse, key.second, by_level[key]);
-      if (rc) {
-        release();
-        return rc;
-      }
-    }
-    mrc = inverse ? add_mx_tops(BATCH_IFFT) : add_mx_low(false);
-    if (mrc) {
-      release();
-      return mrc;
-    }
+  int lrc = build_levels(ctx, tw, gt, dbase, !(flags & STWO_HIP_BATCH_DROP_COEFFS), true, st, levels);
+  if (lrc) {
+    release();
+    return lrc;
   }
   // The trees, step by step (layers max_log .. 0 of a mixed tree with runs of
   // pure node layers in one; leaves and nodes of a lifted one): the steps of one
   // kind that the trees have at the same place share a launch.  Alone, most
-  // trees leave the device idle: 12 trees of 2^13 to 2^19 leaves took 470 us
+  // trees leave the device idle: 12 trees of 2^13 and 2^17 leaves took 470 us
   // one after another, 205 us in shared launches.
   std::vector<TreeWave> waves;
   {
@@ -528,25 +583,8 @@ int batch_create_trees(stwo_hip_ctx *ctx, const BatchTree *trees, size_t n_trees
   b->mem_from_job = from_job;
   const uint32_t keep_coeffs = (flags & STWO_HIP_BATCH_DROP_COEFFS) ? 0u : 1u;
   b->issue = [levels, waves, dbase, keep_coeffs](stwo_hip_ctx *c) -> int {
-    for (const LevelLaunch &ll : levels) {
-      if (ll.matrix) {
-        int rc = ll.mx_layers
-                     ? launch_mx_top(c, nullptr, (const MxTop *)(dbase + ll.groups_off), ll.n_groups, ll.total_wgs,
-                                     ll.mx_layers, ll.mx_inv, ll.mx_fwd)
-                     : launch_mx_low(c, nullptr, (const MxLow *)(dbase + ll.groups_off), ll.n_groups, ll.total_wgs,
-                                     ll.inverse);
-        if (rc) return rc;
-        continue;
-      }
-      int rc = ll.fused ? launch_lde_multi(c, (const FftPass2 *)(dbase + ll.groups_off),
-                                           (const FftPass2 *)(dbase + ll.fwd_off),
-                                           (const uint32_t *)(dbase + ll.wgs_off), ll.n_groups, ll.total_wgs,
-                                           ll.wg_log, ll.kind, keep_coeffs)
-                        : launch_fft_multi(c, ll.inverse, (const FftPass2 *)(dbase + ll.groups_off),
-                                           (const uint32_t *)(dbase + ll.wgs_off), ll.n_groups, ll.total_wgs,
-                                           ll.wg_log, ll.kind);
-      if (rc) return rc;
-    }
+    int frc = issue_levels(c, levels, dbase, keep_coeffs);
+    if (frc) return frc;
     for (const TreeWave &w : waves) {
       int rc = w.n > 1 ? launch_merkle_multi(c, w.step.kind, w.step.layer.lifted, dbase + w.off, w.n, w.wgs)
                        : launch_merkle(c, w.step);
@@ -587,6 +625,78 @@ int batch_create_trees(stwo_hip_ctx *ctx, const BatchTree *trees, size_t n_trees
   }
   *out = b;
   return STWO_HIP_OK;
+}
+
+// The transforms of several groups in shared launches, straight away; *done =
+// false (nothing launched) where their tables do not fit the upload ring or a
+// group's output meets another group's columns, whose order then counts.
+int run_fft_sets(stwo_hip_ctx *ctx, const std::vector<FftSet> &sets, const stwo_hip_twiddles *tw, bool store_coeffs,
+                 bool *done) {
+  *done = false;
+  // [first, end) of every column, with its group and whether it is written
+  struct Span {
+    uintptr_t at, end;
+    uint32_t group, out;
+  };
+  std::vector<Span> spans;
+  for (uint32_t g = 0; g < sets.size(); g++)
+    for (const FftCol &c : sets[g].cols) {
+      const uint32_t b = sets[g].b;
+      const bool in_place = sets[g].stage != BATCH_RFFT;
+      spans.push_back({(uintptr_t)c.in, (uintptr_t)(c.in + ((size_t)1 << sets[g].n)), g, in_place});
+      if (c.out != c.in) spans.push_back({(uintptr_t)c.out, (uintptr_t)(c.out + ((size_t)1 << (sets[g].n + b))), g, 1});
+    }
+  auto by_at = [](const Span &a, const Span &c) { return a.at < c.at; };
+  if (!std::is_sorted(spans.begin(), spans.end(), by_at)) std::sort(spans.begin(), spans.end(), by_at);
+  // The furthest end met so far, and the furthest of the other groups.
+  struct Far {
+    uintptr_t end = 0, end2 = 0;
+    uint32_t group = 0;
+    void add(uintptr_t e, uint32_t g) {
+      if (g == group) {
+        end = std::max(end, e);
+      } else if (e > end) {
+        end2 = end;
+        end = e;
+        group = g;
+      } else {
+        end2 = std::max(end2, e);
+      }
+    }
+    uintptr_t other(uint32_t g) const { return g == group ? end2 : end; }
+  } any, written;
+  for (const Span &s : spans) {
+    if (s.at < (s.out ? any : written).other(s.group)) return STWO_HIP_OK;
+    any.add(s.end, s.group);
+    if (s.out) written.add(s.end, s.group);
+  }
+  Staging st;
+  std::vector<GroupTabs> gt;
+  for (const FftSet &s : sets) gt.push_back(put_group(st, s.n, s.b, s.stage, s.cols));
+  // The matrix passes where their units, over all groups, fill the device: they
+  // are far fewer and longer than the vector passes' workgroups.
+  uint64_t units = 0;
+  for (const GroupTabs &t : gt) {
+    MxPlan mx;
+    if (mx_plan(ctx, tw, t.n, t.stage == BATCH_IFFT ? 0 : t.b, t.stage == BATCH_IFFT, t.count, t.aligned16, true, &mx))
+      units += mx_low_units(t.count, t.n);
+  }
+  const size_t bound = ((st.host.size() + 255) & ~(size_t)255) + levels_bound(gt.size());
+  uint8_t *h = nullptr, *d = nullptr;
+  if (bound > ctx->arena_cap / 2) return STWO_HIP_OK;
+  int rc = upload_begin(ctx, bound, &h, &d);
+  if (rc) return rc;
+  std::vector<LevelLaunch> levels;
+  rc = build_levels(ctx, tw, gt, d, store_coeffs, units >= kMxMinUnits, st, levels);
+  if (!rc && st.host.size() > bound) rc = set_error(ctx, STWO_HIP_EINVAL, "internal: FFT descriptor area overflow");
+  if (rc) {
+    upload_end(ctx, 0);
+    return rc;
+  }
+  memcpy(h, st.host.data(), st.host.size());
+  upload_end(ctx, st.host.size());
+  *done = true;
+  return issue_levels(ctx, levels, d, store_coeffs);
 }
 
 }  // namespace stwo_hip

@@ -152,6 +152,11 @@ int upload_table(stwo_hip_ctx *ctx, const void *src, size_t bytes, void **dptr);
 // device allocation of the library goes through here.
 hipError_t ctx_malloc(stwo_hip_ctx *ctx, void **dptr, size_t bytes);
 int upload_tables(stwo_hip_ctx *ctx, size_t n, const void *const *srcs, const size_t *bytes, void **dptrs);
+// The same in two halves, for tables that hold their own device addresses: room
+// for `bytes` (at most half the ring) at *host, which the device sees at *dev;
+// `used` of it, once written.  No upload or launch in between.
+int upload_begin(stwo_hip_ctx *ctx, size_t bytes, uint8_t **host, uint8_t **dev);
+void upload_end(stwo_hip_ctx *ctx, size_t used);
 // upload_tables for tables that repeat from call to call (column lists of
 // buffers a caller reuses): a call whose tables equal the previous call's
 // under `key` gets the device copy kept from then, with no copy on the

@@ -1268,6 +1268,24 @@ static int run_fft_group(stwo_hip_ctx *ctx, const std::vector<FftCol> &cols, uin
   return STWO_HIP_OK;
 }
 
+// The groups (log size -> columns) of at least 2^4 in shared launches, where
+// there are several; the ones done are taken out.
+static int share_launches(stwo_hip_ctx *ctx, std::map<uint32_t, std::vector<FftCol>> &groups, uint32_t b, int stage,
+                          const stwo_hip_twiddles *tw, bool store_coeffs) {
+  std::vector<FftSet> sets;
+  // largest first: their workgroups start first
+  for (auto g = groups.rbegin(); g != groups.rend() && g->first >= 4; ++g) {
+    if (g->second.size() > 65535) return STWO_HIP_OK;
+    sets.push_back({g->first, b, stage, g->second});
+  }
+  if (sets.size() < 2) return STWO_HIP_OK;
+  bool done = false;
+  int rc = run_fft_sets(ctx, sets, tw, store_coeffs, &done);
+  if (!rc && done)
+    for (const FftSet &st : sets) groups.erase(st.n);
+  return rc;
+}
+
 static int bit_reverse_one(stwo_hip_ctx *ctx, uint32_t *col, uint32_t log_size) {
   if (log_size >= 2 * kBrLog) {
     uint32_t mids = 1u << (log_size - 2 * kBrLog);
@@ -1326,14 +1344,17 @@ int stwo_hip_interpolate_columns(stwo_hip_ctx *ctx, uint32_t *const *cols, const
     groups[log_sizes[i]].push_back({cols[i], cols[i]});
   }
   for (auto &g : groups) {
-    uint32_t N = g.first;
-    stwo_hip_coset dom = {half_odds_initial(N - 1), N - 1};
-    int rc = check_domain(ctx, dom, tw);
+    int rc = check_domain(ctx, {half_odds_initial(g.first - 1), g.first - 1}, tw);
     if (rc) return rc;
+  }
+  int rc = share_launches(ctx, groups, 0, BATCH_IFFT, tw, true);
+  if (rc) return rc;
+  for (auto &g : groups) {
+    const uint32_t N = g.first;
     for (size_t off = 0; off < g.second.size(); off += 65535) {
       std::vector<FftCol> part(g.second.begin() + off,
                                g.second.begin() + std::min(g.second.size(), off + (size_t)65535));
-      rc = run_fft_group(ctx, part, N, N, tw, true, dom);
+      rc = run_fft_group(ctx, part, N, N, tw, true, {half_odds_initial(N - 1), N - 1});
       if (rc) return rc;
     }
   }
@@ -1368,14 +1389,18 @@ int stwo_hip_evaluate_polynomials(stwo_hip_ctx *ctx, const uint32_t *const *coef
     groups[log_sizes[i]].push_back({coeffs[i], outs[i]});
   }
   for (auto &g : groups) {
-    uint32_t n = g.first, N = n + log_blowup;
-    stwo_hip_coset dom = {half_odds_initial(N - 1), N - 1};
-    int rc = check_domain(ctx, dom, tw);
+    const uint32_t N = g.first + log_blowup;
+    int rc = check_domain(ctx, {half_odds_initial(N - 1), N - 1}, tw);
     if (rc) return rc;
+  }
+  int rc = share_launches(ctx, groups, log_blowup, BATCH_RFFT, tw, true);
+  if (rc) return rc;
+  for (auto &g : groups) {
+    const uint32_t n = g.first, N = n + log_blowup;
     for (size_t off = 0; off < g.second.size(); off += 65535) {
       std::vector<FftCol> part(g.second.begin() + off,
                                g.second.begin() + std::min(g.second.size(), off + (size_t)65535));
-      rc = run_fft_group(ctx, part, n, N, tw, false, dom);
+      rc = run_fft_group(ctx, part, n, N, tw, false, {half_odds_initial(N - 1), N - 1});
       if (rc) return rc;
     }
   }
@@ -1386,28 +1411,34 @@ int stwo_hip_extend_evals(stwo_hip_ctx *ctx, uint32_t *const *cols, const uint32
                           uint32_t log_blowup, const stwo_hip_twiddles *tw, uint32_t *const *outs, int store_coeffs) {
   if (!ctx) return STWO_HIP_EINVAL;
   STWO_HIP_CHECK_ARG(ctx, n_cols == 0 || (cols && log_sizes && outs), "extend_evals: NULL arrays");
-  std::map<uint32_t, std::vector<size_t>> groups;
+  std::map<uint32_t, std::vector<FftCol>> groups;
   for (size_t i = 0; i < n_cols; i++) {
     STWO_HIP_CHECK_ARG(ctx, cols[i] && outs[i], "extend_evals: NULL column %zu", i);
     STWO_HIP_CHECK_ARG(ctx, log_sizes[i] >= 1 && log_sizes[i] <= 28 && log_blowup <= 28 &&
                                 log_sizes[i] + log_blowup <= 28,
                        "extend_evals: bad log size %u + %u", log_sizes[i], log_blowup);
-    groups[log_sizes[i]].push_back(i);
+    groups[log_sizes[i]].push_back({cols[i], outs[i]});
   }
   for (auto &g : groups) {
     const uint32_t n = g.first, N = n + log_blowup;
+    int rc = check_domain(ctx, {half_odds_initial(n - 1), n - 1}, tw);
+    if (rc) return rc;
+    rc = check_domain(ctx, {half_odds_initial(N - 1), N - 1}, tw);
+    if (rc) return rc;
+  }
+  int rc = share_launches(ctx, groups, log_blowup, BATCH_LDE, tw, store_coeffs != 0);
+  if (rc) return rc;
+  for (auto &g : groups) {
+    const uint32_t n = g.first, N = n + log_blowup;
     const stwo_hip_coset dom_i = {half_odds_initial(n - 1), n - 1}, dom_f = {half_odds_initial(N - 1), N - 1};
-    int rc = check_domain(ctx, dom_i, tw);
-    if (rc) return rc;
-    rc = check_domain(ctx, dom_f, tw);
-    if (rc) return rc;
     for (size_t off = 0; off < g.second.size(); off += 65535) {
       const size_t e = std::min(g.second.size(), off + (size_t)65535);
       std::vector<FftCol> part;
       std::vector<uint32_t *> po;
       for (size_t k = off; k < e; k++) {
-        part.push_back({cols[g.second[k]], cols[g.second[k]]});
-        po.push_back(outs[g.second[k]]);
+        uint32_t *col = (uint32_t *)g.second[k].in;
+        part.push_back({col, col});
+        po.push_back(g.second[k].out);
       }
       if (n >= 4) {
         rc = run_lde_group(ctx, part, po, n, log_blowup, tw, store_coeffs != 0);

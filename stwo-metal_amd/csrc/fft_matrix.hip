@@ -766,7 +766,7 @@ __global__ void __launch_bounds__(1024) mx_low_multi_kernel(const MxLow *groups,
 
 }  // namespace
 
-constexpr uint64_t kMxMinUnits = 256, kMxBatchUnits = 32;
+constexpr uint64_t kMxBatchUnits = 32;  // kMxMinUnits, shared launch
 
 uint64_t mx_top_units(uint32_t n_cols, uint32_t n, const MxPlan &plan) {
   return plan.top_layers == 8 ? (uint64_t)n_cols << (n - 14) : 0;

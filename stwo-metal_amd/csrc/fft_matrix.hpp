@@ -41,6 +41,9 @@ struct MxPlan {
   bool mid = false;
 };
 
+// Low-pass units (4 columns x 2^12 words) from which the matrix passes pay alone.
+constexpr uint64_t kMxMinUnits = 256;
+
 // Whether a group's transform (log coefficients n, log blowup b; b = 0 for an
 // interpolation) takes the matrix passes, alone or in a batched launch, and
 // their split.

@@ -995,7 +995,7 @@ static int fri_flush(stwo_hip_ctx *ctx, FriChain &c, const stwo_hip_twiddles *tw
 //
 // A chain is a row of dependent launches that leave the device nearly idle, so
 // chains that stand at the same layer size share theirs (the larger ones begin
-// alone): 12 commits of 2^14 to 2^19 one after another took 2.6 ms of
+// alone): 12 commits of 2^13 and 2^17 one after another took 2.6 ms of
 // device time, side by side they take 0.5 ms.
 static int fri_run(stwo_hip_ctx *ctx, FriChain *const *chains, size_t n, const stwo_hip_twiddles *tw) {
   const uint32_t *itw_end = tw->d_itw + tw->len;

@@ -101,6 +101,16 @@ struct BatchTree {
 int batch_create_trees(stwo_hip_ctx *ctx, const BatchTree *trees, size_t n_trees, const stwo_hip_twiddles *tw,
                        int flags, stwo_hip_batch **out);
 
+// Columns {in, out} of one size (in place but for evaluations: in = the column,
+// out = its evaluations) and what to do with them.
+struct FftSet {
+  uint32_t n, b;  // 4 <= n
+  int stage;      // BatchStage
+  std::vector<FftCol> cols;
+};
+int run_fft_sets(stwo_hip_ctx *ctx, const std::vector<FftSet> &sets, const stwo_hip_twiddles *tw, bool store_coeffs,
+                 bool *done);
+
 // stwo_hip_wide_fib_constraint_quotients, writing the quotients over accum
 // instead of adding them when !accumulate (a single component needs no zeroed
 // accumulator); the random coefficient from the host (random_coeff) or

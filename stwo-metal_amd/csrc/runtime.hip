@@ -149,6 +149,33 @@ static size_t table_span(size_t bytes) {
   return sz ? sz : 256;
 }
 
+int upload_begin(stwo_hip_ctx *ctx, size_t bytes, uint8_t **host, uint8_t **dev) {
+  // One contiguous range of the ring for all of a call's tables: a table
+  // handed out earlier is only safe from being overwritten once the kernels
+  // that read it are enqueued (a later copy then follows them in stream
+  // order), so the tables one launch sequence needs must not wrap onto each
+  // other.
+  size_t off = ctx->arena_head;
+  if (off + bytes > ctx->arena_cap) off = 0;
+  // A range that does not extend the pending one (the ring wrapped) starts a
+  // new one: the pending bytes are copied first, so that the wait below also
+  // covers them.
+  int rc = STWO_HIP_OK;
+  if (ctx->pend_end > ctx->pend_begin && off != ctx->pend_end) rc = flush_uploads(ctx);
+  if (rc) return rc;
+  rc = arena_wait_range(ctx, off, off + bytes);
+  if (rc) return rc;
+  if (ctx->pend_end <= ctx->pend_begin) ctx->pend_begin = ctx->pend_end = off;
+  *host = ctx->h_arena + off;
+  *dev = ctx->d_arena + off;
+  return STWO_HIP_OK;
+}
+
+void upload_end(stwo_hip_ctx *ctx, size_t used) {
+  ctx->pend_end += table_span(used) * (used != 0);
+  ctx->arena_head = ctx->pend_end;
+}
+
 int upload_tables(stwo_hip_ctx *ctx, size_t n, const void *const *srcs, const size_t *bytes, void **dptrs) {
   size_t total = 0;
   for (size_t i = 0; i < n; i++) total += table_span(bytes[i]);
@@ -170,29 +197,16 @@ int upload_tables(stwo_hip_ctx *ctx, size_t n, const void *const *srcs, const si
     }
     return STWO_HIP_OK;
   }
-  // One contiguous range of the ring for all of the call's tables: a table
-  // handed out earlier is only safe from being overwritten once the kernels
-  // that read it are enqueued (a later copy then follows them in stream
-  // order), so the tables one launch sequence needs must not wrap onto each
-  // other.
-  size_t off = ctx->arena_head;
-  if (off + total > ctx->arena_cap) off = 0;
-  // A range that does not extend the pending one (the ring wrapped) starts a
-  // new one: the pending bytes are copied first, so that the wait below also
-  // covers them.
-  int rc = STWO_HIP_OK;
-  if (ctx->pend_end > ctx->pend_begin && off != ctx->pend_end) rc = flush_uploads(ctx);
+  uint8_t *h = nullptr, *d = nullptr;
+  int rc = upload_begin(ctx, total, &h, &d);
   if (rc) return rc;
-  rc = arena_wait_range(ctx, off, off + total);
-  if (rc) return rc;
-  if (ctx->pend_end <= ctx->pend_begin) ctx->pend_begin = off;
+  size_t off = 0;
   for (size_t i = 0; i < n; i++) {
-    if (bytes[i]) memcpy(ctx->h_arena + off, srcs[i], bytes[i]);
-    dptrs[i] = ctx->d_arena + off;
+    if (bytes[i]) memcpy(h + off, srcs[i], bytes[i]);
+    dptrs[i] = d + off;
     off += table_span(bytes[i]);
   }
-  ctx->pend_end = off;
-  ctx->arena_head = off;
+  upload_end(ctx, total);
   return STWO_HIP_OK;
 }
 

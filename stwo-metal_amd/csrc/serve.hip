@@ -203,7 +203,7 @@ int check_job(const stwo_hip_server *s, const stwo_hip_job_desc &d) {
 
 // The callers' device columns of a group into its memory, one launch: a copy
 // call per column costs the stream 1.9 us, 1.2 of 5.2 ms for 624 columns of 2^12
-// to 2^17; this moves them in 13 us (bound by memory).  16 bytes a lane where
+// and 2^15; this moves them in 13 us (bound by memory).  16 bytes a lane where
 // the column is aligned to that.
 struct ColCopy {
   const uint32_t *src;
