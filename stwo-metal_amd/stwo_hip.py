@@ -9,6 +9,7 @@ objects owning a device allocation; numpy uint32 arrays cross the host
 boundary.  There is no CPU fallback: if the library is missing or no GPU is
 visible, loading fails with an exception.
 """
+import array
 import ctypes
 import time
 import os
@@ -230,6 +231,14 @@ def _ptrs(bufs):
     for i, b in enumerate(bufs):
         arr[i] = b.ptr if isinstance(b, DeviceBuf) else b
     return arr
+
+
+def _words(values):
+    """A list of words as a uint32 array (numpy's own conversion takes three times as long)."""
+    try:
+        return np.frombuffer(array.array("I", values), dtype=np.uint32)
+    except TypeError:
+        return np.array(values, dtype=np.uint32)
 
 
 class DeviceBuf:
@@ -530,12 +539,24 @@ class Context:
     def compute_fri_quotients(self, cols, log_sizes, samples_per_col, random_coeff, lifting_log, out4):
         """compute_fri_quotients; samples_per_col: per column a list of
         (x[4], y[4], value[4]) PointSamples; out4: 4 device columns of 2^lifting_log."""
-        flat, counts = [], []
+        # Points repeat from sample to sample, so each run of one is taken once:
+        # 264 samples at one point 205 -> 66 us (98 us with a point object each).
+        pts, runs, vals, counts, px, py = [], [], [], [], None, None
         for ss in samples_per_col:
             counts.append(len(ss))
             for x, y, v in ss:
-                flat.extend(list(x) + list(y) + list(v))
-        fl = np.array(flat or [0], dtype=np.uint32)
+                if x is px and y is py:
+                    runs[-1] += 1
+                else:
+                    pts.extend(x)
+                    pts.extend(y)
+                    runs.append(1)
+                    px, py = x, y
+                vals.extend(v)
+        fl = np.zeros((max(1, sum(runs)), 12), dtype=np.uint32)
+        if runs:
+            fl[:, :8] = np.repeat(_words(pts).reshape(-1, 8), runs, axis=0)
+            fl[:, 8:] = _words(vals).reshape(-1, 4)
         cn = np.array(counts or [0], dtype=np.uint32)
         ls = np.ascontiguousarray(list(log_sizes) or [0], dtype=np.uint32)
         rc = np.ascontiguousarray(random_coeff, dtype=np.uint32)
