@@ -23,6 +23,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "fft_column.hpp"
 #include "fft_matrix.hpp"
 #include "field.hpp"
 #include "internal.hpp"
@@ -62,6 +63,8 @@ struct LevelLaunch {
   // pass with its directions, or the low pass (mx_layers = 0)
   bool matrix = false, mx_inv = false, mx_fwd = false;
   uint32_t mx_layers = 0;
+  // a workgroup per column (groups_off: ColumnFft descriptors), largest N
+  uint32_t column_N = 0;
 };
 
 // One tree's layer tables and shape.
@@ -122,7 +125,7 @@ GroupTabs put_group(Staging &st, uint32_t n, uint32_t b, int stage, const std::v
 // tables per launch (2 directions x 4 levels x 2 workgroup sizes x at most 14
 // schedule kinds, and the fused launches).
 size_t levels_bound(size_t n_groups) {
-  return n_groups * (sizeof(MxTop) + 2 * sizeof(MxLow)) + 8 * 256 + 2 * 4 * n_groups * (sizeof(FftPass2) + 8) +
+  return n_groups * (sizeof(MxTop) + 2 * sizeof(MxLow) + sizeof(ColumnFft)) + 14 * 256 + 2 * 4 * n_groups * (sizeof(FftPass2) + 8) +
          2 * 4 * 2 * 14 * 2 * 256 + 8192;
 }
 
@@ -143,11 +146,28 @@ int build_levels(stwo_hip_ctx *ctx, const stwo_hip_twiddles *tw, const std::vect
     std::vector<PassLaunch> inv, fwd;
     bool fused = false;
     bool matrix = false;  // first and last passes on the matrix cores
+    bool column = false;  // a workgroup per column
     MxPlan mx;
   };
   std::vector<GroupPasses> gp(gt.size());
+  // The smallest sizes take a workgroup per column, up to what one launch of
+  // them may hold (the groups come largest first).
+  size_t column_words = 0;
+  for (size_t gi = gt.size(); gi-- > 0;) {
+    const GroupTabs &t = gt[gi];
+    const bool inv = t.stage != BATCH_RFFT, fwd = t.stage != BATCH_IFFT;
+    const uint32_t N = t.n + (fwd ? t.b : 0);
+    MxPlan mx;
+    if (!column_fft_takes(ctx, t.n, N, t.count, inv, fwd) || column_words + ((size_t)t.count << t.n) > kColumnFftWords ||
+        (matrix && (!inv || mx_plan(ctx, tw, t.n, 0, true, t.count, t.aligned16, true, &mx)) &&
+         (!fwd || mx_plan(ctx, tw, t.n, t.b, false, t.count, t.aligned16, true, &mx))))
+      continue;
+    gp[gi].column = true;
+    column_words += (size_t)t.count << t.n;
+  }
   for (size_t gi = 0; gi < gt.size(); gi++) {
     const GroupTabs &t = gt[gi];
+    if (gp[gi].column) continue;
     for (int dir = 0; dir < 2; dir++) {
       const bool inverse = dir == 0;
       if ((inverse && t.stage == BATCH_RFFT) || (!inverse && t.stage == BATCH_IFFT)) continue;
@@ -301,14 +321,53 @@ int build_levels(stwo_hip_ctx *ctx, const stwo_hip_twiddles *tw, const std::vect
     }
     return STWO_HIP_OK;
   };
+  // Small and large columns apart, a launch's workgroups having the lanes and the
+  // LDS of its largest; together where there is a CU for each (then the further
+  // launch costs more, 5 us).
+  auto add_columns = [&](int stage) {
+    uint64_t cols = 0;
+    for (size_t gi = 0; gi < gt.size(); gi++)
+      if (gp[gi].column && gt[gi].stage == stage) cols += gt[gi].count;
+    const bool apart = cols > 256;
+    for (uint32_t large = 0; large <= (uint32_t)apart; large++) {
+      std::vector<ColumnFft> descs;
+      uint32_t acc = 0, max_N = 0;
+      for (size_t gi = 0; gi < gt.size(); gi++) {
+        const GroupTabs &t = gt[gi];
+        const uint32_t N = t.n + (stage == BATCH_IFFT ? 0 : t.b);
+        if (!gp[gi].column || t.stage != stage || (apart && (N > 10) != large)) continue;
+        descs.push_back(column_fft(tw, (const FftCol *)(dbase + t.ifft_off), (const FftCol *)(dbase + t.rfft_off),
+                                   t.count, t.n, N, store_coeffs));
+        descs.back().wg_start = acc;
+        acc += t.count;
+        max_N = std::max(max_N, N);
+      }
+      if (descs.empty()) continue;
+      LevelLaunch ll{};
+      ll.column_N = max_N;
+      ll.mx_inv = stage != BATCH_RFFT;
+      ll.mx_fwd = stage != BATCH_IFFT;
+      ll.groups_off = st.put(descs.data(), descs.size() * sizeof(ColumnFft));
+      ll.n_groups = (uint32_t)descs.size();
+      ll.total_wgs = acc;
+      levels.push_back(ll);
+    }
+  };
   for (int dir = 0; dir < 2; dir++) {
     const bool inverse = dir == 0;
+    if (inverse) {
+      add_columns(BATCH_IFFT);
+      add_columns(BATCH_LDE);
+    } else {
+      add_columns(BATCH_RFFT);
+    }
     int mrc = inverse ? add_mx_low(true) : add_mx_tops(BATCH_LDE);
     if (!mrc && !inverse) mrc = add_mx_tops(BATCH_RFFT);
     if (mrc) return mrc;
     // (level, workgroup size) -> passes of every group (the fused ones aside)
     std::map<std::pair<uint32_t, uint32_t>, std::vector<PassLaunch>> by_level;
     for (const GroupPasses &g : gp) {
+      if (g.column) continue;
       const std::vector<PassLaunch> &passes = inverse ? g.inv : g.fwd;
       const size_t k0 = (!inverse && g.fused) ? 1 : 0, k1 = passes.size() - ((inverse && g.fused) ? 1 : 0);
       for (size_t k = k0; k < k1; k++) {
@@ -362,6 +421,12 @@ int build_levels(stwo_hip_ctx *ctx, const stwo_hip_twiddles *tw, const std::vect
 
 int issue_levels(stwo_hip_ctx *c, const std::vector<LevelLaunch> &levels, uint8_t *dbase, uint32_t keep_coeffs) {
   for (const LevelLaunch &ll : levels) {
+    if (ll.column_N) {
+      int rc = launch_column_fft_multi(c, (const ColumnFft *)(dbase + ll.groups_off), ll.n_groups, ll.total_wgs,
+                                       ll.column_N, ll.mx_inv, ll.mx_fwd);
+      if (rc) return rc;
+      continue;
+    }
     if (ll.matrix) {
       int rc = ll.mx_layers
                    ? launch_mx_top(c, nullptr, (const MxTop *)(dbase + ll.groups_off), ll.n_groups, ll.total_wgs,

@@ -30,6 +30,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "fft_column.hpp"
 #include "fft_dev.hpp"
 #include "fft_matrix.hpp"
 #include "field.hpp"
@@ -1117,6 +1118,10 @@ static int run_fft_group2(stwo_hip_ctx *ctx, const std::vector<FftCol> &cols, vo
   if (mx_plan(ctx, tw, n, N - n, inverse, cols.size(), aligned16, false, &mx))
     return run_mx_group(ctx, (const FftCol *)dtab, (const FftCol *)dtab_out, (uint32_t)cols.size(), n, N, tw, inverse,
                         mx);
+  if (column_fft_takes(ctx, n, N, cols.size(), inverse, !inverse)) {
+    const FftCol *tab = (const FftCol *)dtab;
+    return launch_column_fft(ctx, column_fft(tw, tab, tab, (uint32_t)cols.size(), n, N, true), inverse, !inverse);
+  }
   std::vector<PassLaunch> passes;
   int rc = make_group_passes(ctx, n, N, inverse, (const FftCol *)dtab, (const FftCol *)dtab_out,
                              (uint32_t)cols.size(), tw_end, aligned16, passes);
@@ -1168,6 +1173,10 @@ static int run_lde_group(stwo_hip_ctx *ctx, const std::vector<FftCol> &cols, con
     if (!rc && mx.mid) rc = launch_mx_mid(ctx, tio, nc, n, N, tw, false);
     return rc ? rc : launch_mx_low(ctx, &lf, nullptr, 0, w2, false);
   }
+  if (column_fft_takes(ctx, n, N, cols.size(), true, true))
+    return launch_column_fft(ctx, column_fft(tw, (const FftCol *)d[0], (const FftCol *)d[1], (uint32_t)cols.size(), n, N,
+                                             store_coeffs),
+                             true, true);
   std::vector<PassLaunch> inv, fwd;
   int rc = make_group_passes(ctx, n, n, true, (const FftCol *)d[0], (const FftCol *)d[0], (uint32_t)cols.size(),
                              tw->d_itw2 + tw->len, aligned16, inv);
@@ -1574,11 +1583,12 @@ int stwo_hip_fft_autotune(stwo_hip_ctx *ctx, const uint32_t *log_sizes, size_t n
           }
       float best = 1e30f, def_ms = 0;
       FftTune best_t = def;
-      // Without a choice the shape may take the matrix passes: then those are
-      // the default that a vector plan has to beat.
+      // Without a choice the shape may take the matrix passes or a workgroup per
+      // column: then those are the default that a vector plan has to beat.
       MxPlan mx;
       ctx->fft_tune.erase(fft_tune_key(n, Nd, inverse));
       const bool matrix = mx_plan(ctx, tw, n, Nd - n, inverse, c, true, false, &mx);
+      const bool column = !matrix && column_fft_takes(ctx, n, Nd, c, inverse, !inverse);
       for (auto &ck : cands) {
         rc = make_group_passes(ctx, n, Nd, inverse, first, inpl, (uint32_t)c, tw_end, true, ps, &ck.second);
         if (rc) return rc;
@@ -1593,15 +1603,21 @@ int stwo_hip_fft_autotune(stwo_hip_ctx *ctx, const uint32_t *log_sizes, size_t n
             },
             &ms);
         if (rc) return rc;
-        if (!matrix && !(ck.first < def_key) && !(def_key < ck.first)) def_ms = ms;
+        if (!matrix && !column && !(ck.first < def_key) && !(def_key < ck.first)) def_ms = ms;
         if (ms < best) {
           best = ms;
           best_t = ck.second;
         }
       }
-      if (matrix) {
+      if (matrix || column) {
+        const ColumnFft cf = column_fft(tw, first, first, (uint32_t)c, n, Nd, true);
         rc = time_launches(
-            ctx, [&]() { return run_mx_group(ctx, first, inpl, (uint32_t)c, n, Nd, tw, inverse, mx); }, &def_ms);
+            ctx,
+            [&]() {
+              return matrix ? run_mx_group(ctx, first, inpl, (uint32_t)c, n, Nd, tw, inverse, mx)
+                            : launch_column_fft(ctx, cf, inverse, !inverse);
+            },
+            &def_ms);
         if (rc) return rc;
       }
       // Another plan must beat the default by kTuneMargin: timed alone a shape
