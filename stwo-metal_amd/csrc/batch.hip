@@ -336,8 +336,7 @@ int build_levels(stwo_hip_ctx *ctx, const stwo_hip_twiddles *tw, const std::vect
         const GroupTabs &t = gt[gi];
         const uint32_t N = t.n + (stage == BATCH_IFFT ? 0 : t.b);
         if (!gp[gi].column || t.stage != stage || (apart && (N > 10) != large)) continue;
-        descs.push_back(column_fft(tw, (const FftCol *)(dbase + t.ifft_off), (const FftCol *)(dbase + t.rfft_off),
-                                   t.count, t.n, N, store_coeffs));
+        descs.push_back(column_fft(tw, (const FftCol *)(dbase + t.rfft_off), t.count, t.n, N, store_coeffs));
         descs.back().wg_start = acc;
         acc += t.count;
         max_N = std::max(max_N, N);
@@ -550,7 +549,7 @@ int batch_create_trees(stwo_hip_ctx *ctx, const BatchTree *trees, size_t n_trees
   // launch's table starts aligned.
   size_t tree_steps_bound = 0;
   if (tl.size() > 1)
-    for (const TreeLaunches &L : tl) tree_steps_bound += 2 * L.lt.size() * (sizeof(MerkleLayer) + 256);
+    for (const TreeLaunches &L : tl) tree_steps_bound += 2 * L.lt.size() * (sizeof(MerkleTree) + 256);
   const size_t desc_bytes = levels_bound(gt.size()) + tree_steps_bound;
   int arc = device_alloc(ctx, tables_bytes + desc_bytes, &dmem, &from_job);
   if (arc) return arc;
@@ -578,21 +577,24 @@ int batch_create_trees(stwo_hip_ctx *ctx, const BatchTree *trees, size_t n_trees
       size_t ti = 0;
       for (int l = (int)L.max_log; l >= 0;) {
         const uint32_t *prev = l == (int)L.max_log ? nullptr : L.layers + tree_layer_off((uint32_t)l + 1);
-        if (ti < L.lt.size() && L.lt[ti].log_size == (uint32_t)l) {
-          const auto &t = L.lt[ti++];
-          steps[k].push_back(merkle_layer_step(prev, (const ColRef *)(dbase + t.off), t.count, (uint32_t)l,
+        const auto *t = ti < L.lt.size() && L.lt[ti].log_size == (uint32_t)l ? &L.lt[ti++] : nullptr;
+        const int next = ti < L.lt.size() ? (int)L.lt[ti].log_size : -1;  // the next layer with columns
+        if (t) {
+          steps[k].push_back(merkle_layer_step(prev, (const ColRef *)(dbase + t->off), t->count, (uint32_t)l,
                                                L.layers + tree_layer_off((uint32_t)l), L.mode, lifted));
-          l--;
-          continue;
+          if (!merkle_tree_step(steps[k].back(), (uint32_t)(next + 1), counters)) {
+            l--;
+            continue;
+          }
+        } else {
+          steps[k].push_back(merkle_nodes_step(L.layers, (uint32_t)l + 1, (uint32_t)(next + 1), L.mode, counters));
         }
-        const int next = ti < L.lt.size() ? (int)L.lt[ti].log_size : -1;
-        steps[k].push_back(merkle_nodes_step(L.layers, (uint32_t)l + 1, (uint32_t)(next + 1), L.mode, counters));
         l = next;
       }
       longest = std::max(longest, steps[k].size());
     }
     for (size_t at = 0; at < longest; at++)
-      for (uint32_t kind = kMerkleLayer; kind <= kMerkleNodes1024; kind++) {
+      for (uint32_t kind = 0; kind < kMerkleKinds; kind++) {
         std::vector<const MerkleStep *> same;
         for (const auto &v : steps)
           if (at < v.size() && v[at].kind == kind) same.push_back(&v[at]);
@@ -604,12 +606,15 @@ int batch_create_trees(stwo_hip_ctx *ctx, const BatchTree *trees, size_t n_trees
                            [](const MerkleStep *a, const MerkleStep *c) { return a->wgs > c->wgs; });
           std::vector<MerkleLayer> ls;
           std::vector<MerkleNodes> ns;
+          std::vector<MerkleTree> ts;
           uint64_t acc = 0;
           for (const MerkleStep *s : same) {
             ls.push_back(s->layer);
             ls.back().wg_start = (uint32_t)acc;
             ns.push_back(s->nodes);
             ns.back().wg_start = (uint32_t)acc;
+            ts.push_back(s->tree);
+            ts.back().wg_start = (uint32_t)acc;
             acc += s->wgs;
           }
           if (acc >= (1ull << 31)) {
@@ -618,7 +623,8 @@ int batch_create_trees(stwo_hip_ctx *ctx, const BatchTree *trees, size_t n_trees
           }
           w.wgs = (uint32_t)acc;
           w.off = kind < kMerkleNodes64 ? st.put(ls.data(), ls.size() * sizeof(MerkleLayer))
-                                        : st.put(ns.data(), ns.size() * sizeof(MerkleNodes));
+                  : kind < kMerkleTree  ? st.put(ns.data(), ns.size() * sizeof(MerkleNodes))
+                                        : st.put(ts.data(), ts.size() * sizeof(MerkleTree));
         }
         waves.push_back(w);
       }

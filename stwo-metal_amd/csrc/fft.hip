@@ -1109,19 +1109,12 @@ static int run_mx_group(stwo_hip_ctx *ctx, const FftCol *d_tab, const FftCol *d_
 
 // Radix-16 path for N >= 4: one launch per pass over all columns of the group.
 static int run_fft_group2(stwo_hip_ctx *ctx, const std::vector<FftCol> &cols, void *dtab, void *dtab_out,
-                          uint32_t n, uint32_t N, const stwo_hip_twiddles *tw, bool inverse) {
-  bool aligned16 = true;
-  for (const FftCol &c : cols)
-    if ((((uintptr_t)c.in) | ((uintptr_t)c.out)) & 15) aligned16 = false;
+                          uint32_t n, uint32_t N, const stwo_hip_twiddles *tw, bool inverse, bool aligned16,
+                          const MxPlan *mx) {
   const uint32_t *tw_end = (inverse ? tw->d_itw2 : tw->d_tw2) + tw->len;
-  MxPlan mx;
-  if (mx_plan(ctx, tw, n, N - n, inverse, cols.size(), aligned16, false, &mx))
+  if (mx)
     return run_mx_group(ctx, (const FftCol *)dtab, (const FftCol *)dtab_out, (uint32_t)cols.size(), n, N, tw, inverse,
-                        mx);
-  if (column_fft_takes(ctx, n, N, cols.size(), inverse, !inverse)) {
-    const FftCol *tab = (const FftCol *)dtab;
-    return launch_column_fft(ctx, column_fft(tw, tab, tab, (uint32_t)cols.size(), n, N, true), inverse, !inverse);
-  }
+                        *mx);
   std::vector<PassLaunch> passes;
   int rc = make_group_passes(ctx, n, N, inverse, (const FftCol *)dtab, (const FftCol *)dtab_out,
                              (uint32_t)cols.size(), tw_end, aligned16, passes);
@@ -1147,6 +1140,11 @@ static int run_lde_group(stwo_hip_ctx *ctx, const std::vector<FftCol> &cols, con
     to[i] = {outs[i], outs[i]};
     if ((((uintptr_t)cols[i].in) | ((uintptr_t)outs[i])) & 15) aligned16 = false;
   }
+  MxPlan mx;
+  const bool matrix = mx_plan(ctx, tw, n, 0, true, cols.size(), aligned16, false, &mx) &&
+                      mx_plan(ctx, tw, n, b, false, cols.size(), aligned16, false, &mx);
+  if (!matrix && column_fft_takes(ctx, n, N, cols.size(), true, true))
+    return run_column_fft(ctx, tw, tf, n, N, store_coeffs, true, true);
   void *d[3];
   {
     const void *srcs[3] = {cols.data(), tf.data(), to.data()};
@@ -1154,9 +1152,7 @@ static int run_lde_group(stwo_hip_ctx *ctx, const std::vector<FftCol> &cols, con
     int rc = upload_tables(ctx, 3, srcs, bytes, d);
     if (rc) return rc;
   }
-  MxPlan mx;
-  if (mx_plan(ctx, tw, n, 0, true, cols.size(), aligned16, false, &mx) &&
-      mx_plan(ctx, tw, n, b, false, cols.size(), aligned16, false, &mx)) {
+  if (matrix) {
     const FftCol *ti = (const FftCol *)d[0], *tfw = (const FftCol *)d[1], *tio = (const FftCol *)d[2];
     const uint32_t nc = (uint32_t)cols.size();
     if (!mx.top_layers) {
@@ -1173,10 +1169,6 @@ static int run_lde_group(stwo_hip_ctx *ctx, const std::vector<FftCol> &cols, con
     if (!rc && mx.mid) rc = launch_mx_mid(ctx, tio, nc, n, N, tw, false);
     return rc ? rc : launch_mx_low(ctx, &lf, nullptr, 0, w2, false);
   }
-  if (column_fft_takes(ctx, n, N, cols.size(), true, true))
-    return launch_column_fft(ctx, column_fft(tw, (const FftCol *)d[0], (const FftCol *)d[1], (uint32_t)cols.size(), n, N,
-                                             store_coeffs),
-                             true, true);
   std::vector<PassLaunch> inv, fwd;
   int rc = make_group_passes(ctx, n, n, true, (const FftCol *)d[0], (const FftCol *)d[0], (uint32_t)cols.size(),
                              tw->d_itw2 + tw->len, aligned16, inv);
@@ -1210,6 +1202,15 @@ static int run_fft_group(stwo_hip_ctx *ctx, const std::vector<FftCol> &cols, uin
                          const stwo_hip_twiddles *tw, bool inverse, stwo_hip_coset dom) {
   if (cols.empty()) return STWO_HIP_OK;
   STWO_HIP_CHECK_ARG(ctx, cols.size() <= 65535, "too many columns in one group (%zu)", cols.size());
+  bool aligned16 = true, matrix = false;
+  MxPlan mx;
+  if (N >= 4) {
+    for (const FftCol &c : cols)
+      if ((((uintptr_t)c.in) | ((uintptr_t)c.out)) & 15) aligned16 = false;
+    matrix = mx_plan(ctx, tw, n, N - n, inverse, cols.size(), aligned16, false, &mx);
+    if (!matrix && column_fft_takes(ctx, n, N, cols.size(), inverse, !inverse))
+      return run_column_fft(ctx, tw, cols, n, N, true, inverse, !inverse);
+  }
   // The group's table and, forward, the in-place table of the passes after
   // the first (entries {out, out}), uploaded together.
   void *dtab = nullptr, *dtab_out = nullptr;
@@ -1248,7 +1249,7 @@ static int run_fft_group(stwo_hip_ctx *ctx, const std::vector<FftCol> &cols, uin
     return launch(ctx, "fft_small", fft_small_kernel, dim3((uint32_t)cols.size()), dim3(64), 0, a);
   }
   if (N >= 4)
-    return run_fft_group2(ctx, cols, dtab, dtab_out, n, N, tw, inverse);
+    return run_fft_group2(ctx, cols, dtab, dtab_out, n, N, tw, inverse, aligned16, matrix ? &mx : nullptr);
   const uint32_t *tree = inverse ? tw->d_itw : tw->d_tw;
   const uint32_t *tw_end = tree + tw->len;
   uint32_t L = inverse ? N : n;
@@ -1610,12 +1611,12 @@ int stwo_hip_fft_autotune(stwo_hip_ctx *ctx, const uint32_t *log_sizes, size_t n
         }
       }
       if (matrix || column) {
-        const ColumnFft cf = column_fft(tw, first, first, (uint32_t)c, n, Nd, true);
+        const std::vector<FftCol> &cf = inverse ? ta : tb;
         rc = time_launches(
             ctx,
             [&]() {
               return matrix ? run_mx_group(ctx, first, inpl, (uint32_t)c, n, Nd, tw, inverse, mx)
-                            : launch_column_fft(ctx, cf, inverse, !inverse);
+                            : run_column_fft(ctx, tw, cf, n, Nd, true, inverse, !inverse);
             },
             &def_ms);
         if (rc) return rc;

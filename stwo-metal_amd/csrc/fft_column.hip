@@ -98,7 +98,7 @@ __device__ __forceinline__ void lds_step(uint32_t *D, const uint32_t *T, uint32_
 
 // Steps pair the layers from the top, so an odd count leaves layer 0 alone.
 template <bool INV, bool FWD>
-__device__ __forceinline__ void column_body(const ColumnFft &p, uint32_t col, uint32_t *S) {
+__device__ __forceinline__ void column_body(const ColumnFft &p, const FftCol *cols, uint32_t col, uint32_t *S) {
   const uint32_t tid = threadIdx.x, nt = blockDim.x, n = p.n, N = FWD ? p.N : n;
   const uint32_t Q = 1u << (n - 2), s_low = n & 1 ? 1 : 2;
   const bool two = !(n & 1);
@@ -108,10 +108,9 @@ __device__ __forceinline__ void column_body(const ColumnFft &p, uint32_t col, ui
   u32x4 ti = {0, 0, 0, 0}, tf = {0, 0, 0, 0};
   if (has_ti) ti = gld4(p.itw_end - ((size_t)1 << (n - 1)), 16 * tid);
   if (has_tf) tf = gld4(p.tw_end - ((size_t)1 << (N - 1)), 16 * tid);
-  const FftCol c = (INV ? p.icols : p.fcols)[col];
+  const FftCol c = cols[col];
   const uint32_t *in = (const uint32_t *)readfirstlane_u64((uint64_t)c.in);
-  uint32_t *coeffs = (uint32_t *)readfirstlane_u64((uint64_t)c.out);
-  uint32_t *out = FWD ? (uint32_t *)readfirstlane_u64((uint64_t)p.fcols[col].out) : nullptr;
+  uint32_t *coeffs = (uint32_t *)in, *out = (uint32_t *)readfirstlane_u64((uint64_t)c.out);
   uint32_t x[2][4];
 #pragma unroll
   for (int it = 0; it < 2; it++) {
@@ -205,13 +204,22 @@ __device__ __forceinline__ uint32_t column_group(const ColumnFft *groups, uint32
 template <bool INV, bool FWD>
 __global__ void __launch_bounds__(kColMaxThreads) column_fft_kernel(ColumnFft p) {
   extern __shared__ __align__(16) uint32_t S[];
-  column_body<INV, FWD>(p, blockIdx.x, S);
+  column_body<INV, FWD>(p, p.cols, blockIdx.x, S);
+}
+// The columns among the arguments: uploading them costs as much as the launch.
+struct InlineFftCols {
+  FftCol c[kInlineCols];
+};
+template <bool INV, bool FWD>
+__global__ void __launch_bounds__(kColMaxThreads) column_fft_inline_kernel(ColumnFft p, InlineFftCols cols) {
+  extern __shared__ __align__(16) uint32_t S[];
+  column_body<INV, FWD>(p, cols.c, blockIdx.x, S);
 }
 template <bool INV, bool FWD>
 __global__ void __launch_bounds__(kColMaxThreads) column_fft_multi_kernel(const ColumnFft *groups, uint32_t n_groups) {
   extern __shared__ __align__(16) uint32_t S[];
   const ColumnFft p = groups[column_group(groups, n_groups)];
-  column_body<INV, FWD>(p, blockIdx.x - p.wg_start, S);
+  column_body<INV, FWD>(p, p.cols, blockIdx.x - p.wg_start, S);
 }
 
 dim3 threads(uint32_t N) { return dim3(std::min(kColMaxThreads, std::max(64u, 1u << (N - 2)))); }
@@ -238,11 +246,10 @@ bool column_fft_takes(const stwo_hip_ctx *ctx, uint32_t n, uint32_t N, size_t n_
   return !(inv && chosen(n, 1)) && !(fwd && chosen(N, 0));
 }
 
-ColumnFft column_fft(const stwo_hip_twiddles *tw, const FftCol *icols, const FftCol *fcols, uint32_t n_cols,
-                     uint32_t n, uint32_t N, bool store) {
+ColumnFft column_fft(const stwo_hip_twiddles *tw, const FftCol *d_cols, uint32_t n_cols, uint32_t n, uint32_t N,
+                     bool store) {
   ColumnFft p{};
-  p.icols = icols;
-  p.fcols = fcols;
+  p.cols = d_cols;
   p.itw_end = tw->d_itw2 + tw->len;
   p.tw_end = tw->d_tw2 + tw->len;
   p.n = n;
@@ -253,9 +260,22 @@ ColumnFft column_fft(const stwo_hip_twiddles *tw, const FftCol *icols, const Fft
   return p;
 }
 
-int launch_column_fft(stwo_hip_ctx *ctx, const ColumnFft &p, bool inv, bool fwd) {
-  const dim3 grid(p.n_cols), block = threads(p.N);
-  const size_t lds = lds_bytes(p.N, inv && fwd);
+int run_column_fft(stwo_hip_ctx *ctx, const stwo_hip_twiddles *tw, const std::vector<FftCol> &cols, uint32_t n,
+                   uint32_t N, bool store, bool inv, bool fwd) {
+  ColumnFft p = column_fft(tw, nullptr, (uint32_t)cols.size(), n, N, store);
+  const dim3 grid(p.n_cols), block = threads(N);
+  const size_t lds = lds_bytes(N, inv && fwd);
+  if (cols.size() <= kInlineCols) {
+    InlineFftCols in{};
+    std::copy(cols.begin(), cols.end(), in.c);
+    if (!fwd) return launch(ctx, name(inv, fwd), column_fft_inline_kernel<true, false>, grid, block, lds, p, in);
+    if (!inv) return launch(ctx, name(inv, fwd), column_fft_inline_kernel<false, true>, grid, block, lds, p, in);
+    return launch(ctx, name(inv, fwd), column_fft_inline_kernel<true, true>, grid, block, lds, p, in);
+  }
+  void *d = nullptr;
+  int rc = upload_table(ctx, cols.data(), cols.size() * sizeof(FftCol), &d);
+  if (rc) return rc;
+  p.cols = (const FftCol *)d;
   if (!fwd) return launch(ctx, name(inv, fwd), column_fft_kernel<true, false>, grid, block, lds, p);
   if (!inv) return launch(ctx, name(inv, fwd), column_fft_kernel<false, true>, grid, block, lds, p);
   return launch(ctx, name(inv, fwd), column_fft_kernel<true, true>, grid, block, lds, p);

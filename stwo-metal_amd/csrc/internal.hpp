@@ -292,7 +292,10 @@ struct ColRef {
   uint32_t pad;
 };
 
-// A tree's launches: a layer with columns, or a run of node layers.
+// Columns that a launch takes among its arguments at most.
+constexpr uint32_t kInlineCols = 64;
+
+// A tree's launches: a layer with columns, a run of node layers, or both.
 struct MerkleLayer {
   const uint32_t *prev;  // layer log_size + 1, or NULL
   const ColRef *cols;
@@ -304,19 +307,29 @@ struct MerkleNodes {
   uint32_t *packed, *counters;
   uint32_t out_log, stop_log, m31, wg_start;
 };
+struct MerkleTree {
+  MerkleLayer layer;  // out: its place in the packed tree
+  uint32_t *counters;
+  uint32_t stop_log, wg_start;
+};
 enum : uint32_t {
-  kMerkleLayer, kMerkleAhead, kMerkleQuad, kMerkleQuadLds, kMerkleNodes64, kMerkleNodes256, kMerkleNodes1024
+  kMerkleLayer, kMerkleAhead, kMerkleQuad, kMerkleQuadLds, kMerkleNodes64, kMerkleNodes256, kMerkleNodes1024,
+  kMerkleTree, kMerkleTreeLds, kMerkleKinds
 };
 struct MerkleStep {
   uint32_t kind, wgs;  // steps of one kind, of different trees, may share a launch
   MerkleLayer layer;   // kinds below kMerkleNodes64
-  MerkleNodes nodes;
+  MerkleNodes nodes;   // up to kMerkleNodes1024
+  MerkleTree tree;     // the others
 };
 MerkleStep merkle_layer_step(const uint32_t *prev, const ColRef *d_cols, uint32_t n_cols, uint32_t log_size,
                              uint32_t *out, int mode, bool lifted);
 MerkleStep merkle_nodes_step(uint32_t *layers, uint32_t top_log, uint32_t stop_log, int mode, uint32_t *counters);
+// Extends a layer's step by the node layers below it down to stop_log, if the
+// two are to share a launch.
+bool merkle_tree_step(MerkleStep &s, uint32_t stop_log, uint32_t *counters);
 int launch_merkle(stwo_hip_ctx *ctx, const MerkleStep &s);
-// n steps of one kind from a table of MerkleLayer or MerkleNodes.
+// n steps of one kind from a table of MerkleLayer, MerkleNodes or MerkleTree.
 int launch_merkle_multi(stwo_hip_ctx *ctx, uint32_t kind, bool lifted, const void *d_steps, uint32_t n, uint32_t wgs);
 
 // Counters of the one-launch trees: a word per group of workgroups that hand

@@ -84,12 +84,9 @@ __device__ __forceinline__ uint32_t ld_col_word(const uint32_t *col, uint32_t id
 // large layers the other waves hide the latency and the extra registers and
 // copies cost more than they save.
 template <bool AHEAD>
-__device__ __forceinline__ void merkle_layer(const MerkleLayer &L, uint32_t wg) {
+__device__ __forceinline__ b2_state layer_hash(const MerkleLayer &L, const ColRef *cols, uint32_t i) {
   const uint32_t *prev = L.prev;
-  const ColRef *cols = L.cols;
-  const uint32_t n_cols = L.n_cols, lifted = L.lifted, n = 1u << L.log_size;
-  const uint32_t i = wg * 256 + threadIdx.x;
-  if (i >= n) return;
+  const uint32_t n_cols = L.n_cols, lifted = L.lifted;
   // The words of columns c0 .. c0 + 15 at this row (zeros past n_cols).
   auto load_cols = [&](uint32_t c0, uint32_t (&dst)[16]) {
     const uint32_t cnt = min(16u, n_cols - c0);
@@ -130,20 +127,22 @@ __device__ __forceinline__ void merkle_layer(const MerkleLayer &L, uint32_t wg) 
     t += 4 * cnt;
     b2_compress(s, m, t, c0 + 16 >= n_cols);
   }
-  store_hash(L.out + 8 * (size_t)i, s, L.m31);
+  if (L.m31)
+#pragma unroll
+    for (int k = 0; k < 8; k++) s.h[k] = b2_reduce_word(s.h[k]);
+  return s;
 }
 
 // Layers of few nodes, where a node's chain of blocks is the launch's
 // critical path: one node per quad (b2_compress_quad, about 410
 // instructions per lane instead of 960 on one lane), each block's column
-// words loaded one compression ahead.  Same inputs and outputs as
-// merkle_layer_kernel; the grid has 4 lanes per node.
-__device__ __forceinline__ void merkle_layer_quad(const MerkleLayer &L, uint32_t wg) {
+// words loaded one compression ahead.  Same hash as layer_hash, words j and
+// 4 + j of it in lane j.
+__device__ __forceinline__ void layer_hash_quad(const MerkleLayer &L, const ColRef *cols, uint32_t i, uint32_t &lo,
+                                                uint32_t &hi) {
+  const uint32_t j = threadIdx.x & 3;
   const uint32_t *prev = L.prev;
-  const ColRef *cols = L.cols;
-  const uint32_t n_cols = L.n_cols, lifted = L.lifted, m31 = L.m31, n = 1u << L.log_size;
-  const uint32_t i = (wg * 256 + threadIdx.x) >> 2, j = threadIdx.x & 3;
-  if (i >= n) return;  // a quad's four lanes share i and leave together
+  const uint32_t n_cols = L.n_cols, lifted = L.lifted;
   auto load_cols = [&](uint32_t c0, uint32_t (&dst)[16]) {
     const uint32_t cnt = min(16u, n_cols - c0);
 #pragma unroll
@@ -157,7 +156,8 @@ __device__ __forceinline__ void merkle_layer_quad(const MerkleLayer &L, uint32_t
       dst[k] = v;
     }
   };
-  uint32_t lo = b2_iv_lo(j), hi = b2_iv_hi(j);
+  lo = b2_iv_lo(j);
+  hi = b2_iv_hi(j);
   uint32_t m[16], nx[16];
   uint32_t t = 0;
   if (n_cols) load_cols(0, nx);
@@ -178,13 +178,10 @@ __device__ __forceinline__ void merkle_layer_quad(const MerkleLayer &L, uint32_t
     t += 4 * cnt;
     b2_compress_quad(lo, hi, m, t, c0 + 16 >= n_cols);
   }
-  if (m31) {
+  if (L.m31) {
     lo = b2_reduce_word(lo);
     hi = b2_reduce_word(hi);
   }
-  g_u32 *o = as_global(L.out + 8 * (size_t)i);
-  o[j] = lo;
-  o[4 + j] = hi;
 }
 
 // Small mixed-degree layers with many columns (up to 2^14 nodes): the chain
@@ -194,19 +191,22 @@ __device__ __forceinline__ void merkle_layer_quad(const MerkleLayer &L, uint32_t
 // through LDS in chunks of MQ_CHUNK columns: the chunk's column pointers
 // first, then every column's 64 words (one coalesced 256-byte run per wave
 // and load, 32 loads in flight per lane), so a chunk costs about two memory
-// round trips and its blocks then read their words from LDS.  Same inputs
-// and outputs as merkle_layer_kernel (mixed layers only, not lifted).
+// round trips and its blocks then read their words from LDS.  Same hash
+// as layer_hash (mixed layers only, not lifted).
 constexpr uint32_t MQ_CHUNK = 240;  // 15 blocks; 61,440 B of words + 1,920 B of pointers
-__device__ __forceinline__ void merkle_layer_quad_lds(const MerkleLayer &L, uint32_t wg) {
-  __shared__ const uint32_t *ptrs[MQ_CHUNK];
-  __shared__ uint32_t tile[MQ_CHUNK * 64];
+struct QuadTile {
+  const uint32_t *ptrs[MQ_CHUNK];
+  uint32_t tile[MQ_CHUNK * 64];
+};
+__device__ __forceinline__ void layer_hash_quad_lds(const MerkleLayer &L, uint32_t i0, QuadTile &S, uint32_t &lo,
+                                                    uint32_t &hi) {
   const uint32_t *prev = L.prev;
   const ColRef *cols = L.cols;
-  const uint32_t n_cols = L.n_cols, m31 = L.m31, n = 1u << L.log_size;
-  const uint32_t tid = threadIdx.x, node = tid >> 2, j = tid & 3;
-  const uint32_t i0 = wg * 64, i = i0 + node;
+  const uint32_t n_cols = L.n_cols, n = 1u << L.log_size;
+  const uint32_t tid = threadIdx.x, node = tid >> 2, j = tid & 3, i = i0 + node;
   const bool active = i < n;  // every lane stays for the barriers
-  uint32_t lo = b2_iv_lo(j), hi = b2_iv_hi(j);
+  lo = b2_iv_lo(j);
+  hi = b2_iv_hi(j);
   uint32_t m[16];
   uint32_t t = 0;
   if (prev) {
@@ -224,38 +224,93 @@ __device__ __forceinline__ void merkle_layer_quad_lds(const MerkleLayer &L, uint
   for (uint32_t cb = 0; cb < n_cols; cb += MQ_CHUNK) {
     const uint32_t cnt = min(MQ_CHUNK, n_cols - cb), words = cnt * 64;
     __syncthreads();  // the previous chunk's words are consumed
-    for (uint32_t c = tid; c < cnt; c += 256) ptrs[c] = cols[cb + c].p;
+    for (uint32_t c = tid; c < cnt; c += 256) S.ptrs[c] = cols[cb + c].p;
     __syncthreads();
     for (uint32_t e0 = 0; e0 < words; e0 += 256 * 32) {
       uint32_t v[32];
 #pragma unroll
       for (uint32_t k = 0; k < 32; k++) {
         const uint32_t e = e0 + tid + 256 * k;  // column e >> 6 is uniform over the wave
-        v[k] = (e < words && row < n) ? ld_col_word(ptrs[e >> 6], row) : 0u;
+        v[k] = (e < words && row < n) ? ld_col_word(S.ptrs[e >> 6], row) : 0u;
       }
 #pragma unroll
       for (uint32_t k = 0; k < 32; k++) {
         const uint32_t e = e0 + tid + 256 * k;
-        if (e < words) tile[e] = v[k];
+        if (e < words) S.tile[e] = v[k];
       }
     }
     __syncthreads();
     for (uint32_t b = 0; b < cnt; b += 16) {
       const uint32_t bc = min(16u, cnt - b);
 #pragma unroll
-      for (uint32_t k = 0; k < 16; k++) m[k] = k < bc ? tile[(b + k) * 64 + node] : 0u;
+      for (uint32_t k = 0; k < 16; k++) m[k] = k < bc ? S.tile[(b + k) * 64 + node] : 0u;
       t += 4 * bc;
       if (active) b2_compress_quad(lo, hi, m, t, cb + b + 16 >= n_cols);
     }
   }
-  if (!active) return;
-  if (m31) {
+  if (L.m31) {
     lo = b2_reduce_word(lo);
     hi = b2_reduce_word(hi);
   }
-  g_u32 *o = as_global(L.out + 8 * (size_t)i);
-  o[j] = lo;
-  o[4 + j] = hi;
+}
+
+// One layer: its nodes alone.
+template <bool AHEAD>
+__device__ __forceinline__ void merkle_layer(const MerkleLayer &L, uint32_t wg) {
+  const uint32_t i = wg * 256 + threadIdx.x;
+  if (i >= 1u << L.log_size) return;
+  store_hash(L.out + 8 * (size_t)i, layer_hash<AHEAD>(L, L.cols, i), 0);
+}
+__device__ __forceinline__ void store_quad(uint32_t *out, uint32_t i, uint32_t lo, uint32_t hi) {
+  g_u32 *o = as_global(out + 8 * (size_t)i);
+  o[threadIdx.x & 3] = lo;
+  o[4 + (threadIdx.x & 3)] = hi;
+}
+__device__ __forceinline__ void merkle_layer_quad(const MerkleLayer &L, uint32_t wg) {
+  const uint32_t i = (wg * 256 + threadIdx.x) >> 2;
+  if (i >= 1u << L.log_size) return;  // a quad's four lanes share i and leave together
+  uint32_t lo, hi;
+  layer_hash_quad(L, L.cols, i, lo, hi);
+  store_quad(L.out, i, lo, hi);
+}
+__device__ __forceinline__ void merkle_layer_quad_lds(const MerkleLayer &L, uint32_t wg) {
+  __shared__ QuadTile S;
+  const uint32_t i = wg * 64 + (threadIdx.x >> 2);
+  uint32_t lo, hi;
+  layer_hash_quad_lds(L, wg * 64, S, lo, hi);
+  if (i < 1u << L.log_size) store_quad(L.out, i, lo, hi);
+}
+
+// A layer of at most 2^14 nodes and the run of node layers below it, down to
+// stop_log, in one launch (out lies in the packed tree): a workgroup hashes 64
+// nodes of the layer, a quad each (LDS: with the columns staged through it), and
+// goes on as merkle_nodes does.  The layer's digests are not read back, and the
+// second launch and its first loads go: a tree over 16 columns of 2^11 takes
+// 17.4 us, in two launches 5.6 + 14.6.
+template <bool LDS>
+__device__ __forceinline__ void merkle_tree(const MerkleTree &T, const ColRef *cols, uint32_t wg) {
+  // the column words are consumed when the digests come
+  constexpr size_t kBytes = LDS && sizeof(QuadTile) > sizeof(TreeLds) ? sizeof(QuadTile) : sizeof(TreeLds);
+  __shared__ __align__(16) uint8_t mem[kBytes];
+  TreeLds &S = *reinterpret_cast<TreeLds *>(mem);
+  const MerkleLayer &L = T.layer;
+  const uint32_t n = 1u << L.log_size, first = wg * 64, q = threadIdx.x >> 2, j = threadIdx.x & 3, i = first + q;
+  uint32_t lo, hi;
+  if constexpr (LDS) {
+    layer_hash_quad_lds(L, first, *reinterpret_cast<QuadTile *>(mem), lo, hi);
+    __syncthreads();
+  } else if (i < n) {
+    layer_hash_quad(L, cols, i, lo, hi);
+  }
+  if (i < n) {
+    store_quad(L.out, i, lo, hi);
+    tree_row(S, 0, q)[j] = lo;
+    tree_row(S, 0, q)[4 + j] = hi;
+  }
+  const uint32_t cnt = min(64u, n), lv = min(31 - __clz(cnt), L.log_size - T.stop_log), l = L.log_size - lv;
+  uint32_t *packed = L.out - tree_layer_off(L.log_size);
+  const uint32_t buf = tree_levels(S, 0, cnt, first, L.log_size, lv, packed, L.m31, l > T.stop_log);
+  tree_finish(S, buf, wg, l, T.stop_log, packed, L.m31, T.counters);
 }
 
 // Node layers out_log .. stop_log below `prev` (of log size out_log + 1), each
@@ -350,6 +405,23 @@ __global__ void __launch_bounds__(256) merkle_layer_quad_lds_multi_kernel(const 
   const MerkleLayer L = step_of(t, n);
   merkle_layer_quad_lds(L, blockIdx.x - L.wg_start);
 }
+template <bool LDS>
+__global__ void __launch_bounds__(kTreeThreads) merkle_tree_kernel(MerkleTree T) {
+  merkle_tree<LDS>(T, T.layer.cols, blockIdx.x);
+}
+template <bool LDS>
+__global__ void __launch_bounds__(kTreeThreads) merkle_tree_multi_kernel(const MerkleTree *t, uint32_t n) {
+  const MerkleTree T = step_of(t, n);
+  merkle_tree<LDS>(T, T.layer.cols, blockIdx.x - T.wg_start);
+}
+// The columns among the arguments: their upload costs a small commit as much as
+// its leaves.
+struct InlineCols {
+  ColRef c[kInlineCols];
+};
+__global__ void __launch_bounds__(kTreeThreads) merkle_tree_inline_kernel(MerkleTree T, InlineCols cols) {
+  merkle_tree<false>(T, cols.c, blockIdx.x);
+}
 template <uint32_t NODES>
 __global__ void __launch_bounds__(kTreeThreads) merkle_nodes_kernel(MerkleNodes L) {
   merkle_nodes<NODES>(L, blockIdx.x);
@@ -393,8 +465,20 @@ MerkleStep merkle_nodes_step(uint32_t *layers, uint32_t top_log, uint32_t stop_l
   return s;
 }
 
+// Up to 2^14 nodes, where the node layers alone also take a quad for each of 64.
+// With a lane for each of 256 above that there is nothing to gain: 2^17 leaves of
+// 16 columns 37.6 us, in two launches 9.2 + 27.5.
+bool merkle_tree_step(MerkleStep &s, uint32_t stop_log, uint32_t *counters) {
+  const uint32_t lg = s.layer.log_size;
+  if (lg > 14 || stop_log >= lg) return false;
+  s.tree = {s.layer, counters, stop_log, 0};
+  s.kind = s.layer.n_cols > 16 && !s.layer.lifted ? kMerkleTreeLds : kMerkleTree;
+  s.wgs = 1u << (lg > 6 ? lg - 6 : 0);
+  return true;
+}
+
 static const char *step_name(uint32_t kind, bool lifted) {
-  return kind >= kMerkleNodes64 ? "merkle_nodes" : lifted ? "merkle_lifted_leaves" : "merkle_commit_on_layer";
+  return kind >= kMerkleTree ? "merkle_tree" : kind >= kMerkleNodes64 ? "merkle_nodes" : lifted ? "merkle_lifted_leaves" : "merkle_commit_on_layer";
 }
 
 int launch_merkle(stwo_hip_ctx *ctx, const MerkleStep &s) {
@@ -407,7 +491,9 @@ int launch_merkle(stwo_hip_ctx *ctx, const MerkleStep &s) {
     case kMerkleQuadLds: return launch(ctx, name, merkle_layer_quad_lds_kernel, grid, block, 0, s.layer);
     case kMerkleNodes64: return launch(ctx, name, merkle_nodes_kernel<64>, grid, block, 0, s.nodes);
     case kMerkleNodes256: return launch(ctx, name, merkle_nodes_kernel<256>, grid, block, 0, s.nodes);
-    default: return launch(ctx, name, merkle_nodes_kernel<1024>, grid, block, 0, s.nodes);
+    case kMerkleNodes1024: return launch(ctx, name, merkle_nodes_kernel<1024>, grid, block, 0, s.nodes);
+    case kMerkleTree: return launch(ctx, name, merkle_tree_kernel<false>, grid, block, 0, s.tree);
+    default: return launch(ctx, name, merkle_tree_kernel<true>, grid, block, 0, s.tree);
   }
 }
 
@@ -416,6 +502,7 @@ int launch_merkle_multi(stwo_hip_ctx *ctx, uint32_t kind, bool lifted, const voi
   const dim3 grid(wgs), block(256);
   const MerkleLayer *l = (const MerkleLayer *)d_steps;
   const MerkleNodes *t = (const MerkleNodes *)d_steps;
+  const MerkleTree *r = (const MerkleTree *)d_steps;
   switch (kind) {
     case kMerkleLayer: return launch(ctx, name, merkle_layer_multi_kernel<false>, grid, block, 0, l, n);
     case kMerkleAhead: return launch(ctx, name, merkle_layer_multi_kernel<true>, grid, block, 0, l, n);
@@ -423,7 +510,9 @@ int launch_merkle_multi(stwo_hip_ctx *ctx, uint32_t kind, bool lifted, const voi
     case kMerkleQuadLds: return launch(ctx, name, merkle_layer_quad_lds_multi_kernel, grid, block, 0, l, n);
     case kMerkleNodes64: return launch(ctx, name, merkle_nodes_multi_kernel<64>, grid, block, 0, t, n);
     case kMerkleNodes256: return launch(ctx, name, merkle_nodes_multi_kernel<256>, grid, block, 0, t, n);
-    default: return launch(ctx, name, merkle_nodes_multi_kernel<1024>, grid, block, 0, t, n);
+    case kMerkleNodes1024: return launch(ctx, name, merkle_nodes_multi_kernel<1024>, grid, block, 0, t, n);
+    case kMerkleTree: return launch(ctx, name, merkle_tree_multi_kernel<false>, grid, block, 0, r, n);
+    default: return launch(ctx, name, merkle_tree_multi_kernel<true>, grid, block, 0, r, n);
   }
 }
 
@@ -433,17 +522,31 @@ static int check_mode(stwo_hip_ctx *ctx, int mode) {
   return STWO_HIP_OK;
 }
 
+// A layer with columns, and the node layers below it down to stop_log, where they
+// share a launch; *done: whether they did.
 static int launch_layer(stwo_hip_ctx *ctx, const uint32_t *prev, const std::vector<ColRef> &cols, uint32_t log_size,
-                        uint32_t *out, int mode, bool lifted) {
+                        uint32_t *out, int mode, bool lifted, uint32_t stop_log, bool *done) {
   int rc = check_mode(ctx, mode);
   if (rc) return rc;
-  void *dtab = nullptr;
+  MerkleStep s = merkle_layer_step(prev, nullptr, (uint32_t)cols.size(), log_size, out, mode, lifted);
+  *done = merkle_tree_step(s, stop_log, ctx->d_counters);
+  if (s.kind == kMerkleTree && cols.size() <= kInlineCols) {
+    InlineCols in{};
+    std::copy(cols.begin(), cols.end(), in.c);
+    return launch(ctx, "merkle_tree", merkle_tree_inline_kernel, dim3(s.wgs), dim3(kTreeThreads), 0, s.tree, in);
+  }
   if (!cols.empty()) {
+    void *dtab = nullptr;
     rc = upload_table(ctx, cols.data(), cols.size() * sizeof(ColRef), &dtab);
     if (rc) return rc;
+    s.layer.cols = s.tree.layer.cols = (const ColRef *)dtab;
   }
-  return launch_merkle(
-      ctx, merkle_layer_step(prev, (const ColRef *)dtab, (uint32_t)cols.size(), log_size, out, mode, lifted));
+  return launch_merkle(ctx, s);
+}
+static int launch_layer(stwo_hip_ctx *ctx, const uint32_t *prev, const std::vector<ColRef> &cols, uint32_t log_size,
+                        uint32_t *out, int mode, bool lifted) {
+  bool done;
+  return launch_layer(ctx, prev, cols, log_size, out, mode, lifted, log_size, &done);
 }
 
 static int hash_node_layers(stwo_hip_ctx *ctx, uint32_t *layers, uint32_t top_log, uint32_t stop_log, int mode) {
@@ -482,35 +585,28 @@ int stwo_hip_merkle_commit(stwo_hip_ctx *ctx, const uint32_t *const *cols, const
     STWO_HIP_CHECK_ARG(ctx, cols[c] && log_sizes[c] <= 30, "merkle_commit: bad column %zu", c);
     max_log = std::max(max_log, log_sizes[c]);
   }
-  int l = (int)max_log;
-  while (l >= 0) {
+  for (int l = (int)max_log; l >= 0;) {
     std::vector<ColRef> refs;
     for (size_t c = 0; c < n_cols; c++)  // input order == stable order among equal lengths
       if (log_sizes[c] == (uint32_t)l) refs.push_back({cols[c], 0, 0});
     const uint32_t *prev = (l == (int)max_log) ? nullptr : layers + layer_off(l + 1);
-    if (refs.empty() && prev) {
-      // Run of pure node layers down to the next injected layer (or the root).
-      int next = -1;
-      for (size_t c = 0; c < n_cols; c++)
-        if ((int)log_sizes[c] < l) next = std::max(next, (int)log_sizes[c]);
-      uint32_t stop = (uint32_t)(next + 1);
-      int rc = hash_node_layers(ctx, layers, (uint32_t)l + 1, stop, hash_mode);
-      if (rc) return rc;
-      l = (int)stop - 1;
-      continue;
-    }
-    int rc = launch_layer(ctx, prev, refs, (uint32_t)l, layers + layer_off((uint32_t)l), hash_mode, false);
+    // below it, a run of pure node layers down to the next injected layer (or the root)
+    int next = -1;
+    for (size_t c = 0; c < n_cols; c++)
+      if ((int)log_sizes[c] < l) next = std::max(next, (int)log_sizes[c]);
+    const uint32_t stop = (uint32_t)(next + 1);
+    bool done = false;
+    int rc = launch_layer(ctx, prev, refs, (uint32_t)l, layers + layer_off((uint32_t)l), hash_mode, false, stop, &done);
+    if (!rc && !done) rc = hash_node_layers(ctx, layers, (uint32_t)l, stop, hash_mode);
     if (rc) return rc;
-    l--;
+    l = next;
   }
   return STWO_HIP_OK;
 }
 
-int stwo_hip_merkle_lifted_build_leaves(stwo_hip_ctx *ctx, const uint32_t *const *cols, const uint32_t *log_sizes,
-                                        size_t n_cols, uint32_t lifting_log_size, uint32_t *out, int hash_mode) {
-  if (!ctx) return STWO_HIP_EINVAL;
-  STWO_HIP_CHECK_ARG(ctx, out != nullptr, "lifted_build_leaves: NULL output");
-  if (n_cols == 0) return launch_layer(ctx, nullptr, {}, 0, out, hash_mode, true);
+// The leaves of a lifted tree, and its node layers where they share the launch.
+static int lifted_leaves(stwo_hip_ctx *ctx, const uint32_t *const *cols, const uint32_t *log_sizes, size_t n_cols,
+                         uint32_t lifting_log_size, uint32_t *out, int hash_mode, uint32_t stop_log, bool *done) {
   STWO_HIP_CHECK_ARG(ctx, cols && log_sizes && lifting_log_size <= 30, "lifted_build_leaves: bad arguments");
   std::vector<size_t> order(n_cols);
   for (size_t c = 0; c < n_cols; c++) {
@@ -522,7 +618,16 @@ int stwo_hip_merkle_lifted_build_leaves(stwo_hip_ctx *ctx, const uint32_t *const
   std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return log_sizes[a] < log_sizes[b]; });
   std::vector<ColRef> refs;
   for (size_t c : order) refs.push_back({cols[c], lifting_log_size - log_sizes[c], 0});
-  return launch_layer(ctx, nullptr, refs, lifting_log_size, out, hash_mode, true);
+  return launch_layer(ctx, nullptr, refs, lifting_log_size, out, hash_mode, true, stop_log, done);
+}
+
+int stwo_hip_merkle_lifted_build_leaves(stwo_hip_ctx *ctx, const uint32_t *const *cols, const uint32_t *log_sizes,
+                                        size_t n_cols, uint32_t lifting_log_size, uint32_t *out, int hash_mode) {
+  if (!ctx) return STWO_HIP_EINVAL;
+  STWO_HIP_CHECK_ARG(ctx, out != nullptr, "lifted_build_leaves: NULL output");
+  if (n_cols == 0) return launch_layer(ctx, nullptr, {}, 0, out, hash_mode, true);
+  bool done;
+  return lifted_leaves(ctx, cols, log_sizes, n_cols, lifting_log_size, out, hash_mode, lifting_log_size, &done);
 }
 
 int stwo_hip_merkle_lifted_build_next_layer(stwo_hip_ctx *ctx, const uint32_t *prev, uint32_t out_log_size,
@@ -537,9 +642,11 @@ int stwo_hip_merkle_lifted_commit(stwo_hip_ctx *ctx, const uint32_t *const *cols
   if (!ctx) return STWO_HIP_EINVAL;
   STWO_HIP_CHECK_ARG(ctx, layers != nullptr, "lifted_commit: NULL output");
   if (n_cols == 0) return stwo_hip_merkle_lifted_build_leaves(ctx, cols, log_sizes, 0, 0, layers, hash_mode);
-  int rc = stwo_hip_merkle_lifted_build_leaves(ctx, cols, log_sizes, n_cols, lifting_log_size,
-                                               layers + layer_off(lifting_log_size), hash_mode);
-  if (rc) return rc;
+  STWO_HIP_CHECK_ARG(ctx, lifting_log_size <= 30, "lifted_build_leaves: bad arguments");
+  bool done = false;
+  int rc = lifted_leaves(ctx, cols, log_sizes, n_cols, lifting_log_size, layers + layer_off(lifting_log_size),
+                         hash_mode, 0, &done);
+  if (rc || done) return rc;
   return hash_node_layers(ctx, layers, lifting_log_size, 0, hash_mode);
 }
 
