@@ -132,10 +132,45 @@ static int arena_wait_range(stwo_hip_ctx *ctx, size_t b, size_t e) {
   return STWO_HIP_OK;
 }
 
+// Pending uploads of a few KB travel as kernel arguments: one launch, where a
+// copy call and the event that guards its host bytes keep the next launch
+// waiting about 4 us longer (a commit of 16 x 2^16 with two uploads: 72.0 -> 63.8
+// us).  The host bytes are free again at once.
+template <uint32_t BYTES>
+struct UploadBytes {
+  uint4 v[BYTES / 16];
+};
+template <uint32_t BYTES>
+__global__ void __launch_bounds__(256) upload_kernel(UploadBytes<BYTES> src, uint4 *dst, uint32_t n) {
+  const uint32_t i = threadIdx.x;
+  if (i < n) dst[i] = src.v[i];
+}
+template <uint32_t BYTES>
+static int launch_upload(stwo_hip_ctx *ctx, size_t at, size_t bytes) {
+  UploadBytes<BYTES> src;
+  memcpy(&src, ctx->h_arena + at, bytes);
+  hipLaunchKernelGGL(upload_kernel<BYTES>, dim3(1), dim3(BYTES > 1024 ? 256 : 64), 0, ctx->stream, src,
+                     (uint4 *)(ctx->d_arena + at), (uint32_t)(bytes / 16));
+  return check_launch(ctx, "upload");
+}
+constexpr size_t kUploadArgs = 3584;  // below the 4 KB of a launch's arguments
+
 int flush_uploads(stwo_hip_ctx *ctx) {
   if (ctx->pend_end <= ctx->pend_begin) return STWO_HIP_OK;
-  const size_t b = ctx->pend_begin, e = ctx->pend_end;
+  size_t b = ctx->pend_begin;
+  const size_t e = ctx->pend_end;
   ctx->pend_begin = ctx->pend_end = 0;
+  if (e - b <= 2 * kUploadArgs) {
+    // (tables start and end on 256 bytes)
+    for (; b < e; b += kUploadArgs) {
+      const size_t n = std::min(kUploadArgs, e - b);
+      const int rc = n <= 256    ? launch_upload<256>(ctx, b, n)
+                     : n <= 1024 ? launch_upload<1024>(ctx, b, n)
+                                 : launch_upload<kUploadArgs>(ctx, b, n);
+      if (rc) return rc;
+    }
+    return STWO_HIP_OK;
+  }
   STWO_HIP_TRY(ctx, hipMemcpyAsync(ctx->d_arena + b, ctx->h_arena + b, e - b, hipMemcpyHostToDevice, ctx->stream));
   hipEvent_t ev = take_event(ctx);
   if (!ev) return set_error(ctx, STWO_HIP_EDEVICE, "hipEventCreate failed");
