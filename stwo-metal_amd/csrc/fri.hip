@@ -233,9 +233,9 @@ __device__ __forceinline__ qm31 fri_value(const Qm31ColsConst &src, uint32_t *ds
 // launch, so one workgroup runs every remaining inner layer: the fold that
 // produces the first of them, then per layer the lifted leaves of
 // the 4 coordinate columns, the node layers, the channel step and the line
-// fold into the next layer's evaluation.  The layer's values, its fold's
-// twiddles (loaded while the tree is hashed) and the channel stay in LDS from
-// phase to phase; the trees, roots, channel state and folded evaluations
+// fold into the next layer's evaluation.  The layer's values, all folds'
+// twiddles (read once: a load between the layers would wait for the stores
+// before it) and the channel stay in LDS from phase to phase; the trees, roots, channel state and folded evaluations
 // written are the ones the per-layer launches write.  What bounds it is the
 // chain of compressions: lg + 3 a layer.  Layers of 2^9 and 2^10 cost one
 // workgroup as much as a launch over several costs (four compressions per
@@ -265,7 +265,7 @@ struct TailLds {
 
 // Output i of STEP line folds of the layer in LDS (fold_line_at, from LDS).
 template <int STEP>
-__device__ __forceinline__ qm31 tail_fold(const TailLds &S, uint32_t n, uint32_t i) {
+__device__ __forceinline__ qm31 tail_fold(const TailLds &S, const uint32_t *tw, uint32_t n, uint32_t i) {
   constexpr int W = 1 << STEP;
   qm31 a = qm31_make(S.alpha[0], S.alpha[1], S.alpha[2], S.alpha[3]), v[W];
 #pragma unroll
@@ -275,7 +275,7 @@ __device__ __forceinline__ qm31 tail_fold(const TailLds &S, uint32_t n, uint32_t
 #pragma unroll
   for (int layer = 0; layer < STEP; layer++) {
     const int half = W >> (layer + 1);
-    const uint32_t *lvl = S.tw + (n - (n >> layer));
+    const uint32_t *lvl = tw + (n - (n >> layer));
 #pragma unroll
     for (int j = 0; j < half; j++) {
       const uint32_t xi = lvl[i * half + j];
@@ -298,6 +298,8 @@ __device__ __forceinline__ void fri_tail(const FriTail &t) {
   uint32_t *chan = t.state, *alpha = t.state + kAlphaOff;
   uint32_t n = 1u << t.l[0].lg;
   if (tid < n) {
+    // the folds' twiddles: levels lg, lg - 1, ... end the tree
+    S.tw[tid] = t.itw_end[(ptrdiff_t)tid - (ptrdiff_t)n];
     const uint32_t lg = t.l[0].lg;
     qm31 v, a = qm31_make(0, 0, 0, 0);
     if (t.fold) a = load_qm31(alpha);
@@ -320,10 +322,7 @@ __device__ __forceinline__ void fri_tail(const FriTail &t) {
     const FriTailLayer &L = t.l[li];
     n = 1u << L.lg;
     __syncthreads();
-    // the fold's twiddles: levels lg, lg - 1, ... follow each other
     const uint32_t n_out = n >> L.step;
-    uint32_t tw = 0;
-    if (tid < n - n_out) tw = t.itw_end[(ptrdiff_t)tid - (ptrdiff_t)n];
     // lifted leaves: H(le32 of the 4 coordinates), one 16-byte block
     uint32_t *leaves = L.tree + tree_layer_off(L.lg);
     uint32_t m[16];
@@ -351,7 +350,6 @@ __device__ __forceinline__ void fri_tail(const FriTail &t) {
         tree_row(S.t, 0, i)[4 + j] = hi;
       }
     }
-    S.tw[tid] = tw;
     const uint32_t buf = tree_levels(S.t, 0, n, 0, L.lg, L.lg, L.tree, 0, false);
     if (tid < 4) {
       const uint32_t *root = tree_row(S.t, buf, 0);
@@ -373,12 +371,13 @@ __device__ __forceinline__ void fri_tail(const FriTail &t) {
     }
     __syncthreads();
     qm31 r;
+    const uint32_t *tw = S.tw + ((1u << t.l[0].lg) - n);
     if (tid < n_out) {
       switch (L.step) {
-        case 1: r = tail_fold<1>(S, n, tid); break;
-        case 2: r = tail_fold<2>(S, n, tid); break;
-        case 3: r = tail_fold<3>(S, n, tid); break;
-        default: r = tail_fold<4>(S, n, tid); break;
+        case 1: r = tail_fold<1>(S, tw, n, tid); break;
+        case 2: r = tail_fold<2>(S, tw, n, tid); break;
+        case 3: r = tail_fold<3>(S, tw, n, tid); break;
+        default: r = tail_fold<4>(S, tw, n, tid); break;
       }
     }
     __syncthreads();

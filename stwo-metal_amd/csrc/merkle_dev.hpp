@@ -33,9 +33,9 @@ __device__ __forceinline__ void store_hash(uint32_t *dst, const b2_state &s, uin
 // complete before the count; the last arriver sets the counter back to zero.
 //
 // A meeting costs about 1.5 us (stores out, count, loads); a further launch for
-// the levels above costs 3 to 4.5 us before its first hash.  A level takes 1.0 to
-// 1.3 us, the 380 instructions of one compression one after the other plus the
-// way through LDS.
+// the levels above costs 3 to 4.5 us before its first hash.  A level takes 0.8 us,
+// the 380 instructions of one compression one after the other plus the way
+// through LDS.
 
 constexpr uint32_t kTreeThreads = 256;
 
@@ -80,13 +80,21 @@ __device__ __forceinline__ void tree_keep(TreeLds &S, uint32_t buf, uint32_t row
 // A quad per hash (their latency is the critical path), two after each other
 // on a level of 128.  `handoff`: the last level is read by another workgroup.
 // Starts and ends with a barrier; returns the buffer of the last level.
+//
+// Levels of 16 hashes and fewer are one wave's: in place, since a wave's LDS
+// accesses are in order, and with every lane hashing (those past the level a
+// stale row), so the loop has fixed addresses and no branch but its own. A
+// level is 380 instructions of one compression, 1,500 cycles, and about 300 for
+// the way through LDS; with the loop of the wide levels it was 2,200 in all
+// (a tree over 16 columns of 2^11 17.4 -> 15.0 us).
 __device__ __forceinline__ uint32_t tree_levels(TreeLds &S, uint32_t buf, uint32_t cnt, size_t first, uint32_t lg,
                                                 uint32_t n_levels, uint32_t *packed, uint32_t m31, bool handoff) {
   const uint32_t q = threadIdx.x >> 2, j = threadIdx.x & 3;
   const b2_quad_iv iv = b2_quad_init();
   const uint32_t d0 = b2_quad_d(iv, 64, true);
   __syncthreads();
-  for (uint32_t k = 0; k < n_levels; k++) {
+  uint32_t k = 0;
+  for (; k < n_levels && cnt > 32; k++) {
     cnt >>= 1;
     first >>= 1;
     lg--;
@@ -113,11 +121,37 @@ __device__ __forceinline__ uint32_t tree_levels(TreeLds &S, uint32_t buf, uint32
       }
     }
     buf ^= 1;
-    // 16 hashes and fewer are one wave's, whose LDS accesses are in order
-    if (cnt > 16)
-      __syncthreads();
-    else
+    __syncthreads();
+  }
+  if (threadIdx.x < 64) {
+    uint32_t *keep = tree_row(S, buf, q) + j;
+    for (; k < n_levels; k++) {
+      cnt >>= 1;
+      first >>= 1;
+      lg--;
+      g_u32 *out = as_global(packed + tree_layer_off(lg) + 8 * first);
+      uint32_t m[16];
+      tree_pair(S, buf, q, m);
+      uint32_t lo = iv.lo, hi = iv.hi;
+      b2_compress_quad(iv, lo, hi, m, d0);
+      if (m31) {
+        lo = b2_reduce_word(lo);
+        hi = b2_reduce_word(hi);
+      }
       __builtin_amdgcn_wave_barrier();
+      keep[0] = lo;
+      keep[4] = hi;
+      __builtin_amdgcn_wave_barrier();
+      if (q < cnt) {
+        if (handoff && k + 1 == n_levels) {
+          st_agent((uint32_t *)(out + 8 * q + j), lo);
+          st_agent((uint32_t *)(out + 8 * q + 4 + j), hi);
+        } else {
+          out[8 * q + j] = lo;
+          out[8 * q + 4 + j] = hi;
+        }
+      }
+    }
   }
   __syncthreads();
   return buf;
