@@ -242,6 +242,9 @@ int build_levels(stwo_hip_ctx *ctx, const stwo_hip_twiddles *tw, const std::vect
       ll.inverse = inverse;
       ll.fused = false;
       ll.kind = kd != 0 ? (int)kd : (uniform ? -1 : 0);
+      if (kd == 1 && std::all_of(descs.begin(), descs.end(),
+                                 [&](const FftPass2 &p) { return fft_chunk_takes(p, (uint32_t)acc); }))
+        ll.kind = kFftChunk;
       ll.groups_off = st.put(descs.data(), descs.size() * sizeof(FftPass2));
       ll.wgs_off = st.put(starts.data(), starts.size() * sizeof(uint32_t));
       ll.n_groups = (uint32_t)descs.size();

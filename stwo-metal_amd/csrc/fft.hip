@@ -993,6 +993,7 @@ int make_group_passes(stwo_hip_ctx *ctx, uint32_t n, uint32_t N, bool inverse, c
 }
 
 int launch_fft_pass(stwo_hip_ctx *ctx, bool inverse, const FftPass2 &p, uint32_t wgs, uint32_t wg_log) {
+  if (fft_chunk_takes(p, wgs)) return launch_fft_chunk(ctx, inverse, p, wgs);
   if (wg_log == 8 && p.fixed == 1)
     return inverse ? launch(ctx, "ifft_pass_wg8", fft_pass_kernel<true, 8, 3, 0, 4, 8>, dim3(wgs), dim3(256), 0, p)
                    : launch(ctx, "rfft_pass_wg8", fft_pass_kernel<false, 8, 3, 8, 4, 0>, dim3(wgs), dim3(256), 0, p);
@@ -1049,6 +1050,7 @@ int launch_fft_multi(stwo_hip_ctx *ctx, bool inverse, const FftPass2 *d_groups, 
     if (kind == -1) return STWO_MULTI(9, -1);
     return STWO_MULTI(9, 0);
   }
+  if (kind == kFftChunk) return launch_fft_chunk_multi(ctx, inverse, d_groups, d_wg_start, n_groups, total_wgs);
   if (kind == 1) return inverse ? launch(ctx, name, fft_pass_multi_kernel<true, 8, 3, 0, 4, 8>, grid, b8, 0, d_groups, d_wg_start, n_groups)
                                 : launch(ctx, name, fft_pass_multi_kernel<false, 8, 3, 8, 4, 0>, grid, b8, 0, d_groups, d_wg_start, n_groups);
   if (kind == 3) return inverse ? launch(ctx, name, fft_pass_multi_kernel<true, 8, 2, 6, 7, 1>, grid, b8, 0, d_groups, d_wg_start, n_groups)

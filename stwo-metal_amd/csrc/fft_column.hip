@@ -192,6 +192,101 @@ __device__ __forceinline__ void column_body(const ColumnFft &p, const FftCol *co
   }
 }
 
+// The low pass (layers 0 .. 11 of a larger domain) of few columns: a workgroup
+// of 1,024 lanes per 2^12 words, four words a lane, two layers at a time through
+// LDS with the chunk's twiddles read beside its words.  The register pass gives a
+// lane sixteen words and a workgroup 256, and reads its twiddles stage by stage:
+// a quarter of the waves, each with four times the arithmetic between barriers.
+// 512 of them (16 x 2^17): 12.4 us, here 11.1.
+constexpr uint32_t kChunk = 12, kChunkQuads = 1u << (kChunk - 2);
+struct ChunkLds {
+  uint32_t T[1u << (kChunk - 1)], D[(1u << kChunk) / 16 * 17];
+};
+template <bool INV>
+__device__ __forceinline__ void chunk_body(const FftPass2 &p, uint32_t wg, ChunkLds &S) {
+  const uint32_t q = threadIdx.x, N = p.N, chunk = wg & ((1u << (N - kChunk)) - 1), col = wg >> (N - kChunk);
+  // Words 2q and 2q + 1 of the chunk's part of every level, laid out as the
+  // tree of a domain of 2^12: level s has 2^(11 - s) of them from 2^11 - 2^(12 - s) on.
+  uint32_t t[2];
+#pragma unroll
+  for (int k = 0; k < 2; k++) {
+    const uint32_t i = 2 * q + k, r = (1u << (kChunk - 1)) - i;  // the last word is no level's
+    const uint32_t s = kChunk - (32 - __clz(r - 1));
+    t[k] = r < 2 ? 0u
+                 : gld(p.tw_end - ((size_t)1 << (N - s)),
+                       ((chunk << (kChunk - 1 - s)) + i - ((1u << (kChunk - 1)) - (1u << (kChunk - s)))) << 2);
+  }
+  const FftCol c = p.cols[col];
+  const uint32_t *in = (const uint32_t *)readfirstlane_u64((uint64_t)(c.in + ((size_t)chunk << kChunk)));
+  uint32_t *out = (uint32_t *)readfirstlane_u64((uint64_t)(c.out + ((size_t)chunk << kChunk)));
+  uint32_t x[4];
+  if (!INV) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) x[k] = gld(in, (q + k * kChunkQuads) << 2);
+  } else if (((uintptr_t)in & 15) == 0) {
+    const u32x4 v = gld4(in, q << 4);
+    x[0] = v.x;
+    x[1] = v.y;
+    x[2] = v.z;
+    x[3] = v.w;
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; k++) x[k] = gld(in, (4 * q + k) << 2);
+  }
+  S.T[2 * q] = t[0];
+  S.T[2 * q + 1] = t[1];
+  __syncthreads();
+  const uint32_t *l0 = level(S.T, kChunk, kChunk - 2), *l1 = level(S.T, kChunk, kChunk - 1);
+  if (INV) {
+    low_layers<true>(x, S.T, kChunk, q, true);
+    *reinterpret_cast<u32x4 *>(S.D + pos(4 * q)) = u32x4{x[0], x[1], x[2], x[3]};
+    __syncthreads();
+#pragma unroll
+    for (uint32_t s = 2; s + 2 < kChunk; s += 2) lds_step<true>(S.D, S.T, kChunk, s);
+#pragma unroll
+    for (int k = 0; k < 4; k++) x[k] = S.D[pos(q + k * kChunkQuads)];
+    quad_layers<true>(x, l1[0], l0[0], l0[1]);
+    if (p.scale)
+#pragma unroll
+      for (int k = 0; k < 4; k++) x[k] = m31_mul(x[k], p.scale);
+#pragma unroll
+    for (int k = 0; k < 4; k++) gst(out, (q + k * kChunkQuads) << 2, x[k]);
+    return;
+  }
+  quad_layers<false>(x, l1[0], l0[0], l0[1]);
+#pragma unroll
+  for (int k = 0; k < 4; k++) S.D[pos(q + k * kChunkQuads)] = x[k];
+  __syncthreads();
+#pragma unroll
+  for (uint32_t s = kChunk - 4; s >= 2; s -= 2) lds_step<false>(S.D, S.T, kChunk, s);
+  const u32x4 v = *reinterpret_cast<const u32x4 *>(S.D + pos(4 * q));
+  uint32_t y[4] = {v.x, v.y, v.z, v.w};
+  low_layers<false>(y, S.T, kChunk, q, true);
+  if (((uintptr_t)out & 15) == 0) {
+    gst4(out, q << 4, u32x4{y[0], y[1], y[2], y[3]});
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; k++) gst(out, (4 * q + k) << 2, y[k]);
+  }
+}
+template <bool INV>
+__global__ void __launch_bounds__(kColMaxThreads) fft_chunk_kernel(FftPass2 p) {
+  __shared__ __align__(16) ChunkLds S;
+  chunk_body<INV>(p, blockIdx.x, S);
+}
+template <bool INV>
+__global__ void __launch_bounds__(kColMaxThreads) fft_chunk_multi_kernel(const FftPass2 *groups,
+                                                                         const uint32_t *wg_start, uint32_t n_groups) {
+  __shared__ __align__(16) ChunkLds S;
+  uint32_t g = 0, hi = n_groups;
+  while (hi - g > 1) {
+    const uint32_t mid = (g + hi) / 2;
+    if (wg_start[mid] <= blockIdx.x) g = mid; else hi = mid;
+  }
+  const FftPass2 p = groups[g];
+  chunk_body<INV>(p, blockIdx.x - wg_start[g], S);
+}
+
 __device__ __forceinline__ uint32_t column_group(const ColumnFft *groups, uint32_t n) {
   uint32_t g = 0, hi = n;
   while (hi - g > 1) {
@@ -279,6 +374,23 @@ int run_column_fft(stwo_hip_ctx *ctx, const stwo_hip_twiddles *tw, const std::ve
   if (!fwd) return launch(ctx, name(inv, fwd), column_fft_kernel<true, false>, grid, block, lds, p);
   if (!inv) return launch(ctx, name(inv, fwd), column_fft_kernel<false, true>, grid, block, lds, p);
   return launch(ctx, name(inv, fwd), column_fft_kernel<true, true>, grid, block, lds, p);
+}
+
+bool fft_chunk_takes(const FftPass2 &p, uint32_t total_wgs) {
+  return p.fixed == 1 && p.rep_log == 0 && p.in_log == p.N && total_wgs <= kChunkWgs;
+}
+int launch_fft_chunk(stwo_hip_ctx *ctx, bool inverse, const FftPass2 &p, uint32_t wgs) {
+  const dim3 grid(wgs), block(kColMaxThreads);
+  return inverse ? launch(ctx, "ifft_pass_chunk", fft_chunk_kernel<true>, grid, block, 0, p)
+                 : launch(ctx, "rfft_pass_chunk", fft_chunk_kernel<false>, grid, block, 0, p);
+}
+int launch_fft_chunk_multi(stwo_hip_ctx *ctx, bool inverse, const FftPass2 *d_groups, const uint32_t *d_wg_start,
+                           uint32_t n_groups, uint32_t total_wgs) {
+  const dim3 grid(total_wgs), block(kColMaxThreads);
+  return inverse ? launch(ctx, "ifft_pass_chunk", fft_chunk_multi_kernel<true>, grid, block, 0, d_groups, d_wg_start,
+                          n_groups)
+                 : launch(ctx, "rfft_pass_chunk", fft_chunk_multi_kernel<false>, grid, block, 0, d_groups, d_wg_start,
+                          n_groups);
 }
 
 int launch_column_fft_multi(stwo_hip_ctx *ctx, const ColumnFft *d_groups, uint32_t n_groups, uint32_t wgs,
