@@ -8,13 +8,13 @@
 // (STWO/core/poly/utils.rs:27-38), i.e. sum_j c_j * basis_j with
 // basis_j = prod of g_k over the set bits k of j, g_0 = y, g_1 = x,
 // g_k = pi^(k-1)(x), pi(x) = 2x^2 - 1.  The basis does not depend on the
-// column, so one table of the low 2^11 basis values serves every column: a
-// workgroup takes one 2^11-coefficient block of up to 8 columns of the same
-// size, forms the dot products with the table (64-bit accumulation, one
+// column: a workgroup of the one launch takes several 2^11-coefficient blocks of
+// up to 8 columns of the same size, its lanes holding the low 2^11 basis values,
+// forms the dot products (64-bit accumulation, one
 // multiply-add per limb and coefficient), and multiplies by the product of
-// g_k over the block index's bits; a second kernel sums each column's
-// blocks.  Sums of field elements are exact, so the grouping does not change
-// the result.
+// g_k over the block index's bits; the last workgroup of a run of columns to
+// finish sums the others' shares.  Sums of field elements are exact, so the
+// grouping does not change the result.
 #include <string.h>
 
 #include <algorithm>
@@ -24,15 +24,17 @@
 #include "common.hpp"
 #include "field.hpp"
 #include "internal.hpp"
+#include "merkle_dev.hpp"
 
 namespace stwo_hip {
 
 constexpr uint32_t kEvalBlockLog = 11;  // 2048 coefficients per workgroup and block
 
-struct EvalCol {
-  const uint32_t *coeffs;
-  uint32_t log_size;
-  uint32_t block_begin;  // first block (partial) index of this column
+// A run of n <= kDotCols consecutive columns of one log size: the first of its
+// workgroups, how many it has, and its shares' place (words).
+constexpr uint32_t kDotCols = 8;
+struct EvalRun {
+  uint32_t col0, n, log_size, wg0, wgs, part;
 };
 struct EvalFactors {
   uint32_t g[32][4];  // g_0 = y, g_1 = x, g_k = pi^(k-1)(x)
@@ -43,147 +45,186 @@ __device__ __forceinline__ qm31 ld_factor(const EvalFactors *f, uint32_t k) {
   return qm31_make(f->g[k][0], f->g[k][1], f->g[k][2], f->g[k][3]);
 }
 
-// Basis values of the low kEvalBlockLog bits: basis[t] = prod of g_k over the
-// set bits k of t (k < kEvalBlockLog), 4 words each.  The basis of index
-// j = (b << B) + t is basis[t] times the product of g_k over the set bits of
-// b at positions k >= B, so one table serves every column and block.
-__global__ void __launch_bounds__(256) eval_basis_kernel(const EvalFactors *f, uint32_t *basis, uint32_t n) {
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  qm31 r = qm31_make(1, 0, 0, 0);
-  for (uint32_t k = 0; (t >> k) != 0; k++)
-    if ((t >> k) & 1) r = qm31_mul(r, ld_factor(f, k));
-  for (int w = 0; w < 4; w++) basis[4 * (size_t)t + w] = r.v[w];
-}
-
-// One workgroup: block `block` (2^B coefficients, B = min(log, kEvalBlockLog))
-// of `n` <= kDotCols consecutive columns of the same log size.  Lane t holds
+// Workgroup w of its run takes blocks w, w + wgs, ... (2^B coefficients each, B =
+// min(log, kEvalBlockLog)) of the run's columns.  Lane t holds
 // the basis values of coefficients 8t .. 8t + 7 in registers and, per
 // column, accumulates sum c_j * basis_j limb by limb in 64 bits
 // (v_mad_u64_u32; each product is below 2^62, so three fit before a fold
 // (x & P) + (x >> 31), which keeps the sum below 2^34).  The 256 lanes' sums
-// are reduced through LDS, multiplied by the block's factor and written as
-// the column's partial for the block.
-constexpr uint32_t kDotCols = 8;
-struct EvalWork {
-  uint32_t col0, n, block, log_size;
+// are reduced through LDS, multiplied by the block's factor and added to the
+// workgroup's share, while the next block's loads are on their way.
+//
+// Bound by the multiply-adds and the loads under them, three workgroups a CU:
+// 264 columns of 2^18 (277 MB) take 81 us and 3.5 KB of tables.  In three launches
+// (the basis, a workgroup per block and run, the sums) it was 7.4 + 72.7 + 5.1 us
+// and the gaps between them, with a table entry per block and run (68 KB).
+constexpr uint32_t kEvalFactorBlocks = 64;  // blocks whose factors are held at once
+struct EvalLds {
+  uint32_t red[kDotCols * 4][257];
+  uint32_t sums[kDotCols * 4];
+  uint32_t low[2][16][4];                 // basis of index bits 3..6 and 7..10
+  uint32_t fac[kEvalFactorBlocks][4];
+  uint32_t last;
 };
+__device__ __forceinline__ qm31 ld_qm31(const uint32_t *p) { return qm31_make(p[0], p[1], p[2], p[3]); }
 
-
-__global__ void __launch_bounds__(256) eval_point_dot_kernel(const EvalCol *cols, const EvalWork *work,
-                                                             const EvalFactors *f,
-                                                             const uint32_t *basis, uint32_t *partials) {
-  __shared__ uint32_t red[kDotCols * 4][257];
-  __shared__ uint32_t sums[kDotCols * 4];
-  const EvalWork w = work[blockIdx.x];
-  const uint32_t B = w.log_size < kEvalBlockLog ? w.log_size : kEvalBlockLog;
-  const uint32_t nb = 1u << B;
-  const uint32_t t0 = threadIdx.x * 8;
-  qm31 b[8];
-#pragma unroll
-  for (int i = 0; i < 8; i++) {
-    const uint32_t t = t0 + i;
-    b[i] = t < nb ? qm31_make(basis[4 * t], basis[4 * t + 1], basis[4 * t + 2], basis[4 * t + 3])
-                  : qm31_make(0, 0, 0, 0);
+__global__ void __launch_bounds__(256) eval_point_kernel(const uint32_t *const *cols, const EvalRun *runs,
+                                                         uint32_t n_runs, const EvalFactors *f, uint32_t *partials,
+                                                         uint32_t *counters, uint32_t *out) {
+  __shared__ EvalLds S;
+  const uint32_t tid = threadIdx.x;
+  uint32_t ri = 0, hi = n_runs;
+  while (hi - ri > 1) {
+    const uint32_t mid = (ri + hi) / 2;
+    if (runs[mid].wg0 <= blockIdx.x) ri = mid; else hi = mid;
   }
-  // Every coefficient load of the workgroup is issued before the first
-  // product (one memory latency per workgroup rather than one per column):
+  const EvalRun R = runs[ri];
+  const uint32_t w = blockIdx.x - R.wg0, n = R.n;
+  const uint32_t B = R.log_size < kEvalBlockLog ? R.log_size : kEvalBlockLog, nb = 1u << B;
+  const uint32_t n_blocks = 1u << (R.log_size - B), t0 = tid * 8;
   // 8 words per lane and column, as two 16-byte loads when the block is
   // whole and the column pointer 32-byte aligned (a wave-uniform test).
   uint32_t cv[kDotCols][8];
+  auto load = [&](uint32_t block) {
 #pragma unroll
-  for (uint32_t j = 0; j < kDotCols; j++) {
-    if (j < w.n) {
-      const uint32_t *c = cols[w.col0 + j].coeffs + ((size_t)w.block << B);
-      if (nb == (1u << kEvalBlockLog) && ((uintptr_t)c & 31) == 0) {
-        const u32x4 lo = *(gconst_u4 *)(as_global(c) + t0), hi = *(gconst_u4 *)(as_global(c) + t0 + 4);
-        cv[j][0] = lo.x;
-        cv[j][1] = lo.y;
-        cv[j][2] = lo.z;
-        cv[j][3] = lo.w;
-        cv[j][4] = hi.x;
-        cv[j][5] = hi.y;
-        cv[j][6] = hi.z;
-        cv[j][7] = hi.w;
-      } else {
+    for (uint32_t j = 0; j < kDotCols; j++) {
+      if (j < n) {
+        const uint32_t *c = cols[R.col0 + j] + ((size_t)block << B);
+        if (nb == (1u << kEvalBlockLog) && ((uintptr_t)c & 31) == 0) {
+          const u32x4 lo = *(gconst_u4 *)(as_global(c) + t0), h4 = *(gconst_u4 *)(as_global(c) + t0 + 4);
+          cv[j][0] = lo.x;
+          cv[j][1] = lo.y;
+          cv[j][2] = lo.z;
+          cv[j][3] = lo.w;
+          cv[j][4] = h4.x;
+          cv[j][5] = h4.y;
+          cv[j][6] = h4.z;
+          cv[j][7] = h4.w;
+        } else {
 #pragma unroll
-        for (int i = 0; i < 8; i++) cv[j][i] = (t0 + i < nb) ? as_global(c)[t0 + i] : 0;
+          for (int i = 0; i < 8; i++) cv[j][i] = (t0 + i < nb) ? as_global(c)[t0 + i] : 0;
+        }
       }
     }
+  };
+  load(w);
+  // Factors of blocks w + k wgs: bit i of the block index selects g_{B + i}.
+  auto factors = [&](uint32_t first) {
+    const uint32_t block = first + (tid & (kEvalFactorBlocks - 1)) * R.wgs;
+    if (tid >= kEvalFactorBlocks || block >= n_blocks) return;
+    qm31 r = qm31_make(1, 0, 0, 0);
+    for (uint32_t k = B; k < R.log_size; k++)
+      if ((block >> (k - B)) & 1) r = qm31_mul(r, ld_factor(f, k));
+    for (int k = 0; k < 4; k++) S.fac[tid][k] = r.v[k];
+  };
+  // The basis: of index bits 3..6 and 7..10 by 32 lanes, their products and
+  // those of bits 0..2 in every lane.
+  if (tid >= 128 && tid < 160) {
+    const uint32_t half = (tid >> 4) & 1, e = tid & 15;
+    qm31 r = qm31_make(1, 0, 0, 0);
+    for (uint32_t k = 0; k < 4; k++)
+      if ((e >> k) & 1) r = qm31_mul(r, ld_factor(f, 3 + 4 * half + k));
+    for (int k = 0; k < 4; k++) S.low[half][e][k] = r.v[k];
   }
+  factors(w);
+  __syncthreads();
+  qm31 b[8];
+  b[0] = qm31_mul(ld_qm31(S.low[0][tid & 15]), ld_qm31(S.low[1][tid >> 4]));
 #pragma unroll
-  for (uint32_t j = 0; j < kDotCols; j++) {
-    if (j >= w.n) break;
-    uint64_t acc[4] = {0, 0, 0, 0};
+  for (int k = 0; k < 3; k++)
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
+    for (int i = 0; i < (1 << k); i++) b[(1 << k) + i] = qm31_mul(b[i], ld_factor(f, k));
+  if (t0 + 8 > nb)  // a column below 2^11: no coefficient, no product
 #pragma unroll
-      for (int k = 0; k < 4; k++) acc[k] += (uint64_t)cv[j][i] * b[i].v[k];
-      if (i == 2 || i == 5)
+    for (int i = 0; i < 8; i++)
+      if (t0 + i >= nb) b[i] = qm31_make(0, 0, 0, 0);
+  qm31 share = qm31_make(0, 0, 0, 0);
+  uint32_t k_blk = 0;
+  for (uint32_t block = w; block < n_blocks; block += R.wgs) {
 #pragma unroll
-        for (int k = 0; k < 4; k++) acc[k] = m31_fold64(acc[k]);
+    for (uint32_t j = 0; j < kDotCols; j++) {
+      if (j >= n) break;
+      uint64_t acc[4] = {0, 0, 0, 0};
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) acc[k] += (uint64_t)cv[j][i] * b[i].v[k];
+        if (i == 2 || i == 5)
+#pragma unroll
+          for (int k = 0; k < 4; k++) acc[k] = m31_fold64(acc[k]);
+      }
+#pragma unroll
+      for (int k = 0; k < 4; k++) S.red[4 * j + k][tid] = m31_reduce64(acc[k]);
     }
-#pragma unroll
-    for (int k = 0; k < 4; k++) red[4 * j + k][threadIdx.x] = m31_reduce64(acc[k]);
-  }
-  __syncthreads();
-  // Row r (column r / 4, limb r % 4): 8 lanes sum 32 entries each, then
-  // combine across the 8 lanes (consecutive lanes of one wave).
-  const uint32_t r = threadIdx.x >> 3, seg = threadIdx.x & 7;
-  if (r < 4 * w.n) {
-    uint64_t s = 0;
-#pragma unroll
-    for (int i = 0; i < 32; i++) s += red[r][seg * 32 + i];
-    uint32_t v = m31_reduce64(s);
-#pragma unroll
-    for (int o = 1; o < 8; o <<= 1) v = m31_add(v, __shfl_xor(v, o, 8));
-    if (seg == 0) sums[r] = v;
-  }
-  __syncthreads();
-  if (threadIdx.x < w.n) {
-    const uint32_t j = threadIdx.x;
-    qm31 res = qm31_make(sums[4 * j], sums[4 * j + 1], sums[4 * j + 2], sums[4 * j + 3]);
-    // the block index's set bits select g_B, g_{B+1}, ...
-    for (uint32_t k = B; k < w.log_size; k++)
-      if ((w.block >> (k - B)) & 1) res = qm31_mul(res, ld_factor(f, k));
-    const size_t o = 4 * ((size_t)cols[w.col0 + j].block_begin + w.block);
-    for (int q = 0; q < 4; q++) partials[o + q] = res.v[q];
-  }
-}
-
-// One workgroup per column: the sum of its block partials.
-__global__ void __launch_bounds__(256) eval_point_sum_kernel(const EvalCol *cols, uint32_t n_cols,
-                                                             uint32_t total_blocks, const uint32_t *partials,
-                                                             uint32_t *out) {
-  __shared__ qm31 red[256];
-  const uint32_t ci = blockIdx.x;
-  const uint32_t b0 = cols[ci].block_begin;
-  const uint32_t b1 = ci + 1 < n_cols ? cols[ci + 1].block_begin : total_blocks;
-  qm31 acc = qm31_make(0, 0, 0, 0);
-  for (uint32_t b = b0 + threadIdx.x; b < b1; b += blockDim.x)
-    acc = qm31_add(acc, qm31_make(partials[4 * (size_t)b], partials[4 * (size_t)b + 1], partials[4 * (size_t)b + 2],
-                                  partials[4 * (size_t)b + 3]));
-  red[threadIdx.x] = acc;
-  __syncthreads();
-  for (uint32_t s = 128; s > 0; s >>= 1) {
-    if (threadIdx.x < s) red[threadIdx.x] = qm31_add(red[threadIdx.x], red[threadIdx.x + s]);
+    if (block + R.wgs < n_blocks) load(block + R.wgs);
     __syncthreads();
+    // Row r (column r / 4, limb r % 4): 8 lanes sum 32 entries each, then
+    // combine across the 8 lanes (consecutive lanes of one wave).
+    const uint32_t r = tid >> 3, seg = tid & 7;
+    if (r < 4 * n) {
+      uint64_t s = 0;
+#pragma unroll
+      for (int i = 0; i < 32; i++) s += S.red[r][seg * 32 + i];
+      uint32_t v = m31_reduce64(s);
+#pragma unroll
+      for (int o = 1; o < 8; o <<= 1) v = m31_add(v, __shfl_xor(v, o, 8));
+      if (seg == 0) S.sums[r] = v;
+    }
+    __syncthreads();
+    if (tid < n) share = qm31_add(share, qm31_mul(ld_qm31(S.sums + 4 * tid), ld_qm31(S.fac[k_blk])));
+    if (++k_blk == kEvalFactorBlocks) {
+      k_blk = 0;
+      __syncthreads();
+      factors(block + R.wgs);  // seen after the next block's first barrier
+    }
   }
-  if (threadIdx.x == 0)
-    for (int w = 0; w < 4; w++) out[4 * (size_t)ci + w] = red[0].v[w];
+  if (R.wgs == 1) {
+    if (tid < n)
+      for (int k = 0; k < 4; k++) out[4 * (size_t)(R.col0 + tid) + k] = share.v[k];
+    return;
+  }
+  // The last workgroup of the run to count itself sums the shares (stored and
+  // loaded at agent scope, complete before the count) and clears the counter.
+  uint32_t *part = partials + R.part;
+  if (tid < n)
+    for (int k = 0; k < 4; k++) st_agent(part + ((size_t)w * n + tid) * 4 + k, share.v[k]);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (tid == 0) {
+    const uint32_t old =
+        __hip_atomic_fetch_add(counters + ri, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t last = old + 1 == R.wgs;
+    if (last) st_agent(counters + ri, 0);
+    S.last = last;
+  }
+  __syncthreads();
+  if (!S.last) return;
+  const uint32_t j = tid >> 5, lane = tid & 31;  // 32 lanes a column
+  if (j >= n) return;
+  qm31 sum = qm31_make(0, 0, 0, 0);
+  for (uint32_t i = lane; i < R.wgs; i += 32) {
+    const uint32_t *p = part + ((size_t)i * n + j) * 4;
+    sum = qm31_add(sum, qm31_make(ld_agent(p), ld_agent(p + 1), ld_agent(p + 2), ld_agent(p + 3)));
+  }
+#pragma unroll
+  for (int o = 1; o < 32; o <<= 1)
+#pragma unroll
+    for (int k = 0; k < 4; k++) sum.v[k] = m31_add(sum.v[k], __shfl_xor(sum.v[k], o, 32));
+  if (lane == 0)
+    for (int k = 0; k < 4; k++) out[4 * (size_t)(R.col0 + j) + k] = sum.v[k];
 }
 
 // ---- fixed scratch for the entry point that allocates nothing -------------
 //
-// stwo_hip_eval_at_point_noalloc keeps its basis table, block partials and
+// stwo_hip_eval_at_point_noalloc keeps its workgroups' shares and the
 // per-column sums in this file-scope array (one copy per device, held until
 // the process ends) instead of buffers it would allocate.  Layout in words:
-// basis [0, kNaBasisWords), sums [kNaBasisWords, + 4 n_cols), partials after
-// them.  Host code never passes the array's name to a kernel or a copy (on
+// sums [0, 4 n_cols), shares after them.  The call's limit counts a share per
+// column and block and 2^13 words besides, more than it now takes.  Host code never passes the array's name to a kernel or a copy (on
 // the host it is only a stand-in for the symbol): it uses the per-device
 // address that hipGetSymbolAddress returned at context creation.
 constexpr size_t kNaScratchWords = 1u << 18;  // 1 MiB
-constexpr size_t kNaBasisWords = (size_t)4 << kEvalBlockLog;
+constexpr size_t kNaReserved = (size_t)4 << kEvalBlockLog;
 static __device__ __align__(256) uint32_t scratch[kNaScratchWords];
 
 constexpr int kMaxDevices = 64;
@@ -227,14 +268,10 @@ static int eval_at_point_impl(stwo_hip_ctx *ctx, const uint32_t *const *coeffs, 
                      "eval_at_point: NULL argument");
   if (n_cols == 0) return STWO_HIP_OK;
   STWO_HIP_CHECK_ARG(ctx, n_cols <= 65536, "eval_at_point: %zu columns in one call (at most 65536)", n_cols);
-  std::vector<EvalCol> tab(n_cols);
   uint64_t total = 0;
   uint32_t max_log = 0;
   for (size_t c = 0; c < n_cols; c++) {
     STWO_HIP_CHECK_ARG(ctx, coeffs[c] && log_sizes[c] <= 30, "eval_at_point: column %zu invalid", c);
-    tab[c].coeffs = coeffs[c];
-    tab[c].log_size = log_sizes[c];
-    tab[c].block_begin = (uint32_t)total;
     total += 1ull << (log_sizes[c] > kEvalBlockLog ? log_sizes[c] - kEvalBlockLog : 0);
     max_log = std::max(max_log, log_sizes[c]);
   }
@@ -250,66 +287,69 @@ static int eval_at_point_impl(stwo_hip_ctx *ctx, const uint32_t *const *coeffs, 
       x = qm31_sub(qm31_add(sq, sq), qm31_make(1, 0, 0, 0));
     }
   }
-  // Work items: runs of up to kDotCols consecutive columns of one log size, per block.
-  std::vector<EvalWork> work;
+  // Runs of up to kDotCols consecutive columns of one log size, each with
+  // workgroups for an equal share of the blocks: about three a CU in all (as many
+  // as their registers allow), one where the runs alone are more than the counters.
+  std::vector<EvalRun> runs;
+  uint64_t n_work = 0;  // blocks over all runs
   for (size_t c = 0; c < n_cols;) {
     size_t e = c + 1;
     while (e < n_cols && e - c < kDotCols && log_sizes[e] == log_sizes[c]) e++;
-    const uint32_t lg = log_sizes[c];
-    const uint32_t nblk = 1u << (lg > kEvalBlockLog ? lg - kEvalBlockLog : 0);
-    for (uint32_t k = 0; k < nblk; k++) work.push_back({(uint32_t)c, (uint32_t)(e - c), k, lg});
+    runs.push_back({(uint32_t)c, (uint32_t)(e - c), log_sizes[c], 0, 0, 0});
+    n_work += 1ull << (log_sizes[c] > kEvalBlockLog ? log_sizes[c] - kEvalBlockLog : 0);
     c = e;
   }
-  const uint32_t n_basis = 1u << std::min(max_log, kEvalBlockLog);
+  const uint64_t per = (n_work + 767) / 768;
+  uint32_t wgs = 0;
+  size_t shares = 0;
+  for (EvalRun &r : runs) {
+    const uint64_t nblk = 1ull << (r.log_size > kEvalBlockLog ? r.log_size - kEvalBlockLog : 0);
+    r.wg0 = wgs;
+    r.wgs = runs.size() > kTreeCounters ? 1 : (uint32_t)((nblk + per - 1) / per);
+    r.part = (uint32_t)shares;
+    wgs += r.wgs;
+    shares += (size_t)r.wgs * r.n * 4;
+  }
   if (na_scratch) {
     // Everything must fit the fixed array, and the tables the ring arena
     // (larger ones would take an allocated buffer).
-    STWO_HIP_CHECK_ARG(ctx, kNaBasisWords + 4 * ((uint64_t)n_cols + total) <= kNaScratchWords,
+    STWO_HIP_CHECK_ARG(ctx, kNaReserved + 4 * ((uint64_t)n_cols + total) <= kNaScratchWords,
                        "eval_at_point_noalloc: %zu columns and %llu blocks of 2^11 coefficients need %llu words of "
                        "scratch, more than the %zu available",
                        n_cols, (unsigned long long)total,
-                       (unsigned long long)(kNaBasisWords + 4 * ((uint64_t)n_cols + total)), kNaScratchWords);
+                       (unsigned long long)(kNaReserved + 4 * ((uint64_t)n_cols + total)), kNaScratchWords);
     STWO_HIP_CHECK_ARG(ctx,
-                       tab.size() * sizeof(EvalCol) + work.size() * sizeof(EvalWork) + sizeof(EvalFactors) + 512 <=
-                           ctx->arena_cap / 2,
-                       "eval_at_point_noalloc: %zu work items exceed the table arena", work.size());
+                       16 * (n_cols + n_work) + sizeof(EvalFactors) + 512 <= ctx->arena_cap / 2,
+                       "eval_at_point_noalloc: %zu work items exceed the table arena", (size_t)n_work);
   }
-  void *d_tab = nullptr, *d_work = nullptr, *d_basis = nullptr, *d_part = nullptr, *d_out = nullptr;
+  void *d_tab = nullptr, *d_runs = nullptr, *d_part = nullptr, *d_out = nullptr;
   const EvalFactors *d_f = (const EvalFactors *)d_factors;
   int rc;
   {
-    const void *srcs[3] = {tab.data(), work.data(), &f};
-    const size_t bytes[3] = {tab.size() * sizeof(EvalCol), work.size() * sizeof(EvalWork), sizeof f};
+    const void *srcs[3] = {coeffs, runs.data(), &f};
+    const size_t bytes[3] = {n_cols * sizeof(*coeffs), runs.size() * sizeof(EvalRun), sizeof f};
     void *d[3];
     // with the point on the device (the prove) the tables repeat from call to call
     rc = (d_factors && !na_scratch) ? upload_tables_cached(ctx, "eval_at_point", 2, srcs, bytes, d)
                                     : upload_tables(ctx, d_factors ? 2 : 3, srcs, bytes, d);
     if (rc) return rc;
     d_tab = d[0];
-    d_work = d[1];
+    d_runs = d[1];
     if (!d_factors) d_f = (const EvalFactors *)d[2];
   }
   if (na_scratch) {
-    d_basis = na_scratch;
-    d_out = na_scratch + kNaBasisWords;
-    d_part = na_scratch + kNaBasisWords + 4 * n_cols;
+    d_out = na_scratch;
+    d_part = na_scratch + 4 * n_cols;
   } else {
-    rc = get_scratch(ctx, "eval_point_basis", (size_t)n_basis * 16, &d_basis);
-    if (rc) return rc;
-    rc = get_scratch(ctx, "eval_point_partials", total * 16, &d_part);
+    rc = get_scratch(ctx, "eval_point_partials", shares * 4, &d_part);
     if (rc) return rc;
     rc = get_scratch(ctx, "eval_point_out", n_cols * 16, &d_out);
     if (rc) return rc;
   }
   if (d_values) d_out = d_values;
-  rc = launch(ctx, "eval_at_point_basis", eval_basis_kernel, dim3((n_basis + 255) / 256), dim3(256), 0, d_f,
-              (uint32_t *)d_basis, n_basis);
-  if (rc) return rc;
-  rc = launch(ctx, "eval_at_point_dot", eval_point_dot_kernel, dim3((uint32_t)work.size()), dim3(256), 0,
-              (const EvalCol *)d_tab, (const EvalWork *)d_work, d_f, (const uint32_t *)d_basis, (uint32_t *)d_part);
-  if (rc) return rc;
-  rc = launch(ctx, "eval_at_point_sum", eval_point_sum_kernel, dim3((uint32_t)n_cols), dim3(256), 0,
-              (const EvalCol *)d_tab, (uint32_t)n_cols, (uint32_t)total, (const uint32_t *)d_part, (uint32_t *)d_out);
+  rc = launch(ctx, "eval_at_point", eval_point_kernel, dim3(wgs), dim3(256), 0, (const uint32_t *const *)d_tab,
+              (const EvalRun *)d_runs, (uint32_t)runs.size(), d_f, (uint32_t *)d_part, ctx->d_counters,
+              (uint32_t *)d_out);
   if (rc) return rc;
   if (d_values) return STWO_HIP_OK;
   return stwo_hip_download(ctx, values, (const uint32_t *)d_out, 4 * n_cols);

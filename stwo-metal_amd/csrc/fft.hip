@@ -174,6 +174,12 @@ __global__ void fft_small_kernel(SmallFft a) {
 // 256-byte coalesced runs; tiles on the diagonal swap within themselves.
 // Index split for log n = 2k + r bits: i = [hi: 6 | mid: r' | lo: 6].
 constexpr uint32_t kBrLog = 6;
+// Up to 2^17 elements a lane per pair is ahead, its scattered half within the
+// caches and without the way through LDS (us, lane per pair / tiles: 2^12 2.56 /
+// 2.96, 2^14 2.80 / 3.12, 2^16 2.92 / 3.40, 2^17 3.24 / 3.36, 2^18 3.80 / 3.44, 2^19
+// 6.00 / 3.64).
+constexpr uint32_t kBrTiledMin = 18;
+static_assert(kBrTiledMin >= 2 * kBrLog, "a tile's rows and columns");
 
 __global__ void __launch_bounds__(256) bit_reverse_small_kernel(uint32_t *v, uint32_t log_n) {
   uint32_t n = 1u << log_n;
@@ -1299,7 +1305,7 @@ static int share_launches(stwo_hip_ctx *ctx, std::map<uint32_t, std::vector<FftC
 }
 
 static int bit_reverse_one(stwo_hip_ctx *ctx, uint32_t *col, uint32_t log_size) {
-  if (log_size >= 2 * kBrLog) {
+  if (log_size >= kBrTiledMin) {
     uint32_t mids = 1u << (log_size - 2 * kBrLog);
     return launch(ctx, "bit_reverse_tiled",
                   ((uintptr_t)col & 15) ? bit_reverse_tiled_kernel<false> : bit_reverse_tiled_kernel<true>,
