@@ -313,7 +313,7 @@ struct MerkleTree {
   uint32_t stop_log, wg_start;
 };
 enum : uint32_t {
-  kMerkleLayer, kMerkleAhead, kMerkleQuad, kMerkleQuadLds, kMerkleNodes64, kMerkleNodes256, kMerkleNodes1024,
+  kMerkleLayer, kMerkleAhead, kMerkleQuadLds, kMerkleNodes64, kMerkleNodes256, kMerkleNodes1024,
   kMerkleTree, kMerkleTreeLds, kMerkleKinds
 };
 struct MerkleStep {

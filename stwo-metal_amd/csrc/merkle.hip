@@ -19,6 +19,7 @@
 // subtree through LDS, writing every layer to global memory, and the last of
 // each group of workgroups to finish hashes on (merkle_dev.hpp).
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "blake2s.hpp"
@@ -133,58 +134,39 @@ __device__ __forceinline__ b2_state layer_hash(const MerkleLayer &L, const ColRe
   return s;
 }
 
-// Layers of few nodes, where a node's chain of blocks is the launch's
-// critical path: one node per quad (b2_compress_quad, about 410
-// instructions per lane instead of 960 on one lane), each block's column
-// words loaded one compression ahead.  Same hash as layer_hash, words j and
-// 4 + j of it in lane j.
+// Layers of few nodes, where a node's hash is the launch's critical path: one
+// node per quad (b2_compress_quad, about 380 instructions per lane instead of 960
+// on one lane).  Same hash as layer_hash, of at most 16 columns, words j and 4 + j
+// of it in lane j.
 __device__ __forceinline__ void layer_hash_quad(const MerkleLayer &L, const ColRef *cols, uint32_t i, uint32_t &lo,
                                                 uint32_t &hi) {
   const uint32_t j = threadIdx.x & 3;
-  const uint32_t *prev = L.prev;
-  const uint32_t n_cols = L.n_cols, lifted = L.lifted;
-  auto load_cols = [&](uint32_t c0, uint32_t (&dst)[16]) {
-    const uint32_t cnt = min(16u, n_cols - c0);
+  const uint32_t n_cols = L.n_cols;
+  uint32_t w[16], m[16];
 #pragma unroll
-    for (uint32_t k = 0; k < 16; k++) {
-      uint32_t v = 0;
-      if (k < cnt) {
-        const ColRef cr = cols[c0 + k];
-        uint32_t idx = lifted ? (((i >> (cr.shift + 1)) << 1) + (i & 1)) : i;
-        v = ld_col_word(cr.p, idx);
-      }
-      dst[k] = v;
+  for (uint32_t k = 0; k < 16; k++) {
+    w[k] = 0;
+    if (k < n_cols) {
+      const ColRef cr = cols[k];
+      w[k] = ld_col_word(cr.p, L.lifted ? (((i >> (cr.shift + 1)) << 1) + (i & 1)) : i);
     }
-  };
+  }
   lo = b2_iv_lo(j);
   hi = b2_iv_hi(j);
-  uint32_t m[16], nx[16];
   uint32_t t = 0;
-  if (n_cols) load_cols(0, nx);
-  if (prev) {
-    load_block64(m, prev + 16 * (size_t)i);
+  if (L.prev) {
+    load_block64(m, L.prev + 16 * (size_t)i);
     t = 64;
     b2_compress_quad(lo, hi, m, t, n_cols == 0);
-  } else if (n_cols == 0) {
-#pragma unroll
-    for (int k = 0; k < 16; k++) m[k] = 0;
-    b2_compress_quad(lo, hi, m, 0, true);
   }
-  for (uint32_t c0 = 0; c0 < n_cols; c0 += 16) {
-    const uint32_t cnt = min(16u, n_cols - c0);
-#pragma unroll
-    for (int k = 0; k < 16; k++) m[k] = nx[k];
-    if (c0 + 16 < n_cols) load_cols(c0 + 16, nx);
-    t += 4 * cnt;
-    b2_compress_quad(lo, hi, m, t, c0 + 16 >= n_cols);
-  }
+  if (n_cols || !L.prev) b2_compress_quad(lo, hi, w, t + 4 * n_cols, true);
   if (L.m31) {
     lo = b2_reduce_word(lo);
     hi = b2_reduce_word(hi);
   }
 }
 
-// Small mixed-degree layers with many columns (up to 2^14 nodes): the chain
+// Small layers with many columns (up to 2^14 nodes): the chain
 // of blocks per node is the critical path and, with one block loaded ahead,
 // each block waits on a table load followed by a column load.  Here a
 // workgroup owns 64 consecutive nodes (a quad each) and stages its columns
@@ -192,10 +174,12 @@ __device__ __forceinline__ void layer_hash_quad(const MerkleLayer &L, const ColR
 // first, then every column's 64 words (one coalesced 256-byte run per wave
 // and load, 32 loads in flight per lane), so a chunk costs about two memory
 // round trips and its blocks then read their words from LDS.  Same hash
-// as layer_hash (mixed layers only, not lifted).
-constexpr uint32_t MQ_CHUNK = 240;  // 15 blocks; 61,440 B of words + 1,920 B of pointers
+// as layer_hash.  Lifted trees of 2^13 leaves over 12 to 98 columns, six in a
+// launch: 47 us, with the loads a block ahead 65 us.
+constexpr uint32_t MQ_CHUNK = 240;  // 15 blocks; 61,440 B of words + 2,880 B of pointers and shifts
 struct QuadTile {
   const uint32_t *ptrs[MQ_CHUNK];
+  uint32_t shift[MQ_CHUNK];
   uint32_t tile[MQ_CHUNK * 64];
 };
 __device__ __forceinline__ void layer_hash_quad_lds(const MerkleLayer &L, uint32_t i0, QuadTile &S, uint32_t &lo,
@@ -224,21 +208,34 @@ __device__ __forceinline__ void layer_hash_quad_lds(const MerkleLayer &L, uint32
   for (uint32_t cb = 0; cb < n_cols; cb += MQ_CHUNK) {
     const uint32_t cnt = min(MQ_CHUNK, n_cols - cb), words = cnt * 64;
     __syncthreads();  // the previous chunk's words are consumed
-    for (uint32_t c = tid; c < cnt; c += 256) S.ptrs[c] = cols[cb + c].p;
-    __syncthreads();
-    for (uint32_t e0 = 0; e0 < words; e0 += 256 * 32) {
-      uint32_t v[32];
-#pragma unroll
-      for (uint32_t k = 0; k < 32; k++) {
-        const uint32_t e = e0 + tid + 256 * k;  // column e >> 6 is uniform over the wave
-        v[k] = (e < words && row < n) ? ld_col_word(S.ptrs[e >> 6], row) : 0u;
-      }
-#pragma unroll
-      for (uint32_t k = 0; k < 32; k++) {
-        const uint32_t e = e0 + tid + 256 * k;
-        if (e < words) S.tile[e] = v[k];
-      }
+    for (uint32_t c = tid; c < cnt; c += 256) {
+      const ColRef cr = cols[cb + c];
+      S.ptrs[c] = cr.p;
+      S.shift[c] = cr.shift;
     }
+    __syncthreads();
+    auto stage = [&](auto lifted) {
+      for (uint32_t e0 = 0; e0 < words; e0 += 256 * 32) {
+        uint32_t v[32];
+#pragma unroll
+        for (uint32_t k = 0; k < 32; k++) {
+          const uint32_t e = e0 + tid + 256 * k;  // column e >> 6 is uniform over the wave
+          v[k] = 0;
+          if (e < words && row < n)
+            v[k] = ld_col_word(S.ptrs[e >> 6],
+                               lifted ? ((row >> (S.shift[e >> 6] + 1)) << 1) + (row & 1) : row);
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < 32; k++) {
+          const uint32_t e = e0 + tid + 256 * k;
+          if (e < words) S.tile[e] = v[k];
+        }
+      }
+    };
+    if (L.lifted)
+      stage(std::true_type{});
+    else
+      stage(std::false_type{});
     __syncthreads();
     for (uint32_t b = 0; b < cnt; b += 16) {
       const uint32_t bc = min(16u, cnt - b);
@@ -265,13 +262,6 @@ __device__ __forceinline__ void store_quad(uint32_t *out, uint32_t i, uint32_t l
   g_u32 *o = as_global(out + 8 * (size_t)i);
   o[threadIdx.x & 3] = lo;
   o[4 + (threadIdx.x & 3)] = hi;
-}
-__device__ __forceinline__ void merkle_layer_quad(const MerkleLayer &L, uint32_t wg) {
-  const uint32_t i = (wg * 256 + threadIdx.x) >> 2;
-  if (i >= 1u << L.log_size) return;  // a quad's four lanes share i and leave together
-  uint32_t lo, hi;
-  layer_hash_quad(L, L.cols, i, lo, hi);
-  store_quad(L.out, i, lo, hi);
 }
 __device__ __forceinline__ void merkle_layer_quad_lds(const MerkleLayer &L, uint32_t wg) {
   __shared__ QuadTile S;
@@ -393,11 +383,6 @@ __global__ void __launch_bounds__(256) merkle_layer_multi_kernel(const MerkleLay
   const MerkleLayer L = step_of(t, n);
   merkle_layer<AHEAD>(L, blockIdx.x - L.wg_start);
 }
-__global__ void __launch_bounds__(256) merkle_layer_quad_kernel(MerkleLayer L) { merkle_layer_quad(L, blockIdx.x); }
-__global__ void __launch_bounds__(256) merkle_layer_quad_multi_kernel(const MerkleLayer *t, uint32_t n) {
-  const MerkleLayer L = step_of(t, n);
-  merkle_layer_quad(L, blockIdx.x - L.wg_start);
-}
 __global__ void __launch_bounds__(256) merkle_layer_quad_lds_kernel(MerkleLayer L) {
   merkle_layer_quad_lds(L, blockIdx.x);
 }
@@ -435,18 +420,16 @@ __global__ void __launch_bounds__(kTreeThreads) merkle_nodes_multi_kernel(const 
 static inline size_t layer_off(uint32_t l) { return tree_layer_off(l); }
 
 // Up to 2^14 nodes with more than one block per node, the layer is
-// latency-bound even at four lanes per node: a quad per node (mixed layers
-// with the columns staged through LDS, lifted ones loading a block ahead).  Below 2^16
-// nodes, a lane per node with the loads one block ahead.
+// latency-bound even at four lanes per node: a quad per node, with the columns
+// staged through LDS.  Below 2^16 nodes, a lane per node with the loads one block
+// ahead.
 MerkleStep merkle_layer_step(const uint32_t *prev, const ColRef *d_cols, uint32_t n_cols, uint32_t log_size,
                              uint32_t *out, int mode, bool lifted) {
   MerkleStep s{};
   s.layer = {prev, d_cols, out, n_cols, log_size, (uint32_t)(mode == STWO_HIP_HASH_BLAKE2S_M31), (uint32_t)lifted, 0};
   const uint32_t n = 1u << log_size;
   const bool quad = log_size <= 14 && n_cols > 16;
-  s.kind = quad                             ? (lifted ? kMerkleQuad : kMerkleQuadLds)
-           : log_size < 16 && n_cols > 16 ? kMerkleAhead
-                                            : kMerkleLayer;
+  s.kind = quad ? kMerkleQuadLds : log_size < 16 && n_cols > 16 ? kMerkleAhead : kMerkleLayer;
   s.wgs = quad ? (n + 63) / 64 : (n + 255) / 256;
   return s;
 }
@@ -472,7 +455,7 @@ bool merkle_tree_step(MerkleStep &s, uint32_t stop_log, uint32_t *counters) {
   const uint32_t lg = s.layer.log_size;
   if (lg > 14 || stop_log >= lg) return false;
   s.tree = {s.layer, counters, stop_log, 0};
-  s.kind = s.layer.n_cols > 16 && !s.layer.lifted ? kMerkleTreeLds : kMerkleTree;
+  s.kind = s.layer.n_cols > 16 ? kMerkleTreeLds : kMerkleTree;
   s.wgs = 1u << (lg > 6 ? lg - 6 : 0);
   return true;
 }
@@ -487,7 +470,6 @@ int launch_merkle(stwo_hip_ctx *ctx, const MerkleStep &s) {
   switch (s.kind) {
     case kMerkleLayer: return launch(ctx, name, merkle_layer_kernel<false>, grid, block, 0, s.layer);
     case kMerkleAhead: return launch(ctx, name, merkle_layer_kernel<true>, grid, block, 0, s.layer);
-    case kMerkleQuad: return launch(ctx, name, merkle_layer_quad_kernel, grid, block, 0, s.layer);
     case kMerkleQuadLds: return launch(ctx, name, merkle_layer_quad_lds_kernel, grid, block, 0, s.layer);
     case kMerkleNodes64: return launch(ctx, name, merkle_nodes_kernel<64>, grid, block, 0, s.nodes);
     case kMerkleNodes256: return launch(ctx, name, merkle_nodes_kernel<256>, grid, block, 0, s.nodes);
@@ -506,7 +488,6 @@ int launch_merkle_multi(stwo_hip_ctx *ctx, uint32_t kind, bool lifted, const voi
   switch (kind) {
     case kMerkleLayer: return launch(ctx, name, merkle_layer_multi_kernel<false>, grid, block, 0, l, n);
     case kMerkleAhead: return launch(ctx, name, merkle_layer_multi_kernel<true>, grid, block, 0, l, n);
-    case kMerkleQuad: return launch(ctx, name, merkle_layer_quad_multi_kernel, grid, block, 0, l, n);
     case kMerkleQuadLds: return launch(ctx, name, merkle_layer_quad_lds_multi_kernel, grid, block, 0, l, n);
     case kMerkleNodes64: return launch(ctx, name, merkle_nodes_multi_kernel<64>, grid, block, 0, t, n);
     case kMerkleNodes256: return launch(ctx, name, merkle_nodes_multi_kernel<256>, grid, block, 0, t, n);
