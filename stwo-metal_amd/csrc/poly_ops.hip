@@ -330,10 +330,15 @@ static int barycentric_eval_impl(stwo_hip_ctx *ctx, const uint32_t *const *evals
   for (int k = 0; k < 4; k++) STWO_HIP_CHECK_ARG(ctx, weights[k], "barycentric_eval_at_point: NULL weights");
   for (size_t c = 0; c < n_cols; c++) STWO_HIP_CHECK_ARG(ctx, evals[c], "barycentric_eval_at_point: NULL column");
   const uint32_t n_blocks = 1u << (log_size > kBaryBlockLog ? log_size - kBaryBlockLog : 0);
+  // Columns per workgroup: kBaryWgCols share a block's weights; fewer, down to
+  // one group of them, where that leaves CUs idle (48 columns of 2^12: 25 us in 4
+  // workgroups, 5 in 24).
+  size_t per = kBaryWgCols;
+  while (per > kBaryCols && (n_cols + per - 1) / per * n_blocks < 512) per /= 2;
   std::vector<BaryWork> work;
-  for (uint32_t c = 0; c < n_cols; c += kBaryWgCols)
+  for (size_t c = 0; c < n_cols; c += per)
     for (uint32_t b = 0; b < n_blocks; b++)
-      work.push_back({c, (uint32_t)std::min<size_t>(kBaryWgCols, n_cols - c), b});
+      work.push_back({(uint32_t)c, (uint32_t)std::min(per, n_cols - c), b});
   bool vec = log_size >= kBaryBlockLog;  // whole 2^11-row blocks
   for (int k = 0; k < 4; k++) vec = vec && ((uintptr_t)weights[k] & 15) == 0;
   for (size_t c = 0; c < n_cols; c++) vec = vec && ((uintptr_t)evals[c] & 15) == 0;
