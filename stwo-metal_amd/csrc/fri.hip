@@ -407,6 +407,11 @@ __global__ void __launch_bounds__(kTreeThreads) fri_tails_kernel(const FriTail *
 // that hashes the root, the channel step.  The trees, roots, channel state and
 // folded evaluations written are the ones the separate fold, leaf, node and
 // channel launches write.
+// A channel's starting state: digest, n_draws, 0.
+struct ChanInit {
+  uint32_t w[10];
+};
+
 struct FriLayerJob {
   const uint32_t *src[4];
   uint32_t *dst;  // a fold's output, coordinates 2^lg words apart
@@ -415,6 +420,8 @@ struct FriLayerJob {
 };
 struct FriLayerJobs {
   FriLayerJob j[kFriJobs];
+  // the first layer of a lone commit starts from this channel, not from a state
+  uint32_t digest[8], has_digest;
 };
 
 // LEAVES per workgroup (tree_leaves_log): 64 with a quad per leaf, 256, 1,024.
@@ -434,7 +441,7 @@ __global__ void __launch_bounds__(kTreeThreads) fri_layer_kernel(FriLayerJobs jo
   uint32_t cm[16];
   if (tid < 4)
 #pragma unroll
-    for (int k = 0; k < 8; k++) cm[k] = chan[k];
+    for (int k = 0; k < 8; k++) cm[k] = FOLD == 0 && jobs.has_digest ? jobs.digest[k] : chan[k];
   uint32_t top = lg, cnt = min(LEAVES, n), row0 = first;  // the level held in S
   // lifted leaf: H(le32 of the 4 coordinates), one 16-byte block
   uint32_t m[16];
@@ -513,7 +520,10 @@ __global__ void __launch_bounds__(kTreeThreads) fri_layer_kernel(FriLayerJobs jo
 #pragma unroll
     for (int k = 0; k < 8; k++) chan[k] = digest[k];
     chan[8] = n_draws;
-    if (!ok) chan[9] = 1;
+    if (FOLD == 0 && jobs.has_digest)
+      chan[9] = !ok;
+    else if (!ok)
+      chan[9] = 1;
   }
 }
 
@@ -530,14 +540,6 @@ static int launch_fri_layer(stwo_hip_ctx *ctx, const FriLayerJobs &jobs, uint32_
                 : per == 8 ? fri_layer_kernel<FOLD, 256>
                            : fri_layer_kernel<FOLD, 1024>,
                 grid, block, 0, jobs, itw_end, lg);
-}
-
-// chan = [digest, n_draws, 0] (the device channel's starting state).
-struct ChanInit {
-  uint32_t w[10];
-};
-__global__ void chan_init_kernel(ChanInit init, uint32_t *chan) {
-  if (threadIdx.x < 10) chan[threadIdx.x] = init.w[threadIdx.x];
 }
 
 // The starting states of a group of commits (blockIdx.x): a fresh channel that
@@ -986,8 +988,8 @@ static int fri_flush(stwo_hip_ctx *ctx, FriChain &c, const stwo_hip_twiddles *tw
   return rc;
 }
 
-// Runs the chains (each with its channel in its state) up to their last layers:
-// on the stream, without host round trips.  After each
+// Runs the chains (each with its channel in its state; a lone one with it in
+// `digest`) up to their last layers: on the stream, without host round trips.  After each
 // layer's Merkle commit, the kernel that hashes its root (fri_layer_kernel
 // or the tail) mixes the root into the device copy of the channel and
 // draws the next alpha, which the folds read from device memory.
@@ -996,7 +998,8 @@ static int fri_flush(stwo_hip_ctx *ctx, FriChain &c, const stwo_hip_twiddles *tw
 // chains that stand at the same layer size share theirs (the larger ones begin
 // alone): 12 commits of 2^13 and 2^17 one after another took 2.6 ms of
 // device time, side by side they take 0.5 ms.
-static int fri_run(stwo_hip_ctx *ctx, FriChain *const *chains, size_t n, const stwo_hip_twiddles *tw) {
+static int fri_run(stwo_hip_ctx *ctx, FriChain *const *chains, size_t n, const stwo_hip_twiddles *tw,
+                   const uint8_t *digest = nullptr) {
   const uint32_t *itw_end = tw->d_itw + tw->len;
   int rc;
   for (;;) {
@@ -1014,6 +1017,10 @@ static int fri_run(stwo_hip_ctx *ctx, FriChain *const *chains, size_t n, const s
     const int fold = kind(*lead);
     const uint32_t lg = lead->lg;
     FriLayerJobs jobs{};
+    if (digest && lead->first) {
+      memcpy(jobs.digest, digest, 32);
+      jobs.has_digest = 1;
+    }
     uint32_t nj = 0;
     for (size_t i = 0; i < n && nj < kFriJobs; i++) {
       FriChain &c = *chains[i];
@@ -1142,18 +1149,9 @@ static int fri_commit_impl(stwo_hip_ctx *ctx, uint8_t channel_digest[32], uint32
   rc = get_scratch(ctx, "fri_state", kFriStateWords * 4, &p);
   if (rc) return rc;
   uint32_t *state = c.state = (uint32_t *)p;
-  {
-    // set by a launch, in stream order: no synchronization
-    ChanInit init{};
-    memcpy(init.w, channel_digest, 32);
-    init.w[8] = *channel_n_draws;
-    init.w[9] = 0;
-    rc = launch(ctx, "fri_chan_init", chan_init_kernel, dim3(1), dim3(64), 0, init, state);
-    if (rc) return rc;
-  }
   c.start();
   FriChain *chain = &c;
-  rc = fri_run(ctx, &chain, 1, tw);
+  rc = fri_run(ctx, &chain, 1, tw, channel_digest);
   if (rc) return rc;
   const uint32_t nr = c.nr, lg = c.lg;
   if (grind) grind->found = false;
