@@ -47,22 +47,22 @@ __device__ __forceinline__ qm31 ld_factor(const EvalFactors *f, uint32_t k) {
 
 // Workgroup w of its run takes blocks w, w + wgs, ... (2^B coefficients each, B =
 // min(log, kEvalBlockLog)) of the run's columns.  Lane t holds
-// the basis values of coefficients 8t .. 8t + 7 in registers and, per
+// the basis values of coefficients 4t .. 4t + 3 and 1024 above in registers and, per
 // column, accumulates sum c_j * basis_j limb by limb in 64 bits
-// (v_mad_u64_u32; each product is below 2^62, so three fit before a fold
-// (x & P) + (x >> 31), which keeps the sum below 2^34).  The 256 lanes' sums
+// (v_mad_u64_u32; each product is at most P^2, so four fit, also on top of a fold
+// (x & P) + (x >> 31) of the four before, which is below 2^34).  The 256 lanes' sums
 // are reduced through LDS, multiplied by the block's factor and added to the
 // workgroup's share, while the next block's loads are on their way.
 //
 // Bound by the multiply-adds and the loads under them, three workgroups a CU:
-// 264 columns of 2^18 (277 MB) take 81 us and 3.5 KB of tables.  In three launches
+// 264 columns of 2^18 (277 MB) take 78 us and 3.5 KB of tables.  In three launches
 // (the basis, a workgroup per block and run, the sums) it was 7.4 + 72.7 + 5.1 us
 // and the gaps between them, with a table entry per block and run (68 KB).
 constexpr uint32_t kEvalFactorBlocks = 64;  // blocks whose factors are held at once
 struct EvalLds {
   uint32_t red[kDotCols * 4][257];
   uint32_t sums[kDotCols * 4];
-  uint32_t low[2][16][4];                 // basis of index bits 3..6 and 7..10
+  uint32_t low[2][16][4];                 // basis of index bits 2..5 and 6..9
   uint32_t fac[kEvalFactorBlocks][4];
   uint32_t last;
 };
@@ -81,17 +81,17 @@ __global__ void __launch_bounds__(256) eval_point_kernel(const uint32_t *const *
   const EvalRun R = runs[ri];
   const uint32_t w = blockIdx.x - R.wg0, n = R.n;
   const uint32_t B = R.log_size < kEvalBlockLog ? R.log_size : kEvalBlockLog, nb = 1u << B;
-  const uint32_t n_blocks = 1u << (R.log_size - B), t0 = tid * 8;
+  const uint32_t n_blocks = 1u << (R.log_size - B), t0 = tid * 4, t1 = t0 + 1024;
   // 8 words per lane and column, as two 16-byte loads when the block is
-  // whole and the column pointer 32-byte aligned (a wave-uniform test).
+  // whole and the column pointer 16-byte aligned (a wave-uniform test).
   uint32_t cv[kDotCols][8];
   auto load = [&](uint32_t block) {
 #pragma unroll
     for (uint32_t j = 0; j < kDotCols; j++) {
       if (j < n) {
         const uint32_t *c = cols[R.col0 + j] + ((size_t)block << B);
-        if (nb == (1u << kEvalBlockLog) && ((uintptr_t)c & 31) == 0) {
-          const u32x4 lo = *(gconst_u4 *)(as_global(c) + t0), h4 = *(gconst_u4 *)(as_global(c) + t0 + 4);
+        if (nb == (1u << kEvalBlockLog) && ((uintptr_t)c & 15) == 0) {
+          const u32x4 lo = *(gconst_u4 *)(as_global(c) + t0), h4 = *(gconst_u4 *)(as_global(c) + t1);
           cv[j][0] = lo.x;
           cv[j][1] = lo.y;
           cv[j][2] = lo.z;
@@ -102,7 +102,10 @@ __global__ void __launch_bounds__(256) eval_point_kernel(const uint32_t *const *
           cv[j][7] = h4.w;
         } else {
 #pragma unroll
-          for (int i = 0; i < 8; i++) cv[j][i] = (t0 + i < nb) ? as_global(c)[t0 + i] : 0;
+          for (int i = 0; i < 8; i++) {
+            const uint32_t t = i < 4 ? t0 + i : t1 + i - 4;
+            cv[j][i] = t < nb ? as_global(c)[t] : 0;
+          }
         }
       }
     }
@@ -117,13 +120,13 @@ __global__ void __launch_bounds__(256) eval_point_kernel(const uint32_t *const *
       if ((block >> (k - B)) & 1) r = qm31_mul(r, ld_factor(f, k));
     for (int k = 0; k < 4; k++) S.fac[tid][k] = r.v[k];
   };
-  // The basis: of index bits 3..6 and 7..10 by 32 lanes, their products and
-  // those of bits 0..2 in every lane.
+  // The basis: of index bits 2..5 and 6..9 by 32 lanes, their products and
+  // those of bits 0, 1 and 10 in every lane.
   if (tid >= 128 && tid < 160) {
     const uint32_t half = (tid >> 4) & 1, e = tid & 15;
     qm31 r = qm31_make(1, 0, 0, 0);
     for (uint32_t k = 0; k < 4; k++)
-      if ((e >> k) & 1) r = qm31_mul(r, ld_factor(f, 3 + 4 * half + k));
+      if ((e >> k) & 1) r = qm31_mul(r, ld_factor(f, 2 + 4 * half + k));
     for (int k = 0; k < 4; k++) S.low[half][e][k] = r.v[k];
   }
   factors(w);
@@ -133,11 +136,7 @@ __global__ void __launch_bounds__(256) eval_point_kernel(const uint32_t *const *
 #pragma unroll
   for (int k = 0; k < 3; k++)
 #pragma unroll
-    for (int i = 0; i < (1 << k); i++) b[(1 << k) + i] = qm31_mul(b[i], ld_factor(f, k));
-  if (t0 + 8 > nb)  // a column below 2^11: no coefficient, no product
-#pragma unroll
-    for (int i = 0; i < 8; i++)
-      if (t0 + i >= nb) b[i] = qm31_make(0, 0, 0, 0);
+    for (int i = 0; i < (1 << k); i++) b[(1 << k) + i] = qm31_mul(b[i], ld_factor(f, k < 2 ? k : 10));
   qm31 share = qm31_make(0, 0, 0, 0);
   uint32_t k_blk = 0;
   for (uint32_t block = w; block < n_blocks; block += R.wgs) {
@@ -149,7 +148,7 @@ __global__ void __launch_bounds__(256) eval_point_kernel(const uint32_t *const *
       for (int i = 0; i < 8; i++) {
 #pragma unroll
         for (int k = 0; k < 4; k++) acc[k] += (uint64_t)cv[j][i] * b[i].v[k];
-        if (i == 2 || i == 5)
+        if (i == 3)
 #pragma unroll
           for (int k = 0; k < 4; k++) acc[k] = m31_fold64(acc[k]);
       }
