@@ -369,13 +369,12 @@ __device__ __forceinline__ void mx_get(const uint32_t *L, Words16 &x) {
 // buffer is written again only after the barrier of the exchange in between,
 // which every wave reaches after its reads.  Waves drift by up to an exchange
 // and overlap each other's loads, products and stores (one workgroup fills a
-// CU).  The matrices that all waves share are copied to LDS once (the first
-// kMxTopLds of them); the next tile's rows and the wave's next matrix are
+// CU).  The matrices that all waves share are copied to LDS once; the next tile's rows and the wave's next matrix are
 // loaded ahead, before the stores that a wait for them would otherwise include.
 // 256 x 2^20 at blowup 4: 1.40 ms for 5.4 GB, where the butterfly form of the
 // fused pass (lde_pass_kernel<9, 2>) takes 2.04 ms; the accesses are 256-byte
 // runs 16 KB apart.
-constexpr uint32_t kMxTopLds = 6;
+constexpr uint32_t kMxTopLds = 1 + (1u << kMxMaxBlowup);  // the inverse one, one per output block
 struct MxTopLds {
   uint32_t t[2][256 * 64];
   uint32_t m[kMxTopLds][kMxWords];
@@ -409,7 +408,7 @@ __device__ __forceinline__ void mx_top8_body(const MxTop &p, uint32_t wg, MxTopL
   MxMat M = mx_load(table, INV ? kMxInv8 + w : mx_fwd8(p.b, w));
   // shared matrices: the inverse top one, then the forward ones by block
   constexpr uint32_t F0 = INV ? 1 : 0;
-  const uint32_t n_rep = FWD ? 1u << p.b : 0, n_lds = min(kMxTopLds, F0 + n_rep);
+  const uint32_t n_rep = FWD ? 1u << p.b : 0, n_lds = F0 + n_rep;
   for (uint32_t j = threadIdx.x; j < n_lds * (kMxWords / 4); j += 1024) {
     const uint32_t k = j / (kMxWords / 4), o = j - k * (kMxWords / 4);
     const uint32_t id = INV && k == 0 ? kMxInvTop + n : mx_fwd4(p.b, k - F0);
@@ -417,10 +416,6 @@ __device__ __forceinline__ void mx_top8_body(const MxTop &p, uint32_t wg, MxTopL
     *reinterpret_cast<uint4 *>(&S.m[k][4 * o]) = v;
   }
   __syncthreads();
-  auto top_mat = [&](uint32_t k, uint32_t id) {
-    if (k >= kMxTopLds) return mx_load(table, id);
-    return mx_lds(S.m[k]);
-  };
   for (uint32_t tile = tile0; tile < tile1; tile += step) {
     const uint32_t ci = tile >> blk_log;
     const uint32_t pos = ((tile & ((1u << blk_log) - 1)) << 6) + lane_pos;
@@ -442,7 +437,7 @@ __device__ __forceinline__ void mx_top8_body(const MxTop &p, uint32_t wg, MxTopL
       uint32_t *out = (uint32_t *)readfirstlane_u64((uint64_t)p.fcols[ci].out);
       for (uint32_t rep = 0; rep < n_rep; rep++) {
         const bool last = rep + 1 == n_rep;
-        mx_stage<true, false, G>(top_mat(F0 + rep, mx_fwd4(p.b, rep)), x, y);
+        mx_stage<true, false, G>(mx_lds(S.m[F0 + rep]), x, y);
         mx_put<false>(le + buf, y);
         if (last && tile + step < tile1) load(tile + step);
         __syncthreads();
