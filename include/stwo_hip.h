@@ -134,7 +134,8 @@ int stwo_hip_bit_reverse_secure_column(stwo_hip_ctx *ctx, uint32_t *const coords
  * the tree's root coset (or the root itself). */
 int stwo_hip_interpolate(stwo_hip_ctx *ctx, uint32_t *col, stwo_hip_coset domain, const stwo_hip_twiddles *tw);
 /* PolyOps::interpolate_columns (ops.rs:29-40) over canonic domains
- * CanonicCoset(log_sizes[i]).circle_domain(); one batched launch per pass. */
+ * CanonicCoset(log_sizes[i]).circle_domain(); columns of equal size, and where
+ * it pays of different sizes, share their launches. */
 int stwo_hip_interpolate_columns(stwo_hip_ctx *ctx, uint32_t *const *cols, const uint32_t *log_sizes, size_t n_cols,
                                  const stwo_hip_twiddles *tw);
 /* PolyOps::evaluate / evaluate_into (ops.rs:90-108; CPUB/circle.rs:190-250;
@@ -417,8 +418,8 @@ int stwo_hip_wide_fib_constraint_quotients(stwo_hip_ctx *ctx, const uint32_t *co
  * Returns STWO_HIP_ECONSTRAINTS when prove_ex's own OODS self-check fails (a
  * trace that does not satisfy the AIR).  Synchronizes.  The prove's device
  * buffers (4 + 4 * 2^log_blowup_factor bytes per trace cell, plus the trees
- * and the composition and FRI columns) and its launch plans (the trace and
- * composition commits as hipGraphs) are kept by the context and reused by
+ * and the composition and FRI columns) and its launch plans (of the trace and
+ * composition commits) are kept by the context and reused by
  * its next prove of the same shape; stwo_hip_ctx_destroy releases them.
  *
  * stwo_hip_wide_fib_prove keeps the coefficients
@@ -567,8 +568,8 @@ int stwo_hip_batch_destroy(stwo_hip_ctx *ctx, stwo_hip_batch *batch);
  * order) are admitted together if their memory fits the budget; a head that
  * does not fit waits for memory to be released (later jobs do not overtake
  * it).  A group's commit jobs share one batched plan: their columns' FFT
- * passes of equal size and blowup run in the same launches, each job's tree
- * on its own; then each job's FRI.  A prove job runs alone in its group.
+ * passes of equal size and blowup run in the same launches, and so do the
+ * jobs' trees and their FRI layers of equal size.  A prove job runs alone in its group.
  * Groups on different slots run concurrently on the device.  Every device
  * buffer a job needs -- its columns, evaluations, trees, the plan's tables,
  * FRI and prove scratch -- comes from its group's block of the budget, so

@@ -18,13 +18,16 @@
 // evaluate_into (SIMD/circle.rs:413-440), fused into one pass over the
 // output.
 //
-// MI355X mapping: a pass moves a 4096-element tile (16 KB) of one column
-// through LDS.  The tile owns up to 12 consecutive layers: the lowest pass
-// covers layers [0, 12) on a contiguous chunk; higher layers run in strided
-// passes of <= 6 layers whose tile rows are 64 consecutive elements (256 B
-// coalesced runs).  Columns up to 2^12 take one pass, up to 2^18 two, up to
-// 2^24 three.  blockIdx.y selects the column, so one launch covers a whole
-// group of same-size columns.
+// MI355X mapping: groups with a unit of the low pass for every CU run on the
+// matrix cores (fft_matrix.hip), columns up to 2^12 in calls that leave the device
+// idle take a workgroup each (fft_column.hip), and the rest the register passes
+// below.  A register pass owns a tile of up to 2^13 elements of one column, 16 in
+// each lane's registers, exchanged through LDS: the low pass covers layers [0, 12)
+// on a contiguous tile, higher layers run in strided passes of at most 8 whose tile
+// rows are 64 consecutive elements (256 B coalesced runs).  Columns up to 2^12 take
+// one pass, up to 2^20 two, up to 2^28 three.  A launch covers a whole
+// group of same-size columns, or several groups.  The tile kernel with one layer
+// per LDS round trip is left for domains below 2^4.
 #include <algorithm>
 #include <map>
 #include <vector>

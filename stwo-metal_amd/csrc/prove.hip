@@ -45,9 +45,9 @@
 //
 // Outside a serving job the trace commit (trace LDE + lifted tree) and the
 // composition commit (interpolation of the 4 coordinate columns, evaluation of
-// their 8 halves, lifted tree) each run as a batch plan replayed as a
-// hipGraph; the plans are kept on the context for the next prove of the same
-// shape and buffers.  Within a job they are issued eagerly.
+// their 8 halves, lifted tree) each run as a batch plan; the plans are kept on
+// the context for the next prove of the same shape and buffers.  Within a job
+// the calls they stand for are made one by one.
 #include <string.h>
 
 #include <array>
