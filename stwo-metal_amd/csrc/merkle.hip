@@ -253,10 +253,10 @@ __device__ __forceinline__ void layer_hash_quad_lds(const MerkleLayer &L, uint32
 
 // One layer: its nodes alone.
 template <bool AHEAD>
-__device__ __forceinline__ void merkle_layer(const MerkleLayer &L, uint32_t wg) {
+__device__ __forceinline__ void merkle_layer(const MerkleLayer &L, const ColRef *cols, uint32_t wg) {
   const uint32_t i = wg * 256 + threadIdx.x;
   if (i >= 1u << L.log_size) return;
-  store_hash(L.out + 8 * (size_t)i, layer_hash<AHEAD>(L, L.cols, i), 0);
+  store_hash(L.out + 8 * (size_t)i, layer_hash<AHEAD>(L, cols, i), 0);
 }
 __device__ __forceinline__ void store_quad(uint32_t *out, uint32_t i, uint32_t lo, uint32_t hi) {
   g_u32 *o = as_global(out + 8 * (size_t)i);
@@ -376,12 +376,12 @@ __device__ __forceinline__ const T &step_of(const T *t, uint32_t n) {
 }
 template <bool AHEAD>
 __global__ void __launch_bounds__(256) merkle_layer_kernel(MerkleLayer L) {
-  merkle_layer<AHEAD>(L, blockIdx.x);
+  merkle_layer<AHEAD>(L, L.cols, blockIdx.x);
 }
 template <bool AHEAD>
 __global__ void __launch_bounds__(256) merkle_layer_multi_kernel(const MerkleLayer *t, uint32_t n) {
   const MerkleLayer L = step_of(t, n);
-  merkle_layer<AHEAD>(L, blockIdx.x - L.wg_start);
+  merkle_layer<AHEAD>(L, L.cols, blockIdx.x - L.wg_start);
 }
 __global__ void __launch_bounds__(256) merkle_layer_quad_lds_kernel(MerkleLayer L) {
   merkle_layer_quad_lds(L, blockIdx.x);
@@ -400,10 +400,14 @@ __global__ void __launch_bounds__(kTreeThreads) merkle_tree_multi_kernel(const M
   merkle_tree<LDS>(T, T.layer.cols, blockIdx.x - T.wg_start);
 }
 // The columns among the arguments: their upload costs a small commit as much as
-// its leaves.
+// its leaves (2.3 us and a launch's gap; leaves of 16 columns of 2^17 take 9.7).
 struct InlineCols {
   ColRef c[kInlineCols];
 };
+template <bool AHEAD>
+__global__ void __launch_bounds__(256) merkle_layer_inline_kernel(MerkleLayer L, InlineCols cols) {
+  merkle_layer<AHEAD>(L, cols.c, blockIdx.x);
+}
 __global__ void __launch_bounds__(kTreeThreads) merkle_tree_inline_kernel(MerkleTree T, InlineCols cols) {
   merkle_tree<false>(T, cols.c, blockIdx.x);
 }
@@ -511,10 +515,15 @@ static int launch_layer(stwo_hip_ctx *ctx, const uint32_t *prev, const std::vect
   if (rc) return rc;
   MerkleStep s = merkle_layer_step(prev, nullptr, (uint32_t)cols.size(), log_size, out, mode, lifted);
   *done = merkle_tree_step(s, stop_log, ctx->d_counters);
-  if (s.kind == kMerkleTree && cols.size() <= kInlineCols) {
+  const bool in_args = s.kind == kMerkleTree || s.kind == kMerkleLayer || s.kind == kMerkleAhead;
+  if (in_args && cols.size() <= kInlineCols) {
     InlineCols in{};
     std::copy(cols.begin(), cols.end(), in.c);
-    return launch(ctx, "merkle_tree", merkle_tree_inline_kernel, dim3(s.wgs), dim3(kTreeThreads), 0, s.tree, in);
+    const dim3 grid(s.wgs), block(256);
+    const char *name = step_name(s.kind, lifted);
+    if (s.kind == kMerkleTree) return launch(ctx, name, merkle_tree_inline_kernel, grid, block, 0, s.tree, in);
+    return launch(ctx, name, s.kind == kMerkleAhead ? merkle_layer_inline_kernel<true> : merkle_layer_inline_kernel<false>,
+                  grid, block, 0, s.layer, in);
   }
   if (!cols.empty()) {
     void *dtab = nullptr;
