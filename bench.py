@@ -263,13 +263,11 @@ def serving(rates=(10.0, 30.0, 60.0), n_jobs=200, budget=96 << 30, n_slots=4):
 
 # Profiling names of the library's launches -> kernel symbols in rocprofv3 output.
 ROCPROF_NAMES = {
-    "rfft_pass_wg8": "void stwo_hip::fft_pass_kernel<false, 8, 3, 8, 4, 0>(stwo_hip::FftPass2)",
-    "rfft_pass_wg9": "void stwo_hip::fft_pass_kernel<false, 9, 2, 9, 5, 0>(stwo_hip::FftPass2)",
-    "ifft_pass_wg8": "void stwo_hip::fft_pass_kernel<true, 8, 3, 0, 4, 8>(stwo_hip::FftPass2)",
-    "lde_pass_wg9": "void stwo_hip::lde_pass_kernel<9, 2>(stwo_hip::FftPass2, stwo_hip::FftPass2, unsigned int)",
-    "ifft_pass_wg9": "void stwo_hip::fft_pass_kernel<true, 9, 2, 5, 9, 0>(stwo_hip::FftPass2)",
+    "ifft_pass_mx_low": "void stwo_hip::(anonymous namespace)::mx_low_kernel<true>(...)",
+    "lde_pass_mx_top": "void stwo_hip::(anonymous namespace)::mx_top8_kernel<true, true>(...)",
+    "rfft_pass_mx_low": "void stwo_hip::(anonymous namespace)::mx_low_kernel<false>(...)",
     "merkle_commit_on_layer": "void stwo_hip::merkle_layer_kernel<false>(...)",
-    "merkle_nodes": "stwo_hip::merkle_nodes_kernel(...)",
+    "merkle_nodes": "void stwo_hip::merkle_nodes_kernel<1024u>(...)",
 }
 TRAFFIC_FILE = os.path.join(REPO, "profiles", "traffic_lde_merkle_256x2e20_b4.json")
 
@@ -708,7 +706,7 @@ def main():
             "parallelism": "single GPU",
         },
         "roofline": {
-            "bound": "valu",
+            "bound": "hbm" if dom_name.endswith("mx_low") else "valu",
             "kernel": dom_name,
             "rocprof_name": ROCPROF_NAMES.get(dom_name, dom_name),
             "launch_ms": round(dom_launch_ms, 4),
