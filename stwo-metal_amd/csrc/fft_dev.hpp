@@ -43,6 +43,13 @@ __device__ __forceinline__ u32x4 gld4(const uint32_t *base, uint32_t byte_off) {
 __device__ __forceinline__ void gst4(uint32_t *base, uint32_t byte_off, u32x4 v) {
   *(g_u4 *)((g_u8 *)as_global(base) + byte_off) = v;
 }
+// The same for words that the launch touches once.
+__device__ __forceinline__ u32x4 gld4_once(const uint32_t *base, uint32_t byte_off) {
+  return __builtin_nontemporal_load((gconst_u4 *)((gconst_u8 *)as_global(base) + byte_off));
+}
+__device__ __forceinline__ void gst4_once(uint32_t *base, uint32_t byte_off, u32x4 v) {
+  __builtin_nontemporal_store(v, (g_u4 *)((g_u8 *)as_global(base) + byte_off));
+}
 
 __device__ __forceinline__ void load_level(uint32_t *dst, int cnt, const uint32_t *tw_end, uint32_t N, uint32_t s,
                                            uint32_t gb) {

@@ -293,20 +293,38 @@ struct Words16 {
 };
 
 // Words of 4 rows `step` words apart (uniform) from lane offset `off` words.
+//
+// ONCE: non-temporal, for the words between the fused pass's reads and the
+// evaluations: the intermediates that a pass hands on and the low pass's
+// output.  Each is touched once per launch, and kept in the caches they push
+// out the matrices (0.7 MB, read by every wave for every tile) and each other.
+// With either side alone the gain is lost where a set fits the 256 MB cache
+// (100 x 2^17 at blowup 2: stores only 95 us, both 87, neither 91); both: 256 x
+// 2^20 at blowup 4 commit 6.10 -> 5.96 ms, 1,024 uneven columns 1,666 -> 1,600
+// us, a 256 x 2^18 prove 2.07 -> 2.01 ms.  The caller's own columns (an
+// inverse's input, the coefficients of a forward pass alone) are read the
+// ordinary way: they may well be in the cache (forward-only reads as ONCE: 91
+// -> 98 us).
+template <bool ONCE = false>
 __device__ __forceinline__ void mx_ld(const uint32_t *col, uint32_t step, uint32_t off, Words16 &x) {
 #pragma unroll
   for (uint32_t q = 0; q < 4; q++) {
-    const u32x4 v = gld4(col + (size_t)q * step, off << 2);
+    const uint32_t *r = col + (size_t)q * step;
+    const u32x4 v = ONCE ? gld4_once(r, off << 2) : gld4(r, off << 2);
     x.w[q][0] = v.x;
     x.w[q][1] = v.y;
     x.w[q][2] = v.z;
     x.w[q][3] = v.w;
   }
 }
+template <bool ONCE = false>
 __device__ __forceinline__ void mx_st(uint32_t *col, uint32_t step, uint32_t off, const Words16 &x) {
 #pragma unroll
-  for (uint32_t q = 0; q < 4; q++)
-    gst4(col + (size_t)q * step, off << 2, u32x4{x.w[q][0], x.w[q][1], x.w[q][2], x.w[q][3]});
+  for (uint32_t q = 0; q < 4; q++) {
+    const u32x4 v{x.w[q][0], x.w[q][1], x.w[q][2], x.w[q][3]};
+    uint32_t *r = col + (size_t)q * step;
+    if (ONCE) gst4_once(r, off << 2, v); else gst4(r, off << 2, v);
+  }
 }
 
 // Applies M to each of the 4 vector groups.  SIGN: the input words still have
@@ -371,9 +389,10 @@ __device__ __forceinline__ void mx_get(const uint32_t *L, Words16 &x) {
 // and overlap each other's loads, products and stores (one workgroup fills a
 // CU).  The matrices that all waves share are copied to LDS once; the next tile's rows and the wave's next matrix are
 // loaded ahead, before the stores that a wait for them would otherwise include.
-// 256 x 2^20 at blowup 4: 1.40 ms for 5.4 GB, where the butterfly form of the
-// fused pass (lde_pass_kernel<9, 2>) takes 2.04 ms; the accesses are 256-byte
-// runs 16 KB apart.
+// 256 x 2^20 at blowup 4: 1.18 ms for 5.5 GB, 4.7 TB/s (a large copy: 4.9;
+// 1.38 ms with ordinary loads and stores), where the butterfly form of the fused
+// pass (lde_pass_kernel<9, 2>) takes 2.04 ms; the accesses are 256-byte runs 16
+// KB apart.
 constexpr uint32_t kMxTopLds = 1 + (1u << kMxMaxBlowup);  // the inverse one, one per output block
 struct MxTopLds {
   uint32_t t[2][256 * 64];
@@ -402,7 +421,7 @@ __device__ __forceinline__ void mx_top8_body(const MxTop &p, uint32_t wg, MxTopL
   auto load = [&](uint32_t tile) {
     const uint32_t *in = (const uint32_t *)readfirstlane_u64((uint64_t)icols[tile >> blk_log].in);
     const uint32_t pos = ((tile & ((1u << blk_log) - 1)) << 6) + lane_pos;
-    mx_ld(in, INV ? u_step : e_step, (INV ? u_row : e_row) + pos, x);
+    mx_ld<INV && FWD>(in, INV ? u_step : e_step, (INV ? u_row : e_row) + pos, x);
   };
   load(tile0);
   MxMat M = mx_load(table, INV ? kMxInv8 + w : mx_fwd8(p.b, w));
@@ -445,7 +464,7 @@ __device__ __forceinline__ void mx_top8_body(const MxTop &p, uint32_t wg, MxTopL
         buf ^= 256 * 64;
         mx_stage<false, true, G>(M, y, y);
         M = mx_load(table, INV && last ? kMxInv8 + w : mx_fwd8(p.b, (last ? 0 : (rep + 1) * 16) + w));
-        mx_st(out + ((size_t)rep << n), u_step, u_row + pos, y);
+        mx_st<true>(out + ((size_t)rep << n), u_step, u_row + pos, y);
       }
     }
   }
@@ -461,7 +480,8 @@ __device__ __forceinline__ void mx_top4_body(const MxTop &p, uint32_t wg) {
   const uint32_t pos = ((unit & ((1u << blk_log) - 1)) << 6) + ((threadIdx.x & 15) << 2);
   Words16 x, y;
   const uint32_t step = 1u << row_log, off = ((threadIdx.x & 48) >> 2 << row_log) + pos;  // rows 4 g + q
-  mx_ld((const uint32_t *)readfirstlane_u64((uint64_t)(INV ? p.icols[ci].in : p.fcols[ci].in)), step, off, x);
+  const uint32_t *in = (const uint32_t *)readfirstlane_u64((uint64_t)(INV ? p.icols[ci].in : p.fcols[ci].in));
+  mx_ld<INV && FWD>(in, step, off, x);
   if (INV) {
     const MxMat T = mx_load(p.mats, kMxInvTop + n);
     mx_stage<true, true>(T, x, y);
@@ -473,7 +493,7 @@ __device__ __forceinline__ void mx_top4_body(const MxTop &p, uint32_t wg) {
     for (uint32_t rep = 0; rep < 1u << p.b; rep++) {
       const MxMat T = mx_load(p.mats, mx_fwd4(p.b, rep));
       mx_stage<true, true>(T, x, y);
-      mx_st(out + ((size_t)rep << n), step, off, y);
+      mx_st<true>(out + ((size_t)rep << n), step, off, y);
     }
   }
 }
@@ -592,7 +612,7 @@ __device__ __forceinline__ void mx_low_body(const MxLow &p, uint32_t wg, MxLowLd
 #pragma unroll
     for (uint32_t q = 0; q < 4; q++) {
       const uint32_t o = INV ? in_chunk + bfly0 + 4 * q : in_chunk + ((4 * g + q) << 8) + rpos;
-      const u32x4 v = gld4(in, o << 2);
+      const u32x4 v = INV ? gld4(in, o << 2) : gld4_once(in, o << 2);
       xin[4 * q] = v.x;
       xin[4 * q + 1] = v.y;
       xin[4 * q + 2] = v.z;
@@ -698,7 +718,7 @@ __device__ __forceinline__ void mx_low_body(const MxLow &p, uint32_t wg, MxLowLd
         if (cb + k >= col1) break;
         const uint4 v = *reinterpret_cast<const uint4 *>(&blk[k * kMxCol + st_off]);
         uint32_t *out = (uint32_t *)readfirstlane_u64((uint64_t)S.col[cb + k - col0].out);
-        gst4(out, ((tile << 12) + (w << 8) + (lane << 2)) << 2, u32x4{v.x, v.y, v.z, v.w});
+        gst4_once(out, ((tile << 12) + (w << 8) + (lane << 2)) << 2, u32x4{v.x, v.y, v.z, v.w});
       }
     } else {
       uint32_t x[16];
