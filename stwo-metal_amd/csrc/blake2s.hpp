@@ -15,6 +15,14 @@
 
 namespace stwo_hip {
 
+// One instruction (the compiler makes two of a ^ b ^ c here).
+__host__ __device__ __forceinline__ uint32_t b2_xor3(uint32_t a, uint32_t b, uint32_t c) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+#else
+  return a ^ b ^ c;
+#endif
+}
 __host__ __device__ __forceinline__ uint32_t b2_rotr(uint32_t x, uint32_t n) { return (x >> n) | (x << (32 - n)); }
 
 #define STWO_B2_IV0 0x6A09E667u
@@ -85,7 +93,7 @@ __host__ __device__ __forceinline__ void b2_compress(b2_state &s, const uint32_t
   STWO_B2_ROUND(6, 15, 14, 9, 11, 3, 0, 8, 12, 2, 13, 7, 1, 4, 10, 5)
   STWO_B2_ROUND(10, 2, 8, 4, 7, 6, 1, 5, 15, 11, 9, 14, 3, 12, 13, 0)
 #pragma unroll
-  for (int i = 0; i < 8; i++) s.h[i] ^= v[i] ^ v[i + 8];
+  for (int i = 0; i < 8; i++) s.h[i] = b2_xor3(s.h[i], v[i], v[i + 8]);
 }
 
 // ---- one compression on the 4 lanes of an aligned quad ----------------------

@@ -70,12 +70,13 @@ __device__ __forceinline__ b2_state hash_pair(const b2_state &a, const b2_state 
   return hash_block(m, m31);
 }
 
-// Word idx of a column.  Layers are at most 2^30 rows, so the byte offset
+// Word at byte `off` of a column.  Layers are at most 2^30 rows, so the offset
 // fits 32 bits: the load takes the column pointer as an SGPR base and a
 // 32-bit lane offset (no per-column 64-bit address arithmetic).
-__device__ __forceinline__ uint32_t ld_col_word(const uint32_t *col, uint32_t idx) {
-  return *(gconst_u32 *)((gconst_u8 *)as_global(col) + (idx << 2));
+__device__ __forceinline__ uint32_t ld_col_byte(const uint32_t *col, uint32_t off) {
+  return *(gconst_u32 *)((gconst_u8 *)as_global(col) + off);
 }
+__device__ __forceinline__ uint32_t ld_col_word(const uint32_t *col, uint32_t idx) { return ld_col_byte(col, idx << 2); }
 
 // Mixed-degree layer: optional previous layer, then the layer's columns.
 // `lifted` selects the lifted leaf index for column words.
@@ -84,13 +85,44 @@ __device__ __forceinline__ uint32_t ld_col_word(const uint32_t *col, uint32_t id
 // nodes, where a node's chain of blocks is the launch's critical path; on
 // large layers the other waves hide the latency and the extra registers and
 // copies cost more than they save.
-template <bool AHEAD>
+// TABLE: the columns' table is in device memory (not among the arguments,
+// whose address must not be taken).
+template <bool AHEAD, bool TABLE>
 __device__ __forceinline__ b2_state layer_hash(const MerkleLayer &L, const ColRef *cols, uint32_t i) {
   const uint32_t *prev = L.prev;
   const uint32_t n_cols = L.n_cols, lifted = L.lifted;
-  // The words of columns c0 .. c0 + 15 at this row (zeros past n_cols).
+  // The words of columns c0 .. c0 + 15 at this row (zeros past n_cols).  A full
+  // block reads its 16 table entries together, and where the columns lie at the
+  // layer's own size they share one offset: entry by entry, each with its wait
+  // and its offset, a block cost 48 more instructions beside the compression's
+  // 976.  256 columns of 2^20 committed at blowup 4: 6.07 -> 6.00 ms.
   auto load_cols = [&](uint32_t c0, uint32_t (&dst)[16]) {
     const uint32_t cnt = min(16u, n_cols - c0);
+    if (cnt == 16) {
+      uint64_t ref[32];  // a ColRef each two, by scalar loads of 64 bytes
+      if (TABLE) {
+        typedef const __attribute__((address_space(4))) uint64_t const_u64;
+        const_u64 *src = (const_u64 *)readfirstlane_u64((uint64_t)(cols + c0));
+#pragma unroll
+        for (uint32_t k = 0; k < 32; k++) ref[k] = src[k];
+      } else {
+        __builtin_memcpy(ref, cols + c0, sizeof(ref));
+      }
+      uint32_t shifts = 0;
+#pragma unroll
+      for (uint32_t k = 0; k < 16; k++) shifts |= (uint32_t)ref[2 * k + 1];
+      uint32_t row4 = i << 2, odd4 = (i & 1) << 2;
+      asm("" : "+v"(row4), "+v"(odd4));  // stays a 32-bit offset beside the pointer in SGPRs
+      if (lifted && shifts) {
+#pragma unroll
+        for (uint32_t k = 0; k < 16; k++)
+          dst[k] = ld_col_byte((const uint32_t *)ref[2 * k], ((i >> ((uint32_t)ref[2 * k + 1] + 1)) << 3) + odd4);
+      } else {
+#pragma unroll
+        for (uint32_t k = 0; k < 16; k++) dst[k] = ld_col_byte((const uint32_t *)ref[2 * k], row4);
+      }
+      return;
+    }
 #pragma unroll
     for (uint32_t k = 0; k < 16; k++) {
       uint32_t v = 0;
@@ -252,11 +284,11 @@ __device__ __forceinline__ void layer_hash_quad_lds(const MerkleLayer &L, uint32
 }
 
 // One layer: its nodes alone.
-template <bool AHEAD>
+template <bool AHEAD, bool TABLE>
 __device__ __forceinline__ void merkle_layer(const MerkleLayer &L, const ColRef *cols, uint32_t wg) {
   const uint32_t i = wg * 256 + threadIdx.x;
   if (i >= 1u << L.log_size) return;
-  store_hash(L.out + 8 * (size_t)i, layer_hash<AHEAD>(L, cols, i), 0);
+  store_hash(L.out + 8 * (size_t)i, layer_hash<AHEAD, TABLE>(L, cols, i), 0);
 }
 __device__ __forceinline__ void store_quad(uint32_t *out, uint32_t i, uint32_t lo, uint32_t hi) {
   g_u32 *o = as_global(out + 8 * (size_t)i);
@@ -376,12 +408,12 @@ __device__ __forceinline__ const T &step_of(const T *t, uint32_t n) {
 }
 template <bool AHEAD>
 __global__ void __launch_bounds__(256) merkle_layer_kernel(MerkleLayer L) {
-  merkle_layer<AHEAD>(L, L.cols, blockIdx.x);
+  merkle_layer<AHEAD, true>(L, L.cols, blockIdx.x);
 }
 template <bool AHEAD>
 __global__ void __launch_bounds__(256) merkle_layer_multi_kernel(const MerkleLayer *t, uint32_t n) {
   const MerkleLayer L = step_of(t, n);
-  merkle_layer<AHEAD>(L, L.cols, blockIdx.x - L.wg_start);
+  merkle_layer<AHEAD, true>(L, L.cols, blockIdx.x - L.wg_start);
 }
 __global__ void __launch_bounds__(256) merkle_layer_quad_lds_kernel(MerkleLayer L) {
   merkle_layer_quad_lds(L, blockIdx.x);
@@ -406,7 +438,7 @@ struct InlineCols {
 };
 template <bool AHEAD>
 __global__ void __launch_bounds__(256) merkle_layer_inline_kernel(MerkleLayer L, InlineCols cols) {
-  merkle_layer<AHEAD>(L, cols.c, blockIdx.x);
+  merkle_layer<AHEAD, false>(L, cols.c, blockIdx.x);
 }
 __global__ void __launch_bounds__(kTreeThreads) merkle_tree_inline_kernel(MerkleTree T, InlineCols cols) {
   merkle_tree<false>(T, cols.c, blockIdx.x);

@@ -122,3 +122,34 @@ def test_jobs_side_by_side(ctx):
         assert r.n_fri_roots == len(roots) and list(r.fri_roots[:8 * len(roots)]) == list(roots.ravel()), job
         assert list(r.last_layer_poly[:last.size]) == list(last.ravel()), job
         assert bytes(r.final_digest) == digest, job
+
+
+# Leaf layers of full blocks of 16 columns: at the layer's own size or above it in
+# one block or several, a remainder after them, tables among the arguments (up to 64
+# columns) and in memory, layers that load a block ahead (2^15) and not (2^17)
+FULL = [[17] * 16, [15] * 33, [17] * 64, [17] * 65, [15] * 96, [12] * 3 + [15] * 14 + [17] * 20, [9] * 16 + [16] * 17,
+        [5] * 30 + [16] * 18 + [17] * 32]
+
+
+@pytest.mark.parametrize("logs", FULL, ids=["%dx%d" % (len(f), max(f)) for f in FULL])
+def test_full_blocks(ctx, logs):
+    for mode in (sh.HASH_BLAKE2S, sh.HASH_BLAKE2S_M31):
+        _tree(ctx, logs, "mixed", mode)
+        _tree(ctx, logs, "lifted", mode)
+
+
+def test_full_blocks_side_by_side(ctx):
+    """The same of several trees in one launch: jobs of one group."""
+    jobs, ids, want = [(14, 33), (14, 16), (15, 40), (15, 17)], [], []
+    with sh.Server(0, 1 << 30, 17, 1, max_group=len(jobs)) as srv:
+        srv.hold(True)
+        for n, n_cols in jobs:
+            cols, outs = _evals(n, 1, n_cols)
+            want.append(oracle.lifted_commit(outs, n + 1)[:8])
+            bufs = [ctx.to_device(c) for c in cols]
+            ctx.sync()
+            ids.append((srv.submit(n_cols, n, 1, 0, sh.FriConfig(1, 1, 3, 1), cols=bufs), bufs))
+        srv.hold(False)
+        for (i, _), root, job in zip(ids, want, jobs):
+            r = srv.wait(i)
+            assert r.status == 0 and list(r.trace_root) == list(root), job
