@@ -301,7 +301,10 @@ struct Words16 {
 // With either side alone the gain is lost where a set fits the 256 MB cache
 // (100 x 2^17 at blowup 2: stores only 95 us, both 87, neither 91); both: 256 x
 // 2^20 at blowup 4 commit 6.10 -> 5.96 ms, 1,024 uneven columns 1,666 -> 1,600
-// us, a 256 x 2^18 prove 2.07 -> 2.01 ms.  The caller's own columns (an
+// us, a 256 x 2^18 prove 2.07 -> 2.01 ms; sets that stay in the cache either way
+// are within 3% (20 x 2^18 at 2 46 -> 45 us, 40 x 2^17 at 4 70 -> 72).  A branch
+// on the size inside the kernels cost the prove 35 us and gave those nothing
+// back.  The caller's own columns (an
 // inverse's input, the coefficients of a forward pass alone) are read the
 // ordinary way: they may well be in the cache (forward-only reads as ONCE: 91
 // -> 98 us).
