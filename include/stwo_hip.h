@@ -647,6 +647,16 @@ int stwo_hip_debug_fft_plan(uint32_t n, uint32_t N, int inverse, uint32_t *out, 
  * 0 = the default of each. */
 int stwo_hip_debug_fft_plan_tuned(uint32_t n, uint32_t N, int inverse, uint32_t t0, uint32_t smax, uint32_t wg,
                                   uint32_t *out, uint32_t max_passes, uint32_t *n_passes);
+/* The launches that hash a tree (6 words per launch), from a layer down to
+ * stop_log: what = 0, the node layers below layer top_log; 1, layer top_log over
+ * n columns and the node layers below it; 2, a FRI layer of 2^top_log leaves
+ * beside n - 1 others (stop_log = 0).  plan_log: 0 for a call on a context,
+ * else the log size of the tallest tree of a plan (of the FRI column).  Words:
+ * the first level hashed, the level a workgroup hashes down to alone, the last
+ * level, workgroups, the counters on which workgroups meet, and the counters
+ * that there are.  Launches nothing. */
+int stwo_hip_debug_tree_plan(int what, uint32_t top_log, uint32_t stop_log, uint32_t n, uint32_t plan_log,
+                             uint32_t *out, uint32_t max_steps, uint32_t *n_steps);
 
 /* ---- FFT autotuning --------------------------------------------------------------
  * No counterpart in the reference (whose Metal backend fixes its kernel

@@ -548,11 +548,11 @@ int batch_create_trees(stwo_hip_ctx *ctx, const BatchTree *trees, size_t n_trees
   size_t tables_bytes = (st.host.size() + 255) & ~(size_t)255;
   void *dmem = nullptr;
   bool from_job = false;
-  // A tree's steps: its layers with columns and a run of nodes after each; every
-  // launch's table starts aligned.
+  // A tree's steps: its layers with columns and a run of nodes after each, at most
+  // two launches of it; every launch's table starts aligned.
   size_t tree_steps_bound = 0;
   if (tl.size() > 1)
-    for (const TreeLaunches &L : tl) tree_steps_bound += 2 * L.lt.size() * (sizeof(MerkleTree) + 256);
+    for (const TreeLaunches &L : tl) tree_steps_bound += 3 * L.lt.size() * (sizeof(MerkleTree) + 256);
   const size_t desc_bytes = levels_bound(gt.size()) + tree_steps_bound;
   int arc = device_alloc(ctx, tables_bytes + desc_bytes, &dmem, &from_job);
   if (arc) return arc;
@@ -576,6 +576,7 @@ int batch_create_trees(stwo_hip_ctx *ctx, const BatchTree *trees, size_t n_trees
     for (size_t k = 0; k < tl.size(); k++) {
       const TreeLaunches &L = tl[k];
       uint32_t *counters = (uint32_t *)(dbase + L.counters_off);
+      const uint32_t n_counters = tree_counters(L.max_log);
       const bool lifted = L.kind == STWO_HIP_TREE_LIFTED;
       size_t ti = 0;
       for (int l = (int)L.max_log; l >= 0;) {
@@ -585,14 +586,16 @@ int batch_create_trees(stwo_hip_ctx *ctx, const BatchTree *trees, size_t n_trees
         if (t) {
           steps[k].push_back(merkle_layer_step(prev, (const ColRef *)(dbase + t->off), t->count, (uint32_t)l,
                                                L.layers + tree_layer_off((uint32_t)l), L.mode, lifted));
-          if (!merkle_tree_step(steps[k].back(), (uint32_t)(next + 1), counters)) {
+          if (!merkle_tree_step(steps[k].back(), (uint32_t)(next + 1), counters, n_counters)) {
             l--;
             continue;
           }
+          l = next;
         } else {
-          steps[k].push_back(merkle_nodes_step(L.layers, (uint32_t)l + 1, (uint32_t)(next + 1), L.mode, counters));
+          steps[k].push_back(
+              merkle_nodes_step(L.layers, (uint32_t)l + 1, (uint32_t)(next + 1), L.mode, counters, n_counters));
+          l = (int)steps[k].back().nodes.stop_log - 1;
         }
-        l = next;
       }
       longest = std::max(longest, steps[k].size());
     }

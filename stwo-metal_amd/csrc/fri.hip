@@ -530,10 +530,7 @@ __global__ void __launch_bounds__(kTreeThreads) fri_layer_kernel(FriLayerJobs jo
 template <int FOLD>
 static int launch_fri_layer(stwo_hip_ctx *ctx, const FriLayerJobs &jobs, uint32_t n_jobs, const uint32_t *itw_end,
                             uint32_t lg) {
-  // The workgroup's size is the one for a single layer of as many leaves as the
-  // launch holds: six layers of 2^17 take 78 us in 1,024s, 95 us in 256s; six of
-  // 2^13, 22 us in 256s, 25 us in 64s.
-  const uint32_t per = std::min(tree_leaves_log(lg + (31 - __builtin_clz(n_jobs))), lg >= 10 ? 10u : 8u);
+  const uint32_t per = fri_leaves_log(lg, n_jobs);
   const dim3 grid(1u << (lg > per ? lg - per : 0), n_jobs), block(kTreeThreads);
   return launch(ctx, "fri_layer",
                 per == 6   ? fri_layer_kernel<FOLD, 64>

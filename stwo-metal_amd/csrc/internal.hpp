@@ -324,22 +324,49 @@ struct MerkleStep {
 };
 MerkleStep merkle_layer_step(const uint32_t *prev, const ColRef *d_cols, uint32_t n_cols, uint32_t log_size,
                              uint32_t *out, int mode, bool lifted);
-MerkleStep merkle_nodes_step(uint32_t *layers, uint32_t top_log, uint32_t stop_log, int mode, uint32_t *counters);
+// Node layers from top_log - 1 down to s.nodes.stop_log, which is above stop_log
+// where n_counters are too few for the whole run.
+MerkleStep merkle_nodes_step(uint32_t *layers, uint32_t top_log, uint32_t stop_log, int mode, uint32_t *counters,
+                             uint32_t n_counters);
 // Extends a layer's step by the node layers below it down to stop_log, if the
 // two are to share a launch.
-bool merkle_tree_step(MerkleStep &s, uint32_t stop_log, uint32_t *counters);
+bool merkle_tree_step(MerkleStep &s, uint32_t stop_log, uint32_t *counters, uint32_t n_counters);
 int launch_merkle(stwo_hip_ctx *ctx, const MerkleStep &s);
 // n steps of one kind from a table of MerkleLayer, MerkleNodes or MerkleTree.
 int launch_merkle_multi(stwo_hip_ctx *ctx, uint32_t kind, bool lifted, const void *d_steps, uint32_t n, uint32_t wgs);
 
 // Counters of the one-launch trees: a word per group of workgroups that hand
-// their digests on, stage by stage; 2^12 + 2^5 + 1 for 2^30 leaves, and at most
-// 2^(lg / 2) for 2^lg (a tree's stages take equal shares of the levels above the
-// first 2^6, 2^8 or 2^10 digests).
+// their digests on, stage by stage.  A stage takes tree_stage(l, stop) levels of
+// a run from the workgroups' level l down to `stop`: equal shares, at most 8 each.
+// A run down to the root needs 2^12 + 2^6 + 1 words at 2^30 leaves, but one that
+// ends at a layer with columns may be a single level over all its workgroups'
+// digests (2^25 nodes down to 2^14: 2^14 words); merkle_nodes_step and
+// merkle_tree_step end a launch at its workgroups' own level where the run needs
+// more than there are.
+__host__ __device__ inline uint32_t tree_stage(uint32_t l, uint32_t stop) {
+  const uint32_t rem = l - stop, stages = (rem + 7) / 8;
+  return (rem + stages - 1) / stages;
+}
+inline uint64_t tree_counters_needed(uint32_t l, uint32_t stop) {
+  uint64_t n = 0;
+  while (l > stop) {
+    l -= tree_stage(l, stop);
+    n += (uint64_t)1 << l;
+  }
+  return n;
+}
+// The words kept for the trees of up to 2^lg leaves: by a context, for all of
+// its stream's, and by a plan or a FRI commit, for one tree of 2^lg.
 constexpr uint32_t kTreeCounters = 1u << 13;
 inline uint32_t tree_counters(uint32_t lg) { return std::min(kTreeCounters, 1u << ((lg + 1) / 2)); }
 // log2 of the first digests a workgroup of a one-launch tree of 2^lg takes.
 inline uint32_t tree_leaves_log(uint32_t lg) { return lg <= 14 ? 6 : lg < 18 ? 8 : 10; }
+// The same for n_jobs FRI layers of 2^lg in a launch: the size for a single layer of
+// as many leaves as the launch holds (six layers of 2^17 take 78 us in 1,024s, 95 us
+// in 256s; six of 2^13, 22 us in 256s, 25 us in 64s).
+inline uint32_t fri_leaves_log(uint32_t lg, uint32_t n_jobs) {
+  return std::min(tree_leaves_log(lg + (31 - __builtin_clz(n_jobs))), lg >= 10 ? 10u : 8u);
+}
 
 __host__ __device__ inline size_t tree_layer_off(uint32_t l) { return (((size_t)1 << l) - 1) * 8; }
 

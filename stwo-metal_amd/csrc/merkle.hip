@@ -471,28 +471,33 @@ MerkleStep merkle_layer_step(const uint32_t *prev, const ColRef *d_cols, uint32_
 }
 
 // Node layers top_log-1 .. stop_log (< top_log) of a packed tree whose layer
-// top_log is filled.  counters: tree_counters(top_log) zeros, left zero, used by
-// no launch that may overlap this one.
-MerkleStep merkle_nodes_step(uint32_t *layers, uint32_t top_log, uint32_t stop_log, int mode, uint32_t *counters) {
+// top_log is filled.  counters: n_counters zeros, left zero, used by no launch
+// that may overlap this one.  A run that needs more ends at its workgroups' own
+// level (then no workgroup meets another) and leaves the rest to a further
+// launch, which costs 4 us where the levels before it take milliseconds.
+MerkleStep merkle_nodes_step(uint32_t *layers, uint32_t top_log, uint32_t stop_log, int mode, uint32_t *counters,
+                             uint32_t n_counters) {
   MerkleStep s{};
   const uint32_t out_log = top_log - 1;
   // (four nodes per lane take the two levels above along)
   const uint32_t per = std::min<uint32_t>(tree_leaves_log(out_log), out_log >= stop_log + 2 ? 10 : 8);
+  const uint32_t own = out_log > per ? out_log - per : 0;  // the workgroups' level
+  if (own > stop_log && tree_counters_needed(own, stop_log) > n_counters) stop_log = own;
   s.nodes = {layers, counters, out_log, stop_log, (uint32_t)(mode == STWO_HIP_HASH_BLAKE2S_M31), 0};
   s.kind = per == 6 ? kMerkleNodes64 : per == 8 ? kMerkleNodes256 : kMerkleNodes1024;
-  s.wgs = 1u << (out_log > per ? out_log - per : 0);
+  s.wgs = 1u << own;
   return s;
 }
 
 // Up to 2^14 nodes, where the node layers alone also take a quad for each of 64.
 // With a lane for each of 256 above that there is nothing to gain: 2^17 leaves of
 // 16 columns 37.6 us, in two launches 9.2 + 27.5.
-bool merkle_tree_step(MerkleStep &s, uint32_t stop_log, uint32_t *counters) {
-  const uint32_t lg = s.layer.log_size;
-  if (lg > 14 || stop_log >= lg) return false;
+bool merkle_tree_step(MerkleStep &s, uint32_t stop_log, uint32_t *counters, uint32_t n_counters) {
+  const uint32_t lg = s.layer.log_size, own = lg > 6 ? lg - 6 : 0;
+  if (lg > 14 || stop_log >= lg || tree_counters_needed(own, stop_log) > n_counters) return false;
   s.tree = {s.layer, counters, stop_log, 0};
   s.kind = s.layer.n_cols > 16 ? kMerkleTreeLds : kMerkleTree;
-  s.wgs = 1u << (lg > 6 ? lg - 6 : 0);
+  s.wgs = 1u << own;
   return true;
 }
 
@@ -546,7 +551,7 @@ static int launch_layer(stwo_hip_ctx *ctx, const uint32_t *prev, const std::vect
   int rc = check_mode(ctx, mode);
   if (rc) return rc;
   MerkleStep s = merkle_layer_step(prev, nullptr, (uint32_t)cols.size(), log_size, out, mode, lifted);
-  *done = merkle_tree_step(s, stop_log, ctx->d_counters);
+  *done = merkle_tree_step(s, stop_log, ctx->d_counters, kTreeCounters);
   const bool in_args = s.kind == kMerkleTree || s.kind == kMerkleLayer || s.kind == kMerkleAhead;
   if (in_args && cols.size() <= kInlineCols) {
     InlineCols in{};
@@ -573,8 +578,12 @@ static int launch_layer(stwo_hip_ctx *ctx, const uint32_t *prev, const std::vect
 
 static int hash_node_layers(stwo_hip_ctx *ctx, uint32_t *layers, uint32_t top_log, uint32_t stop_log, int mode) {
   int rc = check_mode(ctx, mode);
-  if (rc || top_log <= stop_log) return rc;
-  return launch_merkle(ctx, merkle_nodes_step(layers, top_log, stop_log, mode, ctx->d_counters));
+  while (!rc && top_log > stop_log) {
+    const MerkleStep s = merkle_nodes_step(layers, top_log, stop_log, mode, ctx->d_counters, kTreeCounters);
+    rc = launch_merkle(ctx, s);
+    top_log = s.nodes.stop_log;
+  }
+  return rc;
 }
 
 }  // namespace stwo_hip
@@ -670,6 +679,50 @@ int stwo_hip_merkle_lifted_commit(stwo_hip_ctx *ctx, const uint32_t *const *cols
                          hash_mode, 0, &done);
   if (rc || done) return rc;
   return hash_node_layers(ctx, layers, lifting_log_size, 0, hash_mode);
+}
+
+int stwo_hip_debug_tree_plan(int what, uint32_t top_log, uint32_t stop_log, uint32_t n, uint32_t plan_log,
+                             uint32_t *out, uint32_t max_steps, uint32_t *n_steps) {
+  if (!out || !n_steps || what < 0 || what > 2 || top_log > 30 || stop_log > top_log || plan_log > 30 ||
+      (what == 2 && (n < 1 || n > 16 || stop_log)))
+    return STWO_HIP_EINVAL;
+  const uint32_t there = plan_log ? tree_counters(plan_log) : kTreeCounters;
+  uint32_t k = 0;
+  auto put = [&](uint32_t first, uint32_t own, uint32_t stop, uint32_t wgs) {
+    own = std::max(own, stop);  // a workgroup ends at the run's end
+    if (k < max_steps) {
+      uint32_t *o = out + 6 * k;
+      o[0] = first;
+      o[1] = own;
+      o[2] = stop;
+      o[3] = wgs;
+      o[4] = (uint32_t)tree_counters_needed(own, stop);
+      o[5] = there;
+    }
+    k++;
+  };
+  auto log2 = [](uint32_t v) { return 31u - (uint32_t)__builtin_clz(v); };
+  uint32_t top = top_log;
+  if (what == 2) {
+    const uint32_t per = fri_leaves_log(top, n), own = top > per ? top - per : 0;
+    put(top, own, 0, 1u << own);
+    top = 0;
+  } else if (what == 1) {
+    MerkleStep s = merkle_layer_step(nullptr, nullptr, n, top, nullptr, STWO_HIP_HASH_BLAKE2S, false);
+    if (merkle_tree_step(s, stop_log, nullptr, there)) {
+      put(top, log2(s.wgs), s.tree.stop_log, s.wgs);
+      top = s.tree.stop_log;
+    } else {
+      put(top, top, top, s.wgs);
+    }
+  }
+  while (top > stop_log) {
+    const MerkleStep s = merkle_nodes_step(nullptr, top, stop_log, STWO_HIP_HASH_BLAKE2S, nullptr, there);
+    put(s.nodes.out_log, log2(s.wgs), s.nodes.stop_log, s.wgs);
+    top = s.nodes.stop_log;
+  }
+  *n_steps = k;
+  return k <= max_steps ? STWO_HIP_OK : STWO_HIP_EINVAL;
 }
 
 }  // extern "C"

@@ -159,15 +159,15 @@ __device__ __forceinline__ uint32_t tree_levels(TreeLds &S, uint32_t buf, uint32
 
 // The rest of the tree above the workgroup's subtree, whose one digest is node
 // b of level l (stored by tree_levels with handoff, in buffer buf), down to
-// level `stop`.  Stages take equal shares of the levels, at most 8 each.
+// level `stop`, in stages of tree_stage levels.  counters: tree_counters_needed(l, stop)
+// zeros, left zero.
 // Returns the buffer whose row 0 is then this workgroup's last digest (the root
 // when stop = 0), or -1 in the workgroups that another one goes on for.
 __device__ __forceinline__ int tree_finish(TreeLds &S, uint32_t buf, uint32_t b, uint32_t l, uint32_t stop,
                                            uint32_t *packed, uint32_t m31, uint32_t *counters) {
   const uint32_t tid = threadIdx.x;
   while (l > stop) {
-    const uint32_t rem = l - stop, stages = (rem + 7) / 8, s = (rem + stages - 1) / stages;
-    const uint32_t group = b >> s;
+    const uint32_t s = tree_stage(l, stop), group = b >> s;
     // every lane's handed-over words have left before the count
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
