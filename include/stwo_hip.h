@@ -665,8 +665,11 @@ int stwo_hip_debug_tree_plan(int what, uint32_t top_log, uint32_t stop_log, uint
  * context, where every later plan of that shape uses it (interpolate,
  * evaluate, extend_evals, batch_create).  For each distinct log size n of
  * log_sizes (n >= 4): interpolate of 2^n and evaluate of 2^n at log_blowup.
- * Candidates: low-pass tile 2^10..2^13 (default 2^12), strided passes of at
- * most 5..8 layers (default 8), the tile's own workgroup size or 512 lanes.
+ * Candidates: butterfly passes of low-pass tile 2^10..2^13 (default 2^12),
+ * strided passes of at most 5..8 layers (default 8), the tile's own workgroup
+ * size or 512 lanes.  The default runs groups that are large enough on the
+ * matrix cores, small columns in a workgroup each, and others as the default
+ * butterfly passes.
  * Each runs on as many synthetic columns as the set has of that size (at most
  * 2^26 words, in a context scratch buffer); the fastest of 3 timed runs after
  * a warm-up counts.  Another plan replaces the default only when it is at
@@ -677,7 +680,9 @@ int stwo_hip_debug_tree_plan(int what, uint32_t top_log, uint32_t stop_log, uint
 int stwo_hip_fft_autotune(stwo_hip_ctx *ctx, const uint32_t *log_sizes, size_t n_cols, uint32_t log_blowup,
                           const stwo_hip_twiddles *tw, uint32_t *report, size_t max_report, size_t *n_report);
 /* Sets planner choices (6 words per entry: n, N, inverse, t0 10..13, smax
- * 5..8, wg 0 or 9), e.g. a table saved from an earlier stwo_hip_fft_autotune;
+ * 5..8, wg 0 or 9), e.g. a table saved from an earlier stwo_hip_fft_autotune:
+ * (12, 8, 0), which it reports where the default won, leaves a shape on the
+ * default, any other choice stands in its place.
  * stwo_hip_fft_tune_clear returns every shape to the defaults. */
 int stwo_hip_fft_tune_set(stwo_hip_ctx *ctx, const uint32_t *entries, size_t n_entries);
 int stwo_hip_fft_tune_clear(stwo_hip_ctx *ctx);

@@ -1602,6 +1602,8 @@ int stwo_hip_fft_autotune(stwo_hip_ctx *ctx, const uint32_t *log_sizes, size_t n
       const bool matrix = mx_plan(ctx, tw, n, Nd - n, inverse, c, true, false, &mx);
       const bool column = !matrix && column_fft_takes(ctx, n, Nd, c, inverse, !inverse);
       for (auto &ck : cands) {
+        const bool is_def = !(ck.first < def_key) && !(def_key < ck.first);
+        if (is_def && (matrix || column)) continue;  // not what the default runs
         rc = make_group_passes(ctx, n, Nd, inverse, first, inpl, (uint32_t)c, tw_end, true, ps, &ck.second);
         if (rc) return rc;
         float ms = 0;
@@ -1615,7 +1617,7 @@ int stwo_hip_fft_autotune(stwo_hip_ctx *ctx, const uint32_t *log_sizes, size_t n
             },
             &ms);
         if (rc) return rc;
-        if (!matrix && !column && !(ck.first < def_key) && !(def_key < ck.first)) def_ms = ms;
+        if (is_def) def_ms = ms;
         if (ms < best) {
           best = ms;
           best_t = ck.second;
@@ -1640,9 +1642,8 @@ int stwo_hip_fft_autotune(stwo_hip_ctx *ctx, const uint32_t *log_sizes, size_t n
       if (def_ms > 0 && best > def_ms * (1.0f - kTuneMargin)) {
         best = def_ms;
         best_t = def;
-      } else {
-        best_t.chosen = 1;
       }
+      best_t.chosen = !best_t.is_default();
       ctx->fft_tune[fft_tune_key(n, Nd, inverse)] = best_t;
       if (report && nr < max_report) {
         uint32_t *o = report + 8 * nr;
@@ -1669,7 +1670,7 @@ int stwo_hip_fft_tune_set(stwo_hip_ctx *ctx, const uint32_t *entries, size_t n_e
     t.t0 = (uint8_t)e[3];
     t.smax = (uint8_t)e[4];
     t.wg = (uint8_t)e[5];
-    t.chosen = 1;
+    t.chosen = !t.is_default();
     ctx->fft_tune[fft_tune_key(e[0], e[1], e[2] != 0)] = t;
   }
   return STWO_HIP_OK;
