@@ -682,7 +682,9 @@ int stwo_hip_fft_autotune(stwo_hip_ctx *ctx, const uint32_t *log_sizes, size_t n
 /* Sets planner choices (6 words per entry: n, N, inverse, t0 10..13, smax
  * 5..8, wg 0 or 9), e.g. a table saved from an earlier stwo_hip_fft_autotune:
  * (12, 8, 0), which it reports where the default won, leaves a shape on the
- * default, any other choice stands in its place.
+ * default, any other choice stands in its place.  A choice is of butterfly
+ * passes, timed alone: groups that share a launch of the matrix cores or of the
+ * small columns' workgroups (batch_create; calls over several sizes) stay there.
  * stwo_hip_fft_tune_clear returns every shape to the defaults. */
 int stwo_hip_fft_tune_set(stwo_hip_ctx *ctx, const uint32_t *entries, size_t n_entries);
 int stwo_hip_fft_tune_clear(stwo_hip_ctx *ctx);

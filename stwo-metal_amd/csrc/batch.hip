@@ -158,7 +158,7 @@ int build_levels(stwo_hip_ctx *ctx, const stwo_hip_twiddles *tw, const std::vect
     const bool inv = t.stage != BATCH_RFFT, fwd = t.stage != BATCH_IFFT;
     const uint32_t N = t.n + (fwd ? t.b : 0);
     MxPlan mx;
-    if (!column_fft_takes(ctx, t.n, N, t.count, inv, fwd) || column_words + ((size_t)t.count << t.n) > kColumnFftWords ||
+    if (!column_fft_takes(ctx, t.n, N, t.count, inv, fwd, true) || column_words + ((size_t)t.count << t.n) > kColumnFftWords ||
         (matrix && (!inv || mx_plan(ctx, tw, t.n, 0, true, t.count, t.aligned16, true, &mx)) &&
          (!fwd || mx_plan(ctx, tw, t.n, t.b, false, t.count, t.aligned16, true, &mx))))
       continue;

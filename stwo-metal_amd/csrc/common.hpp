@@ -34,7 +34,8 @@ struct FftTune {
   uint8_t t0 = 12;   // tile log of the contiguous low pass (10..13)
   uint8_t smax = 8;  // most layers per strided pass (5..8)
   uint8_t wg = 0;    // workgroup log: 0 = max(8, T - 4); 9 = 512 lanes for every tile size
-  uint8_t chosen = 0;  // another plan than the default: it stands in place of the matrix passes and of a workgroup per column
+  uint8_t chosen = 0;  // another plan than the default: it stands in place of the matrix passes
+                       // and of a workgroup per column, but for groups in shared launches
   bool is_default() const { return t0 == 12 && smax == 8 && wg == 0; }
 };
 inline uint64_t fft_tune_key(uint32_t n, uint32_t N, bool inverse) {

@@ -1154,7 +1154,7 @@ static int run_lde_group(stwo_hip_ctx *ctx, const std::vector<FftCol> &cols, con
   MxPlan mx;
   const bool matrix = mx_plan(ctx, tw, n, 0, true, cols.size(), aligned16, false, &mx) &&
                       mx_plan(ctx, tw, n, b, false, cols.size(), aligned16, false, &mx);
-  if (!matrix && column_fft_takes(ctx, n, N, cols.size(), true, true))
+  if (!matrix && column_fft_takes(ctx, n, N, cols.size(), true, true, false))
     return run_column_fft(ctx, tw, tf, n, N, store_coeffs, true, true);
   void *d[3];
   {
@@ -1219,7 +1219,7 @@ static int run_fft_group(stwo_hip_ctx *ctx, const std::vector<FftCol> &cols, uin
     for (const FftCol &c : cols)
       if ((((uintptr_t)c.in) | ((uintptr_t)c.out)) & 15) aligned16 = false;
     matrix = mx_plan(ctx, tw, n, N - n, inverse, cols.size(), aligned16, false, &mx);
-    if (!matrix && column_fft_takes(ctx, n, N, cols.size(), inverse, !inverse))
+    if (!matrix && column_fft_takes(ctx, n, N, cols.size(), inverse, !inverse, false))
       return run_column_fft(ctx, tw, cols, n, N, true, inverse, !inverse);
   }
   // The group's table and, forward, the in-place table of the passes after
@@ -1600,7 +1600,7 @@ int stwo_hip_fft_autotune(stwo_hip_ctx *ctx, const uint32_t *log_sizes, size_t n
       MxPlan mx;
       ctx->fft_tune.erase(fft_tune_key(n, Nd, inverse));
       const bool matrix = mx_plan(ctx, tw, n, Nd - n, inverse, c, true, false, &mx);
-      const bool column = !matrix && column_fft_takes(ctx, n, Nd, c, inverse, !inverse);
+      const bool column = !matrix && column_fft_takes(ctx, n, Nd, c, inverse, !inverse, false);
       for (auto &ck : cands) {
         const bool is_def = !(ck.first < def_key) && !(def_key < ck.first);
         if (is_def && (matrix || column)) continue;  // not what the default runs

@@ -332,8 +332,11 @@ const char *name(bool inv, bool fwd) { return !fwd ? "ifft_pass_column" : inv ? 
 // 62.4 -> 53.5; 2^11 x 1,024 58.5 -> 51.4, x 4,096 118 -> 125; 2^12 x 16 32.7 ->
 // 29.2, x 512 53.1 -> 47.7 (from 1,024 on the matrix passes). 2^13 alone, one
 // workgroup's largest: 32.9 -> 34.5.
-bool column_fft_takes(const stwo_hip_ctx *ctx, uint32_t n, uint32_t N, size_t n_cols, bool inv, bool fwd) {
+bool column_fft_takes(const stwo_hip_ctx *ctx, uint32_t n, uint32_t N, size_t n_cols, bool inv, bool fwd,
+                      bool batched) {
   if (n < 4 || n > 12 || N > kColMaxLog || n_cols << n > kColumnFftWords) return false;
+  // a vector plan chosen for the shape stands in a launch of its own (as in mx_plan)
+  if (batched) return true;
   auto chosen = [&](uint32_t M, int inverse) {
     auto it = ctx->fft_tune.find(fft_tune_key(n, M, inverse));
     return it != ctx->fft_tune.end() && it->second.chosen;

@@ -23,7 +23,8 @@ struct ColumnFft {
 // Coefficients in one launch at most.
 constexpr size_t kColumnFftWords = (size_t)1 << 21;
 // Whether a group is taken (alone, or at the side of others in one launch).
-bool column_fft_takes(const stwo_hip_ctx *ctx, uint32_t n, uint32_t N, size_t n_cols, bool inv, bool fwd);
+bool column_fft_takes(const stwo_hip_ctx *ctx, uint32_t n, uint32_t N, size_t n_cols, bool inv, bool fwd,
+                      bool batched);
 ColumnFft column_fft(const stwo_hip_twiddles *tw, const FftCol *d_cols, uint32_t n_cols, uint32_t n, uint32_t N,
                      bool store);
 // One group, its columns given on the host.

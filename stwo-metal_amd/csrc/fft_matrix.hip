@@ -804,9 +804,12 @@ bool mx_plan(const stwo_hip_ctx *ctx, const stwo_hip_twiddles *tw, uint32_t n, u
   if (!tw->d_mx || !aligned16 || n < kMxMinLog || n > kMxMaxLog || b > kMxMaxBlowup || n_cols < 3) return false;
   const uint64_t units = mx_low_units((uint32_t)n_cols, n);
   if (units < (batched ? kMxBatchUnits : kMxMinUnits)) return false;
-  // A vector plan set for the shape stands.
+  // A vector plan chosen for the shape stands in a launch of its own.  It was timed
+  // there: in a shared launch it would only take the group out of the others' (the
+  // plan of 1,024 uneven columns 1.68 ms, 1.73 with three groups taken out; with them
+  // kept in 1.60 beside 1.66).
   auto it = ctx->fft_tune.find(fft_tune_key(n, n + b, inverse));
-  if (it != ctx->fft_tune.end() && it->second.chosen) return false;
+  if (!batched && it != ctx->fft_tune.end() && it->second.chosen) return false;
   plan->top_layers = n == 12 ? 0 : n <= 16 ? 4 : 8;
   plan->t0 = n <= 20 ? n - plan->top_layers : 12;
   plan->mid = n > 20;

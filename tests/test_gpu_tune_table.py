@@ -70,3 +70,31 @@ def test_report_set_back(sets):
         other.fft_tune_set([r[:6] for r in report])
         assert _launches(other, sets) == _launches(ctx, sets)
         tw.destroy()
+
+
+def test_choices_leave_shared_launches_alone(sets):
+    """A plan over all the groups: another choice for each shape moves none out of the
+    launches that they share."""
+    logs = [n for n, C in GROUPS for _ in range(C)]
+    evs = [e for _, es, _, _ in sets for e in es]
+    want = [w for _, _, _, ws in sets for w in ws]
+    with sh.Context(0) as ctx:
+        tw = ctx.precompute_twiddles(sh.half_odds(max(logs) + B - 1))
+        cols, outs = [ctx.alloc(1 << n) for n in logs], [ctx.alloc(2 << n) for n in logs]
+        layers = ctx.alloc(sh.tree_words(max(logs) + B))
+        names = []
+        for t0, smax, wg in ((12, 8, 0), (12, 5, 9)):
+            ctx.fft_tune_set([(n, N, inv, t0, smax, wg) for n, _ in GROUPS for N, inv in ((n, 1), (n + B, 0))])
+            plan = ctx.batch_create(cols, logs, B, tw, outs, layers, use_graph=False)
+            for c, e in zip(cols, evs):
+                c.upload(e)
+            ctx.prof_enable()
+            ctx.prof_reset()
+            plan.run()
+            names.append({k for k in ctx.prof_read() if "mx" in k or "column" in k})
+            ctx.prof_enable(False)
+            for o, w in zip(outs, want):
+                assert np.array_equal(o.download(), w)
+            plan.destroy()
+        assert names[0] == names[1] and any("mx" in k for k in names[0]) and any("column" in k for k in names[0])
+        tw.destroy()
