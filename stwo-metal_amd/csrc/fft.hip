@@ -1289,21 +1289,36 @@ static int run_fft_group(stwo_hip_ctx *ctx, const std::vector<FftCol> &cols, uin
   return STWO_HIP_OK;
 }
 
-// The groups (log size -> columns) of at least 2^4 in shared launches, where
-// there are several; the ones done are taken out.
-static int share_launches(stwo_hip_ctx *ctx, std::map<uint32_t, std::vector<FftCol>> &groups, uint32_t b, int stage,
-                          const stwo_hip_twiddles *tw, bool store_coeffs) {
-  std::vector<FftSet> sets;
-  // largest first: their workgroups start first
-  for (auto g = groups.rbegin(); g != groups.rend() && g->first >= 4; ++g) {
-    if (g->second.size() > 65535) return STWO_HIP_OK;
-    sets.push_back({g->first, b, stage, g->second});
+// The groups (log size -> columns) of a call, smallest first as far as one may read
+// what another writes: those below 2^4 one after the other, then the rest in shared
+// launches where there are several and they do not meet, else one after the other.
+// one(log size, at most 65,535 columns): a group by itself.
+template <typename One>
+static int run_groups(stwo_hip_ctx *ctx, std::map<uint32_t, std::vector<FftCol>> &groups, uint32_t b, int stage,
+                      const stwo_hip_twiddles *tw, bool store_coeffs, One one) {
+  auto alone = [&](uint32_t n, const std::vector<FftCol> &cols) {
+    if (cols.size() <= 65535) return one(n, cols);
+    int rc = STWO_HIP_OK;
+    for (size_t off = 0; off < cols.size() && !rc; off += 65535)
+      rc = one(n, std::vector<FftCol>(cols.begin() + off, cols.begin() + std::min(cols.size(), off + (size_t)65535)));
+    return rc;
+  };
+  int rc = STWO_HIP_OK;
+  auto rest = groups.begin();
+  for (; rest != groups.end() && rest->first < 4 && !rc; ++rest) rc = alone(rest->first, rest->second);
+  if (rc) return rc;
+  bool share = std::distance(rest, groups.end()) > 1;
+  for (auto g = rest; g != groups.end(); ++g) share = share && g->second.size() <= 65535;
+  if (share) {
+    std::vector<FftSet> sets;
+    // largest first: their workgroups start first
+    for (auto g = groups.rbegin(); g != groups.rend() && g->first >= 4; ++g)
+      sets.push_back({g->first, b, stage, g->second});
+    bool done = false;
+    rc = run_fft_sets(ctx, sets, tw, store_coeffs, &done);
+    if (rc || done) return rc;
   }
-  if (sets.size() < 2) return STWO_HIP_OK;
-  bool done = false;
-  int rc = run_fft_sets(ctx, sets, tw, store_coeffs, &done);
-  if (!rc && done)
-    for (const FftSet &st : sets) groups.erase(st.n);
+  for (; rest != groups.end() && !rc; ++rest) rc = alone(rest->first, rest->second);
   return rc;
 }
 
@@ -1368,18 +1383,9 @@ int stwo_hip_interpolate_columns(stwo_hip_ctx *ctx, uint32_t *const *cols, const
     int rc = check_domain(ctx, {half_odds_initial(g.first - 1), g.first - 1}, tw);
     if (rc) return rc;
   }
-  int rc = share_launches(ctx, groups, 0, BATCH_IFFT, tw, true);
-  if (rc) return rc;
-  for (auto &g : groups) {
-    const uint32_t N = g.first;
-    for (size_t off = 0; off < g.second.size(); off += 65535) {
-      std::vector<FftCol> part(g.second.begin() + off,
-                               g.second.begin() + std::min(g.second.size(), off + (size_t)65535));
-      rc = run_fft_group(ctx, part, N, N, tw, true, {half_odds_initial(N - 1), N - 1});
-      if (rc) return rc;
-    }
-  }
-  return STWO_HIP_OK;
+  return run_groups(ctx, groups, 0, BATCH_IFFT, tw, true, [&](uint32_t N, const std::vector<FftCol> &part) {
+    return run_fft_group(ctx, part, N, N, tw, true, {half_odds_initial(N - 1), N - 1});
+  });
 }
 
 int stwo_hip_evaluate(stwo_hip_ctx *ctx, const uint32_t *coeffs, uint32_t coeffs_log_size, stwo_hip_coset domain,
@@ -1414,18 +1420,10 @@ int stwo_hip_evaluate_polynomials(stwo_hip_ctx *ctx, const uint32_t *const *coef
     int rc = check_domain(ctx, {half_odds_initial(N - 1), N - 1}, tw);
     if (rc) return rc;
   }
-  int rc = share_launches(ctx, groups, log_blowup, BATCH_RFFT, tw, true);
-  if (rc) return rc;
-  for (auto &g : groups) {
-    const uint32_t n = g.first, N = n + log_blowup;
-    for (size_t off = 0; off < g.second.size(); off += 65535) {
-      std::vector<FftCol> part(g.second.begin() + off,
-                               g.second.begin() + std::min(g.second.size(), off + (size_t)65535));
-      rc = run_fft_group(ctx, part, n, N, tw, false, {half_odds_initial(N - 1), N - 1});
-      if (rc) return rc;
-    }
-  }
-  return STWO_HIP_OK;
+  return run_groups(ctx, groups, log_blowup, BATCH_RFFT, tw, true, [&](uint32_t n, const std::vector<FftCol> &part) {
+    const uint32_t N = n + log_blowup;
+    return run_fft_group(ctx, part, n, N, tw, false, {half_odds_initial(N - 1), N - 1});
+  });
 }
 
 int stwo_hip_extend_evals(stwo_hip_ctx *ctx, uint32_t *const *cols, const uint32_t *log_sizes, size_t n_cols,
@@ -1447,33 +1445,19 @@ int stwo_hip_extend_evals(stwo_hip_ctx *ctx, uint32_t *const *cols, const uint32
     rc = check_domain(ctx, {half_odds_initial(N - 1), N - 1}, tw);
     if (rc) return rc;
   }
-  int rc = share_launches(ctx, groups, log_blowup, BATCH_LDE, tw, store_coeffs != 0);
-  if (rc) return rc;
-  for (auto &g : groups) {
-    const uint32_t n = g.first, N = n + log_blowup;
-    const stwo_hip_coset dom_i = {half_odds_initial(n - 1), n - 1}, dom_f = {half_odds_initial(N - 1), N - 1};
-    for (size_t off = 0; off < g.second.size(); off += 65535) {
-      const size_t e = std::min(g.second.size(), off + (size_t)65535);
-      std::vector<FftCol> part;
-      std::vector<uint32_t *> po;
-      for (size_t k = off; k < e; k++) {
-        uint32_t *col = (uint32_t *)g.second[k].in;
-        part.push_back({col, col});
-        po.push_back(g.second[k].out);
-      }
-      if (n >= 4) {
-        rc = run_lde_group(ctx, part, po, n, log_blowup, tw, store_coeffs != 0);
-      } else {
-        rc = run_fft_group(ctx, part, n, n, tw, true, dom_i);
-        if (rc) return rc;
-        std::vector<FftCol> pf;
-        for (size_t k = 0; k < part.size(); k++) pf.push_back({part[k].in, po[k]});
-        rc = run_fft_group(ctx, pf, n, N, tw, false, dom_f);
-      }
-      if (rc) return rc;
+  return run_groups(ctx, groups, log_blowup, BATCH_LDE, tw, store_coeffs != 0,
+                    [&](uint32_t n, const std::vector<FftCol> &cols) {
+    const uint32_t N = n + log_blowup;
+    std::vector<FftCol> part;
+    std::vector<uint32_t *> po;
+    for (const FftCol &c : cols) {
+      part.push_back({c.in, (uint32_t *)c.in});
+      po.push_back(c.out);
     }
-  }
-  return STWO_HIP_OK;
+    if (n >= 4) return run_lde_group(ctx, part, po, n, log_blowup, tw, store_coeffs != 0);
+    const int r = run_fft_group(ctx, part, n, n, tw, true, {half_odds_initial(n - 1), n - 1});
+    return r ? r : run_fft_group(ctx, cols, n, N, tw, false, {half_odds_initial(N - 1), N - 1});
+  });
 }
 
 // ---- autotuning ----------------------------------------------------------------
