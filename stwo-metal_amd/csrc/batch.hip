@@ -718,10 +718,10 @@ int run_fft_sets(stwo_hip_ctx *ctx, const std::vector<FftSet> &sets, const stwo_
   std::vector<Span> spans;
   for (uint32_t g = 0; g < sets.size(); g++)
     for (const FftCol &c : sets[g].cols) {
-      const uint32_t b = sets[g].b;
-      const bool in_place = sets[g].stage != BATCH_RFFT;
-      spans.push_back({(uintptr_t)c.in, (uintptr_t)(c.in + ((size_t)1 << sets[g].n)), g, in_place});
-      if (c.out != c.in) spans.push_back({(uintptr_t)c.out, (uintptr_t)(c.out + ((size_t)1 << (sets[g].n + b))), g, 1});
+      const bool evaluates = sets[g].stage != BATCH_IFFT;
+      spans.push_back({(uintptr_t)c.in, (uintptr_t)(c.in + ((size_t)1 << sets[g].n)), g, sets[g].stage != BATCH_RFFT});
+      if (evaluates)  // also where it lies over the input
+        spans.push_back({(uintptr_t)c.out, (uintptr_t)(c.out + ((size_t)1 << (sets[g].n + sets[g].b))), g, 1});
     }
   auto by_at = [](const Span &a, const Span &c) { return a.at < c.at; };
   if (!std::is_sorted(spans.begin(), spans.end(), by_at)) std::sort(spans.begin(), spans.end(), by_at);

@@ -1,6 +1,6 @@
 """Column lists of several sizes where one group's words are another's: the groups run
-smallest first, also those below 2^4, whose launches are their own.  Against the
-oracle, group by group."""
+smallest first, also those below 2^4, whose launches are their own, and columns
+evaluated in place.  Against the oracle, group by group."""
 import os
 import sys
 
@@ -31,6 +31,8 @@ CASES = {
     "small's output in large's input": (1, [(9, 1024, 4096), (6, 128, 512), (2, 0, 1032)]),
     "large's output over small's input": (1, [(9, 4096, 0), (6, 6000, 6400), (2, 100, 7000)]),
     "both among the smallest": (2, [(7, 4096, 2048), (5, 1024, 1200), (3, 64, 4100), (2, 32, 64)]),
+    "in place, one column inside another": (0, [(9, 0, 0), (6, 64, 64), (3, 72, 72)]),
+    "in place over 2^4 alone": (0, [(9, 1024, 1024), (6, 1088, 1088)]),
 }
 
 
