@@ -63,8 +63,8 @@ struct LevelLaunch {
   // pass with its directions, or the low pass (mx_layers = 0)
   bool matrix = false, mx_inv = false, mx_fwd = false;
   uint32_t mx_layers = 0;
-  // a workgroup per column (groups_off: ColumnFft descriptors), largest N
-  uint32_t column_N = 0;
+  // a workgroup per column (groups_off: ColumnFft descriptors), largest n and N
+  uint32_t column_n = 0, column_N = 0;
 };
 
 // One tree's layer tables and shape.
@@ -334,7 +334,7 @@ int build_levels(stwo_hip_ctx *ctx, const stwo_hip_twiddles *tw, const std::vect
     const bool apart = cols > 256;
     for (uint32_t large = 0; large <= (uint32_t)apart; large++) {
       std::vector<ColumnFft> descs;
-      uint32_t acc = 0, max_N = 0;
+      uint32_t acc = 0, max_n = 0, max_N = 0;
       for (size_t gi = 0; gi < gt.size(); gi++) {
         const GroupTabs &t = gt[gi];
         const uint32_t N = t.n + (stage == BATCH_IFFT ? 0 : t.b);
@@ -342,10 +342,12 @@ int build_levels(stwo_hip_ctx *ctx, const stwo_hip_twiddles *tw, const std::vect
         descs.push_back(column_fft(tw, (const FftCol *)(dbase + t.rfft_off), t.count, t.n, N, store_coeffs));
         descs.back().wg_start = acc;
         acc += t.count;
+        max_n = std::max(max_n, t.n);
         max_N = std::max(max_N, N);
       }
       if (descs.empty()) continue;
       LevelLaunch ll{};
+      ll.column_n = max_n;
       ll.column_N = max_N;
       ll.mx_inv = stage != BATCH_RFFT;
       ll.mx_fwd = stage != BATCH_IFFT;
@@ -425,7 +427,7 @@ int issue_levels(stwo_hip_ctx *c, const std::vector<LevelLaunch> &levels, uint8_
   for (const LevelLaunch &ll : levels) {
     if (ll.column_N) {
       int rc = launch_column_fft_multi(c, (const ColumnFft *)(dbase + ll.groups_off), ll.n_groups, ll.total_wgs,
-                                       ll.column_N, ll.mx_inv, ll.mx_fwd);
+                                       ll.column_n, ll.column_N, ll.mx_inv, ll.mx_fwd);
       if (rc) return rc;
       continue;
     }

@@ -20,7 +20,7 @@
 namespace stwo_hip {
 namespace {
 
-constexpr uint32_t kColMaxLog = 13;  // 59 KB of LDS at most
+constexpr uint32_t kColMaxLog = 13;  // domain; 59 KB of LDS at most (coefficients up to 2^12)
 constexpr uint32_t kColMaxThreads = 1024;
 
 // Position of element i: 4 words of padding every 64 spread the strides of
@@ -318,10 +318,11 @@ __global__ void __launch_bounds__(kColMaxThreads) column_fft_multi_kernel(const 
 }
 
 dim3 threads(uint32_t N) { return dim3(std::min(kColMaxThreads, std::max(64u, 1u << (N - 2)))); }
-// For every group of at most N: its own transforms' twiddles are shorter.
-size_t lds_bytes(uint32_t N, bool both) {
-  return (((size_t)1 << (N - 1)) * (both ? 2 : 1) + ((size_t)1 << N) / 16 * 17 + 4) * 4;
+// For every group of at most n and N: the twiddles of each transform, the words.
+constexpr size_t lds_bytes(uint32_t n, uint32_t N, bool inv, bool fwd) {
+  return ((inv ? (size_t)1 << (n - 1) : 0) + (fwd ? (size_t)1 << (N - 1) : 0) + ((size_t)1 << N) / 16 * 17 + 4) * 4;
 }
+static_assert(lds_bytes(kColMaxLog - 1, kColMaxLog, true, true) <= 59 << 10, "two workgroups of the largest a CU");
 const char *name(bool inv, bool fwd) { return !fwd ? "ifft_pass_column" : inv ? "lde_pass_column" : "rfft_pass_column"; }
 
 }  // namespace
@@ -362,7 +363,7 @@ int run_column_fft(stwo_hip_ctx *ctx, const stwo_hip_twiddles *tw, const std::ve
                    uint32_t N, bool store, bool inv, bool fwd) {
   ColumnFft p = column_fft(tw, nullptr, (uint32_t)cols.size(), n, N, store);
   const dim3 grid(p.n_cols), block = threads(N);
-  const size_t lds = lds_bytes(N, inv && fwd);
+  const size_t lds = lds_bytes(n, N, inv, fwd);
   if (cols.size() <= kInlineCols) {
     InlineFftCols in{};
     std::copy(cols.begin(), cols.end(), in.c);
@@ -397,9 +398,9 @@ int launch_fft_chunk_multi(stwo_hip_ctx *ctx, bool inverse, const FftPass2 *d_gr
 }
 
 int launch_column_fft_multi(stwo_hip_ctx *ctx, const ColumnFft *d_groups, uint32_t n_groups, uint32_t wgs,
-                            uint32_t max_N, bool inv, bool fwd) {
+                            uint32_t max_n, uint32_t max_N, bool inv, bool fwd) {
   const dim3 grid(wgs), block = threads(max_N);
-  const size_t lds = lds_bytes(max_N, inv && fwd);
+  const size_t lds = lds_bytes(max_n, max_N, inv, fwd);
   if (!fwd)
     return launch(ctx, name(inv, fwd), column_fft_multi_kernel<true, false>, grid, block, lds, d_groups, n_groups);
   if (!inv)

@@ -30,9 +30,9 @@ ColumnFft column_fft(const stwo_hip_twiddles *tw, const FftCol *d_cols, uint32_t
 // One group, its columns given on the host.
 int run_column_fft(stwo_hip_ctx *ctx, const stwo_hip_twiddles *tw, const std::vector<FftCol> &cols, uint32_t n,
                    uint32_t N, bool store, bool inv, bool fwd);
-// n_groups groups from a table on the device; max_N: their largest N.
+// n_groups groups from a table on the device; max_n, max_N: their largest n and N.
 int launch_column_fft_multi(stwo_hip_ctx *ctx, const ColumnFft *d_groups, uint32_t n_groups, uint32_t wgs,
-                            uint32_t max_N, bool inv, bool fwd);
+                            uint32_t max_n, uint32_t max_N, bool inv, bool fwd);
 
 // The 12-layer low pass (FftPass2::fixed == 1) in workgroups of 1,024 lanes, for
 // launches of at most kChunkWgs: up to there it is 1 to 8% ahead of the register
