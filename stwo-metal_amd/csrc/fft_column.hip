@@ -336,6 +336,14 @@ const char *name(bool inv, bool fwd) { return !fwd ? "ifft_pass_column" : inv ? 
 bool column_fft_takes(const stwo_hip_ctx *ctx, uint32_t n, uint32_t N, size_t n_cols, bool inv, bool fwd,
                       bool batched) {
   if (n < 4 || n > 12 || N > kColMaxLog || n_cols << n > kColumnFftWords) return false;
+  // At a large blowup a column is a long chain of a few lanes: 2^(n-2) of them write
+  // its 2^(N-n) blocks one after another (of 2^4 words, four lanes of 64). Where
+  // there are more columns than the CUs hold at once, that is the time (us, register
+  // passes -> here; the line lies between the two of each size): 2^4 at blowup 2^5 x
+  // 16,384 121 -> 121, x 32,768 155 -> 199; at 2^8 x 4,096 584 -> 512, x 8,192 590 -> 966;
+  // 2^5 at 2^7 x 8,192 648 -> 478, x 16,384 675 -> 913; 2^6 at 2^5 x 16,384 196 -> 182, x
+  // 32,768 264 -> 331.
+  if (n_cols > (n == 4 ? 4096 : 8192) && n_cols << N > (size_t)1 << (n == 4 ? 23 : 25)) return false;
   // a vector plan chosen for the shape stands in a launch of its own (as in mx_plan)
   if (batched) return true;
   auto chosen = [&](uint32_t M, int inverse) {
