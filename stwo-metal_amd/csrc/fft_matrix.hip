@@ -798,10 +798,17 @@ uint64_t mx_low_units(uint32_t n_cols, uint32_t N) { return (uint64_t)((n_cols +
 // 34.7 -> 33.3; 256 (2^16 x 64) 39.8 -> 35.1 / 49.1 -> 42.8; 1,024 (2^20 x 16)
 // 88.3 -> 61.6 / 149 -> 115.  A batched launch shares its workgroups between
 // groups, so there a group of kMxBatchUnits is taken along.  One or two columns
-// would leave most of the low pass's four column slots empty.
+// would leave most of the low pass's four column slots empty; from 2^22 on, where
+// three passes over memory are the time either way, three do too, and at 2^24 five
+// (us, vector -> matrix, interpolation / evaluation at blowup 1, 2 and 4: 3 x 2^21 60 ->
+// 56 / 58 -> 54, 88 -> 88 and 150 -> 154, 3 x 2^22 95 -> 92 / 90 -> 89, 151 -> 155 and 288 ->
+// 306, 4 x 2^22 116 -> 106 / 110 -> 103, 193 -> 178 and 380 -> 351, 3 x 2^23 160 -> 167 / 153
+// -> 164, 296 -> 314 and 588 -> 598, 5 x 2^24 501 -> 565 / 500 -> 551, 975 -> 989 and 1,910 ->
+// 1,891, 6 x 2^24 596 -> 605 / 595 -> 591, 1,165 -> 1,086 and 2,289 -> 2,067).
 bool mx_plan(const stwo_hip_ctx *ctx, const stwo_hip_twiddles *tw, uint32_t n, uint32_t b, bool inverse, size_t n_cols,
              bool aligned16, bool batched, MxPlan *plan) {
   if (!tw->d_mx || !aligned16 || n < kMxMinLog || n > kMxMaxLog || b > kMxMaxBlowup || n_cols < 3) return false;
+  if ((n >= 22 && n_cols < 4) || (n >= 24 && n_cols == 5)) return false;
   const uint64_t units = mx_low_units((uint32_t)n_cols, n);
   if (units < (batched ? kMxBatchUnits : kMxMinUnits)) return false;
   // A vector plan chosen for the shape stands in a launch of its own.  It was timed
