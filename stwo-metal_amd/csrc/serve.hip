@@ -309,7 +309,10 @@ int run_commit_group(stwo_hip_server *s, stwo_hip_ctx *ctx, Group &g) {
     uint32_t *tree = (uint32_t *)p;
     p += align256(words_tree(L) * 4);
     int rc = load_columns(ctx, d, d.n_cols, in, range, copies);
-    if (rc) return rc;
+    if (rc) {
+      (void)stwo_hip_sync(ctx);  // the jobs' copies before it: the group's memory goes to another slot
+      return rc;
+    }
     for (uint32_t c = 0; c < d.n_cols; c++) {
       cols[k].push_back(in + ((size_t)c << n));
       outs[k].push_back(out + ((size_t)c << L));
@@ -374,7 +377,10 @@ int run_prove_group(stwo_hip_server *s, stwo_hip_ctx *ctx, Group &g) {
     b = ab + n;
   }
   p += align256(((size_t)2 << d.log_size) * 4);
-  if (rc) return rc;
+  if (rc) {
+    (void)stwo_hip_sync(ctx);
+    return rc;
+  }
   job_mem_begin(ctx, p, g.mem + g.bytes - p);
   uint8_t digest[32] = {0};
   uint32_t n_draws = 0;
@@ -387,7 +393,8 @@ int run_prove_group(stwo_hip_server *s, stwo_hip_ctx *ctx, Group &g) {
     memcpy(j.res.final_digest, digest, 32);
   }
   if (proof) stwo_hip_stark_proof_destroy(proof);
-  if (rc == STWO_HIP_OK) rc = stwo_hip_sync(ctx);
+  const int src = stwo_hip_sync(ctx);  // also after a failure, as above
+  if (rc == STWO_HIP_OK) rc = src;
   job_mem_end(ctx);
   return rc;
 }
