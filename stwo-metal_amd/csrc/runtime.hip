@@ -132,13 +132,10 @@ static int arena_wait_range(stwo_hip_ctx *ctx, size_t b, size_t e) {
   return STWO_HIP_OK;
 }
 
-// Pending uploads of up to 3.5 KB travel as kernel arguments: one launch, where a
+// Pending uploads of a few KB travel as kernel arguments: one launch, where a
 // copy call and the event that guards its host bytes keep the next launch
 // waiting about 4 us longer (a commit of 16 x 2^16 with two uploads: 72.0 -> 63.8
-// us).  The host bytes are free again at once.  Two launches for twice that save a
-// lone call 1.4 us, but calls that follow one another wait 3 to 4 us longer for the
-// host (interpolation of 256 x 2^8: alone 19.5 us, 20.9 with the copy; one of eight
-// 17.8, 14.6 with the copy).
+// us).  The host bytes are free again at once.
 template <uint32_t BYTES>
 struct UploadBytes {
   uint4 v[BYTES / 16];
@@ -160,13 +157,21 @@ constexpr size_t kUploadArgs = 3584;  // below the 4 KB of a launch's arguments
 
 int flush_uploads(stwo_hip_ctx *ctx) {
   if (ctx->pend_end <= ctx->pend_begin) return STWO_HIP_OK;
-  const size_t b = ctx->pend_begin, e = ctx->pend_end, n = e - b;
+  size_t b = ctx->pend_begin;
+  const size_t e = ctx->pend_end;
   ctx->pend_begin = ctx->pend_end = 0;
-  // (tables start and end on 256 bytes)
-  if (n <= 256) return launch_upload<256>(ctx, b, n);
-  if (n <= 1024) return launch_upload<1024>(ctx, b, n);
-  if (n <= kUploadArgs) return launch_upload<kUploadArgs>(ctx, b, n);
-  STWO_HIP_TRY(ctx, hipMemcpyAsync(ctx->d_arena + b, ctx->h_arena + b, n, hipMemcpyHostToDevice, ctx->stream));
+  if (e - b <= 2 * kUploadArgs) {
+    // (tables start and end on 256 bytes)
+    for (; b < e; b += kUploadArgs) {
+      const size_t n = std::min(kUploadArgs, e - b);
+      const int rc = n <= 256    ? launch_upload<256>(ctx, b, n)
+                     : n <= 1024 ? launch_upload<1024>(ctx, b, n)
+                                 : launch_upload<kUploadArgs>(ctx, b, n);
+      if (rc) return rc;
+    }
+    return STWO_HIP_OK;
+  }
+  STWO_HIP_TRY(ctx, hipMemcpyAsync(ctx->d_arena + b, ctx->h_arena + b, e - b, hipMemcpyHostToDevice, ctx->stream));
   hipEvent_t ev = take_event(ctx);
   if (!ev) return set_error(ctx, STWO_HIP_EDEVICE, "hipEventCreate failed");
   STWO_HIP_TRY(ctx, hipEventRecord(ev, ctx->stream));
