@@ -245,14 +245,14 @@ def _flat_samples(samples_per_col):
     """Per column a list of (x[4], y[4], value[4]) as rows of 12 words, and each list's length.
 
     Points repeat from sample to sample, so each run of one object is taken once (264
-    samples at one point 205 -> 66 us; 98 us with a point object each), as long as
+    samples at one point 205 -> 70 us; 102 us with a point object each), as long as
     lists and tuples hold them: whatever else is iterated may fill one object anew
     for every sample."""
     pts, runs, vals, counts, px, py = [], [], [], [], None, None
-    held = type(samples_per_col) in (list, tuple)
+    plain = {list, tuple}
+    keep = type(samples_per_col) in plain and set(map(type, samples_per_col)) <= plain
     for ss in samples_per_col:
         counts.append(len(ss))
-        keep = held and type(ss) in (list, tuple)
         for x, y, v in ss:
             if x is px and y is py:
                 runs[-1] += 1
