@@ -135,7 +135,12 @@ static int arena_wait_range(stwo_hip_ctx *ctx, size_t b, size_t e) {
 // Pending uploads of a few KB travel as kernel arguments: one launch, where a
 // copy call and the event that guards its host bytes keep the next launch
 // waiting about 4 us longer (a commit of 16 x 2^16 with two uploads: 72.0 -> 63.8
-// us).  The host bytes are free again at once.
+// us).  The host bytes are free again at once.  Two launches up to twice their
+// size: a copy amid a call's launches costs the stream about 10 us (samples and
+// quotients of 264 columns 294 us, with a copy above 3.5 KB 304; a served burst 1,086
+// and 1,113).  Short calls that follow one another without a wait are bound by the
+// host there and lose 3 us (interpolation of 256 x 2^8, one of eight: 17.8, with a
+// copy 14.6; alone 19.5 and 20.9).
 template <uint32_t BYTES>
 struct UploadBytes {
   uint4 v[BYTES / 16];
