@@ -15,9 +15,10 @@
 // the wave -> scalar loads).
 //
 // A run of node layers without injected columns, to the next injected layer or
-// the root, is one launch of `merkle_nodes_kernel`: each workgroup hashes a
-// subtree through LDS, writing every layer to global memory, and the last of
-// each group of workgroups to finish hashes on (merkle_dev.hpp).
+// the root, is one launch of `merkle_nodes_kernel` (two where its workgroups would
+// meet on more counters than there are): each workgroup hashes a subtree through
+// LDS, writing every layer to global memory, and the last of each group of
+// workgroups to finish hashes on (merkle_dev.hpp).
 #include <algorithm>
 #include <type_traits>
 #include <vector>
